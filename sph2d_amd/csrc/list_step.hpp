@@ -566,6 +566,204 @@ __global__ void __launch_bounds__(kBlock) pair_list_kernel(StepParams P, Ctrl* _
     }
 }
 
+// W and the gradient factor F (grad W = (r_i - r_j) F) of kernel type skf at
+// |r| = dist, with rinv = 1 / |r| (infinite for coincident particles) and
+// q = |r| / h: the pieces of kernel_w and kernel_gradf (physics.hpp) without
+// their divisions.
+template <class R>
+__device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R dist, R rinv, R q, R& W, R& F) {
+    const R t = R(2) - q, ih = K.inv_h;
+    switch (skf) {
+    case 2:
+        W = K.f_gauss * exp(-q * q);
+        F = R(-2) * ih * ih * W;
+        break;
+    case 3: {
+        const R s = R(0.5) * t, s3 = s * s * s, g = R(2) * q + R(1);
+        W = q > R(2) ? R(0) : K.f_wend * (s3 * s) * g;
+        F = q < R(1.e-6f) || q >= R(2) ? R(0) : R(2) * K.f_wend * ih * rinv * (s3 * s - g * s3);
+        break;
+    }
+    case 4:
+        W = q <= R(2) ? K.f_desb * (t * t * t) : R(0);
+        F = q < R(2) ? K.f_desb * rinv * ih * (R(-3) * t * t) : R(0);
+        break;
+    default:
+        if (q <= R(1)) {
+            W = K.f_cubic * (R(2) / R(3) - q * q + q * q * q * R(0.5));
+            F = K.f_cubic * (ih * ih) * (R(-2) + R(1.5) * q);
+        } else {
+            W = q <= R(2) ? K.f_cubic * (R(1) / R(6) * (t * t * t)) : R(0);
+            F = q <= R(2) ? -K.f_cubic * rinv * ih * (t * t * R(0.5)) : R(0);
+        }
+        break;
+    }
+}
+
+// Pair pass from the lists with every switch of pair_kernel: any smoothing
+// kernel per term, both pressure approximations, artificial pressure,
+// summation, continuity and delta-SPH density.  Same terms and neighbours as
+// pair_kernel on the same FP64 positions.  An entry gathers the neighbour's
+// position, state and pred record; entries in groups of G as in
+// for_each_listed.  Terms whose kernel type is the pressure's share one
+// evaluation, and no term divides: the cell walk over ~55 candidates with a
+// division or more per term took 167 us at 187,530 particles (FP64, Wendland
+// kernels, delta-SPH, artificial pressure), the ~20 entries of a list 53.
+template <class R>
+__global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
+    StepParams P, Ctrl* __restrict__ ctrl, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
+    const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
+    real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots) {
+    if (ctrl->halted) return;
+    if (ctrl->list_overflow) {  // the build of this step ran out of room: run it without lists
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            ctrl->halted = 1;
+            ctrl->status = kStatusListOverflow;
+        }
+        return;
+    }
+    const uint32_t lb = xcd_block(P.blocks_per_xcd);
+    if (lb >= P.nblocks) return;
+    const uint32_t s = lb * kBlock + threadIdx.x;
+    const bool live = s < P.n;
+    const KernelConsts<R> K = kernel_consts<R>(P);
+    const R m = (R)P.mass;
+    R ax = R(0), ay = -(R)P.g, drho = R(0), avx = R(0), avy = R(0), amu = R(0);
+    bool overflow = false;
+    double2 pj = make_double2(0, 0);
+    real4<R> vaj{}, prj{};
+    if (live) {
+        pj = X.pos[s];
+        vaj = X.va[s];
+        prj = rec[s].pr;
+    }
+    const int tj = (int)vaj.w;
+    const uint32_t cnt = live && tj != 0 ? nbc[s] : 0u;
+    if (cnt) {
+        const bool cont = P.density_treatment != 0, delta = P.density_treatment == 2;
+        const R rhohj = fabs(prj.z), pjres = prj.w * (rhohj * rhohj);
+        const R alpha_c = (R)P.av_alpha * (R)P.av_c, beta = (R)P.av_beta, eta2 = (R)P.av_eta2;
+        const R two_eps_m = R(2) * (R)P.xsph_eps * m, lj_r0 = (R)P.lj_r0, lj_D = (R)P.lj_D;
+        const R dhc2m = R(2) * (R)P.dhc * m, ap_iw = P.art_pressure ? (R)(1.0 / P.ap_wdelta) : R(0);
+        const uint32_t cap = P.max_nbr - 1;
+        const uint32_t row = P.n * 4u;
+        constexpr uint32_t G = 2;
+        static_assert(2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
+        uint32_t off = s * 4u, hits = 0;
+        uint32_t e[G];
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) e[u] = list_entry(nbl, off + u * row);
+        off += G * row;
+#pragma unroll 1
+        for (uint32_t k = 0; k < cnt; k += G) {
+            double2 pos[G];
+            real4<R> va[G], pr[G];
+            uint32_t en[G];
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) {
+                const uint32_t i = e[u] & kSlotMask;
+                pos[u] = X.pos[i];
+                va[u] = X.va[i];
+                pr[u] = rec[i].pr;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) en[u] = list_entry(nbl, off + u * row);
+            off += G * row;
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) {
+                const double dxd = __dsub_rn(pos[u].x, pj.x), dyd = __dsub_rn(pos[u].y, pj.y);
+                const int ti = (int)va[u].w;
+                if (!((k + u < cnt) & (ti != 0) & (dist2_exact(dxd, dyd) < P.cut2))) continue;
+                if (hits == cap) {
+                    overflow = true;
+                    continue;
+                }
+                ++hits;
+                const R dx = (R)dxd, dy = (R)dyd;  // r_i - r_j
+                const R d2 = (R)(dxd * dxd + dyd * dyd);
+                const bool apart = d2 > R(0);
+                const R rinv = apart ? fast_rsqrt<R>(d2) : R(INFINITY);
+                const R dist = apart ? d2 * rinv : R(0);
+                const R q = dist * K.inv_h;
+                R W, F;
+                kernel_wf<R>(K, P.skf_intf, dist, rinv, q, W, F);
+                // continuity density with v and rho of the current step
+                if (cont) {
+                    R Wd = W, Fd = F;
+                    if (P.skf_density != P.skf_intf) kernel_wf<R>(K, P.skf_density, dist, rinv, q, Wd, Fd);
+                    const R gx = dx * Fd, gy = dy * Fd;
+                    drho += m * ((va[u].x - vaj.x) * gx + (va[u].y - vaj.y) * gy);
+                    if (delta) {
+                        const R rf = -(dx * gx + dy * gy) * (rinv * rinv);
+                        drho += dhc2m * ((va[u].z - vaj.z) * fast_rcp<R>(va[u].z) * rf);
+                    }
+                }
+                // Lennard-Jones wall force on fluid from boundary particles
+                if (P.lj_on && tj > 0 && ti < 0 && dist < lj_r0) {
+                    const R rn = lj_r0 * rinv;
+                    const R rn2 = rn * rn, rn4 = rn2 * rn2;
+                    const R f = lj_D * (rn4 * rn4 * rn4 - rn4) * (rinv * rinv);
+                    ax -= dx * f;
+                    ay -= dy * f;
+                }
+                // pressure: p / rho^2 of both from the pred records
+                const R rhohi = fabs(pr[u].z);
+                R pf = P.intf_approx == 1 ? (pjres + pr[u].w * (rhohi * rhohi)) * fast_rcp<R>(rhohj * rhohi)
+                                          : pr[u].w + prj.w;
+                if (P.art_pressure && (pr[u].w < R(0) || prj.w < R(0))) {
+                    R Wa = W, Fa = F;
+                    if (P.skf_ap != P.skf_intf) kernel_wf<R>(K, P.skf_ap, dist, rinv, q, Wa, Fa);
+                    const R api = pr[u].w < R(0) ? -(R)P.ap_coef * pr[u].w : R(0);
+                    const R apj = prj.w < R(0) ? -(R)P.ap_coef * prj.w : R(0);
+                    pf += (api + apj) * pow(Wa * ap_iw, (R)P.ap_index);
+                }
+                R cx = F * pf * m;
+                // artificial viscosity and XSPH with the predicted velocity and density
+                const R dvx = pr[u].x - prj.x, dvy = pr[u].y - prj.y;
+                const R inv_rs = fast_rcp<R>(rhohi + rhohj);
+                if (P.av_on) {
+                    const R vr = dvx * dx + dvy * dy;  // (v_j - v_i) . (r_j - r_i)
+                    if (vr < R(0)) {
+                        const R mu = K.h * vr * fast_rcp<R>(d2 + eta2);
+                        amu = fmax(amu, fabs(mu));
+                        R Wv = W, Fv = F;
+                        if (P.skf_av != P.skf_intf) kernel_wf<R>(K, P.skf_av, dist, rinv, q, Wv, Fv);
+                        cx += Fv * ((beta * mu - alpha_c) * mu * R(2) * inv_rs) * m;
+                    }
+                }
+                ax += dx * cx;
+                ay += dy * cx;
+                if (P.xsph_on && ti > 0) {
+                    R Wx = W, Fx = F;
+                    if (P.skf_xsph != P.skf_intf) kernel_wf<R>(K, P.skf_xsph, dist, rinv, q, Wx, Fx);
+                    const R c = two_eps_m * inv_rs * Wx;
+                    avx += dvx * c;
+                    avy += dvy * c;
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
+        }
+    }
+    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (P.dt_method == 2 && P.dt_dynamic_mode == 1)
+        block_max2_to_slots(live ? sqrt((double)ax * ax + (double)ay * ay) : 0.0, live ? (double)amu : 0.0, maxslots,
+                            lb);
+    if (live) {
+        real4<R> d;
+        d.x = ax;
+        d.y = ay;
+        d.z = drho;
+        d.w = amu;
+        der[s] = d;
+        real2<R> x;
+        x.x = avx;
+        x.y = avy;
+        xs[s] = x;
+        if (P.density_treatment != 0) pres[s] = eos_p<R>(vaj.z, (R)P.rho0, (R)P.eos_B);
+    }
+}
+
 // whole_step of every slot from X into A (in place on list steps), the cell
 // key for the next build, the step's largest displacement, and the records
 // of the next step's pair pass: near (the new position relative to the home
