@@ -38,10 +38,10 @@ class DifferentiableRun:
         self.sim.set_piston(self.omega, a, b)
         return self.sim.adjoint_forward(self.nsteps, self.every, self.spec)
 
-    def backward(self, eta_bar: np.ndarray, ncoef: int) -> dict:
+    def backward(self, eta_bar: np.ndarray, ncoef: int, state: bool = True) -> dict:
         """Gradients for eta_bar = dL/d eta: the ncoef coefficients of a and
-        of b (every paddle's, paddle-major) and the initial state."""
-        return self.sim.adjoint_backward(eta_bar, ncoef)
+        of b (every paddle's, paddle-major) and, with state, the initial state."""
+        return self.sim.adjoint_backward(eta_bar, ncoef, state)
 
 
 def _torch():
@@ -79,7 +79,8 @@ class PistonGauges:
                     # call's tape since: record this call's trajectory again
                     if ctx.run.sim.tape_generation != ctx.tape:
                         ctx.run.forward(*ctx.coefs)
-                    g = ctx.run.backward(eta_bar.detach().double().cpu().numpy(), ctx.ncoef)
+                    # only the coefficients' gradients leave the device
+                    g = ctx.run.backward(eta_bar.detach().double().cpu().numpy(), ctx.ncoef, state=False)
                     ga = torch.from_numpy(g["a"]).to(dtype=ctx.dtype, device=ctx.device)
                     gb = torch.from_numpy(g["b"]).to(dtype=ctx.dtype, device=ctx.device)
                     return ga, gb, None

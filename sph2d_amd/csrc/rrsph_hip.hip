@@ -2405,8 +2405,18 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
     std::vector<double> ps((size_t)N * kMaxSegments);
     HIP_TRY(hipMemcpyAsync(ps.data(), T.piston_sum, ps.size() * sizeof(double), hipMemcpyDeviceToHost,
                            ctx->stream));
-    std::vector<double> lam(lw * n);
-    HIP_TRY(hipMemcpyAsync(lam.data(), T.lam[cur], lam.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if (grad_r0 || grad_v0 || grad_rho0) {
+        const size_t D = d3 ? 3 : 2;
+        unpack_gradients_kernel<<<nb, kBlock, 0, ctx->stream>>>(P.n, T.lam[cur], lw, (uint32_t)D, ctx->st_r,
+                                                                ctx->st_v, ctx->st_rho);
+        HIP_TRY(hipGetLastError());
+        if (grad_r0)
+            HIP_TRY(hipMemcpyAsync(grad_r0, ctx->st_r, D * n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        if (grad_v0)
+            HIP_TRY(hipMemcpyAsync(grad_v0, ctx->st_v, D * n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        if (grad_rho0)
+            HIP_TRY(hipMemcpyAsync(grad_rho0, ctx->st_rho, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    }
     uint32_t flag = 0;
     HIP_TRY(hipMemcpyAsync(&flag, T.flag, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -2423,15 +2433,6 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
             if (grad_a) grad_a[g * nh + k] = ga;
             if (grad_b) grad_b[g * nh + k] = gb;
         }
-    }
-    const uint32_t D = d3 ? 3 : 2;
-    const uint32_t vo = d3 ? 3 : 2, ro = d3 ? 6 : 4;  // offsets of v and rho in lam
-    for (size_t i = 0; i < n; ++i) {
-        for (uint32_t c = 0; c < D; ++c) {
-            if (grad_r0) grad_r0[D * i + c] = lam[lw * i + c];
-            if (grad_v0) grad_v0[D * i + c] = lam[lw * i + vo + c];
-        }
-        if (grad_rho0) grad_rho0[i] = lam[lw * i + ro];
     }
     // leave the context as the forward left it (restore_state makes the next
     // step sort, and build when it runs list steps)

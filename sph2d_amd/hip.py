@@ -363,13 +363,16 @@ class HipStep:
                                                      _dp(eta)))
         return eta
 
-    def adjoint_backward(self, eta_bar: np.ndarray, ncoef: int) -> Dict[str, np.ndarray]:
+    def adjoint_backward(self, eta_bar: np.ndarray, ncoef: int, state: bool = True) -> Dict[str, np.ndarray]:
         """Gradients of the loss whose derivative with respect to the gauges
         is eta_bar: the ncoef piston coefficients of a and of b (every
-        paddle's, paddle-major) and the initial state."""
+        paddle's, paddle-major) and, with state, the initial state."""
         eta_bar = np.ascontiguousarray(eta_bar, dtype=np.float64)
         ga, gb = np.zeros(MAX_HARMONICS), np.zeros(MAX_HARMONICS)
         d = self.dim
+        if not state:
+            self._check(self.L.rrsph_hip_adjoint_backward(self.ctx, _dp(eta_bar), _dp(ga), _dp(gb), None, None, None))
+            return {"a": ga[:ncoef], "b": gb[:ncoef]}
         gr, gv, grho = np.zeros((self.n, d)), np.zeros((self.n, d)), np.zeros(self.n)
         self._check(self.L.rrsph_hip_adjoint_backward(self.ctx, _dp(eta_bar), _dp(ga), _dp(gb), _dp(gr), _dp(gv),
                                                       _dp(grho)))
