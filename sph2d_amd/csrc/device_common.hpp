@@ -50,9 +50,7 @@ struct Ctrl {
     // reductions of the step in flight
     unsigned long long amax_bits;   // max |a| (non-negative double bits)
     unsigned long long mumax_bits;  // max |mu|
-    uint32_t outside;       // particles outside the geometry after whole_step
-    uint32_t nbr_overflow;  // a particle had more than max_neighbours - 1 neighbours
-    uint32_t grid_overflow; // a live particle lay outside the cell grid
+    uint32_t outside;       // particles outside the geometry after whole_step (sorted steps)
     uint32_t resort_count;  // slots that changed cell key since the last sort
     // snapshot of the step in flight (written by the prologue)
     double cur_time;
@@ -68,11 +66,20 @@ struct Ctrl {
     // neighbour-list steps
     double disp_acc;        // sum over the steps since the last list build of each step's largest displacement
     double disp_last;       // the largest displacement of the last committed list or build step
-    uint32_t list_overflow; // the last build found more candidates for some particle than its list holds
     uint32_t list_valid;    // the lists describe the current slot order (a build ran; no sort since)
     uint32_t cur_renorm;    // this step's summation density is renormalised
-    uint32_t renorm_pad;
+    // flags that blocks of a step raise on the control block between steps;
+    // the integrator of a list step, which publishes the words before them
+    // (publish_ctrl), leaves them alone
+    uint32_t nbr_overflow;  // a particle had more than max_neighbours - 1 neighbours
+    uint32_t grid_overflow; // a live particle lay outside the cell grid
+    uint32_t outside_l[2];  // list steps: as outside, by the parity of the step index
+    uint32_t list_overflow; // the last build found more candidates for some particle than its list holds
+    uint32_t flags_pad;
 };
+
+// Particles outside the geometry after the step awaiting its commit.
+__host__ __device__ inline uint32_t ctrl_outside(const Ctrl& c) { return c.outside + c.outside_l[c.step & 1]; }
 
 constexpr int kMaxSegments = 8;  // paddles of a segmented piston
 

@@ -33,9 +33,9 @@
 // from its home cell), where it takes the FP64 positions and the reference's
 // test; the rounding of xi stays far below that band (2e-6 of the cut-off).
 //
-// Step kernels: list_prologue -> [density_sum_list] -> pair_list ->
-// integrate_list (in place; it also writes the next step's records, so no
-// reorder runs between builds).  A build step runs list_prologue -> radix
+// Step kernels: [density_sum_list] -> pair_list -> integrate_list (in place;
+// it also writes the next step's records, so no reorder runs between builds),
+// the first of them with the step's prologue (list_step_begin).  A build step runs list_prologue -> radix
 // sort -> reorder_list_kernel -> list_build_kernel -> the same step kernels
 // on the reordered copy, integrating into A.
 #pragma once
@@ -140,49 +140,160 @@ __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, cons
     fill_cell_starts(P, s, live, k, skey, LB);
 }
 
-// Prologue of a list step or a build step (one block of kBlock threads):
-// the previous step's largest displacement (reduced from its slots), the
-// commit of the previous step, the staleness test of the lists (a list
-// step also halts when no build has run since the last sort, e.g. a build
-// launched while the run was stopped), and the clearing of this step's
-// reduction slots.
-__global__ void __launch_bounds__(kBlock) list_prologue(StepParams P, Ctrl* __restrict__ ctrl,
-                                                        unsigned long long* __restrict__ dslots,
-                                                        unsigned long long* __restrict__ maxslots, uint32_t build) {
+// ------------------------------------------------------------------ control of list steps
+// A list step has no prologue launch: between steps the control block
+// `next` holds the last step's outcome; the step's first kernel (pair or
+// summation pass) reads only `next` and the displacement slots, every block
+// deciding by itself whether the step runs (list_step_halts), and its block 0
+// writes the commit and this step's snapshot to a second block `cur`; the
+// later kernels of the step read `cur`, and the integrator's block 0 publishes
+// `cur` with the step's outcome in `next`.  So no kernel writes what its
+// other blocks read.  A prologue launch of one block took 4.8 us and 1.2 us
+// of launch gap at the head of every step (97 us at 1M particles FP32, 42 at
+// 188k, 22 at 7k); build steps keep one (list_prologue), since their sort
+// needs the decision.
+//
+// What several blocks of a step raise lies outside the published words: the
+// flags at the end of Ctrl, and slots by the parity of the step index -
+// displacement slots dslots (a set per parity: the integrator of step k fills
+// set k, the first kernel of step k + 1 reads it and clears the other) and
+// dt reduction slots maxslots (the pair pass of step k fills set k, its
+// integrator reads it and clears the other).
+constexpr uint32_t kMaxSlotSet = 4 * kMaxSlots;  // offset between the two sets of dt reduction slots
+constexpr uint32_t kCtrlFlagWord = offsetof(Ctrl, nbr_overflow) / 8;
+static_assert(offsetof(Ctrl, nbr_overflow) % 8 == 0 && offsetof(Ctrl, dt_new) % 8 == 0 &&
+                  offsetof(Ctrl, pending) % 8 == 0 && offsetof(Ctrl, halted) == offsetof(Ctrl, pending) + 4 &&
+                  offsetof(Ctrl, status) % 8 == 0,
+              "publish_ctrl's words");
+
+// The largest displacement of the step that `next` holds (block-wide).
+__device__ __forceinline__ double list_dmax(const Ctrl* next, const unsigned long long* __restrict__ dslots) {
     __shared__ double s_m[kBlock / kWave];
-    const unsigned long long word = ctrl_word(ctrl);
-    double d = dbits(dslots[threadIdx.x]);
+    double d = dbits(dslots[(uint32_t)(next->step & 1) * kMaxSlots + threadIdx.x]);
     for (int off = 32; off > 0; off >>= 1) d = fmax(d, __shfl_xor(d, off));
     if (__lane_id() == 0) s_m[threadIdx.x / kWave] = d;
     __syncthreads();
+    double dmax = s_m[0];
+    for (int w = 1; w < kBlock / kWave; ++w) dmax = fmax(dmax, s_m[w]);
+    return dmax;
+}
+
+// The prologue of a list step (build: of a build step) in one block: the
+// commit of the step that `next` holds, the staleness test of the lists (a
+// list step also halts when no build has run since the last sort, e.g. a
+// build launched while the run was stopped), the snapshot into `cur`.
+__device__ __forceinline__ void list_block_prologue(const StepParams& P, const Ctrl* next, Ctrl* cur, double dmax,
+                                                    bool build) {
+    const unsigned long long word = ctrl_word(next);
     uint32_t valid = 0;
     block_prologue(
-        P, ctrl, word,
+        P, cur, word,
         [&](Ctrl& c) {
-            double dmax = s_m[0];
-            for (int w = 1; w < kBlock / kWave; ++w) dmax = fmax(dmax, s_m[w]);
             if (!c.halted && c.pending) {  // the step being committed moved no particle further than dmax
                 c.disp_acc += dmax;
                 c.disp_last = dmax;
             }
             valid = c.list_valid;
+            // a list step whose predecessor overflowed does not get here (its
+            // integrator halted); other blocks of this kernel may be raising
+            // the flag for this step already
+            if (!build) c.nbr_overflow = 0;
         },
         [&](Ctrl& c) {
             if (c.halted) return;
             c.list_valid = build ? 1u : valid;
             if (build) {
                 c.disp_acc = 0.0;
-                c.list_overflow = 0;
             } else if (!valid || !(c.disp_acc < P.skin_half)) {
                 c.halted = 1;
                 c.status = kStatusRebuild;
                 if (c.wall_disappear) c.nwm_done = 0;  // the re-run prologue fires it again
             }
         });
-    maxslots[threadIdx.x] = 0;
-    maxslots[kMaxSlots + threadIdx.x] = 0;
-    dslots[threadIdx.x] = 0;
-    dslots[kMaxSlots + threadIdx.x] = 0;
+}
+
+// Whether list_block_prologue (not a build) halts, from the same fields
+// (none of which the blocks of this kernel write).
+__device__ __forceinline__ bool list_step_halts(const StepParams& P, const Ctrl& N, double dmax) {
+    if (N.halted) return true;
+    double t = N.time, disp = N.disp_acc;
+    if (N.pending) {
+        if (P.consistency_check && ctrl_outside(N) > 0 && P.consistency_treatment == 1) return true;
+        t += N.dt_new;
+        disp += dmax;
+    }
+    return t > N.t_end || !N.list_valid || !(disp < P.skin_half);
+}
+
+// At the head of a list step's first kernel (every thread of the block):
+// false when the step halts, else its step index in `step`.
+__device__ __forceinline__ bool list_step_begin(const StepParams& P, Ctrl* next, Ctrl* cur,
+                                                unsigned long long* __restrict__ dslots, unsigned long long& step) {
+    const double dmax = list_dmax(next, dslots);
+    step = next->step + (next->pending ? 1 : 0);
+    const bool halts = list_step_halts(P, *next, dmax);
+    if (blockIdx.x == 0) {
+        list_block_prologue(P, next, cur, dmax, false);
+        if (!halts) {  // this step's set; the blocks of this kernel read the other one
+            dslots[(uint32_t)(step & 1) * kMaxSlots + threadIdx.x] = 0;
+            if (threadIdx.x == 0) next->outside_l[step & 1] = 0;
+        }
+    }
+    return !halts;
+}
+
+// The prologue of a build step (one block of kBlock threads): it also
+// clears every reduction slot and the flags of the build.
+__global__ void __launch_bounds__(kBlock) list_prologue(StepParams P, Ctrl* __restrict__ next, Ctrl* __restrict__ cur,
+                                                        unsigned long long* __restrict__ dslots,
+                                                        unsigned long long* __restrict__ maxslots) {
+    const double dmax = list_dmax(next, dslots);
+    list_block_prologue(P, next, cur, dmax, true);
+    if (cur->halted) return;
+    for (uint32_t k = 0; k < 2; ++k) {
+        dslots[k * kMaxSlots + threadIdx.x] = 0;
+        maxslots[k * kMaxSlotSet + threadIdx.x] = 0;
+        maxslots[k * kMaxSlotSet + kMaxSlots + threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) {
+        next->outside_l[0] = next->outside_l[1] = 0;
+        next->list_overflow = 0;
+    }
+}
+
+// At the head of a later kernel of a list or build step: false when the
+// step halted.
+__device__ __forceinline__ bool list_step_goes(const Ctrl* cur) { return !cur->halted; }
+
+// A build that found more entries for some particle than its list holds:
+// the step halts before its pair pass and runs without lists.
+__device__ __forceinline__ bool list_build_overflowed(const Ctrl* next, Ctrl* cur) {
+    if (!next->list_overflow) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        cur->halted = 1;
+        cur->status = kStatusListOverflow;
+    }
+    return true;
+}
+
+// The summation density of step `step` is renormalised (as prologue_commit
+// decides it).
+__device__ __forceinline__ bool step_renorm(const StepParams& P, unsigned long long step) {
+    return P.renorm && (step + 1) % P.renorm_every == 0;
+}
+
+// The integrator's block 0: `next` becomes `cur` with the step's outcome
+// (dt: committed by the next step's prologue), or with the halt `status`.
+__device__ __forceinline__ void publish_ctrl(const Ctrl* cur, Ctrl* next, double dt, uint32_t halt_status) {
+    if (threadIdx.x >= kCtrlFlagWord) return;
+    unsigned long long w = reinterpret_cast<const unsigned long long*>(cur)[threadIdx.x];
+    if (!cur->halted) {
+        if (threadIdx.x == offsetof(Ctrl, dt_new) / 8 && halt_status == 0)
+            w = (unsigned long long)__double_as_longlong(dt);
+        if (threadIdx.x == offsetof(Ctrl, pending) / 8) w = halt_status ? (1ull << 32) : 1ull;  // pending | halted << 32
+        if (threadIdx.x == offsetof(Ctrl, status) / 8 && halt_status) w = (w & ~0xffffffffull) | halt_status;
+    }
+    reinterpret_cast<unsigned long long*>(next)[threadIdx.x] = w;
 }
 
 // Cell index (clamped to the grid) of coordinate r.
@@ -197,13 +308,14 @@ __device__ __forceinline__ int clamped_cell(double r, double rmin, double cell, 
 // within a column).  The cells visited are those within list_reach of the
 // particle (3 or 4 per axis, the reach being under two cells).
 template <class R>
-__global__ void __launch_bounds__(kBlock) list_build_kernel(StepParams P, Ctrl* __restrict__ ctrl,
+__global__ void __launch_bounds__(kBlock) list_build_kernel(StepParams P, Ctrl* __restrict__ next,
+                                                            const Ctrl* __restrict__ cur,
                                                             const double2* __restrict__ pos,
                                                             const real4<R>* __restrict__ va,
                                                             const uint32_t* __restrict__ skey,
                                                             const uint32_t* __restrict__ LB, uint32_t* __restrict__ nbl,
                                                             uint32_t* __restrict__ nbc) {
-    if (ctrl->halted) return;
+    if (cur->halted) return;
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     const uint32_t s = lb * kBlock + threadIdx.x;
@@ -252,7 +364,7 @@ __global__ void __launch_bounds__(kBlock) list_build_kernel(StepParams P, Ctrl* 
             }
         }
     }
-    if (cnt > P.list_cap || bad) atomicOr(&ctrl->list_overflow, 1u);
+    if (cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
     nbc[s] = min(cnt, P.list_cap);
 }
 
@@ -440,17 +552,24 @@ __device__ __forceinline__ void list_pair_term(const FastPair<R>& K, PairSums<R>
 // (ModelParams.tex:124-133, rho_i the density before the step).  Cubic
 // spline.  Aliveness and the old densities come from va (pred is being
 // rewritten by this pass).
-template <class R>
-__global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* __restrict__ ctrl, ListState<R> X,
+template <class R, bool FIRST>
+__global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X,
                                                            ListRec<R>* __restrict__ rec, R* __restrict__ pres,
                                                            const uint32_t* __restrict__ nbl,
-                                                           const uint32_t* __restrict__ nbc) {
-    if (ctrl->halted) return;
+                                                           const uint32_t* __restrict__ nbc,
+                                                           unsigned long long* __restrict__ dslots) {
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     __shared__ float2 s_off[64];
     fill_cell_offsets(P, s_off);
-    __syncthreads();
+    unsigned long long step;
+    if constexpr (FIRST) {
+        if (!list_step_begin(P, next, cur, dslots, step)) return;
+    } else {
+        if (!list_step_goes(cur)) return;
+        step = cur->step;
+        __syncthreads();
+    }
     const uint32_t s = lb * kBlock + threadIdx.x;
     if (s >= P.n) return;
     const KernelConsts<R> K = kernel_consts<R>(P);
@@ -458,7 +577,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* _
     const real4<R> vaj = X.va[s];
     const R w0 = kernel_w<R>(K, P.skf_density, R(0));
     R rho = m * w0;
-    const bool renorm = ctrl->cur_renorm != 0;
+    const bool renorm = step_renorm(P, step);
     R wsum = renorm ? m / vaj.z * w0 : R(0);
     bool overflow = false;
     const uint32_t cnt = (int)vaj.w != 0 ? nbc[s] : 0u;
@@ -486,7 +605,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* _
         }
     }
     if (renorm) rho = rho / wsum;
-    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     real4<R> pr = rec[s].pr;
     const R p = eos_p<R>(rho, (R)P.rho0, (R)P.eos_B);
     pr.z = typed_rho<R>(rho, (int)vaj.w);
@@ -500,26 +619,25 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* _
 // pair_fast_kernel), the dt maxima, and the fields for the integrator.  With
 // continuity it also writes the pressure of the current density (the
 // reference's p array).
-template <class R>
-__global__ void __launch_bounds__(kBlock) pair_list_kernel(StepParams P, Ctrl* __restrict__ ctrl, ListState<R> X,
-                                                           const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
-                                                           const uint32_t* __restrict__ nbl,
-                                                           const uint32_t* __restrict__ nbc,
-                                                           real4<R>* __restrict__ der, real2<R>* __restrict__ xs,
-                                                           unsigned long long* __restrict__ maxslots) {
-    if (ctrl->halted) return;
-    if (ctrl->list_overflow) {  // the build of this step ran out of room: run it without lists
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctrl->halted = 1;
-            ctrl->status = kStatusListOverflow;
-        }
-        return;
-    }
+template <class R, bool FIRST>
+__global__ void __launch_bounds__(kBlock) pair_list_kernel(
+    StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
+    const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
+    real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     __shared__ float2 s_off[64];
     fill_cell_offsets(P, s_off);
-    __syncthreads();
+    unsigned long long step;
+    if constexpr (FIRST) {
+        if (!list_step_begin(P, next, cur, dslots, step)) return;
+    } else {
+        if (!list_step_goes(cur)) return;
+        if (list_build_overflowed(next, cur)) return;
+        step = cur->step;
+        __syncthreads();
+    }
+    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
     const uint32_t s = lb * kBlock + threadIdx.x;
     const bool live = s < P.n;
     const FastPair<R> K(P);
@@ -542,7 +660,7 @@ __global__ void __launch_bounds__(kBlock) pair_list_kernel(StepParams P, Ctrl* _
         else
             for_each_listed<R, false>(P, s_off, cap, s, nj, pj, X.pos, rec, nbl, cnt, overflow, term);
     }
-    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const R m = (R)P.mass;
     const R ax = S.ljx + m * S.sx;
     const R ay = -(R)P.g + S.ljy + m * S.sy;
@@ -609,21 +727,22 @@ __device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R d
 // evaluation, and no term divides: the cell walk over ~55 candidates with a
 // division or more per term took 167 us at 187,530 particles (FP64, Wendland
 // kernels, delta-SPH, artificial pressure), the ~20 entries of a list 53.
-template <class R>
+template <class R, bool FIRST>
 __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
-    StepParams P, Ctrl* __restrict__ ctrl, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
+    StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
-    real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots) {
-    if (ctrl->halted) return;
-    if (ctrl->list_overflow) {  // the build of this step ran out of room: run it without lists
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctrl->halted = 1;
-            ctrl->status = kStatusListOverflow;
-        }
-        return;
-    }
+    real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
+    unsigned long long step;
+    if constexpr (FIRST) {
+        if (!list_step_begin(P, next, cur, dslots, step)) return;
+    } else {
+        if (!list_step_goes(cur)) return;
+        if (list_build_overflowed(next, cur)) return;
+        step = cur->step;
+    }
+    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
     const uint32_t s = lb * kBlock + threadIdx.x;
     const bool live = s < P.n;
     const KernelConsts<R> K = kernel_consts<R>(P);
@@ -745,7 +864,7 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
             for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
         }
     }
-    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     if (P.dt_method == 2 && P.dt_dynamic_mode == 1)
         block_max2_to_slots(live ? sqrt((double)ax * ax + (double)ay * ay) : 0.0, live ? (double)amu : 0.0, maxslots,
                             lb);
@@ -764,39 +883,53 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
     }
 }
 
+// At the head of a list step's integrator (every thread): the step's dt;
+// block 0 publishes the control block and clears the next step's dt slots.
+// False when the step halted or halts here (dt below the reference's
+// never-ending bound, more neighbours than max_neighbours - 1).
+__device__ __forceinline__ bool list_dt(const StepParams& P, Ctrl* next, const Ctrl* cur,
+                                        unsigned long long* __restrict__ maxslots, double& dt) {
+    uint32_t halt_status = 0;
+    const bool halted = cur->halted != 0;
+    if (!halted) {
+        const uint32_t par = (uint32_t)(cur->step & 1);
+        if (P.dt_method == 2 && P.dt_dynamic_mode == 1) {
+            double amax, mumax;
+            slots_max2(maxslots + par * kMaxSlotSet, amax, mumax);
+            dt = P.cfl * fmin(sqrt(P.h / amax), P.h / (P.c0 + mumax));
+        } else {
+            dt = cur->cur_dt_const;
+        }
+        const bool never = P.dt_method == 2 && dt <= P.never_ending;
+        const bool nbr_err = P.consistency_check && next->nbr_overflow;
+        halt_status = nbr_err ? 3u : (never ? 4u : 0u);
+        if (blockIdx.x == 0) {
+            maxslots[(par ^ 1) * kMaxSlotSet + threadIdx.x] = 0;
+            maxslots[(par ^ 1) * kMaxSlotSet + kMaxSlots + threadIdx.x] = 0;
+        }
+    }
+    if (blockIdx.x == 0) publish_ctrl(cur, next, dt, halt_status);
+    return !halted && halt_status == 0;
+}
+
 // whole_step of every slot from X into A (in place on list steps), the cell
 // key for the next build, the step's largest displacement, and the records
 // of the next step's pair pass: near (the new position relative to the home
 // cell, the new velocity) and pred (PredictHalfStep.cpp:16-22 with this
 // step's dt, which is the next step's).
 template <class R>
-__global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ctrl* __restrict__ ctrl, ListState<R> X,
+__global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ctrl* __restrict__ next,
+                                                                const Ctrl* __restrict__ cur, ListState<R> X,
                                                                 const real4<R>* __restrict__ der,
                                                                 const real2<R>* __restrict__ xs,
                                                                 ListRec<R>* __restrict__ rec,
                                                                 const uint32_t* __restrict__ home, StateA<R> A,
                                                                 uint32_t* __restrict__ key_next,
-                                                                const unsigned long long* __restrict__ maxslots,
+                                                                unsigned long long* __restrict__ maxslots,
                                                                 unsigned long long* __restrict__ dslots) {
-    Ctrl& c = *ctrl;
-    if (c.halted) return;
+    const Ctrl& c = *cur;
     double dt;
-    if (P.dt_method == 2 && P.dt_dynamic_mode == 1) {
-        double amax, mumax;
-        slots_max2(maxslots, amax, mumax);
-        dt = P.cfl * fmin(sqrt(P.h / amax), P.h / (P.c0 + mumax));
-    } else {
-        dt = c.cur_dt_const;
-    }
-    const bool never = P.dt_method == 2 && dt <= P.never_ending;
-    const bool nbr_err = P.consistency_check && c.nbr_overflow;
-    if (never || nbr_err) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            c.halted = 1;
-            c.status = nbr_err ? 3u : 4u;
-        }
-        return;
-    }
+    if (!list_dt(P, next, cur, maxslots, dt)) return;
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
     uint32_t outside = 0, bad = 0;
     double moved = 0.0;
@@ -830,13 +963,10 @@ __global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ct
         r.nr = near_record<R>(P, o.pos, o.va.x, o.va.y, home[s]);
         rec[s] = r;
     }
-    wave_count_add(&c.outside, outside);
-    if (bad) atomicOr(&c.grid_overflow, 1u);
-    block_max2_to_slots(moved, 0.0, dslots, blockIdx.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        c.dt_new = dt;
-        c.pending = 1;
-    }
+    const uint32_t par = (uint32_t)(c.step & 1);
+    wave_count_add(&next->outside_l[par], outside);
+    if (bad) atomicOr(&next->grid_overflow, 1u);
+    block_max2_to_slots(moved, 0.0, dslots + par * kMaxSlots, blockIdx.x);
 }
 
 }  // namespace rrsph

@@ -17,10 +17,11 @@
 // offsets from a table in LDS, and the FP64 positions and the reference's
 // test (GridFind.cpp:144-176, dist2_exact3) within 1e-5 of the cut-off.
 //
-// Step kernels: list_prologue -> [density_sum_list3] -> pair_list3_kernel
-// -> integrate_list3_kernel (in place).  A build step runs list_prologue ->
-// radix sort -> reorder_list3_kernel -> list_build3_kernel -> the same step
-// kernels on the reordered copy, integrating into A.
+// Step kernels: [density_sum_list3] -> pair_list3_kernel ->
+// integrate_list3_kernel (in place), the first of them with the step's
+// prologue (list_step_begin).  A build step runs list_prologue -> radix sort
+// -> reorder_list3_kernel -> list_build3_kernel -> the same step kernels on
+// the reordered copy, integrating into A.
 #pragma once
 
 #include "list_step.hpp"
@@ -144,14 +145,15 @@ __device__ __forceinline__ int wave_max_i32(int v) {
     return v;
 }
 constexpr uint32_t kBuildL3 = 8;  // candidates in flight per lane (6.6M dam break: 4.06 ms per build, 4.22 at 4)
-__global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl* __restrict__ ctrl,
+__global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl* __restrict__ next,
+                                                             const Ctrl* __restrict__ cur,
                                                              const double4* __restrict__ pos,
                                                              const float4* __restrict__ cand,
                                                              const uint32_t* __restrict__ skey,
                                                              const uint32_t* __restrict__ LB,
                                                              uint32_t* __restrict__ nbl, uint32_t* __restrict__ nbc) {
     __shared__ uint32_t buf[kBuildChunk * kBlock];
-    if (ctrl->halted) return;
+    if (cur->halted) return;
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     const uint32_t s0 = lb * kBlock + threadIdx.x;
@@ -253,7 +255,7 @@ __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl*
     }
     flush();
     if (!inb) return;
-    if (cnt > P.list_cap || bad) atomicOr(&ctrl->list_overflow, 1u);
+    if (cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
     nbc[s] = min(cnt, P.list_cap);
 }
 
@@ -391,25 +393,32 @@ __device__ __forceinline__ void collect_near3(const StepParams& P, bool active, 
 // Summation density from the lists (Density.h:25-61) with the
 // renormalisation of the steps that ask for it (ModelParams.tex:124-133):
 // rho into rec.pr.w (sign-typed), p / rho^2 into rec.nr.w, p into pres.
-template <class R>
-__global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* __restrict__ ctrl, ListState3<R> X,
+template <class R, bool FIRST>
+__global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* next, Ctrl* cur, ListState3<R> X,
                                                             const real4<R>* __restrict__ dens,
                                                             ListRec<R>* __restrict__ rec, R* __restrict__ pres,
                                                             const uint32_t* __restrict__ nbl,
-                                                            const uint32_t* __restrict__ nbc) {
-    if (ctrl->halted) return;
+                                                            const uint32_t* __restrict__ nbc,
+                                                            unsigned long long* __restrict__ dslots) {
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     __shared__ float4 s_off[kCodes3];
     fill_cell_offsets3(P, s_off);
-    __syncthreads();
+    unsigned long long step;
+    if constexpr (FIRST) {
+        if (!list_step_begin(P, next, cur, dslots, step)) return;
+    } else {
+        if (!list_step_goes(cur)) return;
+        step = cur->step;
+        __syncthreads();
+    }
     const uint32_t s = lb * kBlock + threadIdx.x;
     if (s >= P.n) return;
     const R m = (R)P.mass, inv_h = (R)(1.0 / P.h), w_q1 = (R)P.f_cubic, w_q2 = (R)(P.f_cubic / 6.0);
     const real4<R> dj = dens[s];
     const R w0 = w_q1 * (R(2) / R(3));
     R rho = m * w0;
-    const bool renorm = ctrl->cur_renorm != 0;
+    const bool renorm = step_renorm(P, step);
     R wsum = renorm && dj.w != R(0) ? m / fabs(dj.w) * w0 : R(0);
     bool overflow = false;
     const uint32_t cnt = dj.w != R(0) ? nbc[s] : 0u;
@@ -469,7 +478,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     // record's density is 0): it keeps the plain sum, so that its records,
     // which the lists of its former neighbours still name, stay finite
     if (renorm && wsum > R(0)) rho = rho / wsum;
-    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const int itype = (int)X.pos[s].w;
     const R p = eos_p<R>(rho, (R)P.rho0, (R)P.eos_B);
     ListRec<R> r = rec[s];
@@ -536,26 +545,25 @@ __device__ __forceinline__ void list_pair_term3(const FastPair<R>& K, R (&S)[12]
 // (continuity, pressure, artificial viscosity, Lennard-Jones walls, XSPH),
 // the dt maxima and the fields for the integrator.  Entries in groups of
 // G, as for_each_listed.
-template <class R>
-__global__ void __launch_bounds__(kBlock) pair_list3_kernel(StepParams P, Ctrl* __restrict__ ctrl, ListState3<R> X,
-                                                            const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
-                                                            const uint32_t* __restrict__ nbl,
-                                                            const uint32_t* __restrict__ nbc,
-                                                            real4<R>* __restrict__ der, real4<R>* __restrict__ xs,
-                                                            unsigned long long* __restrict__ maxslots) {
-    if (ctrl->halted) return;
-    if (ctrl->list_overflow) {  // the build of this step ran out of room: run it without lists
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctrl->halted = 1;
-            ctrl->status = kStatusListOverflow;
-        }
-        return;
-    }
+template <class R, bool FIRST>
+__global__ void __launch_bounds__(kBlock) pair_list3_kernel(
+    StepParams P, Ctrl* next, Ctrl* cur, ListState3<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
+    const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
+    real4<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     __shared__ float4 s_off[kCodes3];
     fill_cell_offsets3(P, s_off);
-    __syncthreads();
+    unsigned long long step;
+    if constexpr (FIRST) {
+        if (!list_step_begin(P, next, cur, dslots, step)) return;
+    } else {
+        if (!list_step_goes(cur)) return;
+        if (list_build_overflowed(next, cur)) return;
+        step = cur->step;
+        __syncthreads();
+    }
+    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
     const uint32_t s = lb * kBlock + threadIdx.x;
     const bool live = s < P.n;
     const FastPair<R> K(P);
@@ -617,7 +625,7 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(StepParams P, Ctrl* 
         }
         overflow |= over;
     }
-    if (overflow) atomicOr(&ctrl->nbr_overflow, 1u);
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const R m = (R)P.mass;
     const R ax = S[8] + m * S[0];
     const R ay = -(R)P.g + S[9] + m * S[1];
@@ -648,34 +656,19 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(StepParams P, Ctrl* 
 // cell key for the next build, the step's largest displacement, and the
 // next step's records.
 template <class R>
-__global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, Ctrl* __restrict__ ctrl,
+__global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, Ctrl* __restrict__ next,
+                                                                 const Ctrl* __restrict__ cur,
                                                                  ListState3<R> X, const real4<R>* __restrict__ der,
                                                                  const real4<R>* __restrict__ xs,
                                                                  ListRec<R>* __restrict__ rec,
                                                                  real4<R>* __restrict__ dens,
                                                                  const uint32_t* __restrict__ home, StateA3<R> A,
                                                                  uint32_t* __restrict__ key_next,
-                                                                 const unsigned long long* __restrict__ maxslots,
+                                                                 unsigned long long* __restrict__ maxslots,
                                                                  unsigned long long* __restrict__ dslots) {
-    Ctrl& c = *ctrl;
-    if (c.halted) return;
+    const Ctrl& c = *cur;
     double dt;
-    if (P.dt_method == 2 && P.dt_dynamic_mode == 1) {
-        double amax, mumax;
-        slots_max2(maxslots, amax, mumax);
-        dt = P.cfl * fmin(sqrt(P.h / amax), P.h / (P.c0 + mumax));
-    } else {
-        dt = c.cur_dt_const;
-    }
-    const bool never = P.dt_method == 2 && dt <= P.never_ending;
-    const bool nbr_err = P.consistency_check && c.nbr_overflow;
-    if (never || nbr_err) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            c.halted = 1;
-            c.status = nbr_err ? 3u : 4u;
-        }
-        return;
-    }
+    if (!list_dt(P, next, cur, maxslots, dt)) return;
     const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
     uint32_t outside = 0, bad = 0, changed = 0;
     double moved = 0.0;
@@ -698,13 +691,10 @@ __global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, C
         rec[s] = r;
         dens[s] = near3<R>(P, o.pos, typed_rho<R>(o.va.w, itype), h);
     }
-    wave_count_add(&c.outside, outside);
-    if (bad) atomicOr(&c.grid_overflow, 1u);
-    block_max2_to_slots(moved, 0.0, dslots, blockIdx.x);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        c.dt_new = dt;
-        c.pending = 1;
-    }
+    const uint32_t par = (uint32_t)(c.step & 1);
+    wave_count_add(&next->outside_l[par], outside);
+    if (bad) atomicOr(&next->grid_overflow, 1u);
+    block_max2_to_slots(moved, 0.0, dslots + par * kMaxSlots, blockIdx.x);
 }
 
 }  // namespace rrsph

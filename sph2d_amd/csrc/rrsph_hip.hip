@@ -195,6 +195,7 @@ struct rrsph_ctx {
     unsigned long long* maxslots = nullptr;
     uint32_t* LB = nullptr;
     Ctrl* ctrl = nullptr;
+    Ctrl* ctrl_cur = nullptr;   // list steps: the snapshot of the step in flight (list_step.hpp)
     Ctrl* util_ctrl = nullptr;
     Ctrl* host_ctrl = nullptr;  // pinned mirror
     double* scratch = nullptr;  // this device's `scratch` (rrsph_hip_smooth_gauges_noalloc)
@@ -456,40 +457,53 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool b
     const StepParams& P = c->P;
     const uint32_t nb = grid_blocks(P.n, kBlock);
     const uint32_t nb_xcd = P.blocks_per_xcd * kNumXcd;
-    L(K_PROLOGUE, [&] {
-        list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->dslots, c->maxslots, build ? 1u : 0u);
-    });
     ListState<R> X{c->posA, (const real4<R>*)c->vaA, c->oidA};
     ListRec<R>* rec = (ListRec<R>*)c->rec;
     if (build) {
-        enqueue_sort(c, c->ctrl, L);
+        L(K_PROLOGUE, [&] {
+            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->maxslots);
+        });
+        enqueue_sort(c, c->ctrl_cur, L);
         StateA<R> A = stateA<R>(c);
         StateB<R> B = stateB<R>(c, c->pred, c->pres);
         L(K_REORDER, [&] {
-            reorder_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->sorted_keys, c->sorted_perm, A, B,
+            reorder_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
                                                                  rec, c->home, c->LB, c->maxslots);
         });
         L(K_LIST_BUILD, [&] {
-            list_build_kernel<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->posB, (const real4<R>*)c->vaB,
+            list_build_kernel<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->posB, (const real4<R>*)c->vaB,
                                                                    c->sorted_keys, c->LB, c->nbl, c->nbc);
         });
         X = ListState<R>{c->posB, (const real4<R>*)c->vaB, c->oidB};
     }
+    // the first kernel of a list step makes its prologue
+    bool first = !build;
     if (P.density_treatment == 0) {
-        L(K_DENSITY_SUM, [&] {
-            density_sum_list<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, X, rec, (R*)c->pres, c->nbl, c->nbc);
-        });
+        auto density = [&](auto kernel) {
+            L(K_DENSITY_SUM, [&] {
+                kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                         c->dslots);
+            });
+        };
+        if (first) density(density_sum_list<R, true>);
+        else density(density_sum_list<R, false>);
+        first = false;
     }
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
-            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     (real4<R>*)c->der, (real2<R>*)c->xs, c->maxslots);
+            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                     (real4<R>*)c->der, (real2<R>*)c->xs, c->maxslots, c->dslots);
         });
     };
-    if (c->fast_pair) pair(pair_list_kernel<R>);
-    else pair(pair_list_general_kernel<R>);
+    if (c->fast_pair) {
+        if (first) pair(pair_list_kernel<R, true>);
+        else pair(pair_list_kernel<R, false>);
+    } else {
+        if (first) pair(pair_list_general_kernel<R, true>);
+        else pair(pair_list_general_kernel<R, false>);
+    }
     L(K_INTEGRATE, [&] {
-        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, X, (const real4<R>*)c->der,
+        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real4<R>*)c->der,
                                                                (const real2<R>*)c->xs, rec, c->home, stateA<R>(c),
                                                                c->key_next, c->maxslots, c->dslots);
     });
@@ -501,38 +515,48 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     const StepParams& P = c->P;
     const uint32_t nb = grid_blocks(P.n, kBlock);
     const uint32_t nb_xcd = P.blocks_per_xcd * kNumXcd;
-    L(K_PROLOGUE, [&] {
-        list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->dslots, c->maxslots, build ? 1u : 0u);
-    });
     ListState3<R> X{(const double4*)c->posA, (const real4<R>*)c->vaA, c->oidA};
     ListRec<R>* rec = (ListRec<R>*)c->rec;
     real4<R>* dens = (real4<R>*)c->dens;
     if (build) {
-        enqueue_sort(c, c->ctrl, L);
+        L(K_PROLOGUE, [&] {
+            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->maxslots);
+        });
+        enqueue_sort(c, c->ctrl_cur, L);
         StateA3<R> A = stateA3<R>(c);
         StateB3<R> B = stateB3<R>(c, c->pred, c->pw, c->pres);
         L(K_REORDER, [&] {
-            reorder_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->sorted_keys, c->sorted_perm, A, B,
+            reorder_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
                                                                   rec, dens, c->home, c->cand, c->LB, c->maxslots);
         });
         L(K_LIST_BUILD, [&] {
-            list_build3_kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, (const double4*)c->posB, c->cand,
+            list_build3_kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, (const double4*)c->posB, c->cand,
                                                                  c->sorted_keys, c->LB, c->nbl, c->nbc);
         });
         X = ListState3<R>{(const double4*)c->posB, (const real4<R>*)c->vaB, c->oidB};
     }
+    bool first = !build;
     if (P.density_treatment == 0) {
-        L(K_DENSITY_SUM, [&] {
-            density_sum_list3<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, X, dens, rec, (R*)c->pres, c->nbl,
-                                                                   c->nbc);
-        });
+        auto density = [&](auto kernel) {
+            L(K_DENSITY_SUM, [&] {
+                kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, dens, rec, (R*)c->pres, c->nbl,
+                                                         c->nbc, c->dslots);
+            });
+        };
+        if (first) density(density_sum_list3<R, true>);
+        else density(density_sum_list3<R, false>);
+        first = false;
     }
-    L(K_PAIR, [&] {
-        pair_list3_kernel<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                               (real4<R>*)c->der, (real4<R>*)c->xs, c->maxslots);
-    });
+    auto pair = [&](auto kernel) {
+        L(K_PAIR, [&] {
+            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                     (real4<R>*)c->der, (real4<R>*)c->xs, c->maxslots, c->dslots);
+        });
+    };
+    if (first) pair(pair_list3_kernel<R, true>);
+    else pair(pair_list3_kernel<R, false>);
     L(K_INTEGRATE, [&] {
-        integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, X, (const real4<R>*)c->der,
+        integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real4<R>*)c->der,
                                                                 (const real4<R>*)c->xs, rec, dens, c->home,
                                                                 stateA3<R>(c), c->key_next, c->maxslots, c->dslots);
     });
@@ -732,7 +756,7 @@ rrsph_status sync_status(rrsph_ctx* ctx) {
             if (const rrsph_status st = rollback_fused_step(ctx); st != RRSPH_OK) return st;
             return fail(ctx, RRSPH_ERR_TOO_MANY_NEIGHBOURS, status_message(RRSPH_ERR_TOO_MANY_NEIGHBOURS));
         }
-        if (ctx->P.consistency_check && c.outside > 0 && ctx->P.consistency_treatment == 1)
+        if (ctx->P.consistency_check && ctrl_outside(c) > 0 && ctx->P.consistency_treatment == 1)
             return fail(ctx, RRSPH_ERR_OUTSIDE_BOUNDARIES, status_message(RRSPH_ERR_OUTSIDE_BOUNDARIES));
     }
     return RRSPH_OK;
@@ -957,7 +981,7 @@ void free_all(rrsph_ctx* c) {
     void* ptrs[] = {c->posA, c->posB, c->vaA, c->vaB, c->adA, c->pred, c->der, c->xs, c->pred_scratch, c->pres,
                     c->pres_scratch, c->oidA,
                     c->oidB, c->key_next, c->kbuf[0], c->kbuf[1], c->vbuf[0], c->vbuf[1], c->hist, c->digit_total,
-                    c->maxslots, c->LB, c->ctrl,
+                    c->maxslots, c->LB, c->ctrl, c->ctrl_cur,
                     c->util_ctrl, c->red, c->st_r, c->st_v, c->st_rho, c->st_p, c->st_a, c->st_drho, c->st_av,
                     c->st_mu, c->st_itype, c->st_u32, c->skeyA, c->chg, c->chg_mask, c->wpre, c->pw,
                     c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->cand};
@@ -1078,9 +1102,11 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
     ctx->vbuf[1] = dalloc<uint32_t>(n, e);
     ctx->hist = dalloc<uint32_t>((size_t)kRadix * ctx->ntiles, e);
     ctx->digit_total = dalloc<uint32_t>(kRadix, e);
-    ctx->maxslots = dalloc<unsigned long long>(4 * kMaxSlots, e);  // second half: utility sorts
+    // the dt slots, the utility sorts' (cleared, not read), the list steps' second set
+    ctx->maxslots = dalloc<unsigned long long>(kMaxSlotSet + 2 * kMaxSlots, e);
     ctx->LB = dalloc<uint32_t>((size_t)ctx->P.ncells + 2, e);
     ctx->ctrl = dalloc<Ctrl>(1, e);
+    ctx->ctrl_cur = dalloc<Ctrl>(1, e);
     ctx->util_ctrl = dalloc<Ctrl>(1, e);
     ctx->red = dalloc<double>(kDiagSlots * (size_t)kDiagMaxBlocks + 64, e);
     ctx->skeyA = dalloc<uint32_t>(n, e);

@@ -169,11 +169,12 @@ __device__ __forceinline__ bool prologue_commit(const StepParams& P, Ctrl& c) {
             c.status = 3;  // RRSPH_ERR_TOO_MANY_NEIGHBOURS
             return false;
         }
+        const uint32_t outside = ctrl_outside(c);  // of the step being committed
         c.time += c.dt_new;
         c.dt = c.dt_new;
         c.step += 1;
         c.pending = 0;
-        if (P.consistency_check && c.outside > 0 && P.consistency_treatment == 1) {
+        if (P.consistency_check && outside > 0 && P.consistency_treatment == 1) {
             c.halted = 1;
             c.status = 5;  // RRSPH_ERR_OUTSIDE_BOUNDARIES
             return false;
@@ -204,6 +205,7 @@ __device__ __forceinline__ bool prologue_commit(const StepParams& P, Ctrl& c) {
     c.amax_bits = 0;
     c.mumax_bits = 0;
     c.outside = 0;
+    c.outside_l[0] = c.outside_l[1] = 0;
     return true;
 }
 
@@ -221,7 +223,7 @@ __device__ __forceinline__ double fourier_term(const StepParams& P, double t, in
 // with readlane (the values are uniform), the wave commits the previous
 // step and makes this step's snapshot on that copy, the Fourier piston's
 // terms are evaluated one per lane and summed in harmonic order, and lane
-// i writes word i back.  (Updating the block from one thread through
+// i writes word i to `out` (the block itself, or a list step's snapshot).  (Updating the block from one thread through
 // memory, LDS or global, is a chain of dependent round trips.)  `before`
 // and `after` act on the copy.  Every thread of the block calls it; the
 // barrier at the end orders the write-back before the block's later
@@ -239,7 +241,7 @@ __device__ __forceinline__ unsigned long long ctrl_word(const Ctrl* ctrl) {
 }
 
 template <class B, class A>
-__device__ __forceinline__ void block_prologue(const StepParams& P, Ctrl* ctrl, unsigned long long word, B&& before,
+__device__ __forceinline__ void block_prologue(const StepParams& P, Ctrl* out_ctrl, unsigned long long word, B&& before,
                                                A&& after) {
     if (threadIdx.x < kWave) {
         union {
@@ -279,7 +281,7 @@ __device__ __forceinline__ void block_prologue(const StepParams& P, Ctrl* ctrl, 
         unsigned long long out = 0;
 #pragma unroll
         for (uint32_t i = 0; i < kCtrlWords; ++i) out = threadIdx.x == i ? u.w[i] : out;
-        if (threadIdx.x < kCtrlWords) reinterpret_cast<unsigned long long*>(ctrl)[threadIdx.x] = out;
+        if (threadIdx.x < kCtrlWords) reinterpret_cast<unsigned long long*>(out_ctrl)[threadIdx.x] = out;
     }
     __syncthreads();
 }
