@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
         }
     };
     if constexpr (kNear)
-        collect_near3<kAdjChunk>(P, live && tk != 0, P.max_nbr - 1, sc, s_off, nk, nearf, pk, B.pos, nbl, nbc, my,
+        collect_near3<kAdjChunk>(P, live && tk != 0, P.max_nbr - 1, sc, s_off, nk, nearf, B.pos, nbl, nbc, my,
                                  overflow, flush);
     else if (LISTS)
         collect_listed3<kAdjChunk>(P, live && tk != 0, P.max_nbr - 1, sc, pk, B.pos, nbl, nbc, my, overflow, flush);

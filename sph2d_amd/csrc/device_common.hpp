@@ -78,8 +78,11 @@ struct Ctrl {
     uint32_t flags_pad;
 };
 
-// Particles outside the geometry after the step awaiting its commit.
-__host__ __device__ inline uint32_t ctrl_outside(const Ctrl& c) { return c.outside + c.outside_l[c.step & 1]; }
+// Particles outside the geometry after the step awaiting its commit.  (An
+// index computed at run time would put a copy of the block in scratch memory.)
+__host__ __device__ inline uint32_t ctrl_outside(const Ctrl& c) {
+    return c.outside + ((c.step & 1) ? c.outside_l[1] : c.outside_l[0]);
+}
 
 constexpr int kMaxSegments = 8;  // paddles of a segmented piston
 
@@ -98,6 +101,12 @@ struct StepParams {
     // physics
     double h, mass, rho0, g;
     double f_cubic, f_gauss, f_wend, f_desb;
+    // constants of the pair terms, so that no wave divides for them
+    double inv_h;           // 1 / h
+    double c_q1, c_q2, w_q2;  // cubic spline pieces: f / h^2, f / (2 h), f / 6
+    // list pair terms (list_step.hpp): a = c2 (b2 x - a2) x from x = vr /
+    // (d^2 + eta^2), and the factors of the summed terms
+    double lp_a2, lp_b2, lp_mF, lp_mW;
     int32_t skf_density, skf_intf, skf_av, skf_xsph, skf_ap;
     double eos_B;
     int32_t density_treatment;

@@ -108,13 +108,8 @@ __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, cons
                                                               const uint32_t* __restrict__ skey,
                                                               const uint32_t* __restrict__ perm, StateA<R> A,
                                                               StateB<R> B, ListRec<R>* __restrict__ rec,
-                                                              uint32_t* __restrict__ home, uint32_t* __restrict__ LB,
-                                                              unsigned long long* __restrict__ maxslots) {
+                                                              uint32_t* __restrict__ home, uint32_t* __restrict__ LB) {
     if (ctrl->halted) return;
-    if (blockIdx.x == 0) {
-        maxslots[threadIdx.x] = 0;
-        maxslots[kMaxSlots + threadIdx.x] = 0;
-    }
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
     const uint32_t s = live ? s0 : P.n - 1;
@@ -154,28 +149,85 @@ __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, cons
 // needs the decision.
 //
 // What several blocks of a step raise lies outside the published words: the
-// flags at the end of Ctrl, and slots by the parity of the step index -
-// displacement slots dslots (a set per parity: the integrator of step k fills
-// set k, the first kernel of step k + 1 reads it and clears the other) and
-// dt reduction slots maxslots (the pair pass of step k fills set k, its
-// integrator reads it and clears the other).
-constexpr uint32_t kMaxSlotSet = 4 * kMaxSlots;  // offset between the two sets of dt reduction slots
+// flags at the end of Ctrl, and maxima in slots, a set per parity of the step
+// index - displacement slots dslots (the integrator of step k fills set k,
+// the first kernel of step k + 1 reads it and clears the other) and dt
+// reduction slots maxslots (the pair pass of step k fills set k, its
+// integrator reads it and clears the other).  A set is few slots, each in a
+// 256-byte line of its own: every block of the next kernel reads them all, at
+// addresses known before any other load returns, without a reduction across
+// lanes or a barrier (256 adjacent slots, reduced by shuffles through LDS,
+// held every block up for about 1.5 us).
+constexpr uint32_t kSlots = 16, kSlotStride = 32;      // 64-bit words between slots
+constexpr uint32_t kSlotSet = kSlots * kSlotStride;    // words of a set
+constexpr uint32_t kDtSet = 2 * kSlotSet;              // a dt set: largest a^2, then largest mu
+__device__ __forceinline__ double slots_max(const unsigned long long* slots) {
+    unsigned long long w[kSlots];
+#pragma unroll
+    for (uint32_t k = 0; k < kSlots; ++k) w[k] = slots[k * kSlotStride];
+    double m = 0.0;
+#pragma unroll
+    for (uint32_t k = 0; k < kSlots; ++k) m = fmax(m, dbits(w[k]));
+    return m;
+}
+__device__ __forceinline__ void clear_slots(unsigned long long* slots) {
+    if (threadIdx.x < kSlots) slots[threadIdx.x * kSlotStride] = 0;
+}
+
+// The wave's maximum of a non-negative value in every lane's return value of
+// lane 63: data-parallel moves within and across the rows of 16 lanes, no LDS.
+template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <class R> __device__ __forceinline__ R wave_max_lane63(R v) {
+    v = fmax(v, dpp_move<0x111>(v));  // row_shr:1 (lanes without a source get 0)
+    v = fmax(v, dpp_move<0x112>(v));  // row_shr:2
+    v = fmax(v, dpp_move<0x114>(v));  // row_shr:4
+    v = fmax(v, dpp_move<0x118>(v));  // row_shr:8
+    v = fmax(v, dpp_move<0x142>(v));  // row_bcast:15
+    v = fmax(v, dpp_move<0x143>(v));  // row_bcast:31
+    return v;
+}
+// The block's maxima of two non-negative values into a slot of each set.
+template <class A, class B>
+__device__ __forceinline__ void block_max_to_slots(A a, B b, unsigned long long* __restrict__ slots_a,
+                                                   unsigned long long* __restrict__ slots_b, uint32_t blk) {
+    __shared__ double s_a[kBlock / kWave], s_b[kBlock / kWave];
+    a = wave_max_lane63(a);
+    if (slots_b) b = wave_max_lane63(b);
+    if (__lane_id() == kWave - 1) {
+        s_a[threadIdx.x / kWave] = (double)a;
+        s_b[threadIdx.x / kWave] = (double)b;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const double* w = threadIdx.x ? s_b : s_a;
+        double m = w[0];
+        for (int k = 1; k < kBlock / kWave; ++k) m = fmax(m, w[k]);
+        unsigned long long* slots = threadIdx.x ? slots_b : slots_a;
+        if (slots && m > 0.0)
+            atomicMax(&slots[(blk % kSlots) * kSlotStride], (unsigned long long)__double_as_longlong(m));
+    }
+}
+
 constexpr uint32_t kCtrlFlagWord = offsetof(Ctrl, nbr_overflow) / 8;
 static_assert(offsetof(Ctrl, nbr_overflow) % 8 == 0 && offsetof(Ctrl, dt_new) % 8 == 0 &&
                   offsetof(Ctrl, pending) % 8 == 0 && offsetof(Ctrl, halted) == offsetof(Ctrl, pending) + 4 &&
                   offsetof(Ctrl, status) % 8 == 0,
               "publish_ctrl's words");
 
-// The largest displacement of the step that `next` holds (block-wide).
-__device__ __forceinline__ double list_dmax(const Ctrl* next, const unsigned long long* __restrict__ dslots) {
-    __shared__ double s_m[kBlock / kWave];
-    double d = dbits(dslots[(uint32_t)(next->step & 1) * kMaxSlots + threadIdx.x]);
-    for (int off = 32; off > 0; off >>= 1) d = fmax(d, __shfl_xor(d, off));
-    if (__lane_id() == 0) s_m[threadIdx.x / kWave] = d;
-    __syncthreads();
-    double dmax = s_m[0];
-    for (int w = 1; w < kBlock / kWave; ++w) dmax = fmax(dmax, s_m[w]);
-    return dmax;
+// The largest displacement of the step that `next` holds, the slots holding
+// squares (both sets are loaded, so that the loads do not wait for the step
+// index).
+__device__ __forceinline__ double list_dmax(const Ctrl* next, const unsigned long long* dslots) {
+    const double even = slots_max(dslots), odd = slots_max(dslots + kSlotSet);
+    return sqrt((next->step & 1) ? odd : even);
 }
 
 // The prologue of a list step (build: of a build step) in one block: the
@@ -228,14 +280,16 @@ __device__ __forceinline__ bool list_step_halts(const StepParams& P, const Ctrl&
 // At the head of a list step's first kernel (every thread of the block):
 // false when the step halts, else its step index in `step`.
 __device__ __forceinline__ bool list_step_begin(const StepParams& P, Ctrl* next, Ctrl* cur,
-                                                unsigned long long* __restrict__ dslots, unsigned long long& step) {
+                                                unsigned long long* dslots, unsigned long long& step) {
     const double dmax = list_dmax(next, dslots);
-    step = next->step + (next->pending ? 1 : 0);
+    const unsigned long long k = next->step + (next->pending ? 1 : 0);
+    step = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k) |
+           ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(k >> 32)) << 32);
     const bool halts = list_step_halts(P, *next, dmax);
     if (blockIdx.x == 0) {
         list_block_prologue(P, next, cur, dmax, false);
         if (!halts) {  // this step's set; the blocks of this kernel read the other one
-            dslots[(uint32_t)(step & 1) * kMaxSlots + threadIdx.x] = 0;
+            clear_slots(dslots + (uint32_t)(step & 1) * kSlotSet);
             if (threadIdx.x == 0) next->outside_l[step & 1] = 0;
         }
     }
@@ -249,11 +303,11 @@ __global__ void __launch_bounds__(kBlock) list_prologue(StepParams P, Ctrl* __re
                                                         unsigned long long* __restrict__ maxslots) {
     const double dmax = list_dmax(next, dslots);
     list_block_prologue(P, next, cur, dmax, true);
-    if (cur->halted) return;
+    // (also when the step halts: the step after a halt is a build and reads none of them)
     for (uint32_t k = 0; k < 2; ++k) {
-        dslots[k * kMaxSlots + threadIdx.x] = 0;
-        maxslots[k * kMaxSlotSet + threadIdx.x] = 0;
-        maxslots[k * kMaxSlotSet + kMaxSlots + threadIdx.x] = 0;
+        clear_slots(dslots + k * kSlotSet);
+        clear_slots(maxslots + k * kDtSet);
+        clear_slots(maxslots + k * kDtSet + kSlotSet);
     }
     if (threadIdx.x == 0) {
         next->outside_l[0] = next->outside_l[1] = 0;
@@ -394,21 +448,21 @@ __device__ __forceinline__ CutFP32 cut_band(const StepParams& P) {
     return C;
 }
 __device__ __forceinline__ bool list_cut(const StepParams& P, const CutFP32& C, const float2* s_off, uint32_t e,
-                                         const float4& ni, const float4& nj, double2 pj,
+                                         const float4& ni, const float4& nj, uint32_t s,
                                          const double2* __restrict__ pos, float& dx, float& dy) {
     const float2 o = s_off[e >> kSlotBits];
     dx = (ni.x - nj.x) + o.x;
     dy = (ni.y - nj.y) + o.y;
     const float d2 = dx * dx + dy * dy;
     if (!(d2 > C.lo && d2 < C.hi)) return d2 <= C.lo;  // on the band's edge: within a rounding of lo < cut2
-    const double2 q = pos[e & kSlotMask];  // rare: the band around the cut-off
+    const double2 q = pos[e & kSlotMask], pj = pos[s];  // rare: the band around the cut-off
     const double ddx = __dsub_rn(q.x, pj.x), ddy = __dsub_rn(q.y, pj.y);
     dx = (float)ddx;
     dy = (float)ddy;
     return dist2_exact(ddx, ddy) < P.cut2;
 }
 __device__ __forceinline__ bool list_cut(const StepParams& P, const CutFP32&, const float2*, uint32_t,
-                                         const double4& ni, const double4& nj, double2, const double2* __restrict__,
+                                         const double4& ni, const double4& nj, uint32_t, const double2* __restrict__,
                                          double& dx, double& dy) {
     dx = __dsub_rn(ni.x, nj.x);
     dy = __dsub_rn(ni.y, nj.y);
@@ -433,6 +487,84 @@ __device__ __forceinline__ uint32_t list_entry(const uint32_t* __restrict__ nbl,
     return *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(nbl) + byte_off);
 }
 
+// LPP lanes of a wave share a particle's list in the 2D passes: lane l takes
+// the entries l, l + LPP, ..., and the partial sums are added across the
+// lanes (lane_sum).  The lanes of one l are consecutive, so that a row of the
+// lists is still read in runs of 64 / LPP entries.  A pass is bound by the
+// latency of its dependent loads (entry, then record), so with few particles
+// it is the number of rounds per lane that counts, and the lanes that fill
+// the chip are free; with many, the extra lanes only repeat the work per
+// particle.
+template <int LPP> struct LaneGroup {
+    static constexpr uint32_t kParticles = kWave / LPP;  // of a wave
+    uint32_t l, s;                                       // this lane's share of the list, and its particle
+    __device__ explicit LaneGroup(uint32_t lb)
+        : l(__lane_id() / kParticles),
+          s((lb * (kBlock / kWave) + threadIdx.x / kWave) * kParticles + __lane_id() % kParticles) {}
+};
+template <int LPP> __host__ __device__ inline uint32_t group_blocks(uint32_t n) {
+    return (n + kBlock / LPP - 1) / (kBlock / LPP);
+}
+template <int LPP> __host__ __device__ inline uint32_t group_blocks_per_xcd(uint32_t n) {
+    return (group_blocks<LPP>(n) + kNumXcd - 1) / kNumXcd;
+}
+template <int LPP, class R> __device__ __forceinline__ R lane_sum(R v) {
+#pragma unroll
+    for (int off = kWave / LPP; off < kWave; off <<= 1) v += __shfl_xor(v, off);
+    return v;
+}
+template <int LPP, class R> __device__ __forceinline__ R lane_max(R v) {
+#pragma unroll
+    for (int off = kWave / LPP; off < kWave; off <<= 1) v = fmax(v, __shfl_xor(v, off));
+    return v;
+}
+
+// Of the hits of one row of LPP entries of a particle (this lane's: hit),
+// whether this lane's is among the first `cap` of the list, hits counting
+// those of the rows before; every lane of the particle calls it.
+template <int LPP>
+__device__ __forceinline__ bool take_capped(bool hit, uint32_t l, uint32_t cap, uint32_t& hits, bool& over) {
+    uint32_t before = hits;
+    if (LPP == 1) {
+        hits += hit ? 1u : 0u;
+    } else {
+#pragma unroll
+        for (int q = 0; q < LPP; ++q) {
+            const uint32_t h = (uint32_t)__shfl((int)hit, q * (kWave / LPP) + (int)(__lane_id() % (kWave / LPP)));
+            before += q < (int)l ? h : 0u;
+            hits += h;
+        }
+    }
+    const bool take = hit & (before < cap);
+    over |= hit & !take;
+    return take;
+}
+
+// Entries of slot s's list in rounds of G per lane: per round
+// body(k, e, load) - k the list index of the lane's first entry, its entries
+// k, k + LPP, ... in e; load fetches the next round's.  Entries past a list's end name valid slots (padding rows, or entries
+// of an earlier build); with LPP > 1 the loads past the last allocated row
+// read that row instead.
+template <int LPP, uint32_t G, class B>
+__device__ __forceinline__ void list_rounds(const StepParams& P, const uint32_t* __restrict__ nbl, uint32_t s,
+                                            uint32_t l, uint32_t cnt, B&& body) {
+    static_assert(LPP > 1 || 2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
+    const uint32_t row = P.n * 4u, last = (P.list_cap + kListPad - 1) * row + s * 4u;
+    uint32_t off = (l * P.n + s) * 4u;
+    auto load = [&](uint32_t (&e)[G]) {
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) {
+            const uint32_t o = off + u * LPP * row;
+            e[u] = list_entry(nbl, LPP > 1 ? min(o, last) : o);
+        }
+        off += G * LPP * row;
+    };
+    uint32_t e[G];
+    load(e);
+#pragma unroll 1
+    for (uint32_t k = l; k - l < cnt; k += G * LPP) body(k, e, load);
+}
+
 // Visits the entries of slot s's list: f(ListEntry) for every entry (f must
 // add nothing when take is false: every entry runs the same instructions,
 // most entries being neighbours).  kCap: count the neighbours, and entries
@@ -444,106 +576,132 @@ __device__ __forceinline__ uint32_t list_entry(const uint32_t* __restrict__ nbl,
 // loads).  Larger groups keep more gathers in flight per wave but take
 // registers: the pass is bound by load latency, and 2 entries per group
 // (74 VGPRs, 6 waves per SIMD) gave the least time.
-template <class R, bool kCap, class F>
+template <class R, bool kCap, int LPP, class F>
 __device__ __forceinline__ void for_each_listed(const StepParams& P, const float2* s_off, uint32_t cap, uint32_t s,
-                                                const real4<R>& nj, double2 pj, const double2* __restrict__ pos,
+                                                uint32_t l, const real4<R>& nj, const double2* __restrict__ pos,
                                                 const ListRec<R>* __restrict__ rec, const uint32_t* __restrict__ nbl,
-                                                uint32_t cnt, bool& overflow,
-                                                F&& f) {
+                                                uint32_t cnt, bool& overflow, F&& f) {
     constexpr uint32_t G = 2;  // measured at C1-1M FP32: 57.7 us per pass against 58.8 (3), 61.4 (4), 65.1 (1)
-    static_assert(2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
     if (cnt == 0) return;
-    const uint32_t row = P.n * 4u;
-    uint32_t off = s * 4u;
     const CutFP32 C = cut_band(P);
     uint32_t hits = 0;
     bool over = false;
-    uint32_t e[G];
-#pragma unroll
-    for (uint32_t u = 0; u < G; ++u) e[u] = list_entry(nbl, off + u * row);
-    off += G * row;
-#pragma unroll 1
-    for (uint32_t k = 0; k < cnt; k += G) {
+    list_rounds<LPP, G>(P, nbl, s, l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
         ListRec<R> r[G];
         uint32_t en[G];
 #pragma unroll
         for (uint32_t u = 0; u < G; ++u) r[u] = rec[e[u] & kSlotMask];
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) en[u] = list_entry(nbl, off + u * row);
-        off += G * row;
+        load(en);
 #pragma unroll
         for (uint32_t u = 0; u < G; ++u) {
             ListEntry<R> E;
-            const bool in = list_cut(P, C, s_off, e[u], r[u].nr, nj, pj, pos, E.dx, E.dy);
-            const bool hit = in & (r[u].pr.z != R(0)) & (k + u < cnt);
-            if (kCap) {
-                E.take = hit & (hits < cap);
-                over |= hit & !E.take;
-                hits += E.take ? 1u : 0u;
-            } else {
-                E.take = hit;
-            }
+            const bool in = list_cut(P, C, s_off, e[u], r[u].nr, nj, s, pos, E.dx, E.dy);
+            const bool hit = in & (r[u].pr.z != R(0)) & (k + u * LPP < cnt);
+            E.take = kCap ? take_capped<LPP>(hit, l, cap, hits, over) : hit;
             E.nr = r[u].nr;
             E.pr = r[u].pr;
             f(E);
         }
 #pragma unroll
         for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
-    }
+    });
     overflow |= over;
 }
 
-// fast_pair_term (the cubic configuration) for one list entry, without
-// branches except the rare Lennard-Jones case: both pieces of the cubic
-// spline are evaluated and selected, and nothing is added when take is
-// false.  The Lennard-Jones ratios use 1/|r| from the reciprocal square
-// root instead of two divisions.  j's own records: vaj (v, rho, itype) and
-// prj (pred record).
-template <class R>
-__device__ __forceinline__ void list_pair_term(const FastPair<R>& K, PairSums<R>& S, const ListEntry<R>& E,
-                                               const real4<R>& vaj, const real4<R>& prj, int tj) {
-    const R dx = E.dx, dy = E.dy;
-    const bool take = E.take;
-    const R d2 = dx * dx + dy * dy;
-    const R rinv = d2 > R(0) ? fast_rsqrt<R>(d2) : R(0);
-    const R dist = d2 * rinv;
-    const R q = dist * K.inv_h;
-    const R t = R(2) - q;
-    const R t2 = t * t;
-    const bool inner = q <= R(1);
-    const R F1 = K.c_q1 * (R(1.5) * q - R(2));
-    const R F2 = -K.c_q2 * t2 * rinv;
-    const R W1 = K.w_q1 * (R(2) / R(3) - q * q + R(0.5) * q * q * q);
-    const R W2 = K.w_q2 * t2 * t;
-    const R F = take ? (inner ? F1 : F2) : R(0);
-    const R W = inner ? W1 : W2;
-    if (K.cont) S.sd += F * ((E.nr.z - vaj.x) * dx + (E.nr.w - vaj.y) * dy);
-    const R rho_i = fabs(E.pr.z), rho_j = fabs(prj.z);
-    if (K.lj_on && take && tj > 0 && E.pr.z < R(0) && dist < K.lj_r0) {
-        const R rn = K.lj_r0 * rinv;
-        const R rn2 = rn * rn, rn4 = rn2 * rn2;
-        const R f = K.lj_D * (rn4 * rn4 * rn4 - rn4) * (rinv * rinv);
+// The cubic configuration's pair terms (fast_pair_term) for list entries,
+// 2D and 3D, arranged for instruction count, which bounds the passes (a
+// wave of the 2D FP32 pass issued 1,797 VALU instructions, 47 of its 58 us
+// at 1M particles):
+//   * with t = max(1 - q/2, 0) and u = max(1 - q, 0), both free clamps of one
+//     multiply-add, the spline is W = 4f/3 (t^3 - u^3 / 2) and grad W = diff
+//     (-2f/h) (t^2 - u^2) / |r| on both pieces, without selects; constant
+//     factors are applied once per particle (lp_mF, lp_mW);
+//   * an entry that is no neighbour gets |r| = 4 h, where both vanish;
+//   * artificial viscosity from x = min(vr, 0) / (d^2 + eta^2), mu = h x:
+//     the term is zero by itself where particles separate.
+// CONT: continuity density; ALL: artificial viscosity, XSPH and the wall
+// force are all on (else each by its switch).
+template <class R, bool CONT, bool ALL> struct ListPair {
+    static constexpr bool cont = CONT;
+    R ht, hu, hfar, a2, b2, eta2, lj_r0, lj_D;
+    bool lj_on, av_on, xsph_on;
+    __device__ explicit ListPair(const StepParams& P)
+        : ht((R)(-0.5 * P.inv_h)), hu((R)(-P.inv_h)), hfar((R)(4.0 * P.h)), a2((R)P.lp_a2), b2((R)P.lp_b2),
+          eta2((R)P.av_eta2), lj_r0((R)P.lj_r0), lj_D((R)P.lj_D), lj_on(ALL || P.lj_on), av_on(ALL || P.av_on),
+          xsph_on(ALL || P.xsph_on) {}
+};
+// What a pair gives, but for the direction: the gradient factor F (grad W =
+// diff F lp_mF / m), the XSPH weight w of fluid neighbours (W / (rho_i +
+// rho_j), to be scaled by lp_mW), the coefficient of the pressure and
+// viscosity terms, and whether the wall force acts.
+template <class R> struct ListTerm {
+    R F, w, coef, rinv;
+    bool wall;
+};
+template <class R> __device__ __forceinline__ R clamp01(R v) { return fmin(fmax(v, R(0)), R(1)); }
+// min(a, b) for b not NaN; the median takes no canonicalising instruction
+__device__ __forceinline__ float running_min(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, -INFINITY); }
+__device__ __forceinline__ double running_min(double a, double b) { return b < a ? b : a; }
+// d2 = |diff|^2, vr = (v^_i - v^_j) . diff, zi and zj the typed densities, pw the sum
+// of the p / rho^2; xmin collects the least x (mu = h x).
+template <class R, class K_>
+__device__ __forceinline__ ListTerm<R> list_pair(const K_& K, bool take, R d2, R vr, R zi, R zj, R pw, R& xmin) {
+    ListTerm<R> T;
+    // coincident particles: |r| = 0 and t = u, so F = 0
+    T.rinv = fast_rsqrt<R>(d2 + (sizeof(R) == 4 ? R(1e-30f) : R(1e-200)));
+    const R dist = take ? d2 * T.rinv : K.hfar;
+    const R t = clamp01<R>(fma(dist, K.ht, R(1))), u = clamp01<R>(fma(dist, K.hu, R(1)));
+    const R t2 = t * t, u2 = u * u;
+    T.F = T.rinv * (t2 - u2);
+    const R inv_rs = fast_rcp<R>(fabs(zi) + fabs(zj));
+    T.coef = pw;
+    if (K.av_on) {
+        const R x = take ? fmin(vr, R(0)) * fast_rcp<R>(d2 + K.eta2) : R(0);
+        xmin = running_min(xmin, x);
+        T.coef += (K.b2 * x - K.a2) * x * inv_rs;
+    }
+    T.w = K.xsph_on && zi > R(0) ? (t2 * t - R(0.5) * (u2 * u)) * inv_rs : R(0);
+    T.wall = K.lj_on && zj > R(0) && zi < R(0) && dist < K.lj_r0;
+    return T;
+}
+// The wall force's factor on diff (0 for coincident particles).
+template <class R, class K_> __device__ __forceinline__ R list_wall(const K_& K, R d2, R rinv) {
+    const R ri = d2 > R(0) ? rinv : R(0);
+    const R rn = K.lj_r0 * ri;
+    const R rn2 = rn * rn, rn4 = rn2 * rn2;
+    return K.lj_D * (rn4 * rn4 * rn4 - rn4) * (ri * ri);
+}
+
+// One entry in 2D; nj, prj: the particle's own record.
+template <class R> struct ListSums {
+    R sx = 0, sy = 0, sd = 0, xx = 0, xy = 0, xmin = 0, ljx = 0, ljy = 0;
+};
+template <class R, class K_>
+__device__ __forceinline__ void list_pair_term(const K_& K, ListSums<R>& S, const ListEntry<R>& E,
+                                               const real4<R>& nj, const real4<R>& prj) {
+    const R dx = E.dx, dy = E.dy, d2 = dx * dx + dy * dy;
+    const R dvx = E.pr.x - prj.x, dvy = E.pr.y - prj.y;
+    const ListTerm<R> T = list_pair<R>(K, E.take, d2, dvx * dx + dvy * dy, E.pr.z, prj.z, E.pr.w + prj.w, S.xmin);
+    if (K.cont) S.sd += T.F * ((E.nr.z - nj.z) * dx + (E.nr.w - nj.w) * dy);
+    const R fc = T.F * T.coef;
+    S.sx += fc * dx;
+    S.sy += fc * dy;
+    S.xx += dvx * T.w;
+    S.xy += dvy * T.w;
+    if (T.wall) {
+        const R f = list_wall<R>(K, d2, T.rinv);
         S.ljx -= dx * f;
         S.ljy -= dy * f;
     }
-    const R inv_rs = fast_rcp<R>(rho_i + rho_j);
-    R coef = E.pr.w + prj.w;
-    const R dvx = E.pr.x - prj.x, dvy = E.pr.y - prj.y;
-    if (K.av_on) {
-        const R vr = dvx * dx + dvy * dy;
-        const R mu = K.h * vr * fast_rcp<R>(d2 + K.eta2);
-        const bool app = take & (vr < R(0));
-        S.amu = app ? fmax(S.amu, -mu) : S.amu;
-        coef += app ? (K.beta * mu - K.alpha_c) * mu * R(2) * inv_rs : R(0);
-    }
-    const R fc = F * coef;
-    S.sx += fc * dx;
-    S.sy += fc * dy;
-    if (K.xsph_on) {
-        const R cw = (take & (E.pr.z > R(0))) ? W * inv_rs : R(0);
-        S.xx += dvx * cw;
-        S.xy += dvy * cw;
-    }
+}
+
+// The dt reductions of a pair pass: the block's largest a^2 and mu into the
+// step's slots (the integrator takes the square root of the largest: the
+// same value as the largest root).
+template <class R>
+__device__ __forceinline__ void list_dt_maxima(const StepParams& P, double a2, R mu,
+                                               unsigned long long* __restrict__ slots, uint32_t lb) {
+    if (P.dt_method == 2 && P.dt_dynamic_mode == 1) block_max_to_slots(a2, mu, slots, slots + kSlotSet, lb);
 }
 
 // Summation density from the lists (Density.h:25-61): rho = m W(0) +
@@ -552,60 +710,74 @@ __device__ __forceinline__ void list_pair_term(const FastPair<R>& K, PairSums<R>
 // (ModelParams.tex:124-133, rho_i the density before the step).  Cubic
 // spline.  Aliveness and the old densities come from va (pred is being
 // rewritten by this pass).
-template <class R, bool FIRST>
+template <class R, bool FIRST, int LPP>
 __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X,
                                                            ListRec<R>* __restrict__ rec, R* __restrict__ pres,
                                                            const uint32_t* __restrict__ nbl,
                                                            const uint32_t* __restrict__ nbc,
                                                            unsigned long long* __restrict__ dslots) {
-    const uint32_t lb = xcd_block(P.blocks_per_xcd);
-    if (lb >= P.nblocks) return;
+    const uint32_t lb = xcd_block(group_blocks_per_xcd<LPP>(P.n));
+    if (lb >= group_blocks<LPP>(P.n)) return;
     __shared__ float2 s_off[64];
     fill_cell_offsets(P, s_off);
+    const LaneGroup<LPP> g(lb);
+    const uint32_t s = g.s;
+    const bool live = s < P.n;
+    real4<R> vaj{}, nj{};
+    uint32_t cnt = 0;
+    if (live) {
+        vaj = X.va[s];
+        nj = rec[s].nr;
+        cnt = nbc[s];
+    }
     unsigned long long step;
     if constexpr (FIRST) {
         if (!list_step_begin(P, next, cur, dslots, step)) return;
     } else {
         if (!list_step_goes(cur)) return;
         step = cur->step;
-        __syncthreads();
     }
-    const uint32_t s = lb * kBlock + threadIdx.x;
-    if (s >= P.n) return;
+    __syncthreads();  // the offset table
     const KernelConsts<R> K = kernel_consts<R>(P);
     const R m = (R)P.mass;
-    const real4<R> vaj = X.va[s];
     const R w0 = kernel_w<R>(K, P.skf_density, R(0));
-    R rho = m * w0;
     const bool renorm = step_renorm(P, step);
-    R wsum = renorm ? m / vaj.z * w0 : R(0);
+    R rho = R(0), wsum = R(0);
     bool overflow = false;
-    const uint32_t cnt = (int)vaj.w != 0 ? nbc[s] : 0u;
+    if ((int)vaj.w == 0) cnt = 0;
     if (cnt) {
         const CutFP32 C = cut_band(P);
-        const real4<R> nj = rec[s].nr;
-        const double2 pj = X.pos[s];
         const uint32_t cap = P.max_nbr - 1;
-        const uint32_t row = P.n * 4u;
-        uint32_t off = s * 4u;
+        constexpr uint32_t G = 2;
+        const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
         uint32_t hits = 0;
-#pragma unroll 2
-        for (uint32_t k = 0; k < cnt; ++k, off += row) {
-            const uint32_t e = list_entry(nbl, off);
-            const uint32_t i = e & kSlotMask;
-            const real4<R> vai = X.va[i];
-            R dx, dy;
-            const bool hit = list_cut(P, C, s_off, e, rec[i].nr, nj, pj, X.pos, dx, dy) && (int)vai.w != 0;
-            const bool take = hit & (hits < cap);
-            overflow |= hit & !take;
-            hits += take ? 1u : 0u;
-            const R w = take ? kernel_w<R>(K, P.skf_density, pair_dist<R>(dx, dy, 0.0)) : R(0);
-            rho += m * w;
-            if (renorm) wsum += m / vai.z * w;
-        }
+        list_rounds<LPP, G>(P, nbl, s, g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
+            real4<R> ni[G], va[G];
+            uint32_t en[G];
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) {
+                ni[u] = rec[e[u] & kSlotMask].nr;
+                va[u] = X.va[e[u] & kSlotMask];
+            }
+            load(en);
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) {
+                R dx, dy;
+                bool take = list_cut(P, C, s_off, e[u], ni[u], nj, s, X.pos, dx, dy) & ((int)va[u].w != 0) &
+                            (k + u * LPP < cnt);
+                if (capped) take = take_capped<LPP>(take, g.l, cap, hits, overflow);
+                const R w = take ? kernel_w<R>(K, P.skf_density, pair_dist<R>(dx, dy, 0.0)) : R(0);
+                rho += m * w;
+                if (renorm) wsum += m / va[u].z * w;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
+        });
     }
-    if (renorm) rho = rho / wsum;
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
+    rho = m * w0 + lane_sum<LPP>(rho);
+    if (renorm) rho = rho / (m / vaj.z * w0 + lane_sum<LPP>(wsum));
+    if (!live || g.l != 0) return;
     real4<R> pr = rec[s].pr;
     const R p = eos_p<R>(rho, (R)P.rho0, (R)P.eos_B);
     pr.z = typed_rho<R>(rho, (int)vaj.w);
@@ -619,15 +791,26 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* n
 // pair_fast_kernel), the dt maxima, and the fields for the integrator.  With
 // continuity it also writes the pressure of the current density (the
 // reference's p array).
-template <class R, bool FIRST>
-__global__ void __launch_bounds__(kBlock) pair_list_kernel(
+template <class R, bool FIRST, int LPP, bool CONT, bool ALL>
+__global__ void __launch_bounds__(kBlock, LPP == 1 ? (sizeof(R) == 4 ? 6 : 4) : 1) pair_list_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
     real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
-    const uint32_t lb = xcd_block(P.blocks_per_xcd);
-    if (lb >= P.nblocks) return;
+    const uint32_t lb = xcd_block(group_blocks_per_xcd<LPP>(P.n));
+    if (lb >= group_blocks<LPP>(P.n)) return;
     __shared__ float2 s_off[64];
     fill_cell_offsets(P, s_off);
+    const LaneGroup<LPP> g(lb);
+    const uint32_t s = g.s;
+    const bool live = s < P.n;
+    // in flight while the block decides whether the step runs
+    real4<R> prj{}, nj{};
+    uint32_t cnt = 0;
+    if (live) {
+        prj = rec[s].pr;
+        nj = rec[s].nr;
+        cnt = nbc[s];
+    }
     unsigned long long step;
     if constexpr (FIRST) {
         if (!list_step_begin(P, next, cur, dslots, step)) return;
@@ -635,52 +818,41 @@ __global__ void __launch_bounds__(kBlock) pair_list_kernel(
         if (!list_step_goes(cur)) return;
         if (list_build_overflowed(next, cur)) return;
         step = cur->step;
-        __syncthreads();
     }
-    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
-    const uint32_t s = lb * kBlock + threadIdx.x;
-    const bool live = s < P.n;
-    const FastPair<R> K(P);
-    PairSums<R> S;
+    __syncthreads();  // the offset table
+    maxslots += (uint32_t)(step & 1) * kDtSet;
+    const ListPair<R, CONT, ALL> K(P);
+    ListSums<R> S;
     bool overflow = false;
-    real4<R> vaj{}, prj{};
-    if (live) {
-        vaj = X.va[s];
-        prj = rec[s].pr;
-    }
-    const int tj = (int)vaj.w;
-    const uint32_t cnt = live && tj != 0 ? nbc[s] : 0u;
+    if (prj.z == R(0)) cnt = 0;  // died since the build
     const uint32_t cap = P.max_nbr - 1;
     if (cnt) {
-        auto term = [&](const ListEntry<R>& E) { list_pair_term<R>(K, S, E, vaj, prj, tj); };
-        const real4<R> nj = rec[s].nr;
-        const double2 pj = X.pos[s];
+        auto term = [&](const ListEntry<R>& E) { list_pair_term<R>(K, S, E, nj, prj); };
         if (__ballot(cnt > cap))  // some list of the wave may hold more than cap neighbours
-            for_each_listed<R, true>(P, s_off, cap, s, nj, pj, X.pos, rec, nbl, cnt, overflow, term);
+            for_each_listed<R, true, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, overflow, term);
         else
-            for_each_listed<R, false>(P, s_off, cap, s, nj, pj, X.pos, rec, nbl, cnt, overflow, term);
+            for_each_listed<R, false, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, overflow, term);
     }
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
-    const R m = (R)P.mass;
-    const R ax = S.ljx + m * S.sx;
-    const R ay = -(R)P.g + S.ljy + m * S.sy;
-    const R drho = m * S.sd;
-    const R xf = m * R(2) * (R)P.xsph_eps;
-    if (P.dt_method == 2 && P.dt_dynamic_mode == 1)
-        block_max2_to_slots(live ? sqrt((double)ax * ax + (double)ay * ay) : 0.0, live ? (double)S.amu : 0.0,
-                            maxslots, lb);
-    if (live) {
+    const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);
+    const R ax = lane_sum<LPP>(S.ljx + mF * S.sx);
+    const R ay = -(R)P.g + lane_sum<LPP>(S.ljy + mF * S.sy);
+    const R drho = mF * lane_sum<LPP>(S.sd);
+    const R xx = mW * lane_sum<LPP>(S.xx), xy = mW * lane_sum<LPP>(S.xy);
+    const R amu = (R)P.h * lane_max<LPP>(-S.xmin);
+    list_dt_maxima<R>(P, live ? (double)ax * ax + (double)ay * ay : 0.0, live ? amu : R(0), maxslots, lb);
+    if (live && g.l == 0) {
         real4<R> d;
         d.x = ax;
         d.y = ay;
         d.z = drho;
-        d.w = S.amu;
+        d.w = amu;
         der[s] = d;
         real2<R> x;
-        x.x = xf * S.xx;
-        x.y = xf * S.xy;
+        x.x = xx;
+        x.y = xy;
         xs[s] = x;
-        if (P.density_treatment != 0) pres[s] = eos_p<R>(vaj.z, (R)P.rho0, (R)P.eos_B);
+        if (P.density_treatment != 0) pres[s] = eos_p<R>(X.va[s].z, (R)P.rho0, (R)P.eos_B);
     }
 }
 
@@ -727,13 +899,25 @@ __device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R d
 // evaluation, and no term divides: the cell walk over ~55 candidates with a
 // division or more per term took 167 us at 187,530 particles (FP64, Wendland
 // kernels, delta-SPH, artificial pressure), the ~20 entries of a list 53.
-template <class R, bool FIRST>
+template <class R, bool FIRST, int LPP>
 __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
     real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
-    const uint32_t lb = xcd_block(P.blocks_per_xcd);
-    if (lb >= P.nblocks) return;
+    const uint32_t lb = xcd_block(group_blocks_per_xcd<LPP>(P.n));
+    if (lb >= group_blocks<LPP>(P.n)) return;
+    const LaneGroup<LPP> g(lb);
+    const uint32_t s = g.s;
+    const bool live = s < P.n;
+    double2 pj = make_double2(0, 0);
+    real4<R> vaj{}, prj{};
+    uint32_t cnt = 0;
+    if (live) {
+        pj = X.pos[s];
+        vaj = X.va[s];
+        prj = rec[s].pr;
+        cnt = nbc[s];
+    }
     unsigned long long step;
     if constexpr (FIRST) {
         if (!list_step_begin(P, next, cur, dslots, step)) return;
@@ -742,22 +926,13 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
         if (list_build_overflowed(next, cur)) return;
         step = cur->step;
     }
-    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
-    const uint32_t s = lb * kBlock + threadIdx.x;
-    const bool live = s < P.n;
+    maxslots += (uint32_t)(step & 1) * kDtSet;
     const KernelConsts<R> K = kernel_consts<R>(P);
     const R m = (R)P.mass;
-    R ax = R(0), ay = -(R)P.g, drho = R(0), avx = R(0), avy = R(0), amu = R(0);
+    R ax = R(0), ay = R(0), drho = R(0), avx = R(0), avy = R(0), amu = R(0);
     bool overflow = false;
-    double2 pj = make_double2(0, 0);
-    real4<R> vaj{}, prj{};
-    if (live) {
-        pj = X.pos[s];
-        vaj = X.va[s];
-        prj = rec[s].pr;
-    }
     const int tj = (int)vaj.w;
-    const uint32_t cnt = live && tj != 0 ? nbc[s] : 0u;
+    if (tj == 0) cnt = 0;
     if (cnt) {
         const bool cont = P.density_treatment != 0, delta = P.density_treatment == 2;
         const R rhohj = fabs(prj.z), pjres = prj.w * (rhohj * rhohj);
@@ -765,16 +940,10 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
         const R two_eps_m = R(2) * (R)P.xsph_eps * m, lj_r0 = (R)P.lj_r0, lj_D = (R)P.lj_D;
         const R dhc2m = R(2) * (R)P.dhc * m, ap_iw = P.art_pressure ? (R)(1.0 / P.ap_wdelta) : R(0);
         const uint32_t cap = P.max_nbr - 1;
-        const uint32_t row = P.n * 4u;
         constexpr uint32_t G = 2;
-        static_assert(2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
-        uint32_t off = s * 4u, hits = 0;
-        uint32_t e[G];
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) e[u] = list_entry(nbl, off + u * row);
-        off += G * row;
-#pragma unroll 1
-        for (uint32_t k = 0; k < cnt; k += G) {
+        const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
+        uint32_t hits = 0;
+        list_rounds<LPP, G>(P, nbl, s, g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
             double2 pos[G];
             real4<R> va[G], pr[G];
             uint32_t en[G];
@@ -785,19 +954,14 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
                 va[u] = X.va[i];
                 pr[u] = rec[i].pr;
             }
-#pragma unroll
-            for (uint32_t u = 0; u < G; ++u) en[u] = list_entry(nbl, off + u * row);
-            off += G * row;
+            load(en);
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) {
                 const double dxd = __dsub_rn(pos[u].x, pj.x), dyd = __dsub_rn(pos[u].y, pj.y);
                 const int ti = (int)va[u].w;
-                if (!((k + u < cnt) & (ti != 0) & (dist2_exact(dxd, dyd) < P.cut2))) continue;
-                if (hits == cap) {
-                    overflow = true;
-                    continue;
-                }
-                ++hits;
+                bool take = (k + u * LPP < cnt) & (ti != 0) & (dist2_exact(dxd, dyd) < P.cut2);
+                if (capped) take = take_capped<LPP>(take, g.l, cap, hits, overflow);
+                if (!take) continue;
                 const R dx = (R)dxd, dy = (R)dyd;  // r_i - r_j
                 const R d2 = (R)(dxd * dxd + dyd * dyd);
                 const bool apart = d2 > R(0);
@@ -862,13 +1026,17 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
             }
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
-        }
+        });
     }
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
-    if (P.dt_method == 2 && P.dt_dynamic_mode == 1)
-        block_max2_to_slots(live ? sqrt((double)ax * ax + (double)ay * ay) : 0.0, live ? (double)amu : 0.0, maxslots,
-                            lb);
-    if (live) {
+    ax = lane_sum<LPP>(ax);
+    ay = -(R)P.g + lane_sum<LPP>(ay);
+    drho = lane_sum<LPP>(drho);
+    avx = lane_sum<LPP>(avx);
+    avy = lane_sum<LPP>(avy);
+    amu = lane_max<LPP>(amu);
+    list_dt_maxima<R>(P, live ? (double)ax * ax + (double)ay * ay : 0.0, live ? amu : R(0), maxslots, lb);
+    if (live && g.l == 0) {
         real4<R> d;
         d.x = ax;
         d.y = ay;
@@ -888,15 +1056,14 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
 // False when the step halted or halts here (dt below the reference's
 // never-ending bound, more neighbours than max_neighbours - 1).
 __device__ __forceinline__ bool list_dt(const StepParams& P, Ctrl* next, const Ctrl* cur,
-                                        unsigned long long* __restrict__ maxslots, double& dt) {
+                                        unsigned long long* maxslots, double& dt) {
     uint32_t halt_status = 0;
     const bool halted = cur->halted != 0;
     if (!halted) {
         const uint32_t par = (uint32_t)(cur->step & 1);
         if (P.dt_method == 2 && P.dt_dynamic_mode == 1) {
-            double amax, mumax;
-            slots_max2(maxslots + par * kMaxSlotSet, amax, mumax);
-            dt = P.cfl * fmin(sqrt(P.h / amax), P.h / (P.c0 + mumax));
+            const double a2max = slots_max(maxslots + par * kDtSet), mumax = slots_max(maxslots + par * kDtSet + kSlotSet);
+            dt = P.cfl * fmin(sqrt(P.h / sqrt(a2max)), P.h / (P.c0 + mumax));
         } else {
             dt = cur->cur_dt_const;
         }
@@ -904,69 +1071,73 @@ __device__ __forceinline__ bool list_dt(const StepParams& P, Ctrl* next, const C
         const bool nbr_err = P.consistency_check && next->nbr_overflow;
         halt_status = nbr_err ? 3u : (never ? 4u : 0u);
         if (blockIdx.x == 0) {
-            maxslots[(par ^ 1) * kMaxSlotSet + threadIdx.x] = 0;
-            maxslots[(par ^ 1) * kMaxSlotSet + kMaxSlots + threadIdx.x] = 0;
+            clear_slots(maxslots + (par ^ 1) * kDtSet);
+            clear_slots(maxslots + (par ^ 1) * kDtSet + kSlotSet);
         }
     }
     if (blockIdx.x == 0) publish_ctrl(cur, next, dt, halt_status);
     return !halted && halt_status == 0;
 }
 
+// Whether whole_step of a particle looks at its original index: the wall that
+// disappears, wave-maker particles (4 bytes a particle that the others need
+// not read).
+__device__ __forceinline__ bool step_needs_oid(const StepParams& P, const Ctrl& c, int itype) {
+    return c.wall_disappear || (P.boundary_motion && c.piston_active && itype < 0);
+}
+
 // whole_step of every slot from X into A (in place on list steps), the cell
 // key for the next build, the step's largest displacement, and the records
 // of the next step's pair pass: near (the new position relative to the home
 // cell, the new velocity) and pred (PredictHalfStep.cpp:16-22 with this
-// step's dt, which is the next step's).
+// step's dt, which is the next step's).  The step's accelerations are in
+// A.ad already: the pair pass writes them there (its der), since what the
+// step reads of the last ones is in the records.  Bound by HBM traffic: 124
+// bytes a particle in FP32, 208 in FP64 (148 and 249 with A.ad written here
+// and every original index read).  The loads go before the wait for dt.
 template <class R>
-__global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ctrl* __restrict__ next,
-                                                                const Ctrl* __restrict__ cur, ListState<R> X,
-                                                                const real4<R>* __restrict__ der,
-                                                                const real2<R>* __restrict__ xs,
+__global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ctrl* next, const Ctrl* cur,
+                                                                ListState<R> X, const real2<R>* __restrict__ xs,
                                                                 ListRec<R>* __restrict__ rec,
                                                                 const uint32_t* __restrict__ home, StateA<R> A,
                                                                 uint32_t* __restrict__ key_next,
-                                                                unsigned long long* __restrict__ maxslots,
-                                                                unsigned long long* __restrict__ dslots) {
+                                                                unsigned long long* maxslots,
+                                                                unsigned long long* dslots) {
+    const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
+    const bool live = s0 < P.n;
+    const uint32_t s = live ? s0 : P.n - 1;
+    const real4<R> d = A.ad[s];
+    const real2<R> x = xs[s];
+    const double2 p0 = X.pos[s];
+    const real4<R> va = X.va[s];
+    const uint32_t h = home[s];
+    real4<R> pr{};
+    if (P.density_treatment == 0) pr.z = fabs(rec[s].pr.z);  // the summed density (sign-encoded)
     const Ctrl& c = *cur;
     double dt;
     if (!list_dt(P, next, cur, maxslots, dt)) return;
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t par = (uint32_t)(c.step & 1);
     uint32_t outside = 0, bad = 0;
-    double moved = 0.0;
-    if (s < P.n) {
-        const real4<R> d = der[s];
-        const real2<R> x = xs[s];
-        const double2 p0 = X.pos[s];
-        real4<R> pr{};
-        if (P.density_treatment == 0) {  // the summed density (sign-encoded)
-            pr = rec[s].pr;
-            pr.z = fabs(pr.z);
-        }
-        const uint32_t oid = X.oid[s];
-        const Stepped2<R> o = whole_step_one<R>(P, c, p0, X.va[s], pr, oid, d.x, d.y, d.z, x.x, x.y, dt, outside);
+    double moved2 = 0.0;
+    if (live) {
+        const bool reordered = A.oid != X.oid;
+        const uint32_t oid = reordered || step_needs_oid(P, c, (int)va.w) ? X.oid[s] : 0u;
+        const Stepped2<R> o = whole_step_one<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, x.x, x.y, dt, outside);
         A.pos[s] = o.pos;
         A.va[s] = o.va;
-        real4<R> nad;
-        nad.x = d.x;
-        nad.y = d.y;
-        nad.z = d.z;
-        nad.w = R(0);
-        A.ad[s] = nad;
-        if (A.oid != X.oid) A.oid[s] = oid;
-        const int it = (int)o.va.w;
-        key_next[s] = it == 0 ? P.ncells : cell_key(P, o.pos.x, o.pos.y, bad);
+        if (reordered) A.oid[s] = oid;
+        key_next[s] = (int)o.va.w == 0 ? P.ncells : cell_key(P, o.pos.x, o.pos.y, bad);
         const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y;
-        moved = sqrt(mx * mx + my * my);
+        moved2 = mx * mx + my * my;
         R p;
         ListRec<R> r;
         r.pr = predict_record<R>(P, o.va, d.x, d.y, d.z, (R)dt, p);
-        r.nr = near_record<R>(P, o.pos, o.va.x, o.va.y, home[s]);
+        r.nr = near_record<R>(P, o.pos, o.va.x, o.va.y, h);
         rec[s] = r;
     }
-    const uint32_t par = (uint32_t)(c.step & 1);
     wave_count_add(&next->outside_l[par], outside);
     if (bad) atomicOr(&next->grid_overflow, 1u);
-    block_max2_to_slots(moved, 0.0, dslots + par * kMaxSlots, blockIdx.x);
+    block_max_to_slots(moved2, 0.0, dslots + par * kSlotSet, nullptr, blockIdx.x);
 }
 
 }  // namespace rrsph

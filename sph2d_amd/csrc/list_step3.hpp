@@ -83,13 +83,8 @@ __global__ void __launch_bounds__(kBlock) reorder_list3_kernel(StepParams P, con
                                                                const uint32_t* __restrict__ perm, StateA3<R> A,
                                                                StateB3<R> B, ListRec<R>* __restrict__ rec,
                                                                real4<R>* __restrict__ dens, uint32_t* __restrict__ home,
-                                                               float4* __restrict__ cand, uint32_t* __restrict__ LB,
-                                                               unsigned long long* __restrict__ maxslots) {
+                                                               float4* __restrict__ cand, uint32_t* __restrict__ LB) {
     if (ctrl->halted) return;
-    if (blockIdx.x == 0) {
-        maxslots[threadIdx.x] = 0;
-        maxslots[kMaxSlots + threadIdx.x] = 0;
-    }
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
     const uint32_t s = live ? s0 : P.n - 1;
@@ -318,7 +313,7 @@ __device__ __forceinline__ void fill_cell_offsets3(const StepParams& P, float4* 
 // header): FP32 from the records, FP64 on the band; FP64 from the FP64
 // record positions.
 __device__ __forceinline__ bool list_cut3(const StepParams& P, const CutFP32& C, const float4* s_off, uint32_t e,
-                                          const float4& ni, const float4& nj, const double4& pj,
+                                          const float4& ni, const float4& nj, uint32_t s,
                                           const double4* __restrict__ pos, float& dx, float& dy, float& dz) {
     const float4 o = s_off[e >> kSlotBits3];
     dx = (ni.x - nj.x) + o.x;
@@ -326,7 +321,7 @@ __device__ __forceinline__ bool list_cut3(const StepParams& P, const CutFP32& C,
     dz = (ni.z - nj.z) + o.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
     if (!(d2 > C.lo && d2 < C.hi)) return d2 <= C.lo;  // on the band's edge: within a rounding of lo < cut2
-    const double4 q = pos[e & kSlotMask3];  // rare: the band around the cut-off
+    const double4 q = pos[e & kSlotMask3], pj = pos[s];  // rare: the band around the cut-off
     const double ddx = __dsub_rn(q.x, pj.x), ddy = __dsub_rn(q.y, pj.y), ddz = __dsub_rn(q.z, pj.z);
     dx = (float)ddx;
     dy = (float)ddy;
@@ -334,7 +329,7 @@ __device__ __forceinline__ bool list_cut3(const StepParams& P, const CutFP32& C,
     return dist2_exact3(ddx, ddy, ddz) < P.cut2;
 }
 __device__ __forceinline__ bool list_cut3(const StepParams& P, const CutFP32&, const float4*, uint32_t,
-                                          const double4& ni, const double4& nj, const double4&,
+                                          const double4& ni, const double4& nj, uint32_t,
                                           const double4* __restrict__, double& dx, double& dy, double& dz) {
     dx = __dsub_rn(ni.x, nj.x);
     dy = __dsub_rn(ni.y, nj.y);
@@ -350,7 +345,7 @@ __device__ __forceinline__ bool list_cut3(const StepParams& P, const CutFP32&, c
 template <uint32_t kChunk, class F>
 __device__ __forceinline__ void collect_near3(const StepParams& P, bool active, uint32_t cap, uint32_t s,
                                               const float4* s_off, const float4& nk, const float4* __restrict__ nearf,
-                                              const double4& pj, const double4* __restrict__ pos,
+                                              const double4* __restrict__ pos,
                                               const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc,
                                               uint32_t* __restrict__ hits, bool& overflow, F&& flush) {
     static_assert(kChunk >= 2 * kCollectL3, "hit list too short");
@@ -370,7 +365,7 @@ __device__ __forceinline__ void collect_near3(const StepParams& P, bool active, 
 #pragma unroll
         for (uint32_t u = 0; u < kCollectL3; ++u) {
             float dx, dy, dz;
-            const bool in = list_cut3(P, C, s_off, e[u], q[u], nk, pj, pos, dx, dy, dz);
+            const bool in = list_cut3(P, C, s_off, e[u], q[u], nk, s, pos, dx, dy, dz);
             const bool hit = (k + u < cnt) & (q[u].w != 0.f) & in;
             if (hit) {
                 if (done + nh < cap) {
@@ -410,8 +405,8 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     } else {
         if (!list_step_goes(cur)) return;
         step = cur->step;
-        __syncthreads();
     }
+    __syncthreads();  // the offset table
     const uint32_t s = lb * kBlock + threadIdx.x;
     if (s >= P.n) return;
     const R m = (R)P.mass, inv_h = (R)(1.0 / P.h), w_q1 = (R)P.f_cubic, w_q2 = (R)(P.f_cubic / 6.0);
@@ -424,7 +419,6 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     const uint32_t cnt = dj.w != R(0) ? nbc[s] : 0u;
     if (cnt) {
         const CutFP32 C = cut_band(P);
-        const double4 pj = X.pos[s];
         const uint32_t cap = P.max_nbr - 1;
         const uint32_t row = P.n * 4u;
         uint32_t hits = 0;
@@ -433,10 +427,11 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
         // the sums run in list order.  Rows past a list's end name valid
         // slots (padding, or entries of an earlier build); the loads past
         // the last allocated row read that row instead.
-        // 6.6M dam break: FP32 1.13 ms per pass at G = 8 (1.45 at G = 4),
-        // FP64 2.06 ms at G = 4 with incremental offsets (2.21 clamped)
+        // FP32, 2,899,370 particles: 466 us per pass at G = 12 (492 at 8, 538
+        // at 4); FP64, 6.6M: 2.06 ms at G = 4 with incremental offsets (2.21
+        // clamped)
         constexpr bool kWide = sizeof(R) == 4;
-        constexpr uint32_t G = kWide ? 8 : 4;
+        constexpr uint32_t G = kWide ? 12 : 4;
         static_assert(kWide || 2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
         const uint32_t last = P.list_cap + kListPad - 1;
         auto entry = [&](uint32_t k) {
@@ -457,7 +452,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
             for (uint32_t u = 0; u < G; ++u) {
                 R dx, dy, dz;
                 const bool hit =
-                    list_cut3(P, C, s_off, e[u], di[u], dj, pj, X.pos, dx, dy, dz) & (di[u].w != R(0)) & (k + u < cnt);
+                    list_cut3(P, C, s_off, e[u], di[u], dj, s, X.pos, dx, dy, dz) & (di[u].w != R(0)) & (k + u < cnt);
                 const bool take = hit & (hits < cap);
                 overflow |= hit & !take;
                 hits += take ? 1u : 0u;
@@ -488,56 +483,32 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     pres[s] = p;
 }
 
-// fast_pair_term3 (the cubic configuration) for one list entry, without
-// branches except the rare Lennard-Jones case; nothing is added when take
-// is false.  i's records: nr (position half, p / rho^2), pr (v^, s rho^),
-// vai (its current velocity; continuity only).
-template <class R>
-__device__ __forceinline__ void list_pair_term3(const FastPair<R>& K, R (&S)[12], bool take, R dx, R dy, R dz,
+// One entry in 3D (list_pair).  i's records: nr (position half, p / rho^2),
+// pr (v^, s rho^), vai (its current velocity; continuity only).
+template <class R> struct ListSums3 {
+    R sx = 0, sy = 0, sz = 0, sd = 0, xx = 0, xy = 0, xz = 0, xmin = 0, ljx = 0, ljy = 0, ljz = 0;
+};
+template <class R, class K_>
+__device__ __forceinline__ void list_pair_term3(const K_& K, ListSums3<R>& S, bool take, R dx, R dy, R dz,
                                                 const real4<R>& nri, const real4<R>& pri, const real4<R>& vai,
-                                                const real4<R>& vaj, const real4<R>& prj, R pwj, int tj) {
-    // S: sx, sy, sz, sd, xx, xy, xz, amu, ljx, ljy, ljz, (unused)
+                                                const real4<R>& vaj, const real4<R>& prj, R pwj) {
     const R d2 = dx * dx + dy * dy + dz * dz;
-    const R rinv = d2 > R(0) ? fast_rsqrt<R>(d2) : R(0);
-    const R dist = d2 * rinv;
-    const R q = dist * K.inv_h;
-    const R t = R(2) - q;
-    const R t2 = t * t;
-    const bool inner = q <= R(1);
-    const R F1 = K.c_q1 * (R(1.5) * q - R(2));
-    const R F2 = -K.c_q2 * t2 * rinv;
-    const R W1 = K.w_q1 * (R(2) / R(3) - q * q + R(0.5) * q * q * q);
-    const R W2 = K.w_q2 * t2 * t;
-    const R F = take ? (inner ? F1 : F2) : R(0);
-    const R W = inner ? W1 : W2;
-    if (K.cont) S[3] += F * ((vai.x - vaj.x) * dx + (vai.y - vaj.y) * dy + (vai.z - vaj.z) * dz);
-    if (K.lj_on && take && tj > 0 && pri.w < R(0) && dist < K.lj_r0) {
-        const R rn = K.lj_r0 * rinv;
-        const R rn2 = rn * rn, rn4 = rn2 * rn2;
-        const R f = K.lj_D * (rn4 * rn4 * rn4 - rn4) * (rinv * rinv);
-        S[8] -= dx * f;
-        S[9] -= dy * f;
-        S[10] -= dz * f;
-    }
-    const R inv_rs = fast_rcp<R>(fabs(pri.w) + fabs(prj.w));
-    R coef = nri.w + pwj;
     const R dvx = pri.x - prj.x, dvy = pri.y - prj.y, dvz = pri.z - prj.z;
-    if (K.av_on) {
-        const R vr = dvx * dx + dvy * dy + dvz * dz;
-        const R mu = K.h * vr * fast_rcp<R>(d2 + K.eta2);
-        const bool app = take & (vr < R(0));
-        S[7] = app ? fmax(S[7], -mu) : S[7];
-        coef += app ? (K.beta * mu - K.alpha_c) * mu * R(2) * inv_rs : R(0);
-    }
-    const R fc = F * coef;
-    S[0] += fc * dx;
-    S[1] += fc * dy;
-    S[2] += fc * dz;
-    if (K.xsph_on) {
-        const R cw = (take & (pri.w > R(0))) ? W * inv_rs : R(0);
-        S[4] += dvx * cw;
-        S[5] += dvy * cw;
-        S[6] += dvz * cw;
+    const ListTerm<R> T =
+        list_pair<R>(K, take, d2, dvx * dx + dvy * dy + dvz * dz, pri.w, prj.w, nri.w + pwj, S.xmin);
+    if (K.cont) S.sd += T.F * ((vai.x - vaj.x) * dx + (vai.y - vaj.y) * dy + (vai.z - vaj.z) * dz);
+    const R fc = T.F * T.coef;
+    S.sx += fc * dx;
+    S.sy += fc * dy;
+    S.sz += fc * dz;
+    S.xx += dvx * T.w;
+    S.xy += dvy * T.w;
+    S.xz += dvz * T.w;
+    if (T.wall) {
+        const R f = list_wall<R>(K, d2, T.rinv);
+        S.ljx -= dx * f;
+        S.ljy -= dy * f;
+        S.ljz -= dz * f;
     }
 }
 
@@ -545,8 +516,8 @@ __device__ __forceinline__ void list_pair_term3(const FastPair<R>& K, R (&S)[12]
 // (continuity, pressure, artificial viscosity, Lennard-Jones walls, XSPH),
 // the dt maxima and the fields for the integrator.  Entries in groups of
 // G, as for_each_listed.
-template <class R, bool FIRST>
-__global__ void __launch_bounds__(kBlock) pair_list3_kernel(
+template <class R, bool FIRST, bool CONT, bool ALL>
+__global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState3<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
     real4<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
@@ -561,31 +532,31 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
         if (!list_step_goes(cur)) return;
         if (list_build_overflowed(next, cur)) return;
         step = cur->step;
-        __syncthreads();
     }
-    maxslots += (uint32_t)(step & 1) * kMaxSlotSet;
+    __syncthreads();  // the offset table
+    maxslots += (uint32_t)(step & 1) * kDtSet;
     const uint32_t s = lb * kBlock + threadIdx.x;
     const bool live = s < P.n;
-    const FastPair<R> K(P);
-    R S[12] = {};
+    const ListPair<R, CONT, ALL> K(P);
+    ListSums3<R> S;
     bool overflow = false;
-    double4 pj = make_double4(0, 0, 0, 0);
     real4<R> vaj{};
     ListRec<R> rj{};
     if (live) {
-        pj = X.pos[s];
         vaj = X.va[s];
         rj = rec[s];
     }
-    const int tj = (int)pj.w;
-    const uint32_t cnt = live && tj != 0 ? nbc[s] : 0u;
+    const uint32_t cnt = rj.pr.w != R(0) ? nbc[s] : 0u;  // 0: died since the build
     const uint32_t cap = P.max_nbr - 1;
     if (cnt) {
-        // FP32 6.6M dam break: 1.87 ms per pass at G = 8 (168 VGPRs, 3 waves
-        // per SIMD), 2.00 at 4, 2.39 at 2.  Rows past a list's end name
+        // entries in flight per lane at 3 waves per SIMD.  FP32, summation,
+        // 2,899,370 particles: 706 us per pass at G = 6, 724 at 8, 793 at 4;
+        // FP64, 555,686 particles: 310 at 4, 340 at 2 and 3; FP64,
+        // continuity, 943,906 particles (which gathers the velocity too): 635
+        // at 3, 669 at 2, 1032 at 4 (spills).  Rows past a list's end name
         // valid slots (padding, or entries of an earlier build); the loads
         // past the last allocated row read that row instead.
-        constexpr uint32_t G = sizeof(R) == 4 ? 8 : 2;
+        constexpr uint32_t G = sizeof(R) == 4 ? 6 : (CONT ? 3 : 4);
         const uint32_t lastrow = P.list_cap + kListPad - 1;
         const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
         const CutFP32 C = cut_band(P);
@@ -610,7 +581,7 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) {
                 R dx, dy, dz;
-                const bool in = list_cut3(P, C, s_off, e[u], r[u].nr, rj.nr, pj, X.pos, dx, dy, dz);
+                const bool in = list_cut3(P, C, s_off, e[u], r[u].nr, rj.nr, s, X.pos, dx, dy, dz);
                 const bool hit = in & (r[u].pr.w != R(0)) & (k + u < cnt);
                 bool take = hit;
                 if (capped) {
@@ -618,7 +589,7 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
                     over |= hit & !take;
                     hits += take ? 1u : 0u;
                 }
-                list_pair_term3<R>(K, S, take, dx, dy, dz, r[u].nr, r[u].pr, va[u], vaj, rj.pr, rj.nr.w, tj);
+                list_pair_term3<R>(K, S, take, dx, dy, dz, r[u].nr, r[u].pr, va[u], vaj, rj.pr, rj.nr.w);
             }
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
@@ -626,15 +597,14 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
         overflow |= over;
     }
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
-    const R m = (R)P.mass;
-    const R ax = S[8] + m * S[0];
-    const R ay = -(R)P.g + S[9] + m * S[1];
-    const R az = S[10] + m * S[2];
-    const R drho = m * S[3];
-    const R xf = m * R(2) * (R)P.xsph_eps;
-    if (P.dt_method == 2 && P.dt_dynamic_mode == 1)
-        block_max2_to_slots(live ? sqrt((double)ax * ax + (double)ay * ay + (double)az * az) : 0.0,
-                            live ? (double)S[7] : 0.0, maxslots, lb);
+    const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);
+    const R ax = S.ljx + mF * S.sx;
+    const R ay = -(R)P.g + S.ljy + mF * S.sy;
+    const R az = S.ljz + mF * S.sz;
+    const R drho = mF * S.sd;
+    const R amu = (R)P.h * -S.xmin;
+    list_dt_maxima<R>(P, live ? (double)ax * ax + (double)ay * ay + (double)az * az : 0.0, live ? amu : R(0), maxslots,
+                      lb);
     if (live) {
         real4<R> d;
         d.x = ax;
@@ -643,10 +613,10 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
         d.w = drho;
         der[s] = d;
         real4<R> x;
-        x.x = xf * S[4];
-        x.y = xf * S[5];
-        x.z = xf * S[6];
-        x.w = S[7];
+        x.x = mW * S.xx;
+        x.y = mW * S.xy;
+        x.z = mW * S.xz;
+        x.w = amu;
         xs[s] = x;
         if (P.density_treatment != 0) pres[s] = eos_p<R>(vaj.w, (R)P.rho0, (R)P.eos_B);
     }
@@ -654,47 +624,55 @@ __global__ void __launch_bounds__(kBlock) pair_list3_kernel(
 
 // whole_step of every slot from X into A (in place on list steps), the
 // cell key for the next build, the step's largest displacement, and the
-// next step's records.
+// next step's records (dens only where the summation pass reads it); the
+// accelerations are in A.ad already, as in integrate_list_kernel.
 template <class R>
-__global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, Ctrl* __restrict__ next,
-                                                                 const Ctrl* __restrict__ cur,
-                                                                 ListState3<R> X, const real4<R>* __restrict__ der,
-                                                                 const real4<R>* __restrict__ xs,
+__global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, Ctrl* next, const Ctrl* cur,
+                                                                 ListState3<R> X, const real4<R>* __restrict__ xs,
                                                                  ListRec<R>* __restrict__ rec,
                                                                  real4<R>* __restrict__ dens,
                                                                  const uint32_t* __restrict__ home, StateA3<R> A,
                                                                  uint32_t* __restrict__ key_next,
-                                                                 unsigned long long* __restrict__ maxslots,
-                                                                 unsigned long long* __restrict__ dslots) {
+                                                                 unsigned long long* maxslots,
+                                                                 unsigned long long* dslots) {
+    const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
+    const bool live = s0 < P.n;
+    const uint32_t s = live ? s0 : P.n - 1;
+    const real4<R> d = A.ad[s];
+    const real4<R> x = xs[s];
+    const double4 p0 = X.pos[s];
+    const real4<R> va = X.va[s];
+    const uint32_t h = home[s];
+    real4<R> pr{};
+    if (P.density_treatment == 0) pr.w = fabs(rec[s].pr.w);  // the summed density
     const Ctrl& c = *cur;
     double dt;
     if (!list_dt(P, next, cur, maxslots, dt)) return;
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    uint32_t outside = 0, bad = 0, changed = 0;
-    double moved = 0.0;
-    if (s < P.n) {
-        const real4<R> d = der[s];
-        const real4<R> x = xs[s];
-        const double4 p0 = X.pos[s];
-        real4<R> pr{};
-        if (P.density_treatment == 0) pr.w = fabs(rec[s].pr.w);  // the summed density
-        const uint32_t h = home[s];
-        const Stepped3<R> o = integrate_one3<R>(P, c, s, p0, X.va[s], pr, X.oid[s], d.x, d.y, d.z, d.w, x.x, x.y,
-                                                x.z, dt, A, key_next, h, outside, bad, changed);
-        const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y, mz = o.pos.z - p0.z;
-        moved = sqrt(mx * mx + my * my + mz * mz);
+    const uint32_t par = (uint32_t)(c.step & 1);
+    uint32_t outside = 0, bad = 0;
+    double moved2 = 0.0;
+    if (live) {
+        const bool reordered = A.oid != X.oid;
+        const uint32_t oid = reordered || step_needs_oid(P, c, (int)p0.w) ? X.oid[s] : 0u;
+        const Stepped3<R> o =
+            whole_step_one3<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, d.w, x.x, x.y, x.z, dt, outside);
+        A.pos[s] = o.pos;
+        A.va[s] = o.va;
+        if (reordered) A.oid[s] = oid;
         const int itype = (int)o.pos.w;
+        key_next[s] = itype == 0 ? P.ncells : cell_key3(P, o.pos.x, o.pos.y, o.pos.z, bad);
+        const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y, mz = o.pos.z - p0.z;
+        moved2 = mx * mx + my * my + mz * mz;
         R pw, p;
         ListRec<R> r;
         r.pr = predict3<R>(P, o.va, itype, d, (R)dt, pw, p);
         r.nr = near3<R>(P, o.pos, pw, h);
         rec[s] = r;
-        dens[s] = near3<R>(P, o.pos, typed_rho<R>(o.va.w, itype), h);
+        if (P.density_treatment == 0) dens[s] = near3<R>(P, o.pos, typed_rho<R>(o.va.w, itype), h);
     }
-    const uint32_t par = (uint32_t)(c.step & 1);
     wave_count_add(&next->outside_l[par], outside);
     if (bad) atomicOr(&next->grid_overflow, 1u);
-    block_max2_to_slots(moved, 0.0, dslots + par * kMaxSlots, blockIdx.x);
+    block_max_to_slots(moved2, 0.0, dslots + par * kSlotSet, nullptr, blockIdx.x);
 }
 
 }  // namespace rrsph

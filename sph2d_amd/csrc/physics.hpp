@@ -36,7 +36,7 @@ template <class R>
 __device__ __forceinline__ KernelConsts<R> kernel_consts(const StepParams& P) {
     KernelConsts<R> K;
     K.h = (R)P.h;
-    K.inv_h = (R)(1.0 / P.h);
+    K.inv_h = (R)P.inv_h;
     K.f_cubic = (R)P.f_cubic;
     K.f_gauss = (R)P.f_gauss;
     K.f_wend = (R)P.f_wend;

@@ -177,7 +177,8 @@ struct rrsph_ctx {
     bool use_graph = true;
     bool uploaded = false;
     bool stepped = false;
-    bool fields_valid = false;  // der / xs hold the last step's fields in A's slot order
+    bool fields_valid = false;  // der (list steps: adA) / xs hold the last step's fields in A's slot order
+    bool list_fields = false;   // the last step was a list or build step
     uint32_t passes = 0;
     uint32_t ntiles = 0;
     // buffers
@@ -233,12 +234,15 @@ struct rrsph_ctx {
     // list_interval steps (host schedule, adapted to the measured
     // displacement rate); the device halts a step whose lists may be stale
     bool list_mode = false;
+    bool all_terms = false;             // artificial viscosity, XSPH and the wall force are all on
+    int lanes = 1;                      // lanes per particle of the 2D list passes
     bool list_suspended = false;        // the adjoint's tapes and replays run without lists
     uint32_t *nbl = nullptr, *nbc = nullptr;
     void* rec = nullptr;                // records of the list pass (ListRec per slot)
     void* dens = nullptr;               // 3D: records of the summation density pass (real4 per slot)
     uint32_t* home = nullptr;           // each slot's cell at the last build
-    unsigned long long* dslots = nullptr;  // per-step largest displacement (block maxima)
+    unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima, a set per step parity)
+    unsigned long long* dtslots = nullptr; // list steps: dt maxima (likewise)
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
     hipGraph_t graph_list = nullptr, graph_build = nullptr;
     hipGraphExec_t gexec_list = nullptr, gexec_build = nullptr;
@@ -451,6 +455,39 @@ template <class R> void enqueue_step3_t(rrsph_ctx* c, Profiler* prof, bool full_
     }
 }
 
+// The summation and pair passes of a 2D neighbour-list step, LPP lanes per particle.
+template <class R, int LPP, bool ALL> void enqueue_list_passes(rrsph_ctx* c, Launcher& L, const ListState<R>& X, bool build) {
+    const StepParams& P = c->P;
+    const uint32_t nb = group_blocks_per_xcd<LPP>(P.n) * kNumXcd;
+    ListRec<R>* rec = (ListRec<R>*)c->rec;
+    bool first = !build;
+    if (P.density_treatment == 0) {
+        auto density = [&](auto kernel) {
+            L(K_DENSITY_SUM, [&] {
+                kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                     c->dslots);
+            });
+        };
+        if (first) density(density_sum_list<R, true, LPP>);
+        else density(density_sum_list<R, false, LPP>);
+        first = false;
+    }
+    auto pair = [&](auto kernel) {
+        L(K_PAIR, [&] {
+            kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                 (real4<R>*)c->adA, (real2<R>*)c->xs, c->dtslots, c->dslots);
+        });
+    };
+    if (c->fast_pair) {
+        if (P.density_treatment == 0) pair(pair_list_kernel<R, false, LPP, false, ALL>);
+        else if (first) pair(pair_list_kernel<R, true, LPP, true, ALL>);
+        else pair(pair_list_kernel<R, false, LPP, true, ALL>);
+    } else {
+        if (first) pair(pair_list_general_kernel<R, true, LPP>);
+        else pair(pair_list_general_kernel<R, false, LPP>);
+    }
+}
+
 // One neighbour-list step (build: sort, reorder and new lists first).
 template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool build) {
     Launcher L{c, prof};
@@ -461,14 +498,14 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool b
     ListRec<R>* rec = (ListRec<R>*)c->rec;
     if (build) {
         L(K_PROLOGUE, [&] {
-            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->maxslots);
+            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
         });
         enqueue_sort(c, c->ctrl_cur, L);
         StateA<R> A = stateA<R>(c);
         StateB<R> B = stateB<R>(c, c->pred, c->pres);
         L(K_REORDER, [&] {
             reorder_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
-                                                                 rec, c->home, c->LB, c->maxslots);
+                                                                 rec, c->home, c->LB);
         });
         L(K_LIST_BUILD, [&] {
             list_build_kernel<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->posB, (const real4<R>*)c->vaB,
@@ -477,35 +514,13 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool b
         X = ListState<R>{c->posB, (const real4<R>*)c->vaB, c->oidB};
     }
     // the first kernel of a list step makes its prologue
-    bool first = !build;
-    if (P.density_treatment == 0) {
-        auto density = [&](auto kernel) {
-            L(K_DENSITY_SUM, [&] {
-                kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                         c->dslots);
-            });
-        };
-        if (first) density(density_sum_list<R, true>);
-        else density(density_sum_list<R, false>);
-        first = false;
-    }
-    auto pair = [&](auto kernel) {
-        L(K_PAIR, [&] {
-            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     (real4<R>*)c->der, (real2<R>*)c->xs, c->maxslots, c->dslots);
-        });
-    };
-    if (c->fast_pair) {
-        if (first) pair(pair_list_kernel<R, true>);
-        else pair(pair_list_kernel<R, false>);
-    } else {
-        if (first) pair(pair_list_general_kernel<R, true>);
-        else pair(pair_list_general_kernel<R, false>);
-    }
+    if (!c->all_terms && c->fast_pair) enqueue_list_passes<R, 1, false>(c, L, X, build);
+    else if (c->lanes == 8) enqueue_list_passes<R, 8, true>(c, L, X, build);
+    else if (c->lanes == 2) enqueue_list_passes<R, 2, true>(c, L, X, build);
+    else enqueue_list_passes<R, 1, true>(c, L, X, build);
     L(K_INTEGRATE, [&] {
-        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real4<R>*)c->der,
-                                                               (const real2<R>*)c->xs, rec, c->home, stateA<R>(c),
-                                                               c->key_next, c->maxslots, c->dslots);
+        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real2<R>*)c->xs, rec, c->home, stateA<R>(c),
+                                                               c->key_next, c->dtslots, c->dslots);
     });
 }
 
@@ -520,14 +535,14 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     real4<R>* dens = (real4<R>*)c->dens;
     if (build) {
         L(K_PROLOGUE, [&] {
-            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->maxslots);
+            list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
         });
         enqueue_sort(c, c->ctrl_cur, L);
         StateA3<R> A = stateA3<R>(c);
         StateB3<R> B = stateB3<R>(c, c->pred, c->pw, c->pres);
         L(K_REORDER, [&] {
             reorder_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
-                                                                  rec, dens, c->home, c->cand, c->LB, c->maxslots);
+                                                                  rec, dens, c->home, c->cand, c->LB);
         });
         L(K_LIST_BUILD, [&] {
             list_build3_kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, (const double4*)c->posB, c->cand,
@@ -550,15 +565,24 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
             kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     (real4<R>*)c->der, (real4<R>*)c->xs, c->maxslots, c->dslots);
+                                                     (real4<R>*)c->adA, (real4<R>*)c->xs, c->dtslots, c->dslots);
         });
     };
-    if (first) pair(pair_list3_kernel<R, true>);
-    else pair(pair_list3_kernel<R, false>);
+    auto choose = [&](auto summed, auto first_kernel, auto kernel) {
+        if (P.density_treatment == 0) pair(summed);
+        else if (first) pair(first_kernel);
+        else pair(kernel);
+    };
+    if (c->all_terms)
+        choose(pair_list3_kernel<R, false, false, true>, pair_list3_kernel<R, true, true, true>,
+               pair_list3_kernel<R, false, true, true>);
+    else
+        choose(pair_list3_kernel<R, false, false, false>, pair_list3_kernel<R, true, true, false>,
+               pair_list3_kernel<R, false, true, false>);
     L(K_INTEGRATE, [&] {
-        integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real4<R>*)c->der,
+        integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X,
                                                                 (const real4<R>*)c->xs, rec, dens, c->home,
-                                                                stateA3<R>(c), c->key_next, c->maxslots, c->dslots);
+                                                                stateA3<R>(c), c->key_next, c->dtslots, c->dslots);
     });
 }
 
@@ -804,6 +828,14 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     P.f_gauss = d3 ? 1 / (pi * std::sqrt(pi) * (h * h * h)) : 1 / (pi * (h * h));
     P.f_wend = d3 ? 21 / (16 * pi * (h * h * h)) : 7 / (4 * pi * (h * h));
     P.f_desb = d3 ? 15 / (pi * (4 * h) * (4 * h) * (4 * h)) : 5 / (16 * pi * (h * h));
+    P.inv_h = 1.0 / h;
+    P.c_q1 = P.f_cubic / (h * h);
+    P.c_q2 = 0.5 * P.f_cubic / h;
+    P.w_q2 = P.f_cubic / 6.0;
+    P.lp_a2 = 2.0 * h * (p.artificial_shear_visc * p.eos_sound_vel);
+    P.lp_b2 = 2.0 * h * h * p.artificial_bulk_visc;
+    P.lp_mF = -2.0 * P.f_cubic / h * p.mass;
+    P.lp_mW = 2.0 * p.average_velocity_coef * p.mass * (4.0 / 3.0 * P.f_cubic);
     P.skf_density = p.density_skf;
     P.skf_intf = p.intf_skf;
     P.skf_av = p.artificial_viscosity_skf;
@@ -928,6 +960,17 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     if (const char* e = std::getenv("RRSPH_HIP_LIST_SKIN")) skin_frac = std::strtod(e, nullptr);
     ctx->list_mode = (ctx->fast_pair || !d3) && skin_frac > 0.0 && skin_frac < 0.9 && P.n <= (d3 ? kSlotMask3 : kSlotMask);
     if (const char* e = std::getenv("RRSPH_HIP_LIST")) ctx->list_mode = ctx->list_mode && std::strcmp(e, "0") != 0;
+    ctx->all_terms = P.av_on && P.xsph_on && P.lj_on;
+    // lanes per particle of the 2D list passes (LaneGroup), from event-timed
+    // passes with 1, 2 and 8 lanes: 8 below 25,000 particles, where the chip
+    // is not filled (continuity, 6,432 particles FP64 14.2 / 11.8 / 10.1 us,
+    // 22,662 14.9 / 12.6 / 12.3, 54,200 15.6 / 15.3 / 18.7); 2 above (1,020,263
+    // FP64 142.9 / 126.6 / 221.2; summation density 519,203 FP64 56.7 / 45.5 /
+    // 66.9; general pair pass 188,656 FP64 55.8 / 46.4 / 75.3), but for the
+    // FP32 continuity pass, which has the least to do per entry, at large n
+    // (188,656 particles 18.3 / 20.8 / 31.4, 1,020,263 62.5 / 64.5 / 146.7)
+    ctx->lanes = P.n < 25000 ? 8 : 2;
+    if (P.n >= 150000 && ctx->fast_pair && ctx->fp32 && P.density_treatment != 0) ctx->lanes = 1;
     P.list_reach = P.cell * (1.0 + skin_frac);
     P.list_r2 = P.list_reach * P.list_reach * (1.0 + 1e-12);
     P.skin_half = 0.5 * P.cell * skin_frac * (1.0 - 1e-9);
@@ -984,7 +1027,7 @@ void free_all(rrsph_ctx* c) {
                     c->maxslots, c->LB, c->ctrl, c->ctrl_cur,
                     c->util_ctrl, c->red, c->st_r, c->st_v, c->st_rho, c->st_p, c->st_a, c->st_drho, c->st_av,
                     c->st_mu, c->st_itype, c->st_u32, c->skeyA, c->chg, c->chg_mask, c->wpre, c->pw,
-                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->cand};
+                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->dtslots, c->cand};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
@@ -1102,8 +1145,7 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
     ctx->vbuf[1] = dalloc<uint32_t>(n, e);
     ctx->hist = dalloc<uint32_t>((size_t)kRadix * ctx->ntiles, e);
     ctx->digit_total = dalloc<uint32_t>(kRadix, e);
-    // the dt slots, the utility sorts' (cleared, not read), the list steps' second set
-    ctx->maxslots = dalloc<unsigned long long>(kMaxSlotSet + 2 * kMaxSlots, e);
+    ctx->maxslots = dalloc<unsigned long long>(4 * kMaxSlots, e);  // second half: utility sorts
     ctx->LB = dalloc<uint32_t>((size_t)ctx->P.ncells + 2, e);
     ctx->ctrl = dalloc<Ctrl>(1, e);
     ctx->ctrl_cur = dalloc<Ctrl>(1, e);
@@ -1121,10 +1163,11 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
         if (dim == 3) ctx->dens = dalloc<double4>(n, e);
         if (dim == 3) ctx->cand = dalloc<float4>(n, e);
         ctx->home = dalloc<uint32_t>(n, e);
-        ctx->dslots = dalloc<unsigned long long>(2 * kMaxSlots, e);
+        ctx->dslots = dalloc<unsigned long long>(2 * kSlotSet, e);
+        ctx->dtslots = dalloc<unsigned long long>(2 * kDtSet, e);
     }
     if (e != hipSuccess) return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-    if (ctx->dslots) HIP_TRY(hipMemset(ctx->dslots, 0, 2 * kMaxSlots * sizeof(unsigned long long)));
+    if (ctx->dslots) HIP_TRY(hipMemset(ctx->dslots, 0, 2 * kSlotSet * sizeof(unsigned long long)));
     if (ctx->nbl) HIP_TRY(hipMemset(ctx->nbl, 0, (size_t)(ctx->P.list_cap + kListPad) * n * sizeof(uint32_t)));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_ctrl, sizeof(Ctrl), hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_eta, kMaxGauges * sizeof(double), hipHostMallocDefault));
@@ -1248,6 +1291,7 @@ static rrsph_status launch_steps(rrsph_ctx* ctx, uint32_t nsteps) {
         if (nsteps) {
             ctx->stepped = true;
             ctx->fields_valid = true;
+            ctx->list_fields = true;
         }
         return RRSPH_OK;
     }
@@ -1267,6 +1311,7 @@ static rrsph_status launch_steps(rrsph_ctx* ctx, uint32_t nsteps) {
     if (nsteps) {
         ctx->stepped = true;
         ctx->fields_valid = true;
+        ctx->list_fields = false;
     }
     return RRSPH_OK;
 }
@@ -1298,6 +1343,7 @@ static rrsph_status launch_list_step(rrsph_ctx* ctx, bool build, uint64_t abs_st
     ctx->need_full = false;
     ctx->stepped = true;
     ctx->fields_valid = true;
+    ctx->list_fields = true;
     return RRSPH_OK;
 }
 
@@ -1500,20 +1546,21 @@ rrsph_status rrsph_hip_fields(rrsph_ctx* ctx, double* a, double* drho, double* a
         return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: enable rrsph_hip_set_export_fields before stepping");
     const size_t n = ctx->P.n, dim = ctx->P.dim;
     const uint32_t nb = grid_blocks(ctx->P.n, kBlock);
+    const void* der = ctx->list_fields ? ctx->adA : ctx->der;
     if (dim == 3 && ctx->fp32)
-        fields3_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const float4*)ctx->der,
+        fields3_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const float4*)der,
                                                               (const float4*)ctx->xs, ctx->st_a, ctx->st_drho,
                                                               ctx->st_av, ctx->st_mu);
     else if (dim == 3)
-        fields3_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const double4*)ctx->der,
+        fields3_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const double4*)der,
                                                                (const double4*)ctx->xs, ctx->st_a, ctx->st_drho,
                                                                ctx->st_av, ctx->st_mu);
     else if (ctx->fp32)
-        fields_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const float4*)ctx->der,
+        fields_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const float4*)der,
                                                              (const float4*)ctx->xs, ctx->st_a, ctx->st_drho,
                                                              ctx->st_av, ctx->st_mu);
     else
-        fields_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const double4*)ctx->der,
+        fields_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->oidA, (const double4*)der,
                                                               (const double4*)ctx->xs, ctx->st_a, ctx->st_drho,
                                                               ctx->st_av, ctx->st_mu);
     HIP_TRY(hipGetLastError());
@@ -1746,6 +1793,7 @@ rrsph_status rrsph_hip_profile_steps(rrsph_ctx* ctx, uint32_t nsteps, double* av
     if (nsteps) {
         ctx->stepped = true;
         ctx->fields_valid = true;
+        ctx->list_fields = list_active(ctx);
     }
     std::vector<double> sum(K_NUM_CLASSES, 0.0);
     std::vector<uint32_t> cnt(K_NUM_CLASSES, 0);
@@ -1958,6 +2006,7 @@ static rrsph_status launch_taped_step(rrsph_ctx* ctx, uint64_t base, bool& launc
     ctx->need_full = false;
     ctx->stepped = true;
     ctx->fields_valid = true;
+    ctx->list_fields = false;
     launched = true;
     return RRSPH_OK;
 }

@@ -260,11 +260,9 @@ template <class R> struct Stepped3 {
     real4<R> va;
 };
 template <class R>
-__device__ __forceinline__ Stepped3<R> integrate_one3(const StepParams& P, const Ctrl& c, uint32_t s, double4 pos,
-                                               real4<R> va, const real4<R>& pred, uint32_t oid, R ax, R ay, R az,
-                                               R drho, R avx, R avy, R avz, double dt, StateA3<R> A,
-                                               uint32_t* __restrict__ key_next, uint32_t key_old, uint32_t& outside,
-                                               uint32_t& bad, uint32_t& changed) {
+__device__ __forceinline__ Stepped3<R> whole_step_one3(const StepParams& P, const Ctrl& c, double4 pos, real4<R> va,
+                                                       const real4<R>& pred, uint32_t oid, R ax, R ay, R az, R drho,
+                                                       R avx, R avy, R avz, double dt, uint32_t& outside) {
     const double vdt_d = c.cur_first ? dt * 0.5 : dt;
     const R vdt = (R)vdt_d;
     int itype = (int)pos.w;
@@ -309,13 +307,25 @@ __device__ __forceinline__ Stepped3<R> integrate_one3(const StepParams& P, const
         pos.x < P.xmax && pos.x > P.xmin && pos.y < P.ymax && pos.y > P.ymin && pos.z < P.zmax && pos.z > P.zmin;
     if (!inside) outside += 1;
     pos.w = (double)itype;
-    A.pos[s] = pos;
     real4<R> nva;
     nva.x = vx;
     nva.y = vy;
     nva.z = vz;
     nva.w = rho;
-    A.va[s] = nva;
+    return Stepped3<R>{pos, nva};
+}
+
+// whole_step of slot s into state A, and the slot's key for the next sort.
+template <class R>
+__device__ __forceinline__ void integrate_one3(const StepParams& P, const Ctrl& c, uint32_t s, double4 pos,
+                                               real4<R> va, const real4<R>& pred, uint32_t oid, R ax, R ay, R az,
+                                               R drho, R avx, R avy, R avz, double dt, StateA3<R> A,
+                                               uint32_t* __restrict__ key_next, uint32_t key_old, uint32_t& outside,
+                                               uint32_t& bad, uint32_t& changed) {
+    const Stepped3<R> o =
+        whole_step_one3<R>(P, c, pos, va, pred, oid, ax, ay, az, drho, avx, avy, avz, dt, outside);
+    A.pos[s] = o.pos;
+    A.va[s] = o.va;
     real4<R> nad;
     nad.x = ax;
     nad.y = ay;
@@ -323,10 +333,9 @@ __device__ __forceinline__ Stepped3<R> integrate_one3(const StepParams& P, const
     nad.w = drho;
     A.ad[s] = nad;
     A.oid[s] = oid;
-    const uint32_t key = itype == 0 ? P.ncells : cell_key3(P, pos.x, pos.y, pos.z, bad);
+    const uint32_t key = (int)o.pos.w == 0 ? P.ncells : cell_key3(P, o.pos.x, o.pos.y, o.pos.z, bad);
     key_next[s] = key;
     changed = key != key_old ? 1u : 0u;
-    return Stepped3<R>{pos, nva};
 }
 
 // ------------------------------------------------------------------ pair pass

