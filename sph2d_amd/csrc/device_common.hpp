@@ -160,6 +160,12 @@ struct StepParams {
     uint32_t list_cap;
 };
 
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
+    return v;
+}
+
 // XCD-aware block index: the hardware deals consecutive workgroups to the 8
 // XCDs round-robin; this mapping gives each XCD one contiguous slice of the
 // sorted particle range so neighbour data is shared inside one L2.

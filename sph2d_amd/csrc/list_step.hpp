@@ -540,30 +540,158 @@ __device__ __forceinline__ bool take_capped(bool hit, uint32_t l, uint32_t cap, 
     return take;
 }
 
+// The entries of slot s's list, a row of LPP entries at a time: entry k + l
+// for k a multiple of LPP, the row's offset in a scalar register (so that an
+// entry costs no vector instruction but its load).  Rows past a list's end
+// name valid slots (padding rows, or entries of an earlier build); the loads
+// past the last allocated row read the last one instead.
+template <int LPP> struct ListRows {
+    __amdgpu_buffer_rsrc_t lists;
+    uint32_t row, last, col;  // bytes of a row; the last row to start from; this lane's byte offset in one
+    __device__ ListRows(const StepParams& P, const uint32_t* nbl, uint32_t s, uint32_t l)
+        : lists(__builtin_amdgcn_make_buffer_rsrc((void*)nbl, 0, (int)((P.list_cap + kListPad) * P.n * 4u), 0x00027000)),
+          row(P.n * 4u),
+          last(P.list_cap + kListPad - LPP),
+          col((l * P.n + min(s, P.n - 1)) * 4u) {}
+    __device__ __forceinline__ uint32_t operator()(uint32_t k) const {
+        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(lists, (int)col, (int)(min(k, last) * row), 0);
+    }
+};
+
 // Entries of slot s's list in rounds of G per lane: per round
 // body(k, e, load) - k the list index of the lane's first entry, its entries
-// k, k + LPP, ... in e; load fetches the next round's.  Entries past a list's end name valid slots (padding rows, or entries
-// of an earlier build); with LPP > 1 the loads past the last allocated row
-// read that row instead.
-template <int LPP, uint32_t G, class B>
-__device__ __forceinline__ void list_rounds(const StepParams& P, const uint32_t* __restrict__ nbl, uint32_t s,
-                                            uint32_t l, uint32_t cnt, B&& body) {
-    static_assert(LPP > 1 || 2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
-    const uint32_t row = P.n * 4u, last = (P.list_cap + kListPad - 1) * row + s * 4u;
-    uint32_t off = (l * P.n + s) * 4u;
+// k, k + LPP, ... in e; load fetches the next round's.
+template <int LPP, uint32_t G, class Rows, class B>
+__device__ __forceinline__ void list_rounds(const Rows& rows, uint32_t l, uint32_t cnt, B&& body) {
+    uint32_t k = 0, e[G];
     auto load = [&](uint32_t (&e)[G]) {
 #pragma unroll
-        for (uint32_t u = 0; u < G; ++u) {
-            const uint32_t o = off + u * LPP * row;
-            e[u] = list_entry(nbl, LPP > 1 ? min(o, last) : o);
-        }
-        off += G * LPP * row;
+        for (uint32_t u = 0; u < G; ++u) e[u] = rows(k + (G + u) * LPP);
     };
-    uint32_t e[G];
-    load(e);
+#pragma unroll
+    for (uint32_t u = 0; u < G; ++u) e[u] = rows(u * LPP);
 #pragma unroll 1
-    for (uint32_t k = l; k - l < cnt; k += G * LPP) body(k, e, load);
+    for (; k < cnt; k += G * LPP) body(k + l, e, load);
 }
+
+// ------------------------------------------------------------------ wave gathers
+// FP64 records fetched by the lanes of a wave together.  A lane that loads
+// its own record of W 16-byte words takes W instructions, each with a
+// cache-line access per lane or nearly (45 for 64 lanes, neighbouring lanes'
+// neighbours lying close), and those accesses bound the plain passes, not
+// bytes or arithmetic.  Here W consecutive lanes load the words of one
+// record, the first instruction those of their first lane's, and so on, so
+// that an instruction touches 64 / W records, each once.  The loads go
+// straight to LDS (16 bytes per lane in lane order) and each lane reads its
+// own record there.  Record t is lane t % W's of its W lanes: instruction
+// t % W put its words at lanes t - t % W on, word p in place p ^ (t % W), so
+// that lanes read from different banks.
+template <uint32_t W, uint32_t STRIDE, uint32_t MASK> struct WaveGather {
+    static_assert(W == 2 || W == 4, "words of a gathered record");
+    static constexpr uint32_t kW = W;
+    const char* records;
+    uint4* buf;        // of the wave: W * 64 words per record in flight
+    uint32_t part[W];  // byte offset of the word that this lane loads in the q-th instruction
+    __device__ WaveGather(const void* rec, uint4* wave_buf) : records((const char*)rec), buf(wave_buf) {
+#pragma unroll
+        for (uint32_t q = 0; q < W; ++q) part[q] = ((__lane_id() % W) ^ q) * 16u;
+    }
+    // the value of the q-th of this lane's W lanes
+    template <uint32_t q> __device__ __forceinline__ static uint32_t of_lane(uint32_t v) {
+        constexpr int perm = W == 4 ? q * 0x55 : (q == 0 ? 0xa0 : 0xf5);  // quad_perm [q,q,q,q] or [q,q,q+2,q+2]
+        return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, perm, 0xf, 0xf, true);
+    }
+    template <uint32_t q> __device__ __forceinline__ void fetch_one(uint32_t u, uint32_t off) const {
+        using Global = const __attribute__((address_space(1))) void*;
+        using Lds = __attribute__((address_space(3))) void*;
+        __builtin_amdgcn_global_load_lds((Global)(records + (of_lane<q>(off) | part[q])),
+                                         (Lds)(buf + (u * W + q) * kWave), 16, 0, 0);
+        if constexpr (q + 1 < W) fetch_one<q + 1>(u, off);
+    }
+    // starts the loads of the records that the lanes' entries e name, the u-th in flight
+    __device__ __forceinline__ void fetch(uint32_t u, uint32_t e) const { fetch_one<0>(u, (e & MASK) * STRIDE); }
+    __device__ __forceinline__ void read(uint32_t u, uint4* w) const {
+        const uint32_t t = __lane_id(), q = t % W;
+#pragma unroll
+        for (uint32_t p = 0; p < W; ++p) w[p] = buf[(u * W + q) * kWave + t - q + (p ^ q)];
+    }
+};
+// Records of two arrays under one entry.
+template <class A, class B> struct WaveGatherBoth {
+    static constexpr uint32_t kW = A::kW + B::kW;
+    A a;
+    B b;
+    __device__ __forceinline__ void fetch(uint32_t u, uint32_t e) const {
+        a.fetch(u, e);
+        b.fetch(u, e);
+    }
+    __device__ __forceinline__ void read(uint32_t u, uint4* w) const {
+        a.read(u, w);
+        b.read(u, w + A::kW);
+    }
+};
+__device__ __forceinline__ uint32_t wave_of_block() {  // in a scalar register
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+}
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }    // lgkmcnt(0)
+
+// list_rounds with the records gathered by the wave (every lane calls it;
+// cnt 0: no entries): body(k, e, w) - k the list index of the lane's first
+// entry of the round, e the entries, w the words of their records.  The next
+// round's records are on their way while body works on this one's, which are
+// in registers by then.
+template <int LPP, uint32_t G, class S_, class B>
+__device__ __forceinline__ void gather_rounds(const StepParams& P, const uint32_t* __restrict__ nbl, const S_& src,
+                                              uint32_t s, uint32_t l, uint32_t cnt, B&& body) {
+    const uint32_t cmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u32(cnt));
+    if (cmax == 0) return;
+    const ListRows<LPP> rows(P, nbl, s, l);
+    uint32_t e[G], en[G];
+    auto load = [&](uint32_t k) {
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) en[u] = rows(k + u * LPP);
+    };
+    auto fetch = [&]() {
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) {
+            e[u] = en[u];
+            src.fetch(u, e[u]);
+        }
+    };
+    load(0);
+    fetch();
+    load(G * LPP);
+#pragma unroll 1
+    for (uint32_t k = 0; k < cmax; k += G * LPP) {
+        uint4 w[G][S_::kW];
+        uint32_t ec[G];
+        wait_loads();
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) {
+            src.read(u, w[u]);
+            ec[u] = e[u];
+        }
+        wait_lds();  // the records are in registers: the next ones may land
+        __builtin_amdgcn_sched_barrier(0);
+        if (k + G * LPP < cmax) {
+            fetch();
+            load(k + 2 * G * LPP);
+        }
+        body(k + l, ec, w);
+    }
+}
+__device__ __forceinline__ float4 record_real4(const uint4* w, float) {
+    return make_float4(__uint_as_float(w[0].x), __uint_as_float(w[0].y), __uint_as_float(w[0].z),
+                       __uint_as_float(w[0].w));
+}
+__device__ __forceinline__ double4 record_real4(const uint4* w, double) {
+    auto d = [](uint32_t lo, uint32_t hi) { return __hiloint2double((int)hi, (int)lo); };
+    return make_double4(d(w[0].x, w[0].y), d(w[0].z, w[0].w), d(w[1].x, w[1].y), d(w[1].z, w[1].w));
+}
+// Records in flight per lane of the 2D FP64 pass: 1,020,263 particles, 105 us
+// per pass with 2 (119 with 3; 127 when each lane gathered its own).
+constexpr uint32_t kGather2 = 2;
 
 // Visits the entries of slot s's list: f(ListEntry) for every entry (f must
 // add nothing when take is false: every entry runs the same instructions,
@@ -580,31 +708,42 @@ template <class R, bool kCap, int LPP, class F>
 __device__ __forceinline__ void for_each_listed(const StepParams& P, const float2* s_off, uint32_t cap, uint32_t s,
                                                 uint32_t l, const real4<R>& nj, const double2* __restrict__ pos,
                                                 const ListRec<R>* __restrict__ rec, const uint32_t* __restrict__ nbl,
-                                                uint32_t cnt, bool& overflow, F&& f) {
-    constexpr uint32_t G = 2;  // measured at C1-1M FP32: 57.7 us per pass against 58.8 (3), 61.4 (4), 65.1 (1)
-    if (cnt == 0) return;
+                                                uint32_t cnt, uint4* buf, bool& overflow, F&& f) {
     const CutFP32 C = cut_band(P);
     uint32_t hits = 0;
     bool over = false;
-    list_rounds<LPP, G>(P, nbl, s, l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
-        ListRec<R> r[G];
-        uint32_t en[G];
+    auto entry = [&](uint32_t k, uint32_t e, const real4<R>& nr, const real4<R>& pr) {
+        ListEntry<R> E;
+        const bool in = list_cut(P, C, s_off, e, nr, nj, s, pos, E.dx, E.dy);
+        const bool hit = in & (pr.z != R(0)) & (k < cnt);
+        E.take = kCap ? take_capped<LPP>(hit, l, cap, hits, over) : hit;
+        E.nr = nr;
+        E.pr = pr;
+        f(E);
+    };
+    if constexpr (sizeof(R) == 8) {
+        constexpr uint32_t G = kGather2;
+        gather_rounds<LPP, G>(P, nbl, WaveGather<4, 64, kSlotMask>(rec, buf), s, l, cnt,
+                              [&](uint32_t k, const uint32_t (&e)[G], const auto& w) {
 #pragma unroll
-        for (uint32_t u = 0; u < G; ++u) r[u] = rec[e[u] & kSlotMask];
-        load(en);
+                                  for (uint32_t u = 0; u < G; ++u)
+                                      entry(k + u * LPP, e[u], record_real4(w[u], R(0)), record_real4(w[u] + 2, R(0)));
+                              });
+    } else {
+        constexpr uint32_t G = 2;  // measured at C1-1M FP32: 57.7 us per pass against 58.8 (3), 61.4 (4), 65.1 (1)
+        list_rounds<LPP, G>(ListRows<LPP>(P, nbl, s, l), l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
+            ListRec<R> r[G];
+            uint32_t en[G];
 #pragma unroll
-        for (uint32_t u = 0; u < G; ++u) {
-            ListEntry<R> E;
-            const bool in = list_cut(P, C, s_off, e[u], r[u].nr, nj, s, pos, E.dx, E.dy);
-            const bool hit = in & (r[u].pr.z != R(0)) & (k + u * LPP < cnt);
-            E.take = kCap ? take_capped<LPP>(hit, l, cap, hits, over) : hit;
-            E.nr = r[u].nr;
-            E.pr = r[u].pr;
-            f(E);
-        }
+            for (uint32_t u = 0; u < G; ++u) r[u] = rec[e[u] & kSlotMask];
+            load(en);
 #pragma unroll
-        for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
-    });
+            for (uint32_t u = 0; u < G; ++u) {
+                entry(k + u * LPP, e[u], r[u].nr, r[u].pr);
+                e[u] = en[u];
+            }
+        });
+    }
     overflow |= over;
 }
 
@@ -751,7 +890,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* n
         constexpr uint32_t G = 2;
         const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
         uint32_t hits = 0;
-        list_rounds<LPP, G>(P, nbl, s, g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
+        list_rounds<LPP, G>(ListRows<LPP>(P, nbl, s, g.l), g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
             real4<R> ni[G], va[G];
             uint32_t en[G];
 #pragma unroll
@@ -792,7 +931,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* n
 // continuity it also writes the pressure of the current density (the
 // reference's p array).
 template <class R, bool FIRST, int LPP, bool CONT, bool ALL>
-__global__ void __launch_bounds__(kBlock, LPP == 1 ? (sizeof(R) == 4 ? 6 : 4) : 1) pair_list_kernel(
+__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 4 : LPP == 1 ? 6 : 1) pair_list_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
     real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
@@ -826,12 +965,17 @@ __global__ void __launch_bounds__(kBlock, LPP == 1 ? (sizeof(R) == 4 ? 6 : 4) : 
     bool overflow = false;
     if (prj.z == R(0)) cnt = 0;  // died since the build
     const uint32_t cap = P.max_nbr - 1;
-    if (cnt) {
+    {
+        __shared__ uint4 s_rec[kBlock / kWave][sizeof(R) == 8 ? kGather2 * 4 * kWave : 1];
+        uint4* buf = s_rec[wave_of_block()];
         auto term = [&](const ListEntry<R>& E) { list_pair_term<R>(K, S, E, nj, prj); };
         if (__ballot(cnt > cap))  // some list of the wave may hold more than cap neighbours
-            for_each_listed<R, true, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, overflow, term);
+            for_each_listed<R, true, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, buf, overflow, term);
         else
-            for_each_listed<R, false, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, overflow, term);
+            for_each_listed<R, false, LPP>(P, s_off, cap, s, g.l, nj, X.pos, rec, nbl, cnt, buf, overflow, term);
+        // a dead particle's lanes went along with their wave's: its density is
+        // 0, so that a pair of dead particles gives no number
+        if (cnt == 0) S = ListSums<R>();
     }
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);
@@ -898,9 +1042,9 @@ __device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R d
 // for_each_listed.  Terms whose kernel type is the pressure's share one
 // evaluation, and no term divides: the cell walk over ~55 candidates with a
 // division or more per term took 167 us at 187,530 particles (FP64, Wendland
-// kernels, delta-SPH, artificial pressure), the ~20 entries of a list 53.
+// kernels, delta-SPH, artificial pressure), the ~20 entries of a list 42.
 template <class R, bool FIRST, int LPP>
-__global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
+__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_general_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
     real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
@@ -940,10 +1084,12 @@ __global__ void __launch_bounds__(kBlock) pair_list_general_kernel(
         const R two_eps_m = R(2) * (R)P.xsph_eps * m, lj_r0 = (R)P.lj_r0, lj_D = (R)P.lj_D;
         const R dhc2m = R(2) * (R)P.dhc * m, ap_iw = P.art_pressure ? (R)(1.0 / P.ap_wdelta) : R(0);
         const uint32_t cap = P.max_nbr - 1;
-        constexpr uint32_t G = 2;
+        // FP64 (187,530 particles, Wendland kernels): 42 us per pass with one
+        // entry a round and 3 waves per SIMD, 47 with two and 2 waves
+        constexpr uint32_t G = sizeof(R) == 8 ? 1 : 2;
         const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
         uint32_t hits = 0;
-        list_rounds<LPP, G>(P, nbl, s, g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
+        list_rounds<LPP, G>(ListRows<LPP>(P, nbl, s, g.l), g.l, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
             double2 pos[G];
             real4<R> va[G], pr[G];
             uint32_t en[G];

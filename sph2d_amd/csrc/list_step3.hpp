@@ -385,6 +385,19 @@ __device__ __forceinline__ void collect_near3(const StepParams& P, bool active, 
     flush(nh);
 }
 
+// ListRows with the row's offset added in a vector register: the FP32 passes,
+// which keep 6 or 12 entries in flight, take 703 us at 2,899,370 particles
+// (pair pass) this way and 728 with scalar row offsets.
+struct ListRowsVector {
+    const uint32_t* nbl;
+    uint32_t row, last, col;
+    __device__ ListRowsVector(const StepParams& P, const uint32_t* lists, uint32_t s)
+        : nbl(lists), row(P.n * 4u), last(P.list_cap + kListPad - 1), col(s * 4u) {}
+    __device__ __forceinline__ uint32_t operator()(uint32_t k) const {
+        return list_entry(nbl, min(k, last) * row + col);
+    }
+};
+
 // Summation density from the lists (Density.h:25-61) with the
 // renormalisation of the steps that ask for it (ModelParams.tex:124-133):
 // rho into rec.pr.w (sign-typed), p / rho^2 into rec.nr.w, p into pres.
@@ -407,8 +420,9 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
         step = cur->step;
     }
     __syncthreads();  // the offset table
-    const uint32_t s = lb * kBlock + threadIdx.x;
-    if (s >= P.n) return;
+    const uint32_t s0 = lb * kBlock + threadIdx.x;
+    const bool live = s0 < P.n;
+    const uint32_t s = live ? s0 : P.n - 1;
     const R m = (R)P.mass, inv_h = (R)(1.0 / P.h), w_q1 = (R)P.f_cubic, w_q2 = (R)(P.f_cubic / 6.0);
     const real4<R> dj = dens[s];
     const R w0 = w_q1 * (R(2) / R(3));
@@ -416,59 +430,52 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     const bool renorm = step_renorm(P, step);
     R wsum = renorm && dj.w != R(0) ? m / fabs(dj.w) * w0 : R(0);
     bool overflow = false;
-    const uint32_t cnt = dj.w != R(0) ? nbc[s] : 0u;
-    if (cnt) {
-        const CutFP32 C = cut_band(P);
-        const uint32_t cap = P.max_nbr - 1;
-        const uint32_t row = P.n * 4u;
-        uint32_t hits = 0;
-        // groups of G entries: the group's records gathered together, the
-        // next group's entries loaded behind them (as the pair pass does);
-        // the sums run in list order.  Rows past a list's end name valid
-        // slots (padding, or entries of an earlier build); the loads past
-        // the last allocated row read that row instead.
-        // FP32, 2,899,370 particles: 466 us per pass at G = 12 (492 at 8, 538
-        // at 4); FP64, 6.6M: 2.06 ms at G = 4 with incremental offsets (2.21
-        // clamped)
-        constexpr bool kWide = sizeof(R) == 4;
-        constexpr uint32_t G = kWide ? 12 : 4;
-        static_assert(kWide || 2 * G - 1 <= kListPad, "the entries loaded past a list's end lie in its padding rows");
-        const uint32_t last = P.list_cap + kListPad - 1;
-        auto entry = [&](uint32_t k) {
-            return list_entry(nbl, (kWide ? min(k, last) : k) * row + s * 4u);
-        };
-        uint32_t e[G];
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) e[u] = entry(u);
-#pragma unroll 1
-        for (uint32_t k = 0; k < cnt; k += G) {
+    const uint32_t cnt = live && dj.w != R(0) ? nbc[s] : 0u;
+    const CutFP32 C = cut_band(P);
+    const uint32_t cap = P.max_nbr - 1;
+    uint32_t hits = 0;
+    auto entry_term = [&](uint32_t k, uint32_t e, const real4<R>& di) {
+        R dx, dy, dz;
+        const bool hit = list_cut3(P, C, s_off, e, di, dj, s, X.pos, dx, dy, dz) & (di.w != R(0)) & (k < cnt);
+        const bool take = hit & (hits < cap);
+        overflow |= hit & !take;
+        hits += take ? 1u : 0u;
+        const R q = pair_dist<R>(dx, dy, dz) * inv_h;
+        const R t = R(2) - q;
+        const R w = q <= R(1) ? w_q1 * (R(2) / R(3) - q * q + R(0.5) * q * q * q) : w_q2 * t * t * t;
+        const R wt = take ? w : R(0);
+        rho += m * wt;
+        // (a neighbour that died since the build has density 0 in its
+        // record: only taken entries enter the sum)
+        if (renorm && take) wsum += m / fabs(di.w) * wt;
+    };
+    if constexpr (sizeof(R) == 4) {
+        // 2,899,370 particles: 466 us per pass with 12 in flight (492 with 8, 538 with 4)
+        constexpr uint32_t G = 12;
+        list_rounds<1, G>(ListRowsVector(P, nbl, s), 0, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
             real4<R> di[G];
             uint32_t en[G];
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) di[u] = dens[e[u] & kSlotMask3];
-#pragma unroll
-            for (uint32_t u = 0; u < G; ++u) en[u] = entry(k + G + u);
+            load(en);
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) {
-                R dx, dy, dz;
-                const bool hit =
-                    list_cut3(P, C, s_off, e[u], di[u], dj, s, X.pos, dx, dy, dz) & (di[u].w != R(0)) & (k + u < cnt);
-                const bool take = hit & (hits < cap);
-                overflow |= hit & !take;
-                hits += take ? 1u : 0u;
-                const R q = pair_dist<R>(dx, dy, dz) * inv_h;
-                const R t = R(2) - q;
-                const R w = q <= R(1) ? w_q1 * (R(2) / R(3) - q * q + R(0.5) * q * q * q) : w_q2 * t * t * t;
-                const R wt = take ? w : R(0);
-                rho += m * wt;
-                // (a neighbour that died since the build has density 0 in its
-                // record: only taken entries enter the sum)
-                if (renorm && take) wsum += m / fabs(di[u].w) * wt;
+                entry_term(k + u, e[u], di[u]);
+                e[u] = en[u];
             }
+        });
+    } else {
+        // 555,686 particles: 158 us per pass with 8 in flight (184 with 4, 225
+        // with 12), 181 when each lane gathered its own
+        constexpr uint32_t G = 8;
+        __shared__ uint4 s_rec[kBlock / kWave][G * 2 * kWave];
+        const WaveGather<2, 32, kSlotMask3> src(dens, s_rec[wave_of_block()]);
+        gather_rounds<1, G>(P, nbl, src, s0, 0, cnt, [&](uint32_t k, const uint32_t (&e)[G], const auto& w) {
 #pragma unroll
-            for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
-        }
+            for (uint32_t u = 0; u < G; ++u) entry_term(k + u, e[u], record_real4(w[u], R(0)));
+        });
     }
+    if (!live) return;
     // a particle that died since the build has no sums to renormalise (its
     // record's density is 0): it keeps the plain sum, so that its records,
     // which the lists of its former neighbours still name, stay finite
@@ -514,8 +521,14 @@ __device__ __forceinline__ void list_pair_term3(const K_& K, ListSums3<R>& S, bo
 
 // Pair pass from the 3D lists: the cubic configuration of pair3_kernel
 // (continuity, pressure, artificial viscosity, Lennard-Jones walls, XSPH),
-// the dt maxima and the fields for the integrator.  Entries in groups of
-// G, as for_each_listed.
+// the dt maxima and the fields for the integrator.  Entries in rounds of G,
+// the records gathered by each lane in FP32 (6 in flight: 706 us per pass at
+// 2,899,370 particles, summation; 724 at 8, 793 at 4; by the wave, two lanes a
+// record, 807: the pass is bound by instructions there) and by the wave in
+// FP64 (555,686 particles, summation: 224 us per pass with 4 in flight, 235
+// with 3, 253 with 2; 310 when each lane gathered its own; 943,906 particles,
+// continuity, which gathers the velocity too: 515 with 3, 576 with 2, 633 by
+// lane).  Two blocks per CU hold enough loads in flight then.
 template <class R, bool FIRST, bool CONT, bool ALL>
 __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState3<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
@@ -548,53 +561,64 @@ __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
     }
     const uint32_t cnt = rj.pr.w != R(0) ? nbc[s] : 0u;  // 0: died since the build
     const uint32_t cap = P.max_nbr - 1;
-    if (cnt) {
-        // entries in flight per lane at 3 waves per SIMD.  FP32, summation,
-        // 2,899,370 particles: 706 us per pass at G = 6, 724 at 8, 793 at 4;
-        // FP64, 555,686 particles: 310 at 4, 340 at 2 and 3; FP64,
-        // continuity, 943,906 particles (which gathers the velocity too): 635
-        // at 3, 669 at 2, 1032 at 4 (spills).  Rows past a list's end name
-        // valid slots (padding, or entries of an earlier build); the loads
-        // past the last allocated row read that row instead.
-        constexpr uint32_t G = sizeof(R) == 4 ? 6 : (CONT ? 3 : 4);
-        const uint32_t lastrow = P.list_cap + kListPad - 1;
+    {
         const bool capped = __ballot(cnt > cap) != 0;  // some list of the wave may hold more than cap neighbours
         const CutFP32 C = cut_band(P);
-        const uint32_t row = P.n * 4u;
         uint32_t hits = 0;
-        bool over = false;
-        uint32_t e[G];
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) e[u] = list_entry(nbl, min(u, lastrow) * row + s * 4u);
-#pragma unroll 1
-        for (uint32_t k = 0; k < cnt; k += G) {
-            ListRec<R> r[G];
-            real4<R> va[G]{};
-            uint32_t en[G];
-#pragma unroll
-            for (uint32_t u = 0; u < G; ++u) {
-                r[u] = rec[e[u] & kSlotMask3];
-                if (K.cont) va[u] = X.va[e[u] & kSlotMask3];
+        auto entry = [&](uint32_t k, uint32_t e, const real4<R>& nr, const real4<R>& pr, const real4<R>& va) {
+            R dx, dy, dz;
+            const bool in = list_cut3(P, C, s_off, e, nr, rj.nr, s, X.pos, dx, dy, dz);
+            const bool hit = in & (pr.w != R(0)) & (k < cnt);
+            bool take = hit;
+            if (capped) {
+                take = hit & (hits < cap);
+                overflow |= hit & !take;
+                hits += take ? 1u : 0u;
             }
+            list_pair_term3<R>(K, S, take, dx, dy, dz, nr, pr, va, vaj, rj.pr, rj.nr.w);
+        };
+        if constexpr (sizeof(R) == 8) {
+            constexpr uint32_t G = CONT ? 3 : 4;
+            __shared__ uint4 s_rec[kBlock / kWave][G * (CONT ? 6 : 4) * kWave];
+            uint4* buf = s_rec[wave_of_block()];
+            const WaveGather<4, 64, kSlotMask3> of_rec(rec, buf);
+            auto body = [&](uint32_t k, const uint32_t (&e)[G], const auto& w) {
 #pragma unroll
-            for (uint32_t u = 0; u < G; ++u) en[u] = list_entry(nbl, min(k + G + u, lastrow) * row + s * 4u);
-#pragma unroll
-            for (uint32_t u = 0; u < G; ++u) {
-                R dx, dy, dz;
-                const bool in = list_cut3(P, C, s_off, e[u], r[u].nr, rj.nr, s, X.pos, dx, dy, dz);
-                const bool hit = in & (r[u].pr.w != R(0)) & (k + u < cnt);
-                bool take = hit;
-                if (capped) {
-                    take = hit & (hits < cap);
-                    over |= hit & !take;
-                    hits += take ? 1u : 0u;
+                for (uint32_t u = 0; u < G; ++u) {
+                    real4<R> va{};
+                    if constexpr (CONT) va = record_real4(w[u] + 4, R(0));
+                    entry(k + u, e[u], record_real4(w[u], R(0)), record_real4(w[u] + 2, R(0)), va);
                 }
-                list_pair_term3<R>(K, S, take, dx, dy, dz, r[u].nr, r[u].pr, va[u], vaj, rj.pr, rj.nr.w);
+            };
+            if constexpr (CONT) {
+                using Va = WaveGather<2, 32, kSlotMask3>;
+                const WaveGatherBoth<WaveGather<4, 64, kSlotMask3>, Va> both{of_rec, Va(X.va, buf + G * 4 * kWave)};
+                gather_rounds<1, G>(P, nbl, both, s, 0, cnt, body);
+            } else {
+                gather_rounds<1, G>(P, nbl, of_rec, s, 0, cnt, body);
             }
+            // a dead particle's lane went along with its wave's: its density is
+            // 0, so that a pair of dead particles gives no number
+            if (cnt == 0) S = ListSums3<R>();
+        } else if (cnt) {
+            constexpr uint32_t G = 6;
+            list_rounds<1, G>(ListRowsVector(P, nbl, s), 0, cnt, [&](uint32_t k, uint32_t (&e)[G], auto& load) {
+                ListRec<R> r[G];
+                real4<R> va[G]{};
+                uint32_t en[G];
 #pragma unroll
-            for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
+                for (uint32_t u = 0; u < G; ++u) {
+                    r[u] = rec[e[u] & kSlotMask3];
+                    if (K.cont) va[u] = X.va[e[u] & kSlotMask3];
+                }
+                load(en);
+#pragma unroll
+                for (uint32_t u = 0; u < G; ++u) {
+                    entry(k + u, e[u], r[u].nr, r[u].pr, va[u]);
+                    e[u] = en[u];
+                }
+            });
         }
-        overflow |= over;
     }
     if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);

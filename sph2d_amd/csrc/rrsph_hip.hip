@@ -963,12 +963,13 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     ctx->all_terms = P.av_on && P.xsph_on && P.lj_on;
     // lanes per particle of the 2D list passes (LaneGroup), from event-timed
     // passes with 1, 2 and 8 lanes: 8 below 25,000 particles, where the chip
-    // is not filled (continuity, 6,432 particles FP64 14.2 / 11.8 / 10.1 us,
-    // 22,662 14.9 / 12.6 / 12.3, 54,200 15.6 / 15.3 / 18.7); 2 above (1,020,263
-    // FP64 142.9 / 126.6 / 221.2; summation density 519,203 FP64 56.7 / 45.5 /
-    // 66.9; general pair pass 188,656 FP64 55.8 / 46.4 / 75.3), but for the
-    // FP32 continuity pass, which has the least to do per entry, at large n
-    // (188,656 particles 18.3 / 20.8 / 31.4, 1,020,263 62.5 / 64.5 / 146.7)
+    // is not filled (continuity, 6,432 particles FP64 14.8 / 11.9 / 10.8 us,
+    // 22,662 15.2 / 12.5 / 12.1, 54,200 15.7 / 14.0 / 20.0); 2 above (413,242
+    // FP64 44.3 / 44.6 / -, 1,020,263 108.5 / 104.7 / -; summation density
+    // 519,203 FP32 36.1 / 32.9 / 57.4; general pair pass 413,242 FP32 52.6 /
+    // 42.0 / 76.1), but for the FP32 continuity pass, which has the least to
+    // do per entry, at large n (188,656 particles 18.3 / 19.4 / 31.4,
+    // 1,020,263 61.4 / 61.6 / 146.7)
     ctx->lanes = P.n < 25000 ? 8 : 2;
     if (P.n >= 150000 && ctx->fast_pair && ctx->fp32 && P.density_treatment != 0) ctx->lanes = 1;
     P.list_reach = P.cell * (1.0 + skin_frac);

@@ -145,11 +145,6 @@ __device__ __forceinline__ void for_each_neighbour3(const StepParams& P, uint32_
 // decided by a ballot.  Every lane of the wave calls it; lanes with
 // active = false walk empty ranges.  Same neighbour set, visiting order and
 // overflow rule as for_each_neighbour3.
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
-    return v;
-}
 
 constexpr uint32_t kCollect3 = 4;  // candidates per batch of the 3D walk
 template <uint32_t kChunk, class F>
