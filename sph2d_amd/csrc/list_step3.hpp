@@ -119,27 +119,9 @@ __global__ void __launch_bounds__(kBlock) reorder_list3_kernel(StepParams P, con
 // particle, every live particle i != s within list_reach, in the order of
 // the reference's cell walk (x-major columns, then y, each column's z range
 // contiguous).  The cells visited are those within list_reach (3 or 4 per
-// axis).  The walk is wave-uniform: the slots of a wave share one (x, y)
-// column of cells or a few, so the wave loops over the union of its lanes'
-// columns and, in each, over its longest z range, lanes masked outside
-// their own ranges (same entries and order as a per-lane walk).  Entries
-// go to the lane's column of an LDS buffer first; when a lane's column
-// might overflow, the wave writes the buffered rows out together, so each
-// row's stores from the lanes of a wave are contiguous (written straight
-// from the walk, they left lines partly written in L2).
+// axis; a column off the particle's own needs a shorter z range, corner
+// columns most).
 constexpr uint32_t kCollectL3 = 4;
-constexpr uint32_t kBuildChunk = 32;  // LDS rows per lane
-__device__ __forceinline__ int wave_min_i32(int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off));
-    return v;
-}
-__device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off));
-    return v;
-}
-constexpr uint32_t kBuildL3 = 8;  // candidates in flight per lane (6.6M dam break: 4.06 ms per build, 4.22 at 4)
 __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl* __restrict__ next,
                                                              const Ctrl* __restrict__ cur,
                                                              const double4* __restrict__ pos,
@@ -147,14 +129,13 @@ __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl*
                                                              const uint32_t* __restrict__ skey,
                                                              const uint32_t* __restrict__ LB,
                                                              uint32_t* __restrict__ nbl, uint32_t* __restrict__ nbc) {
-    __shared__ uint32_t buf[kBuildChunk * kBlock];
+    __shared__ BuildLds s_build[kBlock / kWave];
     if (cur->halted) return;
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     const uint32_t s0 = lb * kBlock + threadIdx.x;
     const bool inb = s0 < P.n;
     const uint32_t s = inb ? s0 : P.n - 1;
-    uint32_t cnt = 0;
     bool bad = false;
     const double4 pj = pos[s];
     const bool alive = inb && (int)pj.w != 0;
@@ -162,9 +143,11 @@ __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl*
     const int hz = (int)(kj % (uint32_t)P.ncz);
     const uint32_t hxy = kj / (uint32_t)P.ncz;
     const int hx = (int)(hxy / (uint32_t)P.ncy), hy = (int)hxy - hx * P.ncy;
-    const double reach = P.list_reach * (1.0 + 1e-9);
+    const float4 cj = cand[s];
+    const float cell = (float)P.cell, inv_cell = (float)(1.0 / P.cell);
+    const float reach = (float)(P.list_reach * (1.0 + 1e-5));
     // empty ranges (x0 > x1) for lanes with nothing to list
-    int x0 = 1, x1 = 0, y0 = 1, y1 = 0, z0 = 0, z1 = 0;
+    int x0 = 0, x1 = -1, y0 = 0, y1 = -1, z0 = 0, z1 = 0;
     if (alive) {
         // the list pass takes the FP32 positions relative to the home cell
         // for within 2.1 cells of its origin: a particle outside the cell
@@ -173,85 +156,64 @@ __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl*
         const double ox = pj.x - o.x, oy = pj.y - o.y, oz = pj.z - o.z;
         bad = !(ox > -P.cell && ox < 2.0 * P.cell && oy > -P.cell && oy < 2.0 * P.cell && oz > -P.cell &&
                 oz < 2.0 * P.cell);
-        x0 = clamped_cell(pj.x - reach, P.xmin, P.cell, P.ncx);
-        x1 = clamped_cell(pj.x + reach, P.xmin, P.cell, P.ncx);
-        y0 = clamped_cell(pj.y - reach, P.ymin, P.cell, P.ncy);
-        y1 = clamped_cell(pj.y + reach, P.ymin, P.cell, P.ncy);
-        z0 = clamped_cell(pj.z - reach, P.zmin, P.cell, P.ncz);
-        z1 = clamped_cell(pj.z + reach, P.zmin, P.cell, P.ncz);
+        if (!bad) {
+            x0 = reach_first(cj.x, reach, inv_cell, hx);
+            x1 = reach_last(cj.x, reach, inv_cell, hx, P.ncx);
+            y0 = reach_first(cj.y, reach, inv_cell, hy);
+            y1 = reach_last(cj.y, reach, inv_cell, hy, P.ncy);
+            z0 = reach_first(cj.z, reach, inv_cell, hz);
+            z1 = reach_last(cj.z, reach, inv_cell, hz, P.ncz);
+        }
         bad |= x0 < hx - 2 || x1 > hx + 2 || y0 < hy - 2 || y1 > hy + 2 || z0 < hz - 2 || z1 > hz + 2;
     }
-    uint32_t* my = buf + threadIdx.x;
-    uint32_t nh = 0;
-    auto flush = [&]() {
-#pragma unroll 1
-        for (uint32_t r = 0; r < nh; ++r)
-            if (cnt + r < P.list_cap) nbl[(size_t)(cnt + r) * P.n + s] = my[r * kBlock];
-        cnt += nh;
-        nh = 0;
-    };
-    const int wx0 = wave_min_i32(alive ? x0 : INT_MAX), wx1 = wave_max_i32(alive ? x1 : INT_MIN);
-    const int wy0 = wave_min_i32(alive ? y0 : INT_MAX), wy1 = wave_max_i32(alive ? y1 : INT_MIN);
-    const double reach2 = reach * reach;
-    // candidates are tested in FP32 from the candidate records: r_i - r_s =
-    // (xi_i - xi_s) + (home-cell offset) cell, rounded far below the 1e-5
-    // by which the FP32 reach exceeds list_reach, so the lists hold every
-    // pair within list_reach (and at most a few just beyond, which every
-    // list step tests again)
-    const float4 cj = cand[s];
-    const float cellf = (float)P.cell;
-    const float r2f = (float)(P.list_r2 * (1.0 + 1e-5));
+    ListBuilder out(P, s_build[wave_of_block()], nbl, s);
+    const int wx0 = full_wave_min_i32(x0 <= x1 ? x0 : INT_MAX), wx1 = full_wave_max_i32(x1);
+    const int wy0 = full_wave_min_i32(y0 <= y1 ? y0 : INT_MAX), wy1 = full_wave_max_i32(y1);
+    // positions relative to the column in x and y and to one cell of the
+    // wave in z, from the candidate records (relative to their home cells)
+    const float r2 = (float)(P.list_r2 * (1.0 + build_margin(P.ncz)));
+    const int zref = __builtin_amdgcn_readfirstlane(hz);
+    const float pz = cj.z + (float)(hz - zref) * cell;
 #pragma unroll 1
     for (int x = wx0; x <= wx1; ++x) {
-        // distance from the particle to the column's x slab
-        const double xl = P.xmin + x * P.cell;
-        const double dxm = fmax(0.0, fmax(xl - pj.x, pj.x - (xl + P.cell)));
-        const float ox = (float)(x - hx) * cellf;
+        const bool need_x = x >= x0 && x <= x1;
+        if (!__any(need_x)) continue;
+        const float px = cj.x + (float)(hx - x) * cell;
+        const float dxm = fmaxf(0.f, fmaxf(-px, px - cell));  // distance to the column's x slab
+        const float rem_x = r2 - dxm * dxm;
 #pragma unroll 1
         for (int y = wy0; y <= wy1; ++y) {
-            const double yl = P.ymin + y * P.cell;
-            const double dym = fmax(0.0, fmax(yl - pj.y, pj.y - (yl + P.cell)));
-            const float oy = (float)(y - hy) * cellf;
-            // the z cells of this column within reach: a column off the
-            // particle's own needs a shorter range (corner columns most)
-            const double rem = reach2 - dxm * dxm - dym * dym;
-            bool need = x >= x0 && x <= x1 && y >= y0 && y <= y1 && rem >= 0.0;
-            int za = z0, zb = z1;
+            const float py = cj.y + (float)(hy - y) * cell;
+            const float dym = fmaxf(0.f, fmaxf(-py, py - cell));
+            const float rem = rem_x - dym * dym;
+            const bool need = need_x && y >= y0 && y <= y1 && rem >= 0.f;
+            if (!__any(need)) continue;
+            const uint32_t col = ((uint32_t)x * (uint32_t)P.ncy + (uint32_t)y) * (uint32_t)P.ncz;
+            uint32_t b = 0, e = 0;
             if (need) {
-                const double zr = sqrt(rem) * (1.0 + 1e-9);
-                za = max(z0, clamped_cell(pj.z - zr, P.zmin, P.cell, P.ncz));
-                zb = min(z1, clamped_cell(pj.z + zr, P.zmin, P.cell, P.ncz));
+                // the z cells of this column within reach, a little widened
+                // for the rounding here
+                const float zr = __builtin_amdgcn_sqrtf(rem) * (1.f + 1e-5f) + 1e-5f * cell;
+                const int za = max(z0, hz + (int)floorf((cj.z - zr) * inv_cell));
+                const int zb = min(z1, hz + (int)floorf((cj.z + zr) * inv_cell));
+                b = LB[col + za];
+                e = LB[col + zb + 1];
             }
-            const uint32_t col = need ? ((uint32_t)x * (uint32_t)P.ncy + (uint32_t)y) * (uint32_t)P.ncz : 0u;
-            const uint32_t b = need ? LB[col + za] : 0u;
-            const uint32_t len = need ? LB[col + zb + 1] - b : 0u;
-            const uint32_t code_xy = (uint32_t)(x - hx + 2) + 5u * (uint32_t)(y - hy + 2);
-            const uint32_t lmax = wave_max_u32(len);
-#pragma unroll 1
-            for (uint32_t i = 0; i < lmax; i += kBuildL3) {
-                float4 q[kBuildL3];
-#pragma unroll
-                for (uint32_t u = 0; u < kBuildL3; ++u) q[u] = cand[len ? b + min(i + u, len - 1) : s];
-#pragma unroll
-                for (uint32_t u = 0; u < kBuildL3; ++u) {
-                    const int dcz = __float_as_int(q[u].w) - hz;  // the neighbour's z cell, from its key
-                    const float dx = (q[u].x - cj.x) + ox, dy = (q[u].y - cj.y) + oy;
-                    const float dz = (q[u].z - cj.z) + (float)dcz * cellf;
-                    const bool in = (i + u < len) & (b + i + u != s) & (dx * dx + dy * dy + dz * dz < r2f);
-                    if (in) {
-                        const uint32_t code = code_xy + 25u * (uint32_t)(dcz + 2);
-                        my[nh * kBlock] = (b + i + u) | (code << kSlotBits3);
-                        ++nh;
-                    }
-                }
-                if (__any(nh + kBuildL3 > kBuildChunk)) flush();  // wave-uniform
-            }
+            // the word holds the slot and the z cell; the offsets from the
+            // lane's home cell complete the code (modulo 2^32)
+            const uint32_t add = (uint32_t)((x - hx + 2) + 5 * (y - hy + 2) + 25 * (2 - hz)) << kSlotBits3;
+            out.column<true>(need, b, e, px, py, pz, r2, add, [&](uint32_t i) {
+                const float4 q = cand[i];
+                const int cz = __float_as_int(q.w);
+                return make_float4(q.x, q.y, q.z + (float)(cz - zref) * cell,
+                                   __uint_as_float(i + ((uint32_t)(25 * cz) << kSlotBits3)));
+            });
         }
     }
-    flush();
+    out.flush();
     if (!inb) return;
-    if (cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
-    nbc[s] = min(cnt, P.list_cap);
+    if (out.cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
+    nbc[s] = min(out.cnt, P.list_cap);
 }
 
 // collect_neighbours3 over a particle's list instead of the cell walk: the
