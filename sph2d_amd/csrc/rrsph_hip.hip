@@ -247,6 +247,7 @@ struct rrsph_ctx {
     hipGraph_t graph_list = nullptr, graph_build = nullptr;
     hipGraphExec_t gexec_list = nullptr, gexec_build = nullptr;
     uint64_t build_at = 0;              // step index of the last build launched
+    double tape_skin = 0;               // skin of taped runs (fraction of the cut-off)
     uint64_t list_interval = 8;         // steps between builds
     uint64_t n_list = 0, n_build = 0, n_list_halts = 0;
     AdjTape adj;
@@ -296,6 +297,14 @@ uint32_t grid_blocks(uint32_t n, uint32_t bs) { return (n + bs - 1) / bs; }
 constexpr uint64_t kFullSortRun = 64;
 constexpr uint64_t kFullSortRunMax = 4096;
 constexpr uint64_t kFallbackWindow = 8;
+
+// The reach and the skin of the neighbour lists from the skin's fraction of
+// the cut-off.
+void set_skin(StepParams& P, double skin_frac) {
+    P.list_reach = P.cell * (1.0 + skin_frac);
+    P.list_r2 = P.list_reach * P.list_reach * (1.0 + 1e-12);
+    P.skin_half = 0.5 * P.cell * skin_frac * (1.0 - 1e-9);
+}
 
 // Launch helper that optionally records HIP events around the launch.
 struct Launcher {
@@ -953,10 +962,15 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
                      (p.density_treatment == 0 || p.density_treatment == 1) && std::fabs(p.cell_scale_k - 2.0) == 0.0;
     // neighbour-list steps: every 2D configuration and the cubic one in 3D
     // (187,530 particles with Wendland kernels, delta-SPH and artificial
-    // pressure, FP64: 81 us a step with lists, 205 us sorted); skin as a
-    // fraction of the cut-off (an entry holds a slot in kSlotBits bits in
-    // 2D, kSlotBits3 in 3D)
-    double skin_frac = 0.125;
+    // pressure, FP64: 81 us a step with lists, 205 us sorted); an entry holds
+    // a slot in kSlotBits bits in 2D, kSlotBits3 in 3D.  The skin, a fraction
+    // of the cut-off: a wider one makes builds rarer and lists longer, and in
+    // 3D the lists grow faster.  Per 50 steps of 1,020,263 particles (FP32): 5250
+    // us at 0.125, 5050 at 0.15, 5380 at 0.18; below 25,000 particles, where a
+    // pass is bound by latency, per 200 steps of 6,923: 3940 at 0.125, 3870 at
+    // 0.15, 3640 at 0.23, 3620 at 0.26; 3D, per 25 steps of 555,686 (FP64):
+    // 11110 at 0.06, 11100 at 0.08, 11520 at 0.1, 11630 at 0.125
+    double skin_frac = d3 ? 0.08 : P.n < 25000 ? 0.23 : 0.15;
     if (const char* e = std::getenv("RRSPH_HIP_LIST_SKIN")) skin_frac = std::strtod(e, nullptr);
     ctx->list_mode = (ctx->fast_pair || !d3) && skin_frac > 0.0 && skin_frac < 0.9 && P.n <= (d3 ? kSlotMask3 : kSlotMask);
     if (const char* e = std::getenv("RRSPH_HIP_LIST")) ctx->list_mode = ctx->list_mode && std::strcmp(e, "0") != 0;
@@ -972,10 +986,12 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     // 1,020,263 61.4 / 61.6 / 146.7)
     ctx->lanes = P.n < 25000 ? 8 : 2;
     if (P.n >= 150000 && ctx->fast_pair && ctx->fp32 && P.density_treatment != 0) ctx->lanes = 1;
-    P.list_reach = P.cell * (1.0 + skin_frac);
-    P.list_r2 = P.list_reach * P.list_reach * (1.0 + 1e-12);
-    P.skin_half = 0.5 * P.cell * skin_frac * (1.0 - 1e-9);
-    const double grow = std::pow(1.0 + skin_frac, d3 ? 3 : 2);
+    // a taped run keeps every build's lists, so that its builds cost more: 12
+    // steps and their gradients, 943,906 particles (3D FP32), 30.6 ms at 0.08,
+    // 25.3 at 0.1, 23.1 at 0.125, 23.6 at 0.15
+    ctx->tape_skin = d3 && !std::getenv("RRSPH_HIP_LIST_SKIN") ? 0.125 : skin_frac;
+    set_skin(P, skin_frac);
+    const double grow = std::pow(1.0 + std::max(skin_frac, ctx->tape_skin), d3 ? 3 : 2);
     P.list_cap = (uint32_t)std::ceil(p.max_neighbours * grow) + 8;
     // the list pass addresses the lists (list_cap + kListPad rows) with
     // 32-bit byte offsets: fewer rows where n is large (a build that finds
@@ -2012,6 +2028,22 @@ static rrsph_status launch_taped_step(rrsph_ctx* ctx, uint64_t base, bool& launc
     return RRSPH_OK;
 }
 
+// The skin of taped runs while they launch steps.  Lists built with either
+// skin: a taped range starts with a build, and the wider lists left behind
+// serve the narrower skin.
+struct TapeSkin {
+    StepParams& P;
+    const StepParams before;
+    TapeSkin(rrsph_ctx* ctx) : P(ctx->P), before(ctx->P) {
+        if (ctx->adj.lists) set_skin(P, ctx->tape_skin);
+    }
+    ~TapeSkin() {
+        P.list_reach = before.list_reach;
+        P.list_r2 = before.list_r2;
+        P.skin_half = before.skin_half;
+    }
+};
+
 constexpr uint32_t kHaltCheck = 64;  // tape steps between two looks at the control block
 
 // Launch steps [k0, k1) of the tape, reading the control block back every
@@ -2022,6 +2054,7 @@ constexpr uint32_t kHaltCheck = 64;  // tape steps between two looks at the cont
 static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool forward, void* seg_base,
                                 uint32_t kslot, uint64_t abs0) {
     AdjTape& T = ctx->adj;
+    const TapeSkin skin(ctx);
     const size_t n = ctx->P.n;
     // the forward keeps the states of the last segment (of every step with
     // keep_all): the reverse pass starts there and needs no replay of it
