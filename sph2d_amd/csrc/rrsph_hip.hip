@@ -164,6 +164,16 @@ struct AdjTape {
     uint64_t tbase = 0;
 };
 
+// Captured steps with neighbour lists: a build step, and runs of 1, 2, 4 and
+// 8 list steps.  Between two graphs the stream idles for 3 us or more (8 us
+// where a profiler looks on), between the kernels of one for about 1.
+constexpr uint32_t kListRunMax = 8;
+constexpr uint64_t kFirstChunk = 16;
+struct ListGraphs {
+    hipGraph_t graph[5] = {};
+    hipGraphExec_t exec[5] = {};
+};
+
 struct rrsph_ctx {
     rrsph_params_c prm{};
     StepParams P{};
@@ -244,11 +254,12 @@ struct rrsph_ctx {
     unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima, a set per step parity)
     unsigned long long* dtslots = nullptr; // list steps: dt maxima (likewise)
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
-    hipGraph_t graph_list = nullptr, graph_build = nullptr;
-    hipGraphExec_t gexec_list = nullptr, gexec_build = nullptr;
+    ListGraphs list_graphs[2];          // of plain runs and of taped ones (another skin)
+    bool taping = false;                // ctx->P holds the taped runs' skin
     uint64_t build_at = 0;              // step index of the last build launched
     double tape_skin = 0;               // skin of taped runs (fraction of the cut-off)
     uint64_t list_interval = 8;         // steps between builds
+    uint64_t list_chunk = kFirstChunk;  // steps between looks at the control block
     uint64_t n_list = 0, n_build = 0, n_list_halts = 0;
     AdjTape adj;
 };
@@ -618,8 +629,8 @@ void enqueue_step(rrsph_ctx* c, Profiler* prof, bool full_sort) {
 }
 
 void drop_graph(rrsph_ctx* c) {
-    hipGraphExec_t* ex[] = {&c->gexec, &c->gexec_full, &c->gexec_list, &c->gexec_build};
-    hipGraph_t* gr[] = {&c->graph, &c->graph_full, &c->graph_list, &c->graph_build};
+    hipGraphExec_t* ex[] = {&c->gexec, &c->gexec_full};
+    hipGraph_t* gr[] = {&c->graph, &c->graph_full};
     for (auto* e : ex) {
         if (*e) (void)hipGraphExecDestroy(*e);
         *e = nullptr;
@@ -627,6 +638,13 @@ void drop_graph(rrsph_ctx* c) {
     for (auto* g : gr) {
         if (*g) (void)hipGraphDestroy(*g);
         *g = nullptr;
+    }
+    for (ListGraphs& G : c->list_graphs) {
+        for (auto e : G.exec)
+            if (e) (void)hipGraphExecDestroy(e);
+        for (auto g : G.graph)
+            if (g) (void)hipGraphDestroy(g);
+        G = ListGraphs{};
     }
 }
 
@@ -641,16 +659,25 @@ rrsph_status build_graph(rrsph_ctx* ctx) {
     enqueue_step(ctx, nullptr, true);
     HIP_TRY(hipStreamEndCapture(ctx->stream, &ctx->graph_full));
     HIP_TRY(hipGraphInstantiate(&ctx->gexec_full, ctx->graph_full, nullptr, nullptr, 0));
-    if (ctx->list_mode) {
-        HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_list_step(ctx, nullptr, false);
-        HIP_TRY(hipStreamEndCapture(ctx->stream, &ctx->graph_list));
-        HIP_TRY(hipGraphInstantiate(&ctx->gexec_list, ctx->graph_list, nullptr, nullptr, 0));
-        HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        enqueue_list_step(ctx, nullptr, true);
-        HIP_TRY(hipStreamEndCapture(ctx->stream, &ctx->graph_build));
-        HIP_TRY(hipGraphInstantiate(&ctx->gexec_build, ctx->graph_build, nullptr, nullptr, 0));
+    return RRSPH_OK;
+}
+
+// Launch a build step (build) or `steps` list steps (a power of two up to
+// kListRunMax) through the captured graphs, or directly.
+rrsph_status launch_list_run(rrsph_ctx* ctx, bool build, uint32_t steps) {
+    if (!ctx->use_graph) {
+        for (uint32_t k = 0; k < steps; ++k) enqueue_list_step(ctx, nullptr, build);
+        return RRSPH_OK;
     }
+    ListGraphs& G = ctx->list_graphs[ctx->taping ? 1 : 0];
+    const uint32_t i = build ? 0 : 1 + (uint32_t)__builtin_ctz(steps);
+    if (!G.exec[i]) {
+        HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+        for (uint32_t k = 0; k < steps; ++k) enqueue_list_step(ctx, nullptr, build);
+        HIP_TRY(hipStreamEndCapture(ctx->stream, &G.graph[i]));
+        HIP_TRY(hipGraphInstantiate(&G.exec[i], G.graph[i], nullptr, nullptr, 0));
+    }
+    HIP_TRY(hipGraphLaunch(G.exec[i], ctx->stream));
     return RRSPH_OK;
 }
 
@@ -1283,26 +1310,28 @@ static bool next_is_build(const rrsph_ctx* ctx, uint64_t step) {
 }
 
 static rrsph_status launch_steps(rrsph_ctx* ctx, uint32_t nsteps) {
-    if (ctx->use_graph && !ctx->gexec) {
-        rrsph_status st = build_graph(ctx);
-        if (st != RRSPH_OK) return st;
-    }
     if (list_active(ctx)) {
         // step indices from the committed count of the last synchronisation
         const uint64_t base = committed_steps(*ctx->host_ctrl);
-        for (uint32_t k = 0; k < nsteps; ++k) {
+        for (uint32_t k = 0; k < nsteps;) {
             const bool build = next_is_build(ctx, base + k);
-            if (ctx->use_graph) HIP_TRY(hipGraphLaunch(build ? ctx->gexec_build : ctx->gexec_list, ctx->stream));
-            else enqueue_list_step(ctx, nullptr, build);
+            uint32_t run = 1;  // list steps to the next build, in powers of two
+            if (!build) {
+                const uint64_t left = std::min<uint64_t>(nsteps - k, ctx->build_at + ctx->list_interval - (base + k));
+                while (run < kListRunMax && 2 * run <= left) run *= 2;
+            }
+            const rrsph_status st = launch_list_run(ctx, build, run);
+            if (st != RRSPH_OK) return st;
             if (build) {
                 ctx->build_at = base + k;
                 ++ctx->n_build;
                 ++ctx->n_full;
             } else {
-                ++ctx->n_list;
+                ctx->n_list += run;
             }
-            ++ctx->launched;
+            ctx->launched += run;
             ctx->need_full = false;
+            k += run;
         }
         HIP_TRY(hipGetLastError());
         if (nsteps) {
@@ -1311,6 +1340,10 @@ static rrsph_status launch_steps(rrsph_ctx* ctx, uint32_t nsteps) {
             ctx->list_fields = true;
         }
         return RRSPH_OK;
+    }
+    if (ctx->use_graph && !ctx->gexec) {
+        rrsph_status st = build_graph(ctx);
+        if (st != RRSPH_OK) return st;
     }
     for (uint32_t k = 0; k < nsteps; ++k) {
         const bool full = ctx->need_full || !ctx->incremental || ctx->launched < ctx->full_until;
@@ -1339,12 +1372,8 @@ static uint64_t committed_steps(const Ctrl& c) { return c.step + (c.pending ? 1 
 // follow their own schedule); `abs_step` is its step index since the upload.
 // A build's sort lands in kbuf / vbuf of the last radix pass.
 static rrsph_status launch_list_step(rrsph_ctx* ctx, bool build, uint64_t abs_step) {
-    if (ctx->use_graph && !ctx->gexec) {
-        rrsph_status st = build_graph(ctx);
-        if (st != RRSPH_OK) return st;
-    }
-    if (ctx->use_graph) HIP_TRY(hipGraphLaunch(build ? ctx->gexec_build : ctx->gexec_list, ctx->stream));
-    else enqueue_list_step(ctx, nullptr, build);
+    const rrsph_status st = launch_list_run(ctx, build, 1);
+    if (st != RRSPH_OK) return st;
     HIP_TRY(hipGetLastError());
     if (build) {
         const uint32_t fb = (ctx->passes - 1) & 1u;
@@ -1435,15 +1464,17 @@ static rrsph_status resume_halt(rrsph_ctx* ctx, bool* resumed) {
 }
 
 // Run nsteps steps to completion (or to a halt) and report the status.
-// List steps go in batches of about twice the build interval, so that a
-// halt wastes few launches and the interval follows the flow.
+// List steps go in batches: kFirstChunk steps in a fresh context, about twice the
+// build interval and at least 32 in a steady flow (a look at the control
+// block idles the stream for 25 us), few after a halt, when the interval is
+// still falling and the launches behind the next halt do nothing.
 static rrsph_status run_steps(rrsph_ctx* ctx, uint32_t nsteps) {
     const uint64_t target = committed_steps(*ctx->host_ctrl) + nsteps;
     while (true) {
         const uint64_t now = committed_steps(*ctx->host_ctrl);
         if (now >= target) return RRSPH_OK;
         uint64_t chunk = target - now;
-        if (list_active(ctx)) chunk = std::min<uint64_t>(chunk, std::min<uint64_t>(256, std::max<uint64_t>(16, 2 * ctx->list_interval)));
+        if (list_active(ctx)) chunk = std::min(chunk, ctx->list_chunk);
         rrsph_status st = launch_steps(ctx, (uint32_t)chunk);
         if (st != RRSPH_OK) return st;
         st = sync_status(ctx);
@@ -1452,7 +1483,11 @@ static rrsph_status run_steps(rrsph_ctx* ctx, uint32_t nsteps) {
         st = resume_halt(ctx, &resumed);
         if (st != RRSPH_OK) return st;
         if (!resumed && ctx->host_ctrl->halted) return RRSPH_OK;  // stopped at t_end
-        if (!resumed && list_active(ctx)) adapt_list_interval(ctx);
+        if (!list_active(ctx)) continue;
+        if (!resumed) adapt_list_interval(ctx);
+        const uint64_t two = 2 * ctx->list_interval;
+        ctx->list_chunk = resumed ? std::max<uint64_t>(4, std::min(kFirstChunk, two))
+                                  : std::min<uint64_t>(2 * ctx->list_chunk, std::min<uint64_t>(256, std::max<uint64_t>(32, two)));
     }
 }
 
@@ -2034,10 +2069,14 @@ static rrsph_status launch_taped_step(rrsph_ctx* ctx, uint64_t base, bool& launc
 struct TapeSkin {
     StepParams& P;
     const StepParams before;
-    TapeSkin(rrsph_ctx* ctx) : P(ctx->P), before(ctx->P) {
-        if (ctx->adj.lists) set_skin(P, ctx->tape_skin);
+    bool& taping;
+    TapeSkin(rrsph_ctx* ctx) : P(ctx->P), before(ctx->P), taping(ctx->taping) {
+        if (!ctx->adj.lists) return;
+        set_skin(P, ctx->tape_skin);
+        taping = true;
     }
     ~TapeSkin() {
+        taping = false;
         P.list_reach = before.list_reach;
         P.list_r2 = before.list_r2;
         P.skin_half = before.skin_half;
