@@ -68,20 +68,24 @@ struct Ctrl {
     double disp_last;       // the largest displacement of the last committed list or build step
     uint32_t list_valid;    // the lists describe the current slot order (a build ran; no sort since)
     uint32_t cur_renorm;    // this step's summation density is renormalised
+    uint32_t halt_now;      // the step halted that wrote this (a later one only finds it halted)
+    uint32_t pad0;
     // flags that blocks of a step raise on the control block between steps;
     // the integrator of a list step, which publishes the words before them
     // (publish_ctrl), leaves them alone
     uint32_t nbr_overflow;  // a particle had more than max_neighbours - 1 neighbours
     uint32_t grid_overflow; // a live particle lay outside the cell grid
-    uint32_t outside_l[2];  // list steps: as outside, by the parity of the step index
+    uint32_t outside_l[4];  // list steps: as outside, by the step index modulo 4
     uint32_t list_overflow; // the last build found more candidates for some particle than its list holds
-    uint32_t flags_pad;
+    uint32_t list_long;     // ... more entries than max_neighbours - 1
 };
 
 // Particles outside the geometry after the step awaiting its commit.  (An
 // index computed at run time would put a copy of the block in scratch memory.)
 __host__ __device__ inline uint32_t ctrl_outside(const Ctrl& c) {
-    return c.outside + ((c.step & 1) ? c.outside_l[1] : c.outside_l[0]);
+    const uint32_t odd = (c.step & 2) ? c.outside_l[3] : c.outside_l[1];
+    const uint32_t even = (c.step & 2) ? c.outside_l[2] : c.outside_l[0];
+    return c.outside + ((c.step & 1) ? odd : even);
 }
 
 constexpr int kMaxSegments = 8;  // paddles of a segmented piston
@@ -158,6 +162,7 @@ struct StepParams {
     // skin_half = skin / 2 (less a rounding margin)
     double list_reach, list_r2, skin_half;
     uint32_t list_cap;
+    uint32_t dset_mask;     // displacement slot sets of list steps, less one (list_step.hpp)
 };
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {

@@ -34,7 +34,8 @@
 // test; the rounding of xi stays far below that band (2e-6 of the cut-off).
 //
 // Step kernels: [density_sum_list] -> pair_list -> integrate_list (in place;
-// it also writes the next step's records, so no reorder runs between builds),
+// it also writes the next step's records, so no reorder runs between builds;
+// with a constant dt and no wave maker the pair pass integrates: fused_step_begin),
 // the first of them with the step's prologue (list_step_begin).  A build step runs list_prologue -> radix
 // sort -> reorder_list_kernel -> list_build_kernel -> the same step kernels
 // on the reordered copy, integrating into A.
@@ -46,6 +47,7 @@
 namespace rrsph {
 
 constexpr uint32_t kStatusRebuild = 101;       // internal: re-run this step as a list build
+constexpr uint32_t kStatusUnfused = 103;       // internal: a fused step might have too many neighbours; run steps unfused
 constexpr uint32_t kStatusListOverflow = 102;  // internal: a list ran out of room; run without lists
 
 // The state a list step reads (the reordered copy B on a build step, A after).
@@ -223,9 +225,10 @@ static_assert(offsetof(Ctrl, nbr_overflow) % 8 == 0 && offsetof(Ctrl, dt_new) % 
               "publish_ctrl's words");
 
 // The largest displacement of the step that `next` holds, the slots holding
-// squares (both sets are loaded, so that the loads do not wait for the step
-// index).
-__device__ __forceinline__ double list_dmax(const Ctrl* next, const unsigned long long* dslots) {
+// squares (of two sets both are loaded, so that the loads do not wait for the
+// step index).
+__device__ __forceinline__ double list_dmax(const StepParams& P, const Ctrl* next, const unsigned long long* dslots) {
+    if (P.dset_mask == 3) return sqrt(slots_max(dslots + (uint32_t)(next->step & 3) * kSlotSet));
     const double even = slots_max(dslots), odd = slots_max(dslots + kSlotSet);
     return sqrt((next->step & 1) ? odd : even);
 }
@@ -234,13 +237,22 @@ __device__ __forceinline__ double list_dmax(const Ctrl* next, const unsigned lon
 // commit of the step that `next` holds, the staleness test of the lists (a
 // list step also halts when no build has run since the last sort, e.g. a
 // build launched while the run was stopped), the snapshot into `cur`.
-__device__ __forceinline__ void list_block_prologue(const StepParams& P, const Ctrl* next, Ctrl* cur, double dmax,
-                                                    bool build) {
+// fused: of a step of one kernel (pair_list_kernel, FUSED with CONT), which
+// publishes its outcome here: dt is known, and `next` gets all but the flags,
+// which stay in `flags`.
+__device__ __forceinline__ void list_block_prologue(const StepParams& P, const Ctrl* next, Ctrl* cur,
+                                                    const Ctrl* flags, double dmax, bool build, bool fused) {
     const unsigned long long word = ctrl_word(next);
     uint32_t valid = 0;
+    bool was_halted = false;
     block_prologue(
         P, cur, word,
         [&](Ctrl& c) {
+            was_halted = c.halted != 0;
+            if (fused) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) c.outside_l[k] = flags->outside_l[k];
+            }
             if (!c.halted && c.pending) {  // the step being committed moved no particle further than dmax
                 c.disp_acc += dmax;
                 c.disp_last = dmax;
@@ -252,6 +264,7 @@ __device__ __forceinline__ void list_block_prologue(const StepParams& P, const C
             if (!build) c.nbr_overflow = 0;
         },
         [&](Ctrl& c) {
+            c.halt_now = c.halted && !was_halted;
             if (c.halted) return;
             c.list_valid = build ? 1u : valid;
             if (build) {
@@ -259,38 +272,85 @@ __device__ __forceinline__ void list_block_prologue(const StepParams& P, const C
             } else if (!valid || !(c.disp_acc < P.skin_half)) {
                 c.halted = 1;
                 c.status = kStatusRebuild;
+                c.halt_now = 1;
                 if (c.wall_disappear) c.nwm_done = 0;  // the re-run prologue fires it again
+            } else if (fused && P.consistency_check && flags->list_long) {
+                c.halted = 1;
+                c.status = kStatusUnfused;
+                c.halt_now = 1;
+            } else if (fused) {
+                c.dt_new = c.cur_dt_const;
+                c.pending = 1;
             }
-        });
+        },
+        fused ? kCtrlFlagWord : kCtrlWords);
 }
 
 // Whether list_block_prologue (not a build) halts, from the same fields
 // (none of which the blocks of this kernel write).
-__device__ __forceinline__ bool list_step_halts(const StepParams& P, const Ctrl& N, double dmax) {
+__device__ __forceinline__ bool list_step_halts(const StepParams& P, const Ctrl& N, uint32_t outside, double dmax) {
     if (N.halted) return true;
     double t = N.time, disp = N.disp_acc;
     if (N.pending) {
-        if (P.consistency_check && ctrl_outside(N) > 0 && P.consistency_treatment == 1) return true;
+        if (P.consistency_check && outside > 0 && P.consistency_treatment == 1) return true;
         t += N.dt_new;
         disp += dmax;
     }
     return t > N.t_end || !N.list_valid || !(disp < P.skin_half);
 }
 
+// The index of the step that a kernel starting from `next` runs, in scalar registers.
+__device__ __forceinline__ unsigned long long list_step_index(const Ctrl* next) {
+    const unsigned long long k = next->step + (next->pending ? 1 : 0);
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k) |
+           ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(k >> 32)) << 32);
+}
+
 // At the head of a list step's first kernel (every thread of the block):
 // false when the step halts, else its step index in `step`.
 __device__ __forceinline__ bool list_step_begin(const StepParams& P, Ctrl* next, Ctrl* cur,
                                                 unsigned long long* dslots, unsigned long long& step) {
-    const double dmax = list_dmax(next, dslots);
-    const unsigned long long k = next->step + (next->pending ? 1 : 0);
-    step = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k) |
-           ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(k >> 32)) << 32);
-    const bool halts = list_step_halts(P, *next, dmax);
+    const double dmax = list_dmax(P, next, dslots);
+    step = list_step_index(next);
+    const bool halts = list_step_halts(P, *next, ctrl_outside(*next), dmax);
     if (blockIdx.x == 0) {
-        list_block_prologue(P, next, cur, dmax, false);
-        if (!halts) {  // this step's set; the blocks of this kernel read the other one
-            clear_slots(dslots + (uint32_t)(step & 1) * kSlotSet);
-            if (threadIdx.x == 0) next->outside_l[step & 1] = 0;
+        list_block_prologue(P, next, cur, next, dmax, false, false);
+        if (!halts) {  // this step's sets, and of four the next one's; the blocks of this kernel read neither
+            clear_slots(dslots + (uint32_t)(step & P.dset_mask) * kSlotSet);
+            if (P.dset_mask == 3) clear_slots(dslots + (uint32_t)((step + 1) & 3) * kSlotSet);
+            if (threadIdx.x < 2) next->outside_l[(step + threadIdx.x) & 3] = 0;
+        }
+    }
+    return !halts;
+}
+
+// Fused steps (dt constant, no wave maker): the pair pass integrates too.
+// It writes the next step's records to a second array, so that its other
+// blocks still read this step's, and (FP32, whose near cut-off tests read
+// the neighbours' FP64 positions) the positions to the other of two arrays.
+// Steps go in pairs, back and forth, so that a pair leaves everything where
+// the other kernels expect it; when the second of a pair halts, it puts the
+// positions back instead.  Where the pair pass is the step's only kernel
+// (continuity), the step also reads the control block in one place and
+// publishes in another, for the same reason, and clears the next step's
+// displacement set (of four) while its blocks fill their own; more entries
+// than max_neighbours - 1 in some list halt it (kStatusUnfused): the step
+// could not be undone if a particle had more neighbours.
+//
+// At the head of a fused continuity step (every thread): false when it halts.
+__device__ __forceinline__ bool fused_step_begin(const StepParams& P, const Ctrl* in, Ctrl* out, Ctrl* flags,
+                                                 unsigned long long* dslots, unsigned long long& step) {
+    const double dmax = list_dmax(P, in, dslots);
+    step = list_step_index(in);
+    uint32_t outside = flags->outside_l[0];
+#pragma unroll
+    for (uint32_t k = 1; k < 4; ++k) outside = (in->step & 3) == k ? flags->outside_l[k] : outside;
+    const bool halts = list_step_halts(P, *in, outside, dmax) || (P.consistency_check && flags->list_long);
+    if (blockIdx.x == 0) {
+        list_block_prologue(P, in, out, flags, dmax, false, true);
+        if (!halts) {
+            clear_slots(dslots + (uint32_t)((step + 1) & 3) * kSlotSet);
+            if (threadIdx.x == 0) flags->outside_l[(step + 1) & 3] = 0;
         }
     }
     return !halts;
@@ -301,17 +361,18 @@ __device__ __forceinline__ bool list_step_begin(const StepParams& P, Ctrl* next,
 __global__ void __launch_bounds__(kBlock) list_prologue(StepParams P, Ctrl* __restrict__ next, Ctrl* __restrict__ cur,
                                                         unsigned long long* __restrict__ dslots,
                                                         unsigned long long* __restrict__ maxslots) {
-    const double dmax = list_dmax(next, dslots);
-    list_block_prologue(P, next, cur, dmax, true);
+    const double dmax = list_dmax(P, next, dslots);
+    list_block_prologue(P, next, cur, next, dmax, true, false);
     // (also when the step halts: the step after a halt is a build and reads none of them)
+    for (uint32_t k = 0; k <= P.dset_mask; ++k) clear_slots(dslots + k * kSlotSet);
     for (uint32_t k = 0; k < 2; ++k) {
-        clear_slots(dslots + k * kSlotSet);
         clear_slots(maxslots + k * kDtSet);
         clear_slots(maxslots + k * kDtSet + kSlotSet);
     }
     if (threadIdx.x == 0) {
-        next->outside_l[0] = next->outside_l[1] = 0;
+        for (int k = 0; k < 4; ++k) next->outside_l[k] = 0;
         next->list_overflow = 0;
+        next->list_long = 0;
     }
 }
 
@@ -548,6 +609,7 @@ __global__ void __launch_bounds__(kBlock) list_build_kernel(StepParams P, Ctrl* 
     }
     out.flush();
     if (out.cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
+    if (out.cnt > P.max_nbr - 1) atomicOr(&next->list_long, 1u);
     if (inb) nbc[s] = min(out.cnt, P.list_cap);
 }
 
@@ -1051,16 +1113,72 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* n
     pres[s] = p;
 }
 
+// Where a 2D step leaves the state, the next step's records and keys, and
+// the control block with the flags it raises.
+template <class R> struct ListOut {
+    double2* pos;
+    real4<R>* va;
+    ListRec<R>* rec;
+    const uint32_t* home;
+    uint32_t* key_next;
+    Ctrl* flags;
+    bool second;  // fused steps: the second of a pair
+};
+// whole_step of slot s, its cell key for the next build and the records of
+// the next step's pair pass: near (the new position relative to the home
+// cell, the new velocity) and pred (PredictHalfStep.cpp:16-22 with this
+// step's dt, which is the next step's).  The square of its displacement.
+template <class R>
+__device__ __forceinline__ double step_listed(const StepParams& P, const Ctrl& c, uint32_t s, double2 p0,
+                                              const real4<R>& va, const real4<R>& pr, uint32_t oid, uint32_t h,
+                                              const real4<R>& d, const real2<R>& x, double dt, const ListOut<R>& O,
+                                              uint32_t& outside, uint32_t& bad) {
+    const Stepped2<R> o = whole_step_one<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, x.x, x.y, dt, outside);
+    O.pos[s] = o.pos;
+    O.va[s] = o.va;
+    O.key_next[s] = (int)o.va.w == 0 ? P.ncells : cell_key(P, o.pos.x, o.pos.y, bad);
+    R p;
+    ListRec<R> r;
+    r.pr = predict_record<R>(P, o.va, d.x, d.y, d.z, (R)dt, p);
+    r.nr = near_record<R>(P, o.pos, o.va.x, o.va.y, h);
+    O.rec[s] = r;
+    const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y;
+    return mx * mx + my * my;
+}
+// The flags of step `step` and its largest displacement (every thread).
+__device__ __forceinline__ void finish_listed(const StepParams& P, Ctrl* flags, unsigned long long step,
+                                              uint32_t outside, uint32_t bad, double moved2,
+                                              unsigned long long* dslots, uint32_t blk) {
+    wave_count_add(&flags->outside_l[step & 3], outside);
+    if (bad) atomicOr(&flags->grid_overflow, 1u);
+    block_max_to_slots(moved2, 0.0, dslots + (uint32_t)(step & P.dset_mask) * kSlotSet, nullptr, blk);
+}
+
+// At the head of a fused pair pass behind the summation pass (every thread):
+// as list_dt, dt being constant; too many neighbours were found by the
+// summation pass.
+__device__ __forceinline__ bool fused_pair_begin(const StepParams& P, Ctrl* next, const Ctrl* cur) {
+    const bool halted = cur->halted != 0;
+    const uint32_t halt_status = !halted && P.consistency_check && next->nbr_overflow ? 3u : 0u;
+    if (blockIdx.x == 0) publish_ctrl(cur, next, cur->cur_dt_const, halt_status);
+    return !halted && halt_status == 0;
+}
+
 // Pair pass from the lists: continuity density rate, pressure, artificial
 // viscosity, Lennard-Jones walls and XSPH (the cubic configuration of
 // pair_fast_kernel), the dt maxima, and the fields for the integrator.  With
 // continuity it also writes the pressure of the current density (the
 // reference's p array).
-template <class R, bool FIRST, int LPP, bool CONT, bool ALL>
-__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 4 : LPP == 1 ? 6 : 1) pair_list_kernel(
-    StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
-    const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
-    real2<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
+// FUSED: see fused_step_begin.  200 steps of 6,923 particles (FP64) take 2.35 ms
+// so, 2.88 with an integrator of their own (4 us of a step's 14, and a launch
+// gap); 30 of 134,603 (summation, FP32) 1.50 against 1.58.
+template <class R, bool FIRST, int LPP, bool CONT, bool ALL, bool FUSED>
+__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? (FUSED ? 3 : 4) : LPP == 1 ? (FUSED ? 5 : 6) : 1)
+    pair_list_kernel(StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec,
+                     R* __restrict__ pres, const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc,
+                     real4<R>* __restrict__ der, real2<R>* __restrict__ xs,
+                     unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots,
+                     ListOut<R> O) {
     const uint32_t lb = xcd_block(group_blocks_per_xcd<LPP>(P.n));
     if (lb >= group_blocks<LPP>(P.n)) return;
     __shared__ float2 s_off[64];
@@ -1077,7 +1195,24 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 4 : LPP == 1 ? 6 : 1)
         cnt = nbc[s];
     }
     unsigned long long step;
-    if constexpr (FIRST) {
+    double dt = 0;
+    if constexpr (FUSED) {
+        bool goes, back;  // back: the pair's first step left the positions in the other array
+        if constexpr (CONT) {
+            back = !next->halted;
+            goes = fused_step_begin(P, next, cur, O.flags, dslots, step);
+            dt = next->pending ? next->dt_new : next->dt;
+        } else {
+            back = cur->halt_now || !cur->halted;
+            goes = fused_pair_begin(P, next, cur);
+            step = cur->step;
+            dt = cur->cur_dt_const;
+        }
+        if (!goes) {
+            if (O.second && back && X.pos != O.pos && live && g.l == 0) O.pos[s] = X.pos[s];
+            return;
+        }
+    } else if constexpr (FIRST) {
         if (!list_step_begin(P, next, cur, dslots, step)) return;
     } else {
         if (!list_step_goes(cur)) return;
@@ -1103,7 +1238,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 4 : LPP == 1 ? 6 : 1)
         // 0, so that a pair of dead particles gives no number
         if (cnt == 0) S = ListSums<R>();
     }
-    if (overflow) atomicOr(&next->nbr_overflow, 1u);
+    if (!FUSED && overflow) atomicOr(&next->nbr_overflow, 1u);
     const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);
     const R ax = lane_sum<LPP>(S.ljx + mF * S.sx);
     const R ay = -(R)P.g + lane_sum<LPP>(S.ljy + mF * S.sy);
@@ -1123,6 +1258,20 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 4 : LPP == 1 ? 6 : 1)
         x.y = xy;
         xs[s] = x;
         if (P.density_treatment != 0) pres[s] = eos_p<R>(X.va[s].z, (R)P.rho0, (R)P.eos_B);
+    }
+    if constexpr (FUSED) {
+        uint32_t outside = 0, bad = 0;
+        double moved2 = 0.0;
+        if (live && g.l == 0) {
+            Ctrl c{};  // what whole_step reads of it without a wave maker
+            c.cur_first = step == 0;
+            const real4<R> d{ax, ay, drho, amu};
+            const real2<R> x{xx, xy};
+            real4<R> pr{};
+            if (!CONT) pr.z = fabs(prj.z);  // the summed density
+            moved2 = step_listed<R>(P, c, s, X.pos[s], X.va[s], pr, 0u, O.home[s], d, x, dt, O, outside, bad);
+        }
+        finish_listed(P, O.flags, step, outside, bad, moved2, dslots, lb);
     }
 }
 
@@ -1388,28 +1537,16 @@ __global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ct
     const Ctrl& c = *cur;
     double dt;
     if (!list_dt(P, next, cur, maxslots, dt)) return;
-    const uint32_t par = (uint32_t)(c.step & 1);
     uint32_t outside = 0, bad = 0;
     double moved2 = 0.0;
     if (live) {
         const bool reordered = A.oid != X.oid;
         const uint32_t oid = reordered || step_needs_oid(P, c, (int)va.w) ? X.oid[s] : 0u;
-        const Stepped2<R> o = whole_step_one<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, x.x, x.y, dt, outside);
-        A.pos[s] = o.pos;
-        A.va[s] = o.va;
+        moved2 = step_listed<R>(P, c, s, p0, va, pr, oid, h, d, x, dt, ListOut<R>{A.pos, A.va, rec, home, key_next, next, false},
+                                outside, bad);
         if (reordered) A.oid[s] = oid;
-        key_next[s] = (int)o.va.w == 0 ? P.ncells : cell_key(P, o.pos.x, o.pos.y, bad);
-        const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y;
-        moved2 = mx * mx + my * my;
-        R p;
-        ListRec<R> r;
-        r.pr = predict_record<R>(P, o.va, d.x, d.y, d.z, (R)dt, p);
-        r.nr = near_record<R>(P, o.pos, o.va.x, o.va.y, h);
-        rec[s] = r;
     }
-    wave_count_add(&next->outside_l[par], outside);
-    if (bad) atomicOr(&next->grid_overflow, 1u);
-    block_max_to_slots(moved2, 0.0, dslots + par * kSlotSet, nullptr, blockIdx.x);
+    finish_listed(P, next, c.step, outside, bad, moved2, dslots, blockIdx.x);
 }
 
 }  // namespace rrsph

@@ -213,6 +213,7 @@ __global__ void __launch_bounds__(kBlock) list_build3_kernel(StepParams P, Ctrl*
     out.flush();
     if (!inb) return;
     if (out.cnt > P.list_cap || bad) atomicOr(&next->list_overflow, 1u);
+    if (out.cnt > P.max_nbr - 1) atomicOr(&next->list_long, 1u);
     nbc[s] = min(out.cnt, P.list_cap);
 }
 
@@ -481,6 +482,37 @@ __device__ __forceinline__ void list_pair_term3(const K_& K, ListSums3<R>& S, bo
     }
 }
 
+// As ListOut and step_listed in 3D (dens only where the summation pass reads it).
+template <class R> struct ListOut3 {
+    double4* pos;
+    real4<R>* va;
+    ListRec<R>* rec;
+    real4<R>* dens;
+    const uint32_t* home;
+    uint32_t* key_next;
+    Ctrl* flags;
+    bool second;
+};
+template <class R>
+__device__ __forceinline__ double step_listed3(const StepParams& P, const Ctrl& c, uint32_t s, double4 p0,
+                                               const real4<R>& va, const real4<R>& pr, uint32_t oid, uint32_t h,
+                                               const real4<R>& d, const real4<R>& x, double dt, const ListOut3<R>& O,
+                                               uint32_t& outside, uint32_t& bad) {
+    const Stepped3<R> o = whole_step_one3<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, d.w, x.x, x.y, x.z, dt, outside);
+    O.pos[s] = o.pos;
+    O.va[s] = o.va;
+    const int itype = (int)o.pos.w;
+    O.key_next[s] = itype == 0 ? P.ncells : cell_key3(P, o.pos.x, o.pos.y, o.pos.z, bad);
+    R pw, p;
+    ListRec<R> r;
+    r.pr = predict3<R>(P, o.va, itype, d, (R)dt, pw, p);
+    r.nr = near3<R>(P, o.pos, pw, h);
+    O.rec[s] = r;
+    if (P.density_treatment == 0) O.dens[s] = near3<R>(P, o.pos, typed_rho<R>(o.va.w, itype), h);
+    const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y, mz = o.pos.z - p0.z;
+    return mx * mx + my * my + mz * mz;
+}
+
 // Pair pass from the 3D lists: the cubic configuration of pair3_kernel
 // (continuity, pressure, artificial viscosity, Lennard-Jones walls, XSPH),
 // the dt maxima and the fields for the integrator.  Entries in rounds of G,
@@ -491,17 +523,29 @@ __device__ __forceinline__ void list_pair_term3(const K_& K, ListSums3<R>& S, bo
 // with 3, 253 with 2; 310 when each lane gathered its own; 943,906 particles,
 // continuity, which gathers the velocity too: 515 with 3, 576 with 2, 633 by
 // lane).  Two blocks per CU hold enough loads in flight then.
-template <class R, bool FIRST, bool CONT, bool ALL>
+// FUSED (behind the summation pass): see fused_step_begin; 16 steps of 6.6M
+// particles (FP32) 62.0 -> 60.5 ms, of which 8 are copies.
+template <class R, bool FIRST, bool CONT, bool ALL, bool FUSED>
 __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState3<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
     const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc, real4<R>* __restrict__ der,
-    real4<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots) {
+    real4<R>* __restrict__ xs, unsigned long long* __restrict__ maxslots, unsigned long long* __restrict__ dslots,
+    ListOut3<R> O) {
+    static_assert(!(FUSED && CONT), "a fused 3D step has a summation pass");
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
     __shared__ float4 s_off[kCodes3];
     fill_cell_offsets3(P, s_off);
     unsigned long long step;
-    if constexpr (FIRST) {
+    if constexpr (FUSED) {
+        const bool back = cur->halt_now || !cur->halted;  // as in pair_list_kernel
+        if (!fused_pair_begin(P, next, cur)) {
+            const uint32_t s = lb * kBlock + threadIdx.x;
+            if (O.second && back && X.pos != O.pos && s < P.n) O.pos[s] = X.pos[s];
+            return;
+        }
+        step = cur->step;
+    } else if constexpr (FIRST) {
         if (!list_step_begin(P, next, cur, dslots, step)) return;
     } else {
         if (!list_step_goes(cur)) return;
@@ -582,7 +626,7 @@ __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
             });
         }
     }
-    if (overflow) atomicOr(&next->nbr_overflow, 1u);
+    if (!FUSED && overflow) atomicOr(&next->nbr_overflow, 1u);
     const R mF = (R)P.lp_mF, mW = K.xsph_on ? (R)P.lp_mW : R(0);
     const R ax = S.ljx + mF * S.sx;
     const R ay = -(R)P.g + S.ljy + mF * S.sy;
@@ -605,6 +649,20 @@ __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
         x.w = amu;
         xs[s] = x;
         if (P.density_treatment != 0) pres[s] = eos_p<R>(vaj.w, (R)P.rho0, (R)P.eos_B);
+    }
+    if constexpr (FUSED) {
+        uint32_t outside = 0, bad = 0;
+        double moved2 = 0.0;
+        if (live) {
+            Ctrl c{};  // what whole_step reads of it without a wave maker
+            c.cur_first = step == 0;
+            const real4<R> d{ax, ay, az, drho}, x{mW * S.xx, mW * S.xy, mW * S.xz, amu};
+            real4<R> pr{};
+            pr.w = fabs(rj.pr.w);  // the summed density
+            moved2 = step_listed3<R>(P, c, s, X.pos[s], vaj, pr, 0u, O.home[s], d, x, cur->cur_dt_const, O, outside,
+                                     bad);
+        }
+        finish_listed(P, O.flags, step, outside, bad, moved2, dslots, lb);
     }
 }
 
@@ -634,31 +692,16 @@ __global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, C
     const Ctrl& c = *cur;
     double dt;
     if (!list_dt(P, next, cur, maxslots, dt)) return;
-    const uint32_t par = (uint32_t)(c.step & 1);
     uint32_t outside = 0, bad = 0;
     double moved2 = 0.0;
     if (live) {
         const bool reordered = A.oid != X.oid;
         const uint32_t oid = reordered || step_needs_oid(P, c, (int)p0.w) ? X.oid[s] : 0u;
-        const Stepped3<R> o =
-            whole_step_one3<R>(P, c, p0, va, pr, oid, d.x, d.y, d.z, d.w, x.x, x.y, x.z, dt, outside);
-        A.pos[s] = o.pos;
-        A.va[s] = o.va;
+        moved2 = step_listed3<R>(P, c, s, p0, va, pr, oid, h, d, x, dt,
+                                 ListOut3<R>{A.pos, A.va, rec, dens, home, key_next, next, false}, outside, bad);
         if (reordered) A.oid[s] = oid;
-        const int itype = (int)o.pos.w;
-        key_next[s] = itype == 0 ? P.ncells : cell_key3(P, o.pos.x, o.pos.y, o.pos.z, bad);
-        const double mx = o.pos.x - p0.x, my = o.pos.y - p0.y, mz = o.pos.z - p0.z;
-        moved2 = mx * mx + my * my + mz * mz;
-        R pw, p;
-        ListRec<R> r;
-        r.pr = predict3<R>(P, o.va, itype, d, (R)dt, pw, p);
-        r.nr = near3<R>(P, o.pos, pw, h);
-        rec[s] = r;
-        if (P.density_treatment == 0) dens[s] = near3<R>(P, o.pos, typed_rho<R>(o.va.w, itype), h);
     }
-    wave_count_add(&next->outside_l[par], outside);
-    if (bad) atomicOr(&next->grid_overflow, 1u);
-    block_max_to_slots(moved2, 0.0, dslots + par * kSlotSet, nullptr, blockIdx.x);
+    finish_listed(P, next, c.step, outside, bad, moved2, dslots, blockIdx.x);
 }
 
 }  // namespace rrsph

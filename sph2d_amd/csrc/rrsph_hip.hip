@@ -256,6 +256,9 @@ struct rrsph_ctx {
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
     ListGraphs list_graphs[2];          // of plain runs and of taped ones (another skin)
     bool taping = false;                // ctx->P holds the taped runs' skin
+    bool fuse = false;                  // list steps may run in fused pairs (fused_step_begin)
+    void* rec1 = nullptr;               // fused steps: the second array of records
+    Ctrl* ctrl_alt = nullptr;           // ... and, with continuity, control block
     uint64_t build_at = 0;              // step index of the last build launched
     double tape_skin = 0;               // skin of taped runs (fraction of the cut-off)
     uint64_t list_interval = 8;         // steps between builds
@@ -475,48 +478,90 @@ template <class R> void enqueue_step3_t(rrsph_ctx* c, Profiler* prof, bool full_
     }
 }
 
+// A list step's kind: a build, a list step, or the first or second of a pair
+// of fused ones (fused_step_begin in list_step.hpp).
+enum ListStep { kBuildStep, kPlainStep, kFusedFirst, kFusedSecond };
+
+// The arrays between which fused steps go back and forth: the records, and in
+// FP32 the positions.
+void fused_arrays(rrsph_ctx* c, ListStep kind, void*& rec, void*& rec_out, double2*& pos, double2*& pos_out) {
+    const bool second = kind == kFusedSecond;
+    rec = second ? c->rec1 : c->rec;
+    rec_out = second ? c->rec : c->rec1;
+    pos = second && c->fp32 ? c->posB : c->posA;
+    pos_out = !second && c->fp32 ? c->posB : c->posA;
+}
+
 // The summation and pair passes of a 2D neighbour-list step, LPP lanes per particle.
-template <class R, int LPP, bool ALL> void enqueue_list_passes(rrsph_ctx* c, Launcher& L, const ListState<R>& X, bool build) {
+template <class R, int LPP, bool ALL>
+void enqueue_list_passes(rrsph_ctx* c, Launcher& L, ListState<R> X, ListStep kind) {
     const StepParams& P = c->P;
     const uint32_t nb = group_blocks_per_xcd<LPP>(P.n) * kNumXcd;
     ListRec<R>* rec = (ListRec<R>*)c->rec;
-    bool first = !build;
+    Ctrl *next = c->ctrl, *cur = c->ctrl_cur;
+    ListOut<R> O{};
+    const bool fused = kind == kFusedFirst || kind == kFusedSecond;
+    if (fused) {
+        void *r, *ro;
+        double2 *p, *po;
+        fused_arrays(c, kind, r, ro, p, po);
+        rec = (ListRec<R>*)r;
+        X.pos = p;
+        O = ListOut<R>{po, (real4<R>*)c->vaA, (ListRec<R>*)ro, c->home, c->key_next, c->ctrl, kind == kFusedSecond};
+    }
+    bool first = kind != kBuildStep;
     if (P.density_treatment == 0) {
         auto density = [&](auto kernel) {
             L(K_DENSITY_SUM, [&] {
-                kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     c->dslots);
+                kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc, c->dslots);
             });
         };
         if (first) density(density_sum_list<R, true, LPP>);
         else density(density_sum_list<R, false, LPP>);
         first = false;
+    } else if (fused) {  // the step's only kernel reads the control block here and publishes there
+        next = kind == kFusedSecond ? c->ctrl_alt : c->ctrl;
+        cur = kind == kFusedSecond ? c->ctrl : c->ctrl_alt;
     }
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
-            kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
+                                                 (real4<R>*)c->adA, (real2<R>*)c->xs, c->dtslots, c->dslots, O);
+        });
+    };
+    auto general = [&](auto kernel) {
+        L(K_PAIR, [&] {
+            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
                                                  (real4<R>*)c->adA, (real2<R>*)c->xs, c->dtslots, c->dslots);
         });
     };
+    if constexpr (ALL) {
+        if (fused) {
+            if (P.density_treatment == 0) pair(pair_list_kernel<R, false, LPP, false, true, true>);
+            else pair(pair_list_kernel<R, true, LPP, true, true, true>);
+            return;
+        }
+    }
     if (c->fast_pair) {
-        if (P.density_treatment == 0) pair(pair_list_kernel<R, false, LPP, false, ALL>);
-        else if (first) pair(pair_list_kernel<R, true, LPP, true, ALL>);
-        else pair(pair_list_kernel<R, false, LPP, true, ALL>);
+        if (P.density_treatment == 0) pair(pair_list_kernel<R, false, LPP, false, ALL, false>);
+        else if (first) pair(pair_list_kernel<R, true, LPP, true, ALL, false>);
+        else pair(pair_list_kernel<R, false, LPP, true, ALL, false>);
+    } else if (first) {
+        general(pair_list_general_kernel<R, true, LPP>);
     } else {
-        if (first) pair(pair_list_general_kernel<R, true, LPP>);
-        else pair(pair_list_general_kernel<R, false, LPP>);
+        general(pair_list_general_kernel<R, false, LPP>);
     }
 }
 
-// One neighbour-list step (build: sort, reorder and new lists first).
-template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool build) {
+// One neighbour-list step (a build: sort, reorder and new lists first).
+template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, ListStep kind) {
     Launcher L{c, prof};
     const StepParams& P = c->P;
     const uint32_t nb = grid_blocks(P.n, kBlock);
     const uint32_t nb_xcd = P.blocks_per_xcd * kNumXcd;
     ListState<R> X{c->posA, (const real4<R>*)c->vaA, c->oidA};
     ListRec<R>* rec = (ListRec<R>*)c->rec;
-    if (build) {
+    if (kind == kBuildStep) {
         L(K_PROLOGUE, [&] {
             list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
         });
@@ -534,10 +579,11 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool b
         X = ListState<R>{c->posB, (const real4<R>*)c->vaB, c->oidB};
     }
     // the first kernel of a list step makes its prologue
-    if (!c->all_terms && c->fast_pair) enqueue_list_passes<R, 1, false>(c, L, X, build);
-    else if (c->lanes == 8) enqueue_list_passes<R, 8, true>(c, L, X, build);
-    else if (c->lanes == 2) enqueue_list_passes<R, 2, true>(c, L, X, build);
-    else enqueue_list_passes<R, 1, true>(c, L, X, build);
+    if (!c->all_terms && c->fast_pair) enqueue_list_passes<R, 1, false>(c, L, X, kind);
+    else if (c->lanes == 8) enqueue_list_passes<R, 8, true>(c, L, X, kind);
+    else if (c->lanes == 2) enqueue_list_passes<R, 2, true>(c, L, X, kind);
+    else enqueue_list_passes<R, 1, true>(c, L, X, kind);
+    if (kind == kFusedFirst || kind == kFusedSecond) return;
     L(K_INTEGRATE, [&] {
         integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real2<R>*)c->xs, rec, c->home, stateA<R>(c),
                                                                c->key_next, c->dtslots, c->dslots);
@@ -545,7 +591,7 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, bool b
 }
 
 // One 3D neighbour-list step (build: sort, reorder and new lists first).
-template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool build) {
+template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListStep kind) {
     Launcher L{c, prof};
     const StepParams& P = c->P;
     const uint32_t nb = grid_blocks(P.n, kBlock);
@@ -553,6 +599,17 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     ListState3<R> X{(const double4*)c->posA, (const real4<R>*)c->vaA, c->oidA};
     ListRec<R>* rec = (ListRec<R>*)c->rec;
     real4<R>* dens = (real4<R>*)c->dens;
+    const bool build = kind == kBuildStep, fused = kind == kFusedFirst || kind == kFusedSecond;
+    ListOut3<R> O{};
+    if (fused) {
+        void *r, *ro;
+        double2 *p, *po;
+        fused_arrays(c, kind, r, ro, p, po);
+        rec = (ListRec<R>*)r;
+        X.pos = (const double4*)p;
+        O = ListOut3<R>{(double4*)po,    (real4<R>*)c->vaA, (ListRec<R>*)ro,      dens,
+                        c->home, c->key_next,       c->ctrl, kind == kFusedSecond};
+    }
     if (build) {
         L(K_PROLOGUE, [&] {
             list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
@@ -585,7 +642,7 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
             kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     (real4<R>*)c->adA, (real4<R>*)c->xs, c->dtslots, c->dslots);
+                                                     (real4<R>*)c->adA, (real4<R>*)c->xs, c->dtslots, c->dslots, O);
         });
     };
     auto choose = [&](auto summed, auto first_kernel, auto kernel) {
@@ -593,12 +650,16 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
         else if (first) pair(first_kernel);
         else pair(kernel);
     };
+    if (fused) {
+        pair(pair_list3_kernel<R, false, false, true, true>);
+        return;
+    }
     if (c->all_terms)
-        choose(pair_list3_kernel<R, false, false, true>, pair_list3_kernel<R, true, true, true>,
-               pair_list3_kernel<R, false, true, true>);
+        choose(pair_list3_kernel<R, false, false, true, false>, pair_list3_kernel<R, true, true, true, false>,
+               pair_list3_kernel<R, false, true, true, false>);
     else
-        choose(pair_list3_kernel<R, false, false, false>, pair_list3_kernel<R, true, true, false>,
-               pair_list3_kernel<R, false, true, false>);
+        choose(pair_list3_kernel<R, false, false, false, false>, pair_list3_kernel<R, true, true, false, false>,
+               pair_list3_kernel<R, false, true, false, false>);
     L(K_INTEGRATE, [&] {
         integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X,
                                                                 (const real4<R>*)c->xs, rec, dens, c->home,
@@ -606,14 +667,14 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, bool 
     });
 }
 
-void enqueue_list_step(rrsph_ctx* c, Profiler* prof, bool build) {
+void enqueue_list_step(rrsph_ctx* c, Profiler* prof, ListStep kind) {
     if (c->P.dim == 3) {
-        if (c->fp32) enqueue_list_step3_t<float>(c, prof, build);
-        else enqueue_list_step3_t<double>(c, prof, build);
+        if (c->fp32) enqueue_list_step3_t<float>(c, prof, kind);
+        else enqueue_list_step3_t<double>(c, prof, kind);
         return;
     }
-    if (c->fp32) enqueue_list_step_t<float>(c, prof, build);
-    else enqueue_list_step_t<double>(c, prof, build);
+    if (c->fp32) enqueue_list_step_t<float>(c, prof, kind);
+    else enqueue_list_step_t<double>(c, prof, kind);
 }
 
 bool list_active(const rrsph_ctx* c) { return c->list_mode && !c->list_suspended; }
@@ -628,6 +689,16 @@ void enqueue_step(rrsph_ctx* c, Profiler* prof, bool full_sort) {
     else enqueue_step_t<double>(c, prof, full_sort);
 }
 
+void drop_list_graphs(rrsph_ctx* c) {
+    for (ListGraphs& G : c->list_graphs) {
+        for (auto e : G.exec)
+            if (e) (void)hipGraphExecDestroy(e);
+        for (auto g : G.graph)
+            if (g) (void)hipGraphDestroy(g);
+        G = ListGraphs{};
+    }
+}
+
 void drop_graph(rrsph_ctx* c) {
     hipGraphExec_t* ex[] = {&c->gexec, &c->gexec_full};
     hipGraph_t* gr[] = {&c->graph, &c->graph_full};
@@ -639,13 +710,7 @@ void drop_graph(rrsph_ctx* c) {
         if (*g) (void)hipGraphDestroy(*g);
         *g = nullptr;
     }
-    for (ListGraphs& G : c->list_graphs) {
-        for (auto e : G.exec)
-            if (e) (void)hipGraphExecDestroy(e);
-        for (auto g : G.graph)
-            if (g) (void)hipGraphDestroy(g);
-        G = ListGraphs{};
-    }
+    drop_list_graphs(c);
 }
 
 // Capture one step with the incremental re-sort and one with the full sort.
@@ -665,15 +730,23 @@ rrsph_status build_graph(rrsph_ctx* ctx) {
 // Launch a build step (build) or `steps` list steps (a power of two up to
 // kListRunMax) through the captured graphs, or directly.
 rrsph_status launch_list_run(rrsph_ctx* ctx, bool build, uint32_t steps) {
+    auto enqueue = [&]() {
+        for (uint32_t k = 0; k < steps; ++k) {
+            const ListStep kind = build ? kBuildStep
+                                  : ctx->fuse && !ctx->taping && steps > 1 ? (k & 1 ? kFusedSecond : kFusedFirst)
+                                                                           : kPlainStep;
+            enqueue_list_step(ctx, nullptr, kind);
+        }
+    };
     if (!ctx->use_graph) {
-        for (uint32_t k = 0; k < steps; ++k) enqueue_list_step(ctx, nullptr, build);
+        enqueue();
         return RRSPH_OK;
     }
     ListGraphs& G = ctx->list_graphs[ctx->taping ? 1 : 0];
     const uint32_t i = build ? 0 : 1 + (uint32_t)__builtin_ctz(steps);
     if (!G.exec[i]) {
         HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        for (uint32_t k = 0; k < steps; ++k) enqueue_list_step(ctx, nullptr, build);
+        enqueue();
         HIP_TRY(hipStreamEndCapture(ctx->stream, &G.graph[i]));
         HIP_TRY(hipGraphInstantiate(&G.exec[i], G.graph[i], nullptr, nullptr, 0));
     }
@@ -1013,6 +1086,12 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     // 1,020,263 61.4 / 61.6 / 146.7)
     ctx->lanes = P.n < 25000 ? 8 : 2;
     if (P.n >= 150000 && ctx->fast_pair && ctx->fp32 && P.density_treatment != 0) ctx->lanes = 1;
+    // fused pairs of list steps: the cubic configuration with a constant dt
+    // and no wave maker (in 3D with a summation pass: its continuity pass
+    // gathers the neighbours' state)
+    ctx->fuse = ctx->fast_pair && ctx->all_terms && P.dt_method != 2 && !P.boundary_motion &&
+                (!d3 || P.density_treatment == 0);
+    P.dset_mask = ctx->fuse && P.density_treatment != 0 ? 3 : 1;
     // a taped run keeps every build's lists, so that its builds cost more: 12
     // steps and their gradients, 943,906 particles (3D FP32), 30.6 ms at 0.08,
     // 25.3 at 0.1, 23.1 at 0.125, 23.6 at 0.15
@@ -1071,7 +1150,7 @@ void free_all(rrsph_ctx* c) {
                     c->maxslots, c->LB, c->ctrl, c->ctrl_cur,
                     c->util_ctrl, c->red, c->st_r, c->st_v, c->st_rho, c->st_p, c->st_a, c->st_drho, c->st_av,
                     c->st_mu, c->st_itype, c->st_u32, c->skeyA, c->chg, c->chg_mask, c->wpre, c->pw,
-                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->dtslots, c->cand};
+                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->dtslots, c->cand, c->rec1, c->ctrl_alt};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
@@ -1207,11 +1286,15 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
         if (dim == 3) ctx->dens = dalloc<double4>(n, e);
         if (dim == 3) ctx->cand = dalloc<float4>(n, e);
         ctx->home = dalloc<uint32_t>(n, e);
-        ctx->dslots = dalloc<unsigned long long>(2 * kSlotSet, e);
+        ctx->dslots = dalloc<unsigned long long>(4 * kSlotSet, e);
+        if (ctx->fuse) {
+            ctx->rec1 = dalloc<char>(2 * r4 * n, e);
+            ctx->ctrl_alt = dalloc<Ctrl>(1, e);
+        }
         ctx->dtslots = dalloc<unsigned long long>(2 * kDtSet, e);
     }
     if (e != hipSuccess) return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-    if (ctx->dslots) HIP_TRY(hipMemset(ctx->dslots, 0, 2 * kSlotSet * sizeof(unsigned long long)));
+    if (ctx->dslots) HIP_TRY(hipMemset(ctx->dslots, 0, 4 * kSlotSet * sizeof(unsigned long long)));
     if (ctx->nbl) HIP_TRY(hipMemset(ctx->nbl, 0, (size_t)(ctx->P.list_cap + kListPad) * n * sizeof(uint32_t)));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_ctrl, sizeof(Ctrl), hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_eta, kMaxGauges * sizeof(double), hipHostMallocDefault));
@@ -1449,6 +1532,10 @@ static rrsph_status resume_halt(rrsph_ctx* ctx, bool* resumed) {
         note_resort_overflow(ctx, at);
     } else if (c.status == kStatusRebuild) {
         note_list_stale(ctx, at);
+    } else if (c.status == kStatusUnfused) {
+        ctx->fuse = false;
+        drop_list_graphs(ctx);  // (the stream is idle)
+        ctx->need_full = true;
     } else if (c.status == kStatusListOverflow) {
         ctx->list_mode = false;  // more candidates than a list holds: sort every step from here
         ctx->need_full = true;
@@ -1823,7 +1910,7 @@ rrsph_status rrsph_hip_profile_steps(rrsph_ctx* ctx, uint32_t nsteps, double* av
     for (uint32_t k = 0; k < nsteps; ++k) {
         if (list_active(ctx)) {
             const bool build = next_is_build(ctx, first + k);
-            enqueue_list_step(ctx, &prof, build);
+            enqueue_list_step(ctx, &prof, build ? kBuildStep : kPlainStep);
             if (build) {
                 ctx->build_at = first + k;
                 ++ctx->n_build;

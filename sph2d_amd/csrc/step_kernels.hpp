@@ -205,7 +205,7 @@ __device__ __forceinline__ bool prologue_commit(const StepParams& P, Ctrl& c) {
     c.amax_bits = 0;
     c.mumax_bits = 0;
     c.outside = 0;
-    c.outside_l[0] = c.outside_l[1] = 0;
+    c.outside_l[0] = c.outside_l[1] = c.outside_l[2] = c.outside_l[3] = 0;
     return true;
 }
 
@@ -242,7 +242,7 @@ __device__ __forceinline__ unsigned long long ctrl_word(const Ctrl* ctrl) {
 
 template <class B, class A>
 __device__ __forceinline__ void block_prologue(const StepParams& P, Ctrl* out_ctrl, unsigned long long word, B&& before,
-                                               A&& after) {
+                                               A&& after, uint32_t words = kCtrlWords) {
     if (threadIdx.x < kWave) {
         union {
             Ctrl c;
@@ -281,7 +281,7 @@ __device__ __forceinline__ void block_prologue(const StepParams& P, Ctrl* out_ct
         unsigned long long out = 0;
 #pragma unroll
         for (uint32_t i = 0; i < kCtrlWords; ++i) out = threadIdx.x == i ? u.w[i] : out;
-        if (threadIdx.x < kCtrlWords) reinterpret_cast<unsigned long long*>(out_ctrl)[threadIdx.x] = out;
+        if (threadIdx.x < words) reinterpret_cast<unsigned long long*>(out_ctrl)[threadIdx.x] = out;
     }
     __syncthreads();
 }
