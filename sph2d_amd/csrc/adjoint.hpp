@@ -118,8 +118,12 @@ __host__ __device__ inline uint32_t gauge_blocks(uint32_t n) {
 template <class R>
 __global__ void __launch_bounds__(kBlock) smooth_gauge_partials(uint32_t n, const double2* __restrict__ pos,
                                                                 const real4<R>* __restrict__ va, GaugeSpec G,
-                                                                double* __restrict__ partials) {
+                                                                double* __restrict__ partials, size_t stride) {
     __shared__ GaugeLds L;
+    // row y of the grid: the state y strides further on, its partials in a row of their own
+    pos = (const double2*)((const char*)pos + blockIdx.y * stride);
+    va = (const real4<R>*)((const char*)va + blockIdx.y * stride);
+    partials += (size_t)blockIdx.y * 2 * G.n * gridDim.x;
     gauge_lds_clear(G, L);
     const double inv_r2 = 1.0 / (G.radius * G.radius);
     for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
@@ -151,6 +155,10 @@ __global__ void __launch_bounds__(kBlock) smooth_gauge_final(uint32_t nblocks, G
     __shared__ double s_z[kBlock / kWave], s_w[kBlock / kWave];
     const uint32_t g = blockIdx.x;
     if (g >= G.n) return;
+    partials += (size_t)blockIdx.y * 2 * G.n * nblocks;  // row y of the grid: the next state's
+    eta += (size_t)blockIdx.y * kMaxGauges;
+    zsum += (size_t)blockIdx.y * kMaxGauges;
+    wsum += (size_t)blockIdx.y * kMaxGauges;
     if (ctrl) {
         const size_t row = (size_t)min(ctrl->step - base, (uint64_t)nsteps - 1) * kMaxGauges;
         eta += row;
@@ -264,14 +272,7 @@ struct AdjStep {
 };
 
 // After a step: what its adjoint needs from the control block.
-// Record of the step just launched, at rec[k], k = its step index (the
-// control block's step count, committed at the next prologue) - base,
-// clamped to the tape's nsteps records: a step after a halt does not run,
-// and its record lands on the halted step's, which the resumed range
-// writes again.
-__global__ void adj_record(const Ctrl* __restrict__ ctrl, AdjStep* __restrict__ rec, uint64_t base, uint32_t nsteps) {
-    const Ctrl& c = *ctrl;
-    const uint64_t k = min(c.step - base, (uint64_t)nsteps - 1);
+__device__ __forceinline__ AdjStep step_record(const Ctrl& c) {
     AdjStep r;
     r.t = c.cur_time;
     r.dt = c.dt_new;
@@ -280,7 +281,24 @@ __global__ void adj_record(const Ctrl* __restrict__ ctrl, AdjStep* __restrict__ 
     r.piston = c.piston_active;
     r.halted = c.halted;
     r.pad = 0;
-    rec[k] = r;
+    return r;
+}
+// Record of the step just launched, at rec[k], k = its step index (the
+// control block's step count, committed at the next prologue) - base,
+// clamped to the tape's nsteps records: a step after a halt does not run,
+// and its record lands on the halted step's, which the resumed range
+// writes again.
+__global__ void adj_record(const Ctrl* __restrict__ ctrl, AdjStep* __restrict__ rec, uint64_t base, uint32_t nsteps) {
+    const uint64_t k = min(ctrl->step - base, (uint64_t)nsteps - 1);
+    rec[k] = step_record(*ctrl);
+}
+// Records of every step, from the control blocks kept with the state after
+// each: `first` and on, stride bytes apart, and `last`.
+__global__ void __launch_bounds__(kBlock) tape_records_kernel(const char* __restrict__ first, size_t stride,
+                                                              const char* __restrict__ last,
+                                                              AdjStep* __restrict__ rec, uint32_t nsteps) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < nsteps) rec[k] = step_record(*(const Ctrl*)(k + 1 < nsteps ? first + k * stride : last));
 }
 
 // whole_step reverse.  out_adj[s] = (a_x, a_y, av_x, av_y) adjoints,

@@ -81,8 +81,12 @@ __device__ __forceinline__ double gauge_weight3(const GaugeSpec3& G, uint32_t g,
 // Block partial sums (sum w e, sum w) of every gauge (layout of
 // gauge_block_sums).
 __global__ void __launch_bounds__(kBlock) smooth_gauge_partials3(uint32_t n, const double4* __restrict__ pos,
-                                                                 GaugeSpec3 G, double* __restrict__ partials) {
+                                                                 GaugeSpec3 G, double* __restrict__ partials,
+                                                                 size_t stride) {
     __shared__ GaugeLds L;
+    // row y of the grid: the state y strides further on, its partials in a row of their own
+    pos = (const double4*)((const char*)pos + blockIdx.y * stride);
+    partials += (size_t)blockIdx.y * 2 * G.g.n * gridDim.x;
     gauge_lds_clear(G.g, L);
     const double inv_r2 = 1.0 / (G.g.radius * G.g.radius);
     for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {

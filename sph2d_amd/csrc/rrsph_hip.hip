@@ -124,7 +124,9 @@ struct AdjTape {
     bool seg_last = false;               // seg holds the last segment's states (kept by the forward)
     // seg holds the state before every step of the run (and the sorts):
     // the forward keeps them all when they fit in half the free device
-    // memory (tapes of sorted steps), and the reverse pass replays nothing
+    // memory (with list steps: together with the lists of a build in every
+    // step, so that the lists cannot run out), and the reverse pass replays
+    // nothing (943,906-particle basin, 12 steps in two segments: 23.6 -> 20.2 ms)
     bool keep_all = false;
     // the cell sort each step of seg ran with (keys, permutation): the reverse
     // step reorders its state with them instead of sorting it again
@@ -162,6 +164,9 @@ struct AdjTape {
     hipGraph_t tgraph = nullptr;
     hipGraphExec_t texec = nullptr;
     uint64_t tbase = 0;
+    // list steps with every state kept: the records and gauges of all steps
+    // are taken from the kept states in a few launches behind the last step
+    bool batched() const { return lists && keep_all; }
 };
 
 // Captured steps with neighbour lists: a build step, and runs of 1, 2, 4 and
@@ -254,7 +259,7 @@ struct rrsph_ctx {
     unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima, a set per step parity)
     unsigned long long* dtslots = nullptr; // list steps: dt maxima (likewise)
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
-    ListGraphs list_graphs[2];          // of plain runs and of taped ones (another skin)
+    ListGraphs list_graphs;             // of plain runs
     bool taping = false;                // ctx->P holds the taped runs' skin
     bool fuse = false;                  // list steps may run in fused pairs (fused_step_begin)
     void* rec1 = nullptr;               // fused steps: the second array of records
@@ -690,13 +695,11 @@ void enqueue_step(rrsph_ctx* c, Profiler* prof, bool full_sort) {
 }
 
 void drop_list_graphs(rrsph_ctx* c) {
-    for (ListGraphs& G : c->list_graphs) {
-        for (auto e : G.exec)
-            if (e) (void)hipGraphExecDestroy(e);
-        for (auto g : G.graph)
-            if (g) (void)hipGraphDestroy(g);
-        G = ListGraphs{};
-    }
+    for (auto e : c->list_graphs.exec)
+        if (e) (void)hipGraphExecDestroy(e);
+    for (auto g : c->list_graphs.graph)
+        if (g) (void)hipGraphDestroy(g);
+    c->list_graphs = ListGraphs{};
 }
 
 void drop_graph(rrsph_ctx* c) {
@@ -738,11 +741,13 @@ rrsph_status launch_list_run(rrsph_ctx* ctx, bool build, uint32_t steps) {
             enqueue_list_step(ctx, nullptr, kind);
         }
     };
-    if (!ctx->use_graph) {
+    // a taped step is followed by a copy of its state to an address of its
+    // own, and every run sets new piston coefficients, which a graph would hold
+    if (!ctx->use_graph || ctx->taping) {
         enqueue();
         return RRSPH_OK;
     }
-    ListGraphs& G = ctx->list_graphs[ctx->taping ? 1 : 0];
+    ListGraphs& G = ctx->list_graphs;
     const uint32_t i = build ? 0 : 1 + (uint32_t)__builtin_ctz(steps);
     if (!G.exec[i]) {
         HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
@@ -2018,21 +2023,26 @@ static rrsph_status to_gauge_spec(rrsph_ctx* ctx, const rrsph_gauge_spec* in, Ga
 }
 
 // smooth gauges of state A into eta/zs/ws (device, kMaxGauges entries each)
-// (with ctrl: into row ctrl->step - base of tapes of nsteps rows)
+// (with ctrl: into row ctrl->step - base of tapes of nsteps rows), or with
+// `saved` of `rows` states saved `stride` bytes apart, into consecutive rows
 static rrsph_status enqueue_smooth_gauges(rrsph_ctx* ctx, const GaugeSpec3& G, double* partials, double* eta,
                                           double* zs, double* ws, const Ctrl* ctrl = nullptr, uint64_t base = 0,
-                                          uint32_t nsteps = 0) {
-    const uint32_t nb = gauge_blocks(ctx->P.n);  // partials holds 2 kMaxGauges nb doubles
+                                          uint32_t nsteps = 0, const StateView* saved = nullptr, uint32_t rows = 1,
+                                          size_t stride = 0) {
+    const uint32_t nb = gauge_blocks(ctx->P.n);  // partials holds 2 kMaxGauges nb doubles a row
+    const void* pos = saved ? saved->pos : (const void*)ctx->posA;
+    const void* va = saved ? saved->va : ctx->vaA;
+    const dim3 grid(nb, rows);
     if (ctx->P.dim == 3)
-        smooth_gauge_partials3<<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, (const double4*)ctx->posA, G, partials);
+        smooth_gauge_partials3<<<grid, kBlock, 0, ctx->stream>>>(ctx->P.n, (const double4*)pos, G, partials, stride);
     else if (ctx->fp32)
-        smooth_gauge_partials<float><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->posA, (const float4*)ctx->vaA,
-                                                                      G.g, partials);
+        smooth_gauge_partials<float><<<grid, kBlock, 0, ctx->stream>>>(ctx->P.n, (const double2*)pos,
+                                                                       (const float4*)va, G.g, partials, stride);
     else
-        smooth_gauge_partials<double><<<nb, kBlock, 0, ctx->stream>>>(ctx->P.n, ctx->posA, (const double4*)ctx->vaA,
-                                                                       G.g, partials);
-    smooth_gauge_final<<<std::max(G.g.n, 1u), kBlock, 0, ctx->stream>>>(nb, G.g, partials, eta, zs, ws, ctrl, base,
-                                                                         nsteps);
+        smooth_gauge_partials<double><<<grid, kBlock, 0, ctx->stream>>>(ctx->P.n, (const double2*)pos,
+                                                                        (const double4*)va, G.g, partials, stride);
+    smooth_gauge_final<<<dim3(std::max(G.g.n, 1u), rows), kBlock, 0, ctx->stream>>>(nb, G.g, partials, eta, zs, ws,
+                                                                                     ctrl, base, nsteps);
     HIP_TRY(hipGetLastError());
     return RRSPH_OK;
 }
@@ -2050,7 +2060,6 @@ static rrsph_status adjoint_supported(rrsph_ctx* ctx) {
     return RRSPH_OK;
 }
 
-// one saved state: posA | vaA | adA | oidA | pres | ctrl
 // bytes per particle of the FP64 position array (2D double2, 3D double4)
 // and of one real4 state array (va, ad: FP32 or FP64)
 static size_t pos_bytes(const rrsph_ctx* ctx) { return ctx->P.dim == 3 ? 32 : 16; }
@@ -2058,9 +2067,11 @@ static size_t real4_bytes(const rrsph_ctx* ctx) { return ctx->fp32 ? 16 : 32; }
 // bytes of one saved state: pos | va | ad | oid | pressure | control block
 // (the pressure of the step that produced the state, in its slot order: the
 // reference's p array, which download() returns)
-static size_t state_bytes(const rrsph_ctx* ctx) {
-    return (pos_bytes(ctx) + 2 * real4_bytes(ctx) + 4 + real4_bytes(ctx) / 4) * ctx->P.n + sizeof(Ctrl);
+// (the control block on a 16-byte boundary: tape_records_kernel reads it in place)
+static size_t state_ctrl_offset(const rrsph_ctx* ctx) {
+    return ((pos_bytes(ctx) + 2 * real4_bytes(ctx) + 4 + real4_bytes(ctx) / 4) * ctx->P.n + 15) / 16 * 16;
 }
+static size_t state_bytes(const rrsph_ctx* ctx) { return state_ctrl_offset(ctx) + sizeof(Ctrl); }
 
 // the blob of one saved state: posA | vaA | adA | oidA | pres | ctrl
 static CopyPlan state_plan(rrsph_ctx* ctx, void* blob, bool save) {
@@ -2071,6 +2082,7 @@ static CopyPlan state_plan(rrsph_ctx* ctx, void* blob, bool save) {
     CopyPlan plan;
     size_t off = 0;
     for (int k = 0; k < 6; ++k) {
+        if (k == 5) off = state_ctrl_offset(ctx);
         if (save) plan.add(arrays[k], d + off, bytes[k]);
         else plan.add(d + off, arrays[k], bytes[k]);
         off += bytes[k];
@@ -2189,6 +2201,8 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
     // the copies after a step (its sort, its build's lists) wait for the
     // state copy before the next step and go in the same launch when the
     // ranges fit one; the next step's sort overwrites them only after that
+    if (forward && T.keep_all && T.lists)  // the builds before k0 (those launched after a halt left no lists)
+        T.nseg_lists = k0 > 0 ? (uint32_t)(T.seg_build[k0 - 1] + 1) : 0u;
     CopyPlan pending;
     auto flush = [&]() -> rrsph_status {
         if (pending.n == 0) return RRSPH_OK;
@@ -2205,7 +2219,7 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
         return flush();
     };
     for (uint32_t k = k0; k < k1; ++k) {
-        rrsph_status st;
+        rrsph_status st = RRSPH_OK;
         // after a halt the rest of the range is launches that do nothing:
         // look every kHaltCheck steps, so that a halt early in a long range
         // costs at most that many (the caller resumes from the halted step)
@@ -2227,8 +2241,12 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
         }
         const bool keep = forward ? k >= last0 : true;  // seg holds this step's state
         const size_t slot = forward ? k - last0 : k - kslot;
+        // a batched tape's records come from the kept control blocks, so a range
+        // that resumes at a halted step keeps the state saved before the halt
+        // (the halted step left the state as it was, but not the control block)
+        const bool kept = forward && T.batched() && k == k0 && k0 > 0;
         if (keep) {
-            st = save((char*)seg_base + slot * T.blob);
+            if (!kept) st = save((char*)seg_base + slot * T.blob);
             if (st != RRSPH_OK) return st;
             if (!forward && k + 1 == k1) {  // the state before the segment's last step is all the adjoint needs
                 // that step is not launched: a list step reads the lists of the segment's last build; a
@@ -2250,7 +2268,7 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
         }
         if (st != RRSPH_OK) return st;
         if (keep) {
-            if (slot == 0 || !T.lists) T.nseg_lists = 0;
+            if ((slot == 0 && !T.keep_all) || !T.lists) T.nseg_lists = 0;
             CopyPlan plan;
             if (!T.lists || build) {  // keep the sort of a step whose state seg holds
                 plan.add(ctx->last_keys, T.seg_keys + slot * n, n * sizeof(uint32_t));
@@ -2285,7 +2303,7 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
             if (T.lists) T.seg_build[slot] = (int32_t)T.nseg_lists - 1;
             pending = plan;  // empty before: the state copy before the step took it
         }
-        if (forward && !taped) {
+        if (forward && !taped && !T.batched()) {
             adj_record<<<1, 1, 0, ctx->stream>>>(ctx->ctrl, T.rec, base, T.nsteps);
             st = enqueue_smooth_gauges(ctx, T.spec, T.partials, T.eta, T.zs, T.ws, ctx->ctrl, base, T.nsteps);
             if (st != RRSPH_OK) return st;
@@ -2443,6 +2461,32 @@ rrsph_status rrsph_hip_adjoint_backward(rrsph_ctx* ctx, const double* eta_bar, d
     return adjoint_backward_impl(ctx, eta_bar, grad_a, grad_b, grad_r0, grad_v0, grad_rho0);
 }
 
+constexpr uint32_t kGaugeRows = 64;  // steps whose gauges one launch takes
+
+// The records and gauges of every step of a batched tape, from the states
+// kept before the next step and the final state.  A record and two gauge
+// kernels after each step took 14 us and their launch gaps.
+static rrsph_status tape_records_and_gauges(rrsph_ctx* ctx) {
+    AdjTape& T = ctx->adj;
+    const uint32_t N = T.nsteps;
+    char* final_state = (char*)T.ck.back();
+    const size_t at = state_ctrl_offset(ctx);
+    tape_records_kernel<<<grid_blocks(N, kBlock), kBlock, 0, ctx->stream>>>((const char*)T.seg + T.blob + at, T.blob,
+                                                                            final_state + at, T.rec, N);
+    HIP_TRY(hipGetLastError());
+    for (uint32_t k = 0; k < N;) {
+        const bool last = k + 1 == N;
+        const uint32_t rows = last ? 1u : std::min(kGaugeRows, N - 1 - k);
+        const StateView v = state_view(ctx, last ? final_state : (char*)T.seg + (size_t)(k + 1) * T.blob);
+        const size_t o = (size_t)k * kMaxGauges;
+        const rrsph_status st = enqueue_smooth_gauges(ctx, T.spec, T.partials, T.eta + o, T.zs + o, T.ws + o, nullptr,
+                                                      0, 0, &v, rows, T.blob);
+        if (st != RRSPH_OK) return st;
+        k += rows;
+    }
+    return RRSPH_OK;
+}
+
 // The buffers of a tape of T.nsteps steps with a checkpoint every T.every.
 static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     AdjTape& T = ctx->adj;
@@ -2459,9 +2503,9 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
         // every step's state and sort when they fit in half the free memory
         // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's, and replays)
         size_t free_b = 0, total_b = 0;
-        const double all_b = (double)nsteps * (double)(T.blob + 2 * n * sizeof(uint32_t));
-        T.keep_all = !T.lists && !T.segments && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-                     all_b <= 0.5 * (double)free_b;
+        const size_t lists_b = T.lists ? (size_t)(ctx->P.list_cap + kListPad + 2) * n * sizeof(uint32_t) : 0;
+        const double all_b = (double)nsteps * (double)(T.blob + 2 * n * sizeof(uint32_t) + lists_b);
+        T.keep_all = !T.segments && hipMemGetInfo(&free_b, &total_b) == hipSuccess && all_b <= 0.5 * (double)free_b;
     }
     uint32_t cap = T.keep_all ? nsteps : T.every;  // states seg holds
     const bool alloc_ok = e == hipSuccess;
@@ -2489,7 +2533,7 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     T.zs = dalloc<double>((size_t)nsteps * kMaxGauges, e);
     T.ws = dalloc<double>((size_t)nsteps * kMaxGauges, e);
     T.eta_bar = dalloc<double>((size_t)nsteps * kMaxGauges, e);
-    T.partials = dalloc<double>(2 * kMaxGauges * (size_t)nb, e);
+    T.partials = dalloc<double>(2 * kMaxGauges * (T.batched() ? (size_t)gauge_blocks(ctx->P.n) * kGaugeRows : nb), e);
     T.piston_sum = dalloc<double>((size_t)nsteps * kMaxSegments, e);
     T.lam[0] = dalloc<double>((d3 ? kLam3 : 8) * n, e);
     T.lam[1] = dalloc<double>((d3 ? kLam3 : 8) * n, e);
@@ -2560,6 +2604,10 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
         return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: the run halted during the adjoint forward");
     st = save_state(ctx, T.ck[nck]);
     if (st != RRSPH_OK) return st;
+    if (T.batched()) {
+        st = tape_records_and_gauges(ctx);
+        if (st != RRSPH_OK) return st;
+    }
     T.seg_last = true;
     std::vector<double> h((size_t)nsteps * kMaxGauges);
     HIP_TRY(hipMemcpyAsync(h.data(), T.eta, h.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));

@@ -1,0 +1,65 @@
+"""Tapes of list steps that keep every step's state give what the replays of their segments give: the
+same schedule of builds, the same states, records and gauges; also where lists go stale and steps halt and resume."""
+import numpy as np
+import pytest
+
+from sph2d_amd import generators as G
+from sph2d_amd import hip as H
+from sph2d_amd.adjoint import DifferentiableRun
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(dim, precision):
+    if dim == 2:
+        lay = G.adjoint_tank(delta=0.0075, length=1.5, sigma=0.01, seed=5)
+        xs, zs = [0.03, 0.06, 0.1], None
+    else:
+        lay = G.piston_basin_3d(delta=0.05, length=1.0, width=0.8)
+        xs, zs = [0.1, 0.2, 0.2], [0.3, 0.5, 0.7]
+    prm = lay.params
+    spec = H.gauge_spec(xs, radius=3 * prm.delta, tau=prm.delta / 4, y_ref=prm.depth, zs=zs)
+    sim = H.HipStep(prm, precision=precision)
+    return DifferentiableRun(sim, dict(lay.state), 30, 8, spec, prm.piston_omega), prm
+
+
+def _gradients(run, prm, scale=1.0):
+    a, b = scale * np.array(prm.piston_a), scale * np.array(prm.piston_b)
+    eta = run.forward(a, b)
+    c = np.random.default_rng(5).normal(0.0, 1.0, eta.shape)
+    return eta, run.backward(c, len(a)), run.sim.download()
+
+
+@pytest.mark.parametrize("dim", [3])
+@pytest.mark.parametrize("precision", [H.FP64, H.FP32])
+@pytest.mark.parametrize("skin", [None, "0.004"])
+def test_kept_list_tapes_equal_their_replays(monkeypatch, dim, precision, skin):
+    if skin:
+        monkeypatch.setenv("RRSPH_HIP_LIST_SKIN", skin)
+    res = {}
+    for store in ("all", "segments"):
+        monkeypatch.setenv("RRSPH_HIP_ADJ_STORE", store)
+        run, prm = _run(dim, precision)
+        first = _gradients(run, prm)
+        _gradients(run, prm, 0.3)  # another run on the same tape
+        res[store] = (first, run.sim.list_stats())
+        run.sim.close()
+    ((e1, g1, s1), q1), ((e0, g0, s0), q0) = res["all"], res["segments"]
+    print("list stats", q1, q0, flush=True)
+    assert q1["list_steps"] > 0
+    assert q0["list_steps"] + q0["builds"] > q1["list_steps"] + q1["builds"]  # the replays ran
+    if skin:
+        assert q1["stale_halts"] > 0
+    assert np.array_equal(e1, e0)
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(s1[f], s0[f]), f
+        # A replay does not launch a segment's last step; where that one builds, its reverse walks the cells, in 3D
+        # with FP64 differences of positions instead of the FP32 near records': those are rounded to 2^-24 of up to
+        # 2.1 cells, about 3e-7 of a particle spacing, in each of 30 steps.
+        if dim == 3 and precision == H.FP32:
+            assert np.max(np.abs(g1[f] - g0[f])) <= 1e-5 * np.max(np.abs(g0[f])), f
+        else:
+            assert np.array_equal(g1[f], g0[f]), f
+    for f in ("a", "b"):  # sums over blocks are atomic adds
+        tol = 1e-5 if dim == 3 and precision == H.FP32 else 1e-12
+        assert np.max(np.abs(g1[f] - g0[f])) <= tol * np.max(np.abs(g0[f]))
