@@ -22,6 +22,8 @@
 //   adj_pair  gather over neighbours: every pair is differentiated in both
 //             orientations (the particle as owner of the sum and as
 //             neighbour), then predict and EOS reverse; writes lam_n
+//   adj_prep_list, adj_pair_list  the same on the lists of the build that the
+//             step read, in its slot order
 //   smooth_gauge_* the surrogate eta_g = y_ref + tau log(sum w e / sum w)
 //             with w = (1 - (x - x_g)^2 / R^2)^3 inside |x - x_g| < R and
 //             e = exp((y - y_ref) / tau); tau -> 0 gives max y in the window,
@@ -30,6 +32,7 @@
 #pragma once
 
 #include "device_common.hpp"
+#include "list_step.hpp"
 #include "step_kernels.hpp"
 
 namespace rrsph {
@@ -195,21 +198,12 @@ __global__ void __launch_bounds__(kBlock) smooth_gauge_final(uint32_t nblocks, G
     }
 }
 
-// lam[oid].r += sum_g eta_bar[g] d eta_g / d r (state in sorted order).
-template <class R>
-__global__ void __launch_bounds__(kBlock) smooth_gauge_grad(uint32_t n, const double2* __restrict__ pos,
-                                                            const real4<R>* __restrict__ va,
-                                                            const uint32_t* __restrict__ oid, GaugeSpec G,
-                                                            const double* __restrict__ eta_bar,
-                                                            const double* __restrict__ zsum,
-                                                            const double* __restrict__ wsum,
-                                                            double* __restrict__ lam) {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    if ((int)va[s].w != G.ptype) return;
-    const double2 p = pos[s];
+// (gx, gy) = sum_g eta_bar[g] d eta_g / d r at p; false outside every window.
+__device__ __forceinline__ bool gauge_gradient(const GaugeSpec& G, double2 p, const double* __restrict__ eta_bar,
+                                               const double* __restrict__ zsum, const double* __restrict__ wsum,
+                                               double& gx, double& gy) {
     const double inv_r2 = 1.0 / (G.radius * G.radius);
-    double gx = 0, gy = 0;
+    gx = gy = 0;
     bool seen = false;  // inside a window: only those particles update lam
     for (uint32_t g = 0; g < G.n; ++g) {
         const double dx = p.x - G.x[g];
@@ -223,7 +217,23 @@ __global__ void __launch_bounds__(kBlock) smooth_gauge_grad(uint32_t n, const do
         gy += eta_bar[g] * w * e / z;
         gx += eta_bar[g] * G.tau * wp * (e / z - 1.0 / ws);
     }
-    if (!seen) return;
+    return seen;
+}
+
+// lam[oid].r += sum_g eta_bar[g] d eta_g / d r (state in sorted order).
+template <class R>
+__global__ void __launch_bounds__(kBlock) smooth_gauge_grad(uint32_t n, const double2* __restrict__ pos,
+                                                            const real4<R>* __restrict__ va,
+                                                            const uint32_t* __restrict__ oid, GaugeSpec G,
+                                                            const double* __restrict__ eta_bar,
+                                                            const double* __restrict__ zsum,
+                                                            const double* __restrict__ wsum,
+                                                            double* __restrict__ lam) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= n) return;
+    if ((int)va[s].w != G.ptype) return;
+    double gx, gy;
+    if (!gauge_gradient(G, pos[s], eta_bar, zsum, wsum, gx, gy)) return;
     double* l = lam + 8 * (size_t)oid[s];
     l[0] += gx;
     l[1] += gy;
@@ -301,62 +311,52 @@ __global__ void __launch_bounds__(kBlock) tape_records_kernel(const char* __rest
     if (k < nsteps) rec[k] = step_record(*(const Ctrl*)(k + 1 < nsteps ? first + k * stride : last));
 }
 
-// whole_step reverse.  out_adj[s] = (a_x, a_y, av_x, av_y) adjoints,
-// drho_adj[s]; direct[s] = (r_x, r_y, v_x, v_y, rho) adjoints that do not
-// pass through the pair sums; piston_sum += wave-maker velocity adjoint.
-template <class R>
-__global__ void __launch_bounds__(kBlock) adj_prep(StepParams P, AdjStep T, StateB<R> B,
-                                                   const double* __restrict__ lam_in,
-                                                   double4* __restrict__ out_adj, double* __restrict__ drho_adj,
-                                                   double* __restrict__ direct, double* __restrict__ piston_sum) {
-    __shared__ double s_p[kBlock / kWave];
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    double pist = 0.0;
-    if (s < P.n) {
-        const uint32_t o = B.oid[s];
-        const double* l = lam_in + 8 * (size_t)o;
-        const double rx = l[0], ry = l[1], vx = l[2], vy = l[3], rb = l[4], ax = l[5], ay = l[6], db = l[7];
-        const int t = (int)B.va[s].w;
-        const double vdt = T.first ? T.dt * 0.5 : T.dt;
-        double4 oa;
-        double dvx = 0, dvy = 0;
-        if (t > 0) {
-            const double tx = vx + rx * T.dt, ty = vy + ry * T.dt;  // adjoint of the updated v
-            oa.x = tx * vdt + ax;
-            oa.y = ty * vdt + ay;
-            oa.z = P.xsph_on ? tx : 0.0;
-            oa.w = P.xsph_on ? ty : 0.0;
-            dvx = tx;
-            dvy = ty;
+// whole_step reverse of one particle of type t and original index o with
+// output adjoints l: out = adjoints of (a_x, a_y, av_x, av_y), drho that of
+// drho; d = adjoints of (r_x, r_y, v_x, v_y, rho) that do not pass through
+// the pair sums.  Returns the wave maker's velocity adjoint.
+__device__ __forceinline__ double adj_whole_step(const StepParams& P, const AdjStep& T, int t, uint32_t o,
+                                                 const double* __restrict__ l, double4& out, double& drho, double* d) {
+    const double rx = l[0], ry = l[1], vx = l[2], vy = l[3], rb = l[4], ax = l[5], ay = l[6], db = l[7];
+    const double vdt = T.first ? T.dt * 0.5 : T.dt;
+    double pist = 0.0, dvx = 0, dvy = 0;
+    if (t > 0) {
+        const double tx = vx + rx * T.dt, ty = vy + ry * T.dt;  // adjoint of the updated v
+        out.x = tx * vdt + ax;
+        out.y = ty * vdt + ay;
+        out.z = P.xsph_on ? tx : 0.0;
+        out.w = P.xsph_on ? ty : 0.0;
+        dvx = tx;
+        dvy = ty;
+    } else {
+        out.x = ax;
+        out.y = ay;
+        out.z = 0.0;
+        out.w = 0.0;
+        const bool moving = P.boundary_motion && t < 0;
+        const bool piston = moving && T.piston && o >= P.nwm_start && o < P.nwm_end && o >= P.nfluid;
+        if (piston) {
+            pist = P.nwm_axis == 0 ? vx + rx * T.dt : vy + ry * T.dt;
+        } else if (moving) {
+            dvx = vx + rx * T.dt;
+            dvy = vy + ry * T.dt;
         } else {
-            oa.x = ax;
-            oa.y = ay;
-            oa.z = 0.0;
-            oa.w = 0.0;
-            const bool moving = P.boundary_motion && t < 0;
-            const bool piston = moving && T.piston && o >= P.nwm_start && o < P.nwm_end && o >= P.nfluid;
-            if (piston) {
-                pist = P.nwm_axis == 0 ? vx + rx * T.dt : vy + ry * T.dt;
-            } else if (moving) {
-                dvx = vx + rx * T.dt;
-                dvy = vy + ry * T.dt;
-            } else {
-                dvx = vx;
-                dvy = vy;
-            }
+            dvx = vx;
+            dvy = vy;
         }
-        if (t == 0) {  // no neighbours, no acceleration dependence
-            oa.x = oa.y = 0.0;
-        }
-        out_adj[s] = oa;
-        drho_adj[s] = P.density_treatment != 0 ? rb * vdt + db : 0.0;
-        double* d = direct + 5 * (size_t)s;
-        d[0] = rx;
-        d[1] = ry;
-        d[2] = dvx;
-        d[3] = dvy;
-        d[4] = rb;
     }
+    if (t == 0) out.x = out.y = 0.0;  // no neighbours, no acceleration dependence
+    drho = P.density_treatment != 0 ? rb * vdt + db : 0.0;
+    d[0] = rx;
+    d[1] = ry;
+    d[2] = dvx;
+    d[3] = dvy;
+    d[4] = rb;
+    return pist;
+}
+// piston_sum += the block's wave-maker velocity adjoints (every thread).
+__device__ __forceinline__ void adj_piston_sum(double pist, double* __restrict__ piston_sum) {
+    __shared__ double s_p[kBlock / kWave];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) pist += __shfl_xor(pist, off);
     if (__lane_id() == 0) s_p[threadIdx.x / kWave] = pist;
@@ -366,6 +366,26 @@ __global__ void __launch_bounds__(kBlock) adj_prep(StepParams P, AdjStep T, Stat
         for (int w = 0; w < kBlock / kWave; ++w) b += s_p[w];
         if (b != 0.0) atomicAdd(piston_sum, b);
     }
+}
+
+// whole_step reverse on the re-sorted state: out_adj, drho_adj and direct[5 s]
+// as adj_whole_step gives them.
+template <class R>
+__global__ void __launch_bounds__(kBlock) adj_prep(StepParams P, AdjStep T, StateB<R> B,
+                                                   const double* __restrict__ lam_in,
+                                                   double4* __restrict__ out_adj, double* __restrict__ drho_adj,
+                                                   double* __restrict__ direct, double* __restrict__ piston_sum) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    double pist = 0.0;
+    if (s < P.n) {
+        const uint32_t o = B.oid[s];
+        double4 oa;
+        double drho;
+        pist = adj_whole_step(P, T, (int)B.va[s].w, o, lam_in + 8 * (size_t)o, oa, drho, direct + 5 * (size_t)s);
+        out_adj[s] = oa;
+        drho_adj[s] = drho;
+    }
+    adj_piston_sum(pist, piston_sum);
 }
 
 struct AdjConsts {
@@ -438,19 +458,7 @@ __device__ __forceinline__ void adj_orient(const AdjConsts& K, const AdjPair& Q,
     }
 }
 
-template <class R>
-__global__ void __launch_bounds__(kBlock) adj_pair(StepParams P, AdjStep T, StateB<R> B,
-                                                   const uint32_t* __restrict__ skey,
-                                                   const uint32_t* __restrict__ LB,
-                                                   const double4* __restrict__ out_adj,
-                                                   const double* __restrict__ drho_adj,
-                                                   const double* __restrict__ direct, double* __restrict__ lam_out,
-                                                   uint32_t* __restrict__ overflow_flag) {
-    __shared__ uint32_t hits[kAdjChunk * kBlock];
-    // XCD-aware: each XCD walks one contiguous slice of the slots
-    const uint32_t lb = xcd_block(P.blocks_per_xcd);
-    const uint32_t s = lb * kBlock + threadIdx.x;
-    if (lb >= P.nblocks || s >= P.n) return;
+__device__ __forceinline__ AdjConsts adj_consts(const StepParams& P) {
     AdjConsts K;
     K.h = P.h;
     K.inv_h = 1.0 / P.h;
@@ -468,104 +476,273 @@ __global__ void __launch_bounds__(kBlock) adj_pair(StepParams P, AdjStep T, Stat
     K.av_on = P.av_on;
     K.xsph_on = P.xsph_on;
     K.lj_on = P.lj_on;
-    const double2 pk = B.pos[s];
-    const double4 vak = to_d4<R>(B.va[s]);
-    const double4 prk = to_d4<R>(B.pred[s]);
-    const double pres_k = B.pres[s];
-    const double4 oak = out_adj[s];
-    const double dak = drho_adj[s];
-    const int tk = (int)vak.w;
+    return K;
+}
+
+// What a pair's adjoint reads of a particle: position, predicted velocity u
+// and density rho^, velocity v, p / rho^2, type, and the output adjoints
+// oa = (a, av) and da = drho.
+struct AdjParticle {
+    double2 pos, u, v;
+    double R, pw, da;
+    double4 oa;
+    int t;
+};
+// The pair sums of a particle: adjoints of r, v, u, R and p / R^2.
+struct AdjSums {
     double rbx = 0, rby = 0, vbx = 0, vby = 0, ubx = 0, uby = 0, Rb = 0, Pb = 0;
+};
+// The pair of k and its neighbour i at r_i - r_k = (ex, ey).
+__device__ __forceinline__ void adj_pair_term(const AdjConsts& K, const AdjParticle& k, const AdjParticle& i, double ex,
+                                              double ey, AdjSums& S) {
+    AdjPair Q;
+    Q.d2 = ex * ex + ey * ey;
+    Q.rinv = Q.d2 > 0.0 ? fast_rsqrt<double>(Q.d2) : 0.0;
+    Q.d = Q.d2 * Q.rinv;
+    const double q = Q.d * K.inv_h;
+    const double t = 2.0 - q;
+    if (q <= 1.0) {
+        Q.F = K.c1 * (1.5 * q - 2.0);
+        Q.Fp = 1.5 * K.c1 * K.inv_h;
+        Q.W = K.w1 * (2.0 / 3.0 - q * q + 0.5 * q * q * q);
+    } else {
+        Q.F = -K.c2 * t * t * Q.rinv;
+        Q.Fp = K.c2 * t * (2.0 * Q.rinv * K.inv_h + t * Q.rinv * Q.rinv);
+        Q.W = K.w2 * t * t * t;
+    }
+    Q.IR = fast_rcp<double>(i.R + k.R);
+    const double dux = i.u.x - k.u.x, duy = i.u.y - k.u.y;  // u_i - u_k
+    Q.vr = dux * ex + duy * ey;
+    Q.den = fast_rcp<double>(Q.d2 + K.eta2);
+    Q.mu = K.h * Q.vr * Q.den;
+    Q.app = K.av_on && Q.vr < 0.0;
+    Q.A = Q.app ? 2.0 * Q.IR * (K.beta * Q.mu * Q.mu - K.alpha_c * Q.mu) : 0.0;
+    const double coef = i.pw + k.pw + Q.A;
+    const double dvx = i.v.x - k.v.x, dvy = i.v.y - k.v.y;  // v_i - v_k
+    double ebx, eby, dvbx, dvby, dubx, duby, irb, coefb;
+    // Both orientations of the pair in one evaluation.  k's sum at
+    // k's adjoints is adj_orient at (e, dv, du); i's sum at i's
+    // adjoints is adj_orient at (-e, -dv, -du), entering rb, vb, ub
+    // with the opposite sign and Rb, Pb with the same.  Every
+    // output is linear in the owner's adjoints, and even (the a-
+    // and av-adjoint terms, the wall force) or odd (the
+    // drho-adjoint terms) in (e, dv, du), so the two make one
+    // evaluation at (e, dv, du) with the owner adjoints
+    // m (oa_k - oa_i) and m (drho_k + drho_i), the XSPH adjoint of
+    // whichever owner has a fluid neighbour (i's negated), and the
+    // wall force of whichever owner is the fluid particle (i's
+    // negated).
+    const bool xk = K.xsph_on && i.t > 0, xi = K.xsph_on && k.t > 0;
+    const bool ljk = K.lj_on && k.t > 0 && i.t < 0 && Q.d < K.r0;
+    const bool lji = K.lj_on && i.t > 0 && k.t < 0 && Q.d < K.r0;
+    const double xdx = K.xf * ((xk ? k.oa.z : 0.0) - (xi ? i.oa.z : 0.0));
+    const double xdy = K.xf * ((xk ? k.oa.w : 0.0) - (xi ? i.oa.w : 0.0));
+    adj_orient(K, Q, ex, ey, dvx, dvy, dux, duy, K.m * (k.oa.x - i.oa.x), K.m * (k.oa.y - i.oa.y), K.m * (k.da + i.da),
+               xdx, xdy, ljk ? k.oa.x : -i.oa.x, ljk ? k.oa.y : -i.oa.y, ljk || lji, xk || xi, coef, ebx, eby, dvbx,
+               dvby, dubx, duby, irb, coefb);
+    S.rbx -= ebx;
+    S.rby -= eby;
+    S.vbx -= dvbx;
+    S.vby -= dvby;
+    S.ubx -= dubx;
+    S.uby -= duby;
+    S.Rb -= Q.IR * Q.IR * irb;
+    S.Pb += coefb;
+}
+// The predict and EOS reverse of a particle, into l: P = p / R^2, p =
+// EOS(rho) = B ((rho / rho0)^7 - 1), u = v + a_prev dt/2, R = rho + drho_prev dt/2.
+__device__ __forceinline__ void adj_predict(const StepParams& P, double dt_pred, const AdjSums& S, double Rk, double pres,
+                                            double rho, const double* __restrict__ d, double* __restrict__ l) {
+    const double pb = S.Pb / (Rk * Rk);
+    const double Rb = S.Rb - 2.0 * S.Pb * pres / (Rk * Rk * Rk);
+    const double x = rho / P.rho0;
+    const double x2 = x * x, x3 = x2 * x;
+    const double dpdrho = 7.0 * P.eos_B * x3 * x3 / P.rho0;
+    const double h2 = dt_pred * 0.5;
+    l[0] = d[0] + S.rbx;
+    l[1] = d[1] + S.rby;
+    l[2] = d[2] + S.vbx + S.ubx;
+    l[3] = d[3] + S.vby + S.uby;
+    l[4] = d[4] + (P.density_treatment != 0 ? Rb : 0.0) + pb * dpdrho;
+    l[5] = S.ubx * h2;
+    l[6] = S.uby * h2;
+    l[7] = P.density_treatment != 0 ? Rb * h2 : 0.0;
+}
+
+template <class R>
+__global__ void __launch_bounds__(kBlock) adj_pair(StepParams P, AdjStep T, StateB<R> B,
+                                                   const uint32_t* __restrict__ skey,
+                                                   const uint32_t* __restrict__ LB,
+                                                   const double4* __restrict__ out_adj,
+                                                   const double* __restrict__ drho_adj,
+                                                   const double* __restrict__ direct, double* __restrict__ lam_out,
+                                                   uint32_t* __restrict__ overflow_flag) {
+    __shared__ uint32_t hits[kAdjChunk * kBlock];
+    // XCD-aware: each XCD walks one contiguous slice of the slots
+    const uint32_t lb = xcd_block(P.blocks_per_xcd);
+    const uint32_t s = lb * kBlock + threadIdx.x;
+    if (lb >= P.nblocks || s >= P.n) return;
+    const AdjConsts K = adj_consts(P);
+    auto particle = [&](uint32_t i) {
+        const double4 va = to_d4<R>(B.va[i]), pr = to_d4<R>(B.pred[i]);
+        AdjParticle p;
+        p.pos = B.pos[i];
+        p.u = make_double2(pr.x, pr.y);
+        p.v = make_double2(va.x, va.y);
+        p.R = pr.z;
+        p.pw = pr.w;
+        p.da = drho_adj[i];
+        p.oa = out_adj[i];
+        p.t = (int)va.w;
+        return p;
+    };
+    const AdjParticle k = particle(s);
+    AdjSums S;
     bool overflow = false;
-    if (tk != 0) {
+    if (k.t != 0) {
         uint32_t* my = hits + threadIdx.x;
         auto flush = [&](uint32_t nh) {
 #pragma unroll 1
             for (uint32_t u = 0; u < nh; ++u) {
-                const uint32_t i = my[u * kBlock];
-                const double2 pi = B.pos[i];
-                const double4 vai = to_d4<R>(B.va[i]);
-                const double4 pri = to_d4<R>(B.pred[i]);
-                const double4 oai = out_adj[i];
-                const double dai = drho_adj[i];
-                const int ti = (int)vai.w;
-                const double ex = pi.x - pk.x, ey = pi.y - pk.y;  // r_i - r_k
-                AdjPair Q;
-                Q.d2 = ex * ex + ey * ey;
-                Q.rinv = Q.d2 > 0.0 ? fast_rsqrt<double>(Q.d2) : 0.0;
-                Q.d = Q.d2 * Q.rinv;
-                const double q = Q.d * K.inv_h;
-                const double t = 2.0 - q;
-                if (q <= 1.0) {
-                    Q.F = K.c1 * (1.5 * q - 2.0);
-                    Q.Fp = 1.5 * K.c1 * K.inv_h;
-                    Q.W = K.w1 * (2.0 / 3.0 - q * q + 0.5 * q * q * q);
-                } else {
-                    Q.F = -K.c2 * t * t * Q.rinv;
-                    Q.Fp = K.c2 * t * (2.0 * Q.rinv * K.inv_h + t * Q.rinv * Q.rinv);
-                    Q.W = K.w2 * t * t * t;
-                }
-                Q.IR = fast_rcp<double>(pri.z + prk.z);
-                const double dux = pri.x - prk.x, duy = pri.y - prk.y;  // u_i - u_k
-                Q.vr = dux * ex + duy * ey;
-                Q.den = fast_rcp<double>(Q.d2 + K.eta2);
-                Q.mu = K.h * Q.vr * Q.den;
-                Q.app = K.av_on && Q.vr < 0.0;
-                Q.A = Q.app ? 2.0 * Q.IR * (K.beta * Q.mu * Q.mu - K.alpha_c * Q.mu) : 0.0;
-                const double coef = pri.w + prk.w + Q.A;
-                const double dvx = vai.x - vak.x, dvy = vai.y - vak.y;  // v_i - v_k
-                double ebx, eby, dvbx, dvby, dubx, duby, irb, coefb;
-                // Both orientations of the pair in one evaluation.  k's sum at
-                // k's adjoints is adj_orient at (e, dv, du); i's sum at i's
-                // adjoints is adj_orient at (-e, -dv, -du), entering rb, vb, ub
-                // with the opposite sign and Rb, Pb with the same.  Every
-                // output is linear in the owner's adjoints, and even (the a-
-                // and av-adjoint terms, the wall force) or odd (the
-                // drho-adjoint terms) in (e, dv, du), so the two make one
-                // evaluation at (e, dv, du) with the owner adjoints
-                // m (oa_k - oa_i) and m (drho_k + drho_i), the XSPH adjoint of
-                // whichever owner has a fluid neighbour (i's negated), and the
-                // wall force of whichever owner is the fluid particle (i's
-                // negated).
-                const bool xk = K.xsph_on && ti > 0, xi = K.xsph_on && tk > 0;
-                const bool ljk = K.lj_on && tk > 0 && ti < 0 && Q.d < K.r0;
-                const bool lji = K.lj_on && ti > 0 && tk < 0 && Q.d < K.r0;
-                const double xdx = K.xf * ((xk ? oak.z : 0.0) - (xi ? oai.z : 0.0));
-                const double xdy = K.xf * ((xk ? oak.w : 0.0) - (xi ? oai.w : 0.0));
-                adj_orient(K, Q, ex, ey, dvx, dvy, dux, duy, K.m * (oak.x - oai.x), K.m * (oak.y - oai.y),
-                           K.m * (dak + dai), xdx, xdy, ljk ? oak.x : -oai.x, ljk ? oak.y : -oai.y, ljk || lji,
-                           xk || xi, coef, ebx, eby, dvbx, dvby, dubx, duby, irb, coefb);
-                rbx -= ebx;
-                rby -= eby;
-                vbx -= dvbx;
-                vby -= dvby;
-                ubx -= dubx;
-                uby -= duby;
-                Rb -= Q.IR * Q.IR * irb;
-                Pb += coefb;
+                const AdjParticle i = particle(my[u * kBlock]);
+                adj_pair_term(K, k, i, i.pos.x - k.pos.x, i.pos.y - k.pos.y, S);
             }
         };
-        collect_neighbours<kAdjChunk>(P, P.max_nbr - 1, s, skey[s], pk, B.pos, LB, my, overflow, flush);
+        collect_neighbours<kAdjChunk>(P, P.max_nbr - 1, s, skey[s], k.pos, B.pos, LB, my, overflow, flush);
     }
     if (overflow) atomicOr(overflow_flag, 1u);
-    // P = p / R^2, p = EOS(rho) = B ((rho / rho0)^7 - 1), u = v + a_prev dt/2, R = rho + drho_prev dt/2
-    const double Rk = prk.z;
-    const double pb = Pb / (Rk * Rk);
-    Rb += -2.0 * Pb * pres_k / (Rk * Rk * Rk);
-    const double x = vak.z / P.rho0;
-    const double x2 = x * x, x3 = x2 * x;
-    const double dpdrho = 7.0 * P.eos_B * x3 * x3 / P.rho0;
-    const double* d = direct + 5 * (size_t)s;
-    const double h2 = T.dt_pred * 0.5;
-    double* l = lam_out + 8 * (size_t)B.oid[s];
-    l[0] = d[0] + rbx;
-    l[1] = d[1] + rby;
-    l[2] = d[2] + vbx + ubx;
-    l[3] = d[3] + vby + uby;
-    l[4] = d[4] + (P.density_treatment != 0 ? Rb : 0.0) + pb * dpdrho;
-    l[5] = ubx * h2;
-    l[6] = uby * h2;
-    l[7] = P.density_treatment != 0 ? Rb * h2 : 0.0;
+    adj_predict(P, T.dt_pred, S, k.R, (double)B.pres[s], (double)B.va[s].z, direct + 5 * (size_t)s,
+                lam_out + 8 * (size_t)B.oid[s]);
+}
+
+// ------------------------------------------------------------------ step adjoint over lists
+// The reverse of a step that read neighbour lists, in the slot order of
+// their build.  adj_prep_list takes the kept state as it is (or, for a build
+// step, through the build's permutation) and writes one record per slot with
+// all that the pair adjoint reads of a particle: 128 bytes, which the wave
+// fetches as WaveGather does, in two halves of four words.
+// Per step of 134,042 particles (FP64): reorder 8.9 us, prep 6.9, cell walk
+// 41.2 and gauge gradients 5.0 us before; prep 16.0 and pair with gauges 33.1 now.
+struct alignas(128) AdjRec2 {
+    double2 pos, u, v;
+    double R, pw;      // R = typed_rho: the sign of the type, 0 for a dead particle
+    double4 oa;
+    double da, rho, pres;
+    uint32_t oid;
+    int32_t itype;
+};
+static_assert(sizeof(AdjRec2) == 128, "eight words of a wave gather");
+constexpr uint32_t kAdjListMax = 1u << 25;  // particles whose records' byte offsets fit 32 bits
+__device__ __forceinline__ AdjParticle adj_particle(const AdjRec2& r) {
+    AdjParticle p;
+    p.pos = r.pos;
+    p.u = r.u;
+    p.v = r.v;
+    p.R = fabs(r.R);
+    p.pw = r.pw;
+    p.da = r.da;
+    p.oa = r.oa;
+    p.t = r.R > 0.0 ? 1 : (r.R < 0.0 ? -1 : 0);
+    return p;
+}
+
+// perm: the build step's permutation, or null where the state is in slot order.
+template <class R>
+__global__ void __launch_bounds__(kBlock) adj_prep_list(StepParams P, AdjStep T, StateA<R> A,
+                                                        const uint32_t* __restrict__ perm,
+                                                        const double* __restrict__ lam_in, AdjRec2* __restrict__ rec,
+                                                        double* __restrict__ direct, double* __restrict__ piston_sum) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    double pist = 0.0;
+    if (s < P.n) {
+        const uint32_t src = perm ? min(perm[s], P.n - 1) : s;
+        const real4<R> va = A.va[src], ad = A.ad[src];
+        R p;
+        const real4<R> pr = predict_record<R>(P, va, ad.x, ad.y, ad.z, (R)T.dt_pred, p);
+        AdjRec2 r;
+        r.oid = A.oid[src];
+        r.itype = (int)va.w;
+        r.pos = A.pos[src];
+        r.u = make_double2((double)pr.x, (double)pr.y);
+        r.v = make_double2((double)va.x, (double)va.y);
+        r.R = (double)pr.z;
+        r.pw = (double)pr.w;
+        r.rho = (double)va.z;
+        r.pres = (double)p;
+        pist = adj_whole_step(P, T, (int)va.w, r.oid, lam_in + 8 * (size_t)r.oid, r.oa, r.da, direct + 5 * (size_t)s);
+        rec[s] = r;
+    }
+    adj_piston_sum(pist, piston_sum);
+}
+
+// The pair adjoint over lists, LPP lanes per particle, and the gradient of
+// the gauges of the state it reverses into (gauges: eta_bar null for none).
+// Every entry is decided as the step decided it (FP32 steps too: their test
+// ends in the same FP64 comparison).
+template <int LPP>
+__global__ void __launch_bounds__(kBlock) adj_pair_list(StepParams P, double dt_pred, const AdjRec2* __restrict__ rec,
+                                                        const uint32_t* __restrict__ nbl,
+                                                        const uint32_t* __restrict__ nbc,
+                                                        const double* __restrict__ direct,
+                                                        double* __restrict__ lam_out,
+                                                        uint32_t* __restrict__ overflow_flag, GaugeSpec G,
+                                                        const double* __restrict__ eta_bar,
+                                                        const double* __restrict__ zsum,
+                                                        const double* __restrict__ wsum) {
+    using Half = WaveGather<4, sizeof(AdjRec2), kSlotMask>;
+    __shared__ uint4 s_rec[kBlock / kWave][8 * kWave];
+    const uint32_t lb = xcd_block(group_blocks_per_xcd<LPP>(P.n));
+    if (lb >= group_blocks<LPP>(P.n)) return;
+    const LaneGroup<LPP> g(lb);
+    const bool live = g.s < P.n;
+    const uint32_t s = live ? g.s : P.n - 1;
+    const AdjConsts K = adj_consts(P);
+    const AdjParticle k = adj_particle(rec[s]);
+    const uint32_t cnt = live && k.t != 0 ? nbc[s] : 0u;
+    AdjSums S;
+    uint32_t hits = 0;
+    uint4* buf = s_rec[wave_of_block()];
+    const WaveGatherBoth<Half, Half> src{Half(rec, buf), Half((const char*)rec + 64, buf + 4 * kWave)};
+    gather_rounds<LPP, 1>(P, nbl, src, s, g.l, cnt, [&](uint32_t e0, const uint32_t (&)[1], const auto& w) {
+        const double4 a = record_real4(w[0], 0.0), b = record_real4(w[0] + 2, 0.0);  // (pos, u), (v, R, pw)
+        const double ex = __dsub_rn(a.x, k.pos.x), ey = __dsub_rn(a.y, k.pos.y);
+        if (e0 < cnt && b.z != 0.0 && dist2_exact(ex, ey) < P.cut2) {
+            AdjParticle i;
+            i.pos = make_double2(a.x, a.y);
+            i.u = make_double2(a.z, a.w);
+            i.v = make_double2(b.x, b.y);
+            i.R = fabs(b.z);
+            i.pw = b.w;
+            i.oa = record_real4(w[0] + 4, 0.0);
+            i.da = record_real4(w[0] + 6, 0.0).x;
+            i.t = b.z > 0.0 ? 1 : -1;
+            adj_pair_term(K, k, i, ex, ey, S);
+            ++hits;
+        }
+    });
+    S.rbx = lane_sum<LPP>(S.rbx);
+    S.rby = lane_sum<LPP>(S.rby);
+    S.vbx = lane_sum<LPP>(S.vbx);
+    S.vby = lane_sum<LPP>(S.vby);
+    S.ubx = lane_sum<LPP>(S.ubx);
+    S.uby = lane_sum<LPP>(S.uby);
+    S.Rb = lane_sum<LPP>(S.Rb);
+    S.Pb = lane_sum<LPP>(S.Pb);
+    if (lane_sum<LPP>((int)hits) > (int)(P.max_nbr - 1)) atomicOr(overflow_flag, 1u);
+    if (!live || g.l != 0) return;
+    double l[8];
+    const AdjRec2& own = rec[s];
+    adj_predict(P, dt_pred, S, k.R, own.pres, own.rho, direct + 5 * (size_t)s, l);
+    if (eta_bar && own.itype == G.ptype) {
+        double gx, gy;
+        if (gauge_gradient(G, k.pos, eta_bar, zsum, wsum, gx, gy)) {
+            l[0] += gx;
+            l[1] += gy;
+        }
+    }
+    double2* out = (double2*)(lam_out + 8 * (size_t)own.oid);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) out[c] = make_double2(l[2 * c], l[2 * c + 1]);
 }
 
 }  // namespace rrsph

@@ -1179,16 +1179,34 @@ void enqueue_state_keys(rrsph_ctx* ctx) {
 }  // namespace
 
 // The reverse of one step on its re-sorted state (state precision R, adjoint
-// arithmetic FP64): whole_step reverse, then the pair gather.
+// arithmetic FP64): whole_step reverse, then the pair gather.  In 2D over
+// lists the step's saved state src is read in place, through perm if the step
+// was a build (else null), and the gradient of the gauges of that state comes
+// with the pair gather (eta_bar, zs, ws: their row, or null).  8 lanes a
+// particle below 25,000, where the list passes take them (setup_params).
+constexpr uint32_t kAdjLanes8 = 25000;
 template <class R>
 static void enqueue_reverse_step(rrsph_ctx* ctx, const AdjStep& S, Ctrl* uc, const double* lam_in, double* lam_out,
                                  double* psum, const uint32_t* keys, const uint32_t* perm,
-                                 const AdjTape::Lists* lists, const StateView* src) {
+                                 const AdjTape::Lists* lists, const StateView* src, const double* eta_bar,
+                                 const double* zs, const double* ws) {
     AdjTape& T = ctx->adj;
     const StepParams& P = ctx->P;
     const size_t n = P.n;
     const uint32_t nb = grid_blocks(P.n, kBlock);
     const uint32_t nb_xcd = P.blocks_per_xcd * kNumXcd;  // the pair gathers map blocks to XCDs
+    if (P.dim == 2 && lists) {
+        AdjRec2* rec = (AdjRec2*)T.out_adj;
+        const StateA<R> A{(double2*)src->pos, (real4<R>*)src->va, (real4<R>*)src->ad, src->oid};
+        adj_prep_list<R><<<nb, kBlock, 0, ctx->stream>>>(P, S, A, perm, lam_in, rec, T.direct, psum);
+        auto pair = [&](auto kernel, uint32_t blocks) {
+            kernel<<<blocks * kNumXcd, kBlock, 0, ctx->stream>>>(P, S.dt_pred, rec, lists->nbl, lists->nbc, T.direct,
+                                                                 lam_out, T.flag, T.spec.g, eta_bar, zs, ws);
+        };
+        if (P.n < kAdjLanes8) pair(adj_pair_list<8>, group_blocks_per_xcd<8>(P.n));
+        else pair(adj_pair_list<2>, group_blocks_per_xcd<2>(P.n));
+        return;
+    }
     if (keys) {  // the sort step k ran with, saved by the replay: reorder only
         ctx->sorted_keys = keys;
         ctx->sorted_perm = perm;
@@ -2415,10 +2433,20 @@ rrsph_status rrsph_hip_set_piston(rrsph_ctx* ctx, double omega, uint32_t nharm, 
     return RRSPH_OK;
 }
 
-// The 2D adjoint's tapes and replays run the steps without neighbour lists
-// (a replay must repeat its step exactly, whatever the list schedule was;
-// the 3D tapes record their schedule instead).  Entering and leaving that
-// state forces a full sort and a list build.
+// Whether a tape runs list steps (builds at its checkpoints and by the
+// displacements, the schedule recorded for the replays).
+// In 2D: 60 steps of 134,042 particles forward and back 10.2 -> 8.2 ms, 40 of
+// 18,544 4.1 -> 2.4 and of 5,040, the smallest measured, 4.0 -> 2.2.  Below
+// 4,096 tapes keep to sorted steps, as contexts without lists do.
+constexpr uint32_t kTapeListMin2 = 4096;
+static bool tape_lists(const rrsph_ctx* ctx) {
+    if (!list_active(ctx)) return false;
+    return ctx->P.dim == 3 || (ctx->P.n >= kTapeListMin2 && ctx->P.n <= kAdjListMax);
+}
+
+// Other 2D tapes and replays run without neighbour lists (a replay must
+// repeat its step exactly, whatever the list schedule was).  Entering and
+// leaving that state forces a full sort and a list build.
 struct ListSuspend {
     rrsph_ctx* c;
     bool was;
@@ -2440,7 +2468,7 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
 rrsph_status rrsph_hip_adjoint_forward(rrsph_ctx* ctx, uint32_t nsteps, uint32_t checkpoint_every,
                                        const rrsph_gauge_spec* spec, double* eta) {
     if (!ctx) return RRSPH_ERR_INVALID_ARGUMENT;
-    if (ctx->P.dim == 3) {  // 3D tapes run list steps when the context does (their schedule recorded)
+    if (ctx->P.dim == 3 || tape_lists(ctx)) {
         rrsph_status st = adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
         ctx->need_full = true;
         return st;
@@ -2452,7 +2480,7 @@ rrsph_status rrsph_hip_adjoint_forward(rrsph_ctx* ctx, uint32_t nsteps, uint32_t
 rrsph_status rrsph_hip_adjoint_backward(rrsph_ctx* ctx, const double* eta_bar, double* grad_a, double* grad_b,
                                         double* grad_r0, double* grad_v0, double* grad_rho0) {
     if (!ctx) return RRSPH_ERR_INVALID_ARGUMENT;
-    if (ctx->P.dim == 3) {
+    if (ctx->P.dim == 3 || ctx->adj.lists) {
         rrsph_status st = adjoint_backward_impl(ctx, eta_bar, grad_a, grad_b, grad_r0, grad_v0, grad_rho0);
         ctx->need_full = true;
         return st;
@@ -2527,8 +2555,8 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     T.seg_sorted.assign(cap, 0);
     T.builds.assign(nsteps, 0);
     T.seg_build.assign(cap, -1);
-    if (T.lists) T.iota = dalloc<uint32_t>(n, e);
-    if (T.lists && ctx->fp32) T.nearf = dalloc<float4>(n, e);
+    if (T.lists && d3) T.iota = dalloc<uint32_t>(n, e);
+    if (T.lists && d3 && ctx->fp32) T.nearf = dalloc<float4>(n, e);
     T.eta = dalloc<double>((size_t)nsteps * kMaxGauges, e);
     T.zs = dalloc<double>((size_t)nsteps * kMaxGauges, e);
     T.ws = dalloc<double>((size_t)nsteps * kMaxGauges, e);
@@ -2539,7 +2567,9 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     T.lam[1] = dalloc<double>((d3 ? kLam3 : 8) * n, e);
     T.direct = dalloc<double>((d3 ? kDirect3 : 5) * n, e);
     T.drho_adj = dalloc<double>(n, e);
-    T.out_adj = dalloc<double4>((d3 ? sizeof(AdjRec3<double>) / sizeof(double4) : 1) * n, e);
+    T.out_adj = dalloc<double4>((d3        ? sizeof(AdjRec3<double>) / sizeof(double4)
+                                 : T.lists ? sizeof(AdjRec2) / sizeof(double4)
+                                           : 1) * n, e);
     T.flag = dalloc<uint32_t>(1, e);
     if (e != hipSuccess) {
         free_tape(ctx->adj);
@@ -2551,7 +2581,7 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
         free_tape(ctx->adj);
         return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc (adjoint tape): ") + hipGetErrorString(e));
     }
-    if (T.lists) {
+    if (T.iota) {
         std::vector<uint32_t> id(n);
         for (size_t i = 0; i < n; ++i) id[i] = (uint32_t)i;
         HIP_TRY(hipMemcpy(T.iota, id.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -2574,7 +2604,7 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
     // loop allocates once (the 943,906-particle basin, 12 steps: 32.4 -> 24.3 ms; the tank, 60 steps: 13.0 -> 10.0); another shape frees them first
     const char* store = std::getenv("RRSPH_HIP_ADJ_STORE");
     const bool segments = store && std::strcmp(store, "segments") == 0;
-    const bool lists = list_active(ctx) && ctx->P.dim == 3;
+    const bool lists = tape_lists(ctx);
     AdjTape& T = ctx->adj;
     T.valid = false;
     if (T.allocated && T.nsteps == nsteps && T.every == std::min(checkpoint_every, nsteps) && T.lists == lists &&
@@ -2599,6 +2629,16 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
     T.nseg_lists = 0;
     T.force_build = ~0ull;
     st = adjoint_run_checked(ctx, 0, nsteps, true, T.seg);
+    if (st != RRSPH_OK && T.lists && ctx->P.dim == 2 && ctx->host_ctrl->halted &&
+        ctx->host_ctrl->status == kStatusListOverflow) {
+        // a list ran out of room: the run starts over on sorted steps, which
+        // the context keeps to from here (as resume_halt has it)
+        st = restore_state_sync(ctx, T.ck[0]);
+        if (st != RRSPH_OK) return st;
+        ctx->list_mode = false;
+        ctx->err.clear();
+        return adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
+    }
     if (st != RRSPH_OK) return st;
     if (ctx->host_ctrl->halted)
         return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: the run halted during the adjoint forward");
@@ -2708,13 +2748,19 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
             // sort and reorder state k exactly as its step did (predict with its dt)
             const uint32_t* sk = sorted ? T.seg_keys + slot * n : (lists ? lists->keys : nullptr);
             const uint32_t* sp = sorted ? T.seg_perm + slot * n : (lists ? T.iota : nullptr);
+            // the loss term of state k: in 2D over lists with the pair gather
+            const bool with_gauges = !d3 && lists && k >= 1;
+            const size_t row = k >= 1 ? (size_t)(k - 1) * kMaxGauges : 0;
+            const double *eb = with_gauges ? T.eta_bar + row : nullptr, *zs = T.zs + row, *ws = T.ws + row;
             if (ctx->fp32)
                 enqueue_reverse_step<float>(ctx, T.hrec[k], T.uctrl + k, T.lam[cur], T.lam[1 - cur],
-                                            T.piston_sum + (size_t)k * kMaxSegments, sk, sp, lists, src);
+                                            T.piston_sum + (size_t)k * kMaxSegments, sk, sp, lists, src,
+                                            eb, zs, ws);
             else
                 enqueue_reverse_step<double>(ctx, T.hrec[k], T.uctrl + k, T.lam[cur], T.lam[1 - cur],
-                                             T.piston_sum + (size_t)k * kMaxSegments, sk, sp, lists, src);
-            if (k >= 1) enqueue_gauge_grad(ctx, k - 1, T.lam[1 - cur], src);  // loss term of state k
+                                             T.piston_sum + (size_t)k * kMaxSegments, sk, sp, lists, src,
+                                            eb, zs, ws);
+            if (k >= 1 && !with_gauges) enqueue_gauge_grad(ctx, k - 1, T.lam[1 - cur], src);
             HIP_TRY(hipGetLastError());
             cur = 1 - cur;
         }
