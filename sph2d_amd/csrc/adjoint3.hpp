@@ -65,6 +65,12 @@ __device__ __forceinline__ AdjHit3 adj_hit3(const AdjRec3<float>& r, const doubl
                    (double)r.vp.w};
 }
 
+__device__ __forceinline__ AdjParticle<3> adj_particle(const AdjHit3& h, int t) {
+    return AdjParticle<3>{{h.pos.x, h.pos.y, h.pos.z}, {h.u.x, h.u.y, h.u.z},    {h.v.x, h.v.y, h.v.z},
+                          {h.oa.x, h.oa.y, h.oa.z},    {h.ox.x, h.ox.y, h.ox.z}, h.u.w,
+                          h.pw,                        h.oa.w,                   t};
+}
+
 struct GaugeSpec3 {
     GaugeSpec g;
     double z[kMaxGauges];
@@ -244,72 +250,6 @@ __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, Sta
     }
 }
 
-// One orientation of a pair in 3D (see adj_orient): the owner's sums at the
-// owner's adjoints (Sb = m a-adjoint, s1 = m drho-adjoint, Xb = 2 eps m
-// av-adjoint, Lb = a-adjoint) give the adjoints of e, dv = v_nb - v_own,
-// du = u_nb - u_own, the reciprocal IR and the coefficient.
-struct V3 {
-    double x, y, z;
-};
-__device__ __forceinline__ double dot3(const V3& a, const V3& b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-
-__device__ __forceinline__ void adj_orient3(const AdjConsts& K, const AdjPair& Q, const V3& e, const V3& dv,
-                                            const V3& du, const V3& Sb, double s1, const V3& Xb, const V3& Lb,
-                                            bool lj, bool xsph, double coef, V3& eb, V3& dvb, V3& dub,
-                                            double& irb, double& coefb) {
-    const double Fpe = Q.Fp * Q.rinv;  // grad_e F = Fpe * e
-    // continuity: T1 = F (dv . e)
-    const double dve = dot3(dv, e);
-    dvb = {s1 * Q.F * e.x, s1 * Q.F * e.y, s1 * Q.F * e.z};
-    eb = {s1 * (Q.F * dv.x + dve * Fpe * e.x), s1 * (Q.F * dv.y + dve * Fpe * e.y),
-          s1 * (Q.F * dv.z + dve * Fpe * e.z)};
-    // acceleration: T2 = F coef e
-    const double Se = dot3(Sb, e);
-    eb.x += Q.F * coef * Sb.x + coef * Se * Fpe * e.x;
-    eb.y += Q.F * coef * Sb.y + coef * Se * Fpe * e.y;
-    eb.z += Q.F * coef * Sb.z + coef * Se * Fpe * e.z;
-    coefb = Q.F * Se;
-    dub = {0, 0, 0};
-    irb = 0;
-    // artificial viscosity: A = 2 IR (beta mu^2 - alpha c mu), mu = h vr / (d^2 + eta^2), vr = du . e
-    if (Q.app) {
-        const double Ab = coefb;
-        const double mub = Ab * 2.0 * Q.IR * (2.0 * K.beta * Q.mu - K.alpha_c);
-        irb += Ab * 2.0 * (K.beta * Q.mu * Q.mu - K.alpha_c * Q.mu);
-        const double vrb = mub * K.h * Q.den;
-        const double em = -2.0 * mub * Q.mu * Q.den;
-        eb.x += em * e.x + vrb * du.x;
-        eb.y += em * e.y + vrb * du.y;
-        eb.z += em * e.z + vrb * du.z;
-        dub.x += vrb * e.x;
-        dub.y += vrb * e.y;
-        dub.z += vrb * e.z;
-    }
-    // Lennard-Jones on a fluid owner from a wall neighbour: T3 = -e f(d)
-    if (lj) {
-        const double rn = K.r0 * Q.rinv;
-        const double rn2 = rn * rn, rn4 = rn2 * rn2, rn12 = rn4 * rn4 * rn4;
-        const double f = K.D * (rn12 - rn4) * Q.rinv * Q.rinv;
-        const double fp = K.D * (-14.0 * rn12 + 6.0 * rn4) * Q.rinv * Q.rinv * Q.rinv;  // df/dd
-        const double Le = dot3(Lb, e);
-        eb.x += -f * Lb.x - Le * fp * Q.rinv * e.x;
-        eb.y += -f * Lb.y - Le * fp * Q.rinv * e.y;
-        eb.z += -f * Lb.z - Le * fp * Q.rinv * e.z;
-    }
-    // XSPH from a fluid neighbour: T4 = du W IR
-    if (xsph) {
-        const double xdu = dot3(Xb, du);
-        dub.x += Xb.x * Q.W * Q.IR;
-        dub.y += Xb.y * Q.W * Q.IR;
-        dub.z += Xb.z * Q.W * Q.IR;
-        const double wb = Q.IR * xdu;
-        eb.x += wb * Q.F * e.x;  // grad_e W = F e
-        eb.y += wb * Q.F * e.y;
-        eb.z += wb * Q.F * e.z;
-        irb += Q.W * xdu;
-    }
-}
-
 // Gather over neighbours, both orientations of every pair, then the
 // predict and EOS reverse; writes lam_out.  Every lane of a block runs the
 // wave-uniform walk (lanes past n walk empty ranges).  LISTS: the
@@ -341,36 +281,18 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
     const uint32_t s = lb * kBlock + threadIdx.x;
     const bool live = s < P.n;
     const uint32_t sc = live ? s : P.n - 1;
-    AdjConsts K;
-    K.h = P.h;
-    K.inv_h = 1.0 / P.h;
-    K.c1 = P.f_cubic / (P.h * P.h);
-    K.c2 = 0.5 * P.f_cubic / P.h;
-    K.w1 = P.f_cubic;
-    K.w2 = P.f_cubic / 6.0;
-    K.alpha_c = P.av_alpha * P.av_c;
-    K.beta = P.av_beta;
-    K.eta2 = P.av_eta2;
-    K.r0 = P.lj_r0;
-    K.D = P.lj_D;
-    K.m = P.mass;
-    K.xf = 2.0 * P.mass * P.xsph_eps;
-    K.av_on = P.av_on;
-    K.xsph_on = P.xsph_on;
-    K.lj_on = P.lj_on;
+    const AdjConsts K = adj_consts(P);
     const double4 pk = B.pos[sc];
     const double4 vak = to_d4<R>(B.va[sc]);    // (v, rho)
     const double4 prk = to_d4<R>(B.pred[sc]);  // (u, R)
-    const double Pk = B.pw[sc];                // p / R^2
     const double pres_k = B.pres[sc];
     const AdjHit3 hk = adj_hit3(rec[sc], pk);
     float4 nk{};
     if constexpr (kNear) nk = nearf[sc];
-    const double4 oak = hk.oa;
-    const double4 oxk = hk.ox;
     const int tk = (int)pk.w;
-    V3 rb{0, 0, 0}, vb{0, 0, 0}, ub{0, 0, 0};
-    double Rb = 0, Pb = 0;
+    // (the own velocities and p / R^2 are those of its record)
+    const AdjParticle<3> own = adj_particle(hk, tk);
+    AdjSums<3> S;
     bool overflow = false;
     uint32_t* my = hits + threadIdx.x;
     // the loads of hit u + 1 are issued before the arithmetic of hit u (the
@@ -389,82 +311,25 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
 #pragma unroll 1
         for (uint32_t u = 0; u < nh; ++u) {
             const AdjHit3 h = adj_hit3(rn, pn);
-            const double4 vai = h.v;
-            const double4 pri = h.u;
-            const double Pi = h.pw;
-            const double4 oai = h.oa;
-            const double4 oxi = h.ox;
             int ti;
-            V3 e;  // r_i - r_k
+            double e[3];  // r_i - r_k
             if constexpr (kNear) {
                 const float4 o = s_off[in >> kSlotBits3];
-                e = V3{(double)((qn.x - nk.x) + o.x), (double)((qn.y - nk.y) + o.y), (double)((qn.z - nk.z) + o.z)};
+                e[0] = (double)((qn.x - nk.x) + o.x);
+                e[1] = (double)((qn.y - nk.y) + o.y);
+                e[2] = (double)((qn.z - nk.z) + o.z);
                 ti = (int)qn.w;
             } else {
-                e = V3{h.pos.x - pk.x, h.pos.y - pk.y, h.pos.z - pk.z};
+                e[0] = h.pos.x - pk.x;
+                e[1] = h.pos.y - pk.y;
+                e[2] = h.pos.z - pk.z;
                 ti = (int)h.pos.w;
             }
             in = my[min(u + 1, last) * kBlock];
             rn = rec[kNear ? in & kSlotMask3 : in];
             if constexpr (kNear) qn = nearf[in & kSlotMask3];
             else if constexpr (sizeof(R) == 4) pn = B.pos[in];
-            AdjPair Q;
-            Q.d2 = dot3(e, e);
-            Q.rinv = Q.d2 > 0.0 ? fast_rsqrt<double>(Q.d2) : 0.0;
-            Q.d = Q.d2 * Q.rinv;
-            const double q = Q.d * K.inv_h;
-            const double t = 2.0 - q;
-            if (q <= 1.0) {
-                Q.F = K.c1 * (1.5 * q - 2.0);
-                Q.Fp = 1.5 * K.c1 * K.inv_h;
-                Q.W = K.w1 * (2.0 / 3.0 - q * q + 0.5 * q * q * q);
-            } else {
-                Q.F = -K.c2 * t * t * Q.rinv;
-                Q.Fp = K.c2 * t * (2.0 * Q.rinv * K.inv_h + t * Q.rinv * Q.rinv);
-                Q.W = K.w2 * t * t * t;
-            }
-            Q.IR = fast_rcp<double>(pri.w + prk.w);
-            const V3 du{pri.x - prk.x, pri.y - prk.y, pri.z - prk.z};  // u_i - u_k
-            Q.vr = dot3(du, e);
-            Q.den = fast_rcp<double>(Q.d2 + K.eta2);
-            Q.mu = K.h * Q.vr * Q.den;
-            Q.app = K.av_on && Q.vr < 0.0;
-            Q.A = Q.app ? 2.0 * Q.IR * (K.beta * Q.mu * Q.mu - K.alpha_c * Q.mu) : 0.0;
-            const double coef = Pi + Pk + Q.A;
-            const V3 dv{vai.x - vak.x, vai.y - vak.y, vai.z - vak.z};  // v_i - v_k
-            V3 eb, dvb, dub;
-            double irb, coefb;
-            // Both orientations of the pair in one evaluation.  k's sum at
-            // k's adjoints is adj_orient3 at (e, dv, du); i's sum at i's
-            // adjoints is adj_orient3 at (-e, -dv, -du), entering rb, vb, ub
-            // with the opposite sign and Rb, Pb with the same.  Every output is
-            // linear in the owner's adjoints, and even (the a- and
-            // av-adjoint terms, the wall force) or odd (the drho-adjoint
-            // terms) in (e, dv, du), so the two make one evaluation at
-            // (e, dv, du) with the owner adjoints m (oa_k - oa_i) and
-            // m (drho_k + drho_i), the XSPH adjoint of whichever owner has a
-            // fluid neighbour (i's negated), and the wall force of whichever
-            // owner is the fluid particle (i's negated).
-            const bool xk = K.xsph_on && ti > 0, xi = K.xsph_on && tk > 0;
-            const bool ljk = K.lj_on && tk > 0 && ti < 0 && Q.d < K.r0;
-            const bool lji = K.lj_on && ti > 0 && tk < 0 && Q.d < K.r0;
-            const V3 Xd{K.xf * ((xk ? oxk.x : 0.0) - (xi ? oxi.x : 0.0)),
-                        K.xf * ((xk ? oxk.y : 0.0) - (xi ? oxi.y : 0.0)),
-                        K.xf * ((xk ? oxk.z : 0.0) - (xi ? oxi.z : 0.0))};
-            const V3 L = ljk ? V3{oak.x, oak.y, oak.z} : V3{-oai.x, -oai.y, -oai.z};
-            adj_orient3(K, Q, e, dv, du, V3{K.m * (oak.x - oai.x), K.m * (oak.y - oai.y), K.m * (oak.z - oai.z)},
-                        K.m * (oak.w + oai.w), Xd, L, ljk || lji, xk || xi, coef, eb, dvb, dub, irb, coefb);
-            rb.x -= eb.x;
-            rb.y -= eb.y;
-            rb.z -= eb.z;
-            vb.x -= dvb.x;
-            vb.y -= dvb.y;
-            vb.z -= dvb.z;
-            ub.x -= dub.x;
-            ub.y -= dub.y;
-            ub.z -= dub.z;
-            Rb -= Q.IR * Q.IR * irb;
-            Pb += coefb;
+            adj_pair_term<3>(K, own, adj_particle(h, ti), e, S);
         }
     };
     if constexpr (kNear)
@@ -477,28 +342,12 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
                                        overflow, flush);
     if (overflow) atomicOr(overflow_flag, 1u);
     if (!live) return;
-    // P = p / R^2, p = EOS(rho) = B ((rho / rho0)^7 - 1), u = v + a_prev dt/2, R = rho + drho_prev dt/2
-    const double Rk = prk.w;
-    const double pb = Pb / (Rk * Rk);
-    Rb += -2.0 * Pb * pres_k / (Rk * Rk * Rk);
-    const double x = vak.w / P.rho0;
-    const double x2 = x * x, x3 = x2 * x;
-    const double dpdrho = 7.0 * P.eos_B * x3 * x3 / P.rho0;
-    const double* d = direct + kDirect3 * (size_t)s;
-    const double h2 = T.dt_pred * 0.5;
-    double* l = lam_out + kLam3 * (size_t)B.oid[s];
-    l[0] = d[0] + rb.x;
-    l[1] = d[1] + rb.y;
-    l[2] = d[2] + rb.z;
-    l[3] = d[3] + vb.x + ub.x;
-    l[4] = d[4] + vb.y + ub.y;
-    l[5] = d[5] + vb.z + ub.z;
-    l[6] = d[6] + (P.density_treatment != 0 ? Rb : 0.0) + pb * dpdrho;
-    l[7] = ub.x * h2;
-    l[8] = ub.y * h2;
-    l[9] = ub.z * h2;
-    l[10] = P.density_treatment != 0 ? Rb * h2 : 0.0;
-    l[11] = 0.0;
+    double l[kLam3];
+    adj_predict<3>(P, T.dt_pred, S, prk.w, pres_k, vak.w, direct + kDirect3 * (size_t)s, l);
+    l[kLam3 - 1] = 0.0;
+    double2* out = (double2*)(lam_out + kLam3 * (size_t)B.oid[s]);
+#pragma unroll
+    for (uint32_t c = 0; c < kLam3 / 2; ++c) out[c] = make_double2(l[2 * c], l[2 * c + 1]);
 }
 
 }  // namespace rrsph
