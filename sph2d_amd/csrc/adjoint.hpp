@@ -467,6 +467,7 @@ template <int D> __device__ __forceinline__ double adj_dot(const double (&a)[D],
 template <int D>
 __device__ __forceinline__ void adj_pair_term(const AdjConsts& K, const AdjParticle<D>& k, const AdjParticle<D>& i,
                                               const double (&e)[D], AdjSums<D>& S) {
+#pragma clang fp contract(off)  // the same roundings in every kernel that calls it
     const double d2 = adj_dot<D>(e, e);
     const double rinv = d2 > 0.0 ? fast_rsqrt<double>(d2) : 0.0;
     const double d = d2 * rinv, q = d * K.inv_h, t = 2.0 - q, tr = t * rinv;
@@ -512,7 +513,7 @@ __device__ __forceinline__ void adj_pair_term(const AdjConsts& K, const AdjParti
         for (int c = 0; c < D; ++c) L[c] = k.t > 0 ? k.a[c] : -i.a[c];
         const double rn = K.r0 * rinv, rn2 = rn * rn, rn4 = rn2 * rn2, rn12 = rn4 * rn4 * rn4, ri2 = rinv * rinv;
         const double f = K.lj_Dm * (rn12 - rn4) * ri2;
-        const double g = K.lj_Dm * (-14.0 * rn12 + 6.0 * rn4) * ri2 * ri2 * adj_dot<D>(L, e);  // df/dd / d (L . e)
+        const double g = K.lj_Dm * fma(-14.0, rn12, 6.0 * rn4) * ri2 * ri2 * adj_dot<D>(L, e);  // df/dd / d (L . e)
 #pragma unroll
         for (int c = 0; c < D; ++c) S.r[c] += fma(f, L[c], g * e[c]);
     }
@@ -523,6 +524,7 @@ __device__ __forceinline__ void adj_pair_term(const AdjConsts& K, const AdjParti
 template <int D>
 __device__ __forceinline__ void adj_predict(const StepParams& P, double dt_pred, AdjSums<D> S, double Rk, double pres,
                                             double rho, const double* __restrict__ d, double* __restrict__ l) {
+#pragma clang fp contract(off)
     S.each([&](double v) { return v * P.mass; });
     const double pb = S.P / (Rk * Rk);
     const double Rb = S.R - 2.0 * S.P * pres / (Rk * Rk * Rk);

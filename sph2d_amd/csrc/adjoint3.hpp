@@ -24,16 +24,14 @@ constexpr uint32_t kDirect3 = 8;
 
 // What the pair adjoint of a neighbour reads of slot s, in one record:
 // the output adjoints oa = (a x y z, drho) and ox = (av x y z), p / R^2,
-// the velocity v and the predicted (u, R).  The FP64 step's record holds
-// its position too, all in FP64.  The FP32 step's record is 64 bytes, two
-// slots per cache line (a hit's gather costs by the lines it touches, and
-// the neighbours of a particle lie in runs of slots): the state in its
-// FP32 and the adjoints rounded to FP32 (the arithmetic stays FP64); the
-// FP64 position comes from the packed position array, whose lines the
-// neighbour walk has just read.
+// the velocity v and the predicted (u, R): 128 bytes in FP64.  The FP32
+// step's record is 64 bytes, two slots per cache line (a hit's gather costs
+// by the lines it touches, and the neighbours of a particle lie in runs of
+// slots): the state in its FP32 and the adjoints rounded to FP32 (the
+// arithmetic stays FP64).  The position comes from the packed position
+// array, whose lines the neighbour walk has just read.
 template <class R> struct AdjRec3;
-template <> struct alignas(32) AdjRec3<double> {
-    double4 pos;
+template <> struct alignas(128) AdjRec3<double> {
     double4 oa;
     double ox, oy, oz, pw;
     double4 v;  // (v x y z, unused)
@@ -45,16 +43,15 @@ template <> struct alignas(64) AdjRec3<float> {
     float4 oa;
     float4 ox;  // (av x y z, unused)
 };
-static_assert(sizeof(AdjRec3<float>) == 64, "two records per cache line");
+static_assert(sizeof(AdjRec3<float>) == 64 && sizeof(AdjRec3<double>) == 128, "words of a wave gather");
 
-// The fields of a record, widened to FP64 (pos: the FP64 record's own,
-// else the position array's entry).
+// The fields of a record, widened to FP64, with its position.
 struct AdjHit3 {
     double4 pos, v, u, oa, ox;
     double pw;
 };
-__device__ __forceinline__ AdjHit3 adj_hit3(const AdjRec3<double>& r, const double4&) {
-    return AdjHit3{r.pos, r.v, r.u, r.oa, make_double4(r.ox, r.oy, r.oz, 0.0), r.pw};
+__device__ __forceinline__ AdjHit3 adj_hit3(const AdjRec3<double>& r, const double4& pos) {
+    return AdjHit3{pos, r.v, r.u, r.oa, make_double4(r.ox, r.oy, r.oz, 0.0), r.pw};
 }
 __device__ __forceinline__ AdjHit3 adj_hit3(const AdjRec3<float>& r, const double4& pos) {
     return AdjHit3{pos,
@@ -215,7 +212,6 @@ __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, Sta
             r.oa = make_float4((float)oa.x, (float)oa.y, (float)oa.z, (float)oa.w);
             r.ox = make_float4((float)ox.x, (float)ox.y, (float)ox.z, 0.f);
         } else {
-            r.pos = ps;
             r.oa = oa;
             r.ox = ox.x;
             r.oy = ox.y;
@@ -271,6 +267,8 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
     constexpr bool kNear = LISTS && sizeof(R) == 4;
     __shared__ uint32_t hits[kAdjChunk * kBlock];
     __shared__ float4 s_off[kNear ? kCodes3 : 1];
+    constexpr bool kGathered = LISTS && sizeof(R) == 8;
+    __shared__ uint4 s_rec[kBlock / kWave][kGathered ? 8 * kWave : 1];
     // XCD-aware: each XCD walks one contiguous slice of the slots
     const uint32_t lb = xcd_block(P.blocks_per_xcd);
     if (lb >= P.nblocks) return;
@@ -295,41 +293,79 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
     AdjSums<3> S;
     bool overflow = false;
     uint32_t* my = hits + threadIdx.x;
-    // the loads of hit u + 1 are issued before the arithmetic of hit u (the
-    // kernel runs at 2 waves per SIMD either way, so the registers are free;
-    // a second record in flight needs more registers than 2 waves leave)
+    // Over lists in FP64 the wave fetches the records of its lanes' next hits
+    // together (WaveGather) while it works on this round's: lanes loading their
+    // own made 10 accesses of up to 64 lines a hit, which bound the loop
+    // (509,126 particles 503 -> 427 us).  In FP32, 5 accesses a hit, it made no
+    // difference (943,906 particles: 623 us, 638 and with two records in flight
+    // 632 gathered), nor did 3 waves per SIMD, which spill (791).
     auto flush = [&](uint32_t nh) {
-        if (nh == 0) return;
-        const uint32_t last = nh - 1;
-        // kNear: the hit list holds whole entries (slot and home-cell code)
-        uint32_t in = my[0];
-        AdjRec3<R> rn = rec[kNear ? in & kSlotMask3 : in];
-        double4 pn{};
-        float4 qn{};
-        if constexpr (kNear) qn = nearf[in & kSlotMask3];
-        else if constexpr (sizeof(R) == 4) pn = B.pos[in];
+        if constexpr (kGathered) {
+            const uint32_t nmax = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u32(nh));
+            if (nmax == 0) return;
+            auto hit = [&](uint32_t u) { return u < nh ? my[u * kBlock] : sc; };  // past its hits: its own slot
+            uint4* buf = s_rec[wave_of_block()];
+            using Half = WaveGather<4, sizeof(AdjRec3<R>), kSlotMask3>;
+            const WaveGatherBoth<Half, Half> src{Half(rec, buf), Half((const char*)rec + 64, buf + 4 * kWave)};
+            uint32_t in = hit(0), next = hit(1);
+            double4 pn{};
+            auto fetch = [&]() {
+                pn = B.pos[in];
+                src.fetch(0, in);
+            };
+            fetch();
 #pragma unroll 1
-        for (uint32_t u = 0; u < nh; ++u) {
-            const AdjHit3 h = adj_hit3(rn, pn);
-            int ti;
-            double e[3];  // r_i - r_k
-            if constexpr (kNear) {
-                const float4 o = s_off[in >> kSlotBits3];
-                e[0] = (double)((qn.x - nk.x) + o.x);
-                e[1] = (double)((qn.y - nk.y) + o.y);
-                e[2] = (double)((qn.z - nk.z) + o.z);
-                ti = (int)qn.w;
-            } else {
-                e[0] = h.pos.x - pk.x;
-                e[1] = h.pos.y - pk.y;
-                e[2] = h.pos.z - pk.z;
-                ti = (int)h.pos.w;
+            for (uint32_t u = 0; u < nmax; ++u) {
+                uint4 w[8];
+                wait_loads();
+                src.read(0, w);
+                const double4 p = pn;
+                in = next;
+                next = hit(u + 2);
+                wait_lds();  // the records are in registers: the next ones may land
+                __builtin_amdgcn_sched_barrier(0);
+                if (u + 1 < nmax) fetch();
+                if (u >= nh) continue;
+                AdjRec3<R> r;
+                __builtin_memcpy(&r, w, sizeof r);
+                const double e[3] = {p.x - pk.x, p.y - pk.y, p.z - pk.z};  // r_i - r_k
+                adj_pair_term<3>(K, own, adj_particle(adj_hit3(r, p), (int)p.w), e, S);
             }
-            in = my[min(u + 1, last) * kBlock];
-            rn = rec[kNear ? in & kSlotMask3 : in];
+        } else {
+            // the loads of hit u + 1 are issued before the arithmetic of hit u (the
+            // kernel runs at 2 waves per SIMD either way, so the registers are free;
+            // a second record in flight needs more registers than 2 waves leave)
+            if (nh == 0) return;
+            // kNear: the hit list holds whole entries (slot and home-cell code)
+            uint32_t in = my[0];
+            AdjRec3<R> rn = rec[kNear ? in & kSlotMask3 : in];
+            double4 pn{};
+            float4 qn{};
             if constexpr (kNear) qn = nearf[in & kSlotMask3];
-            else if constexpr (sizeof(R) == 4) pn = B.pos[in];
-            adj_pair_term<3>(K, own, adj_particle(h, ti), e, S);
+            else pn = B.pos[in];
+#pragma unroll 1
+            for (uint32_t u = 0; u < nh; ++u) {
+                const AdjHit3 h = adj_hit3(rn, pn);
+                int ti;
+                double e[3];  // r_i - r_k
+                if constexpr (kNear) {
+                    const float4 o = s_off[in >> kSlotBits3];
+                    e[0] = (double)((qn.x - nk.x) + o.x);
+                    e[1] = (double)((qn.y - nk.y) + o.y);
+                    e[2] = (double)((qn.z - nk.z) + o.z);
+                    ti = (int)qn.w;
+                } else {
+                    e[0] = h.pos.x - pk.x;
+                    e[1] = h.pos.y - pk.y;
+                    e[2] = h.pos.z - pk.z;
+                    ti = (int)h.pos.w;
+                }
+                in = my[min(u + 1, nh - 1) * kBlock];
+                rn = rec[kNear ? in & kSlotMask3 : in];
+                if constexpr (kNear) qn = nearf[in & kSlotMask3];
+                else pn = B.pos[in];
+                adj_pair_term<3>(K, own, adj_particle(h, ti), e, S);
+            }
         }
     };
     if constexpr (kNear)
