@@ -590,7 +590,7 @@ __global__ void __launch_bounds__(kBlock) adj_pair(StepParams P, AdjStep T, Stat
 // all that the pair adjoint reads of a particle: 128 bytes, which the wave
 // fetches as WaveGather does, in two halves of four words.
 // Per step of 134,042 particles (FP64): reorder 8.9 us, prep 6.9, cell walk
-// 41.2 and gauge gradients 5.0 us before; prep 16.0 and pair with gauges 31.2 now.
+// 41.2 and gauge gradients 5.0 us before; prep 9.9 and pair with gauges 30.9 now.
 struct alignas(128) AdjRec2 {
     double2 pos, u, v;
     double R, pw;      // R = typed_rho: the sign of the type, 0 for a dead particle
@@ -606,13 +606,19 @@ __device__ __forceinline__ AdjParticle<2> adj_particle(const AdjRec2& r) {
                           fabs(r.R),          r.pw,           r.da,           r.R > 0.0 ? 1 : (r.R < 0.0 ? -1 : 0)};
 }
 
-// perm: the build step's permutation, or null where the state is in slot order.
+// perm: the build step's permutation, or null where the state is in slot
+// order.  A wave's records go through LDS, so that its stores are contiguous:
+// every lane storing its own wrote 16 bytes of each of 64 lines at a time
+// (134,042 particles 16.0 -> 9.9 us, 40 bytes of direct adjoints left out too).
+// (word p of record t in place p ^ t % 8, for the banks)
 template <class R>
 __global__ void __launch_bounds__(kBlock) adj_prep_list(StepParams P, AdjStep T, StateA<R> A,
                                                         const uint32_t* __restrict__ perm,
                                                         const double* __restrict__ lam_in, AdjRec2* __restrict__ rec,
-                                                        double* __restrict__ direct, double* __restrict__ piston_sum) {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+                                                        double* __restrict__ piston_sum) {
+    __shared__ uint4 s_rec[kBlock / kWave][8 * kWave];
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x, lane = __lane_id();
+    uint4* buf = s_rec[wave_of_block()];
     double pist = 0.0;
     if (s < P.n) {
         const uint32_t src = perm ? min(perm[s], P.n - 1) : s;
@@ -629,8 +635,20 @@ __global__ void __launch_bounds__(kBlock) adj_prep_list(StepParams P, AdjStep T,
         r.pw = (double)pr.w;
         r.rho = (double)va.z;
         r.pres = (double)p;
-        pist = adj_whole_step(P, T, (int)va.w, r.oid, lam_in + 8 * (size_t)r.oid, r.oa, r.da, direct + 5 * (size_t)s);
-        rec[s] = r;
+        double direct[5];  // (the pair adjoint works these out again)
+        pist = adj_whole_step(P, T, r.itype, r.oid, lam_in + 8 * (size_t)r.oid, r.oa, r.da, direct);
+        uint4 w[8];
+        __builtin_memcpy(w, &r, sizeof r);
+#pragma unroll
+        for (uint32_t q = 0; q < 8; ++q) buf[8 * lane + (q ^ (lane & 7))] = w[q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t first = s - lane;  // the wave's first slot
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) {
+        const uint32_t t = 8 * q + lane / 8, w = lane & 7;
+        if (first + t < P.n) ((uint4*)rec)[8 * (size_t)(first + t) + w] = buf[8 * t + (w ^ (t & 7))];
     }
     adj_piston_sum(pist, piston_sum);
 }
@@ -640,10 +658,10 @@ __global__ void __launch_bounds__(kBlock) adj_prep_list(StepParams P, AdjStep T,
 // Every entry is decided as the step decided it (FP32 steps too: their test
 // ends in the same FP64 comparison).
 template <int LPP>
-__global__ void __launch_bounds__(kBlock) adj_pair_list(StepParams P, double dt_pred, const AdjRec2* __restrict__ rec,
+__global__ void __launch_bounds__(kBlock) adj_pair_list(StepParams P, AdjStep T, const AdjRec2* __restrict__ rec,
                                                         const uint32_t* __restrict__ nbl,
                                                         const uint32_t* __restrict__ nbc,
-                                                        const double* __restrict__ direct,
+                                                        const double* __restrict__ lam_in,
                                                         double* __restrict__ lam_out,
                                                         uint32_t* __restrict__ overflow_flag, GaugeSpec G,
                                                         const double* __restrict__ eta_bar,
@@ -677,10 +695,12 @@ __global__ void __launch_bounds__(kBlock) adj_pair_list(StepParams P, double dt_
     S.each([](double v) { return lane_sum<LPP>(v); });
     if (lane_sum<LPP>((int)hits) > (int)(P.max_nbr - 1)) atomicOr(overflow_flag, 1u);
     if (!live || g.l != 0) return;
-    double l[8];
+    double l[8], direct[5], da;
+    double4 oa;
     const AdjRec2& own = rec[s];
+    adj_whole_step(P, T, own.itype, own.oid, lam_in + 8 * (size_t)own.oid, oa, da, direct);
     // (a dead particle has no sums, and no density in its record)
-    adj_predict<2>(P, dt_pred, S, k.t != 0 ? k.R : 1.0, own.pres, own.rho, direct + 5 * (size_t)s, l);
+    adj_predict<2>(P, T.dt_pred, S, k.t != 0 ? k.R : 1.0, own.pres, own.rho, direct, l);
     if (eta_bar && own.itype == G.ptype) {
         double gx, gy;
         if (gauge_gradient(G, own.pos, eta_bar, zsum, wsum, gx, gy)) {

@@ -1198,10 +1198,10 @@ static void enqueue_reverse_step(rrsph_ctx* ctx, const AdjStep& S, Ctrl* uc, con
     if (P.dim == 2 && lists) {
         AdjRec2* rec = (AdjRec2*)T.out_adj;
         const StateA<R> A{(double2*)src->pos, (real4<R>*)src->va, (real4<R>*)src->ad, src->oid};
-        adj_prep_list<R><<<nb, kBlock, 0, ctx->stream>>>(P, S, A, perm, lam_in, rec, T.direct, psum);
+        adj_prep_list<R><<<nb, kBlock, 0, ctx->stream>>>(P, S, A, perm, lam_in, rec, psum);
         auto pair = [&](auto kernel, uint32_t blocks) {
-            kernel<<<blocks * kNumXcd, kBlock, 0, ctx->stream>>>(P, S.dt_pred, rec, lists->nbl, lists->nbc, T.direct,
-                                                                 lam_out, T.flag, T.spec.g, eta_bar, zs, ws);
+            kernel<<<blocks * kNumXcd, kBlock, 0, ctx->stream>>>(P, S, rec, lists->nbl, lists->nbc, lam_in, lam_out,
+                                                                 T.flag, T.spec.g, eta_bar, zs, ws);
         };
         if (P.n < kAdjLanes8) pair(adj_pair_list<8>, group_blocks_per_xcd<8>(P.n));
         else pair(adj_pair_list<2>, group_blocks_per_xcd<2>(P.n));
