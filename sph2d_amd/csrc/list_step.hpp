@@ -41,6 +41,7 @@
 // on the reordered copy, integrating into A.
 #pragma once
 
+#include "cell_sort.hpp"
 #include "device_common.hpp"
 #include "step_kernels.hpp"
 
@@ -104,19 +105,23 @@ template <class R> __device__ __forceinline__ real4<R> predict_record(const Step
 
 // The reorder of a build step: reorder_kernel's gather, prediction,
 // pressure and cell-start table, plus the records of the list pass and each
-// slot's home cell (its cell key).
-template <class R>
+// slot's home cell (its cell key).  COUNTED: behind the counting sort, with
+// perm as its scatter left it; the cell-start table is there, and the
+// permutation goes to perm_out.
+template <class R, bool COUNTED>
 __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, const Ctrl* __restrict__ ctrl,
                                                               const uint32_t* __restrict__ skey,
                                                               const uint32_t* __restrict__ perm, StateA<R> A,
                                                               StateB<R> B, ListRec<R>* __restrict__ rec,
-                                                              uint32_t* __restrict__ home, uint32_t* __restrict__ LB) {
+                                                              uint32_t* __restrict__ home, uint32_t* __restrict__ LB,
+                                                              uint32_t* __restrict__ perm_out) {
     if (ctrl->halted) return;
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
-    const uint32_t s = live ? s0 : P.n - 1;
+    uint32_t s = live ? s0 : P.n - 1;
     const uint32_t k = skey[s];
     const uint32_t src = min(perm[s], P.n - 1);  // a permutation of [0, n); the clamp only guards memory
+    if constexpr (COUNTED) s = cell_place(P, LB, perm, s, k);
     const double2 pos = A.pos[src];
     const real4<R> va = A.va[src];
     const real4<R> ad = A.ad[src];
@@ -133,8 +138,9 @@ __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, cons
         r.pr = pr;
         rec[s] = r;
         home[s] = k;
+        if constexpr (COUNTED) perm_out[s] = src;
     }
-    fill_cell_starts(P, s, live, k, skey, LB);
+    if constexpr (!COUNTED) fill_cell_starts(P, s, live, k, skey, LB);
 }
 
 // ------------------------------------------------------------------ control of list steps

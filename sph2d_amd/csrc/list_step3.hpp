@@ -76,20 +76,22 @@ __device__ __forceinline__ real4<R> predict3(const StepParams& P, const real4<R>
 // The reorder of a 3D build step: reorder3_kernel's gather, pressure and
 // cell-start table, plus the records, each slot's home cell and its
 // candidate record for the build's walk, cand = (position relative to the
-// home cell's origin in FP32, the home cell's z index).
-template <class R>
+// home cell's origin in FP32, the home cell's z index).  COUNTED as in 2D.
+template <class R, bool COUNTED>
 __global__ void __launch_bounds__(kBlock) reorder_list3_kernel(StepParams P, const Ctrl* __restrict__ ctrl,
                                                                const uint32_t* __restrict__ skey,
                                                                const uint32_t* __restrict__ perm, StateA3<R> A,
                                                                StateB3<R> B, ListRec<R>* __restrict__ rec,
                                                                real4<R>* __restrict__ dens, uint32_t* __restrict__ home,
-                                                               float4* __restrict__ cand, uint32_t* __restrict__ LB) {
+                                                               float4* __restrict__ cand, uint32_t* __restrict__ LB,
+                                                               uint32_t* __restrict__ perm_out) {
     if (ctrl->halted) return;
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
-    const uint32_t s = live ? s0 : P.n - 1;
+    uint32_t s = live ? s0 : P.n - 1;
     const uint32_t k = skey[s];
     const uint32_t src = min(perm[s], P.n - 1);  // a permutation of [0, n); the clamp only guards memory
+    if constexpr (COUNTED) s = cell_place(P, LB, perm, s, k);
     const double4 pos = A.pos[src];
     const real4<R> va = A.va[src];
     const real4<R> ad = A.ad[src];
@@ -111,8 +113,9 @@ __global__ void __launch_bounds__(kBlock) reorder_list3_kernel(StepParams P, con
         const double3 o = cell_origin3(P, k);
         cand[s] = make_float4((float)(pos.x - o.x), (float)(pos.y - o.y), (float)(pos.z - o.z),
                               __int_as_float((int)(k % (uint32_t)P.ncz)));
+        if constexpr (COUNTED) perm_out[s] = src;
     }
-    fill_cell_starts(P, s, live, k, skey, LB);
+    if constexpr (!COUNTED) fill_cell_starts(P, s, live, k, skey, LB);
 }
 
 // The lists of a 3D build step on the reordered copy: for each live

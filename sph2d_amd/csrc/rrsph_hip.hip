@@ -258,6 +258,7 @@ struct rrsph_ctx {
     uint32_t* home = nullptr;           // each slot's cell at the last build
     unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima, a set per step parity)
     unsigned long long* dtslots = nullptr; // list steps: dt maxima (likewise)
+    uint32_t* cell_count = nullptr;         // builds with the counting sort: cell counts (zero between builds), scan sums
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
     ListGraphs list_graphs;             // of plain runs
     bool taping = false;                // ctx->P holds the taped runs' skin
@@ -365,6 +366,31 @@ void enqueue_sort(rrsph_ctx* c, Ctrl* ctrl, Launcher& L) {
     }
     c->sorted_keys = src_k;
     c->sorted_perm = src_v;
+}
+
+// The sort of a list build: the counting sort, whose reorder puts the slots
+// of a cell in order (the permutation then lies in cell_sort_perm), or the
+// radix sort where most cells of the grid are empty.
+uint32_t* cell_sort_perm(const rrsph_ctx* c) { return c->vbuf[(c->passes - 1) & 1u]; }
+void enqueue_build_sort(rrsph_ctx* c, Ctrl* ctrl, Launcher& L) {
+    if (!c->cell_count) {
+        enqueue_sort(c, ctrl, L);
+        return;
+    }
+    const StepParams& P = c->P;
+    const uint32_t fb = (c->passes - 1) & 1u, nb = P.blocks_per_xcd * kNumXcd, sb = scan_blocks(P.ncells);
+    uint32_t *skey = c->kbuf[fb], *place = c->kbuf[1 - fb], *slots = c->vbuf[1 - fb];
+    uint32_t* sums = c->cell_count + (size_t)sb * kScanCells;
+    L(K_UPSWEEP, [&] { cell_count_kernel<<<nb, kBlock, 0, c->stream>>>(P, c->key_next, place, c->cell_count, ctrl); });
+    L(K_SCAN, [&] {
+        cell_sums_kernel<<<sb, kBlock, 0, c->stream>>>(c->cell_count, sums, ctrl);
+        cell_starts_kernel<<<sb, kBlock, 0, c->stream>>>(P.ncells, c->cell_count, sums, c->LB, ctrl);
+    });
+    L(K_DOWNSWEEP, [&] {
+        cell_scatter_kernel<<<nb, kBlock, 0, c->stream>>>(P, c->key_next, place, c->LB, skey, slots, ctrl);
+    });
+    c->sorted_keys = skey;
+    c->sorted_perm = slots;
 }
 
 // Incremental re-sort of key_next against skeyA into kbuf[0] / vbuf[0]; its
@@ -570,12 +596,16 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, ListSt
         L(K_PROLOGUE, [&] {
             list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
         });
-        enqueue_sort(c, c->ctrl_cur, L);
+        enqueue_build_sort(c, c->ctrl_cur, L);
         StateA<R> A = stateA<R>(c);
         StateB<R> B = stateB<R>(c, c->pred, c->pres);
         L(K_REORDER, [&] {
-            reorder_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
-                                                                 rec, c->home, c->LB);
+            auto reorder = [&](auto kernel) {
+                kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B, rec, c->home,
+                                                     c->LB, cell_sort_perm(c));
+            };
+            if (c->cell_count) reorder(reorder_list_kernel<R, true>);
+            else reorder(reorder_list_kernel<R, false>);
         });
         L(K_LIST_BUILD, [&] {
             list_build_kernel<R><<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->posB, (const real4<R>*)c->vaB,
@@ -619,12 +649,16 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListS
         L(K_PROLOGUE, [&] {
             list_prologue<<<1, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, c->dslots, c->dtslots);
         });
-        enqueue_sort(c, c->ctrl_cur, L);
+        enqueue_build_sort(c, c->ctrl_cur, L);
         StateA3<R> A = stateA3<R>(c);
         StateB3<R> B = stateB3<R>(c, c->pred, c->pw, c->pres);
         L(K_REORDER, [&] {
-            reorder_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B,
-                                                                  rec, dens, c->home, c->cand, c->LB);
+            auto reorder = [&](auto kernel) {
+                kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B, rec, dens,
+                                                     c->home, c->cand, c->LB, cell_sort_perm(c));
+            };
+            if (c->cell_count) reorder(reorder_list3_kernel<R, true>);
+            else reorder(reorder_list3_kernel<R, false>);
         });
         L(K_LIST_BUILD, [&] {
             list_build3_kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, (const double4*)c->posB, c->cand,
@@ -1155,7 +1189,8 @@ void free_all(rrsph_ctx* c) {
                     c->maxslots, c->LB, c->ctrl, c->ctrl_cur,
                     c->util_ctrl, c->red, c->st_r, c->st_v, c->st_rho, c->st_p, c->st_a, c->st_drho, c->st_av,
                     c->st_mu, c->st_itype, c->st_u32, c->skeyA, c->chg, c->chg_mask, c->wpre, c->pw,
-                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->dtslots, c->cand, c->rec1, c->ctrl_alt};
+                    c->pw_scratch, c->adB, c->nbl, c->nbc, c->rec, c->dens, c->home, c->dslots, c->dtslots, c->cand, c->rec1, c->ctrl_alt,
+                    c->cell_count};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (c->host_ctrl) (void)hipHostFree(c->host_ctrl);
@@ -1315,9 +1350,19 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
             ctx->ctrl_alt = dalloc<Ctrl>(1, e);
         }
         ctx->dtslots = dalloc<unsigned long long>(2 * kDtSet, e);
+        // the counting sort's scan passes over every cell of the grid: 12 bytes a
+        // cell, so that 4 cells a particle take what one radix pass does (24 bytes
+        // a particle read twice and written once); sparser grids keep the radix sort
+        const char* sort = std::getenv("RRSPH_HIP_BUILD_SORT");
+        if ((uint64_t)ctx->P.ncells <= 4ull * n && !(sort && std::strcmp(sort, "radix") == 0)) {
+            const size_t blocks = scan_blocks(ctx->P.ncells);
+            ctx->cell_count = dalloc<uint32_t>(blocks * (kScanCells + 1), e);
+        }
     }
     if (e != hipSuccess) return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
     if (ctx->dslots) HIP_TRY(hipMemset(ctx->dslots, 0, 4 * kSlotSet * sizeof(unsigned long long)));
+    if (ctx->cell_count)
+        HIP_TRY(hipMemset(ctx->cell_count, 0, (size_t)scan_blocks(ctx->P.ncells) * kScanCells * sizeof(uint32_t)));
     if (ctx->nbl) HIP_TRY(hipMemset(ctx->nbl, 0, (size_t)(ctx->P.list_cap + kListPad) * n * sizeof(uint32_t)));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_ctrl, sizeof(Ctrl), hipHostMallocDefault));
     HIP_TRY(hipHostMalloc((void**)&ctx->host_eta, kMaxGauges * sizeof(double), hipHostMallocDefault));
