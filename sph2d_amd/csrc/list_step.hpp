@@ -1481,9 +1481,10 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
 // At the head of a list step's integrator (every thread): the step's dt;
 // block 0 publishes the control block and clears the next step's dt slots.
 // False when the step halted or halts here (dt below the reference's
-// never-ending bound, more neighbours than max_neighbours - 1).
+// never-ending bound, more neighbours than max_neighbours - 1).  keep: a
+// tape's copy of the published words, or null.
 __device__ __forceinline__ bool list_dt(const StepParams& P, Ctrl* next, const Ctrl* cur,
-                                        unsigned long long* maxslots, double& dt) {
+                                        unsigned long long* maxslots, double& dt, Ctrl* keep = nullptr) {
     uint32_t halt_status = 0;
     const bool halted = cur->halted != 0;
     if (!halted) {
@@ -1502,7 +1503,10 @@ __device__ __forceinline__ bool list_dt(const StepParams& P, Ctrl* next, const C
             clear_slots(maxslots + (par ^ 1) * kDtSet + kSlotSet);
         }
     }
-    if (blockIdx.x == 0) publish_ctrl(cur, next, dt, halt_status);
+    if (blockIdx.x == 0) {
+        publish_ctrl(cur, next, dt, halt_status);
+        if (keep) publish_ctrl(cur, keep, dt, halt_status);
+    }
     return !halted && halt_status == 0;
 }
 
@@ -1513,7 +1517,8 @@ __device__ __forceinline__ bool step_needs_oid(const StepParams& P, const Ctrl& 
     return c.wall_disappear || (P.boundary_motion && c.piston_active && itype < 0);
 }
 
-// whole_step of every slot from X into A (in place on list steps), the cell
+// whole_step of every slot from X into A (in place on list steps, but for a
+// tape's, which go from one kept state to the next), the cell
 // key for the next build, the step's largest displacement, and the records
 // of the next step's pair pass: near (the new position relative to the home
 // cell, the new velocity) and pred (PredictHalfStep.cpp:16-22 with this
@@ -1529,7 +1534,7 @@ __global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ct
                                                                 const uint32_t* __restrict__ home, StateA<R> A,
                                                                 uint32_t* __restrict__ key_next,
                                                                 unsigned long long* maxslots,
-                                                                unsigned long long* dslots) {
+                                                                unsigned long long* dslots, Ctrl* keep) {
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
     const uint32_t s = live ? s0 : P.n - 1;
@@ -1542,7 +1547,7 @@ __global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ct
     if (P.density_treatment == 0) pr.z = fabs(rec[s].pr.z);  // the summed density (sign-encoded)
     const Ctrl& c = *cur;
     double dt;
-    if (!list_dt(P, next, cur, maxslots, dt)) return;
+    if (!list_dt(P, next, cur, maxslots, dt, keep)) return;
     uint32_t outside = 0, bad = 0;
     double moved2 = 0.0;
     if (live) {

@@ -681,7 +681,7 @@ __global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, C
                                                                  const uint32_t* __restrict__ home, StateA3<R> A,
                                                                  uint32_t* __restrict__ key_next,
                                                                  unsigned long long* maxslots,
-                                                                 unsigned long long* dslots) {
+                                                                 unsigned long long* dslots, Ctrl* keep) {
     const uint32_t s0 = blockIdx.x * kBlock + threadIdx.x;
     const bool live = s0 < P.n;
     const uint32_t s = live ? s0 : P.n - 1;
@@ -694,7 +694,7 @@ __global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, C
     if (P.density_treatment == 0) pr.w = fabs(rec[s].pr.w);  // the summed density
     const Ctrl& c = *cur;
     double dt;
-    if (!list_dt(P, next, cur, maxslots, dt)) return;
+    if (!list_dt(P, next, cur, maxslots, dt, keep)) return;
     uint32_t outside = 0, bad = 0;
     double moved2 = 0.0;
     if (live) {

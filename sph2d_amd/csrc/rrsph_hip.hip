@@ -270,6 +270,13 @@ struct rrsph_ctx {
     uint64_t list_interval = 8;         // steps between builds
     uint64_t list_chunk = kFirstChunk;  // steps between looks at the control block
     uint64_t n_list = 0, n_build = 0, n_list_halts = 0;
+    // where list and build steps leave the state (pos null: in place)
+    struct Out {
+        double2* pos = nullptr;
+        void *va = nullptr, *ad = nullptr, *pres = nullptr;
+        uint32_t* oid = nullptr;
+        Ctrl* keep = nullptr;           // the control block after the step, for the tape
+    } out;
     AdjTape adj;
 };
 
@@ -293,6 +300,11 @@ template <class R> StateA<R> stateA(rrsph_ctx* c) {
 template <class R> StateB<R> stateB(rrsph_ctx* c, void* pred, void* pres) {
     return StateB<R>{c->posB, (real4<R>*)c->vaB, (real4<R>*)pred, c->oidB, (R*)pres, nullptr};
 }
+// the state a list or build step leaves
+template <class R> StateA<R> stateOut(rrsph_ctx* c) {
+    return c->out.pos ? StateA<R>{c->out.pos, (real4<R>*)c->out.va, (real4<R>*)c->out.ad, c->out.oid} : stateA<R>(c);
+}
+void* pres_out(const rrsph_ctx* c) { return c->out.pos ? c->out.pres : c->pres; }
 // the step's B copy; keeps A.ad too when the fused pass may have to be undone
 template <class R> StateB<R> stepB(rrsph_ctx* c) {
     return StateB<R>{c->posB, (real4<R>*)c->vaB, (real4<R>*)c->pred, c->oidB, (R*)c->pres, (real4<R>*)c->adB};
@@ -300,6 +312,10 @@ template <class R> StateB<R> stepB(rrsph_ctx* c) {
 // 3D: the position buffers hold double4 (two double2 slots per particle)
 template <class R> StateA3<R> stateA3(rrsph_ctx* c) {
     return StateA3<R>{(double4*)c->posA, (real4<R>*)c->vaA, (real4<R>*)c->adA, c->oidA};
+}
+template <class R> StateA3<R> stateOut3(rrsph_ctx* c) {
+    const StateA<R> o = stateOut<R>(c);
+    return StateA3<R>{(double4*)o.pos, o.va, o.ad, o.oid};
 }
 template <class R> StateB3<R> stateB3(rrsph_ctx* c, void* pred, void* pw, void* pres) {
     return StateB3<R>{(double4*)c->posB, (real4<R>*)c->vaB, (real4<R>*)pred, (R*)pw, (R*)pres, c->oidB, nullptr};
@@ -544,7 +560,7 @@ void enqueue_list_passes(rrsph_ctx* c, Launcher& L, ListState<R> X, ListStep kin
     if (P.density_treatment == 0) {
         auto density = [&](auto kernel) {
             L(K_DENSITY_SUM, [&] {
-                kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc, c->dslots);
+                kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)pres_out(c), c->nbl, c->nbc, c->dslots);
             });
         };
         if (first) density(density_sum_list<R, true, LPP>);
@@ -556,14 +572,14 @@ void enqueue_list_passes(rrsph_ctx* c, Launcher& L, ListState<R> X, ListStep kin
     }
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
-            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                 (real4<R>*)c->adA, (real2<R>*)c->xs, c->dtslots, c->dslots, O);
+            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)pres_out(c), c->nbl, c->nbc,
+                                                 stateOut<R>(c).ad, (real2<R>*)c->xs, c->dtslots, c->dslots, O);
         });
     };
     auto general = [&](auto kernel) {
         L(K_PAIR, [&] {
-            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                 (real4<R>*)c->adA, (real2<R>*)c->xs, c->dtslots, c->dslots);
+            kernel<<<nb, kBlock, 0, c->stream>>>(P, next, cur, X, rec, (R*)pres_out(c), c->nbl, c->nbc,
+                                                 stateOut<R>(c).ad, (real2<R>*)c->xs, c->dtslots, c->dslots);
         });
     };
     if constexpr (ALL) {
@@ -598,7 +614,7 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, ListSt
         });
         enqueue_build_sort(c, c->ctrl_cur, L);
         StateA<R> A = stateA<R>(c);
-        StateB<R> B = stateB<R>(c, c->pred, c->pres);
+        StateB<R> B = stateB<R>(c, c->pred, pres_out(c));
         L(K_REORDER, [&] {
             auto reorder = [&](auto kernel) {
                 kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B, rec, c->home,
@@ -620,8 +636,8 @@ template <class R> void enqueue_list_step_t(rrsph_ctx* c, Profiler* prof, ListSt
     else enqueue_list_passes<R, 1, true>(c, L, X, kind);
     if (kind == kFusedFirst || kind == kFusedSecond) return;
     L(K_INTEGRATE, [&] {
-        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real2<R>*)c->xs, rec, c->home, stateA<R>(c),
-                                                               c->key_next, c->dtslots, c->dslots);
+        integrate_list_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, (const real2<R>*)c->xs, rec, c->home, stateOut<R>(c),
+                                                               c->key_next, c->dtslots, c->dslots, c->out.keep);
     });
 }
 
@@ -651,7 +667,7 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListS
         });
         enqueue_build_sort(c, c->ctrl_cur, L);
         StateA3<R> A = stateA3<R>(c);
-        StateB3<R> B = stateB3<R>(c, c->pred, c->pw, c->pres);
+        StateB3<R> B = stateB3<R>(c, c->pred, c->pw, pres_out(c));
         L(K_REORDER, [&] {
             auto reorder = [&](auto kernel) {
                 kernel<<<nb, kBlock, 0, c->stream>>>(P, c->ctrl_cur, c->sorted_keys, c->sorted_perm, A, B, rec, dens,
@@ -670,7 +686,7 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListS
     if (P.density_treatment == 0) {
         auto density = [&](auto kernel) {
             L(K_DENSITY_SUM, [&] {
-                kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, dens, rec, (R*)c->pres, c->nbl,
+                kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, dens, rec, (R*)pres_out(c), c->nbl,
                                                          c->nbc, c->dslots);
             });
         };
@@ -680,8 +696,8 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListS
     }
     auto pair = [&](auto kernel) {
         L(K_PAIR, [&] {
-            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)c->pres, c->nbl, c->nbc,
-                                                     (real4<R>*)c->adA, (real4<R>*)c->xs, c->dtslots, c->dslots, O);
+            kernel<<<nb_xcd, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X, rec, (R*)pres_out(c), c->nbl, c->nbc,
+                                                     stateOut<R>(c).ad, (real4<R>*)c->xs, c->dtslots, c->dslots, O);
         });
     };
     auto choose = [&](auto summed, auto first_kernel, auto kernel) {
@@ -702,7 +718,8 @@ template <class R> void enqueue_list_step3_t(rrsph_ctx* c, Profiler* prof, ListS
     L(K_INTEGRATE, [&] {
         integrate_list3_kernel<R><<<nb, kBlock, 0, c->stream>>>(P, c->ctrl, c->ctrl_cur, X,
                                                                 (const real4<R>*)c->xs, rec, dens, c->home,
-                                                                stateA3<R>(c), c->key_next, c->dtslots, c->dslots);
+                                                                stateOut3<R>(c), c->key_next, c->dtslots, c->dslots,
+                                                                c->out.keep);
     });
 }
 
@@ -2130,25 +2147,33 @@ static size_t real4_bytes(const rrsph_ctx* ctx) { return ctx->fp32 ? 16 : 32; }
 // bytes of one saved state: pos | va | ad | oid | pressure | control block
 // (the pressure of the step that produced the state, in its slot order: the
 // reference's p array, which download() returns)
-// (the control block on a 16-byte boundary: tape_records_kernel reads it in place)
-static size_t state_ctrl_offset(const rrsph_ctx* ctx) {
-    return ((pos_bytes(ctx) + 2 * real4_bytes(ctx) + 4 + real4_bytes(ctx) / 4) * ctx->P.n + 15) / 16 * 16;
-}
-static size_t state_bytes(const rrsph_ctx* ctx) { return state_ctrl_offset(ctx) + sizeof(Ctrl); }
+// Each array on a 32-byte boundary: steps read and write saved states in place.
+constexpr int kStateArrays = 6;
+struct StateLayout {
+    size_t off[kStateArrays + 1], bytes[kStateArrays];
+    explicit StateLayout(const rrsph_ctx* ctx) {
+        const size_t n = ctx->P.n, pb = pos_bytes(ctx), vb = real4_bytes(ctx);
+        const size_t b[kStateArrays] = {pb * n, vb * n, vb * n, 4 * n, vb / 4 * n, sizeof(Ctrl)};
+        off[0] = 0;
+        for (int k = 0; k < kStateArrays; ++k) {
+            bytes[k] = b[k];
+            off[k + 1] = (off[k] + b[k] + 31) / 32 * 32;
+        }
+    }
+};
+static size_t state_ctrl_offset(const rrsph_ctx* ctx) { return StateLayout(ctx).off[kStateArrays - 1]; }
+static size_t state_bytes(const rrsph_ctx* ctx) { return StateLayout(ctx).off[kStateArrays]; }
 
 // the blob of one saved state: posA | vaA | adA | oidA | pres | ctrl
-static CopyPlan state_plan(rrsph_ctx* ctx, void* blob, bool save) {
-    const size_t n = ctx->P.n, pb = pos_bytes(ctx), vb = real4_bytes(ctx);
+// (without the control block if !ctrl)
+static CopyPlan state_plan(rrsph_ctx* ctx, void* blob, bool save, bool ctrl = true) {
+    const StateLayout S(ctx);
     char* d = (char*)blob;
-    void* arrays[6] = {ctx->posA, ctx->vaA, ctx->adA, ctx->oidA, ctx->pres, ctx->ctrl};
-    const size_t bytes[6] = {pb * n, vb * n, vb * n, 4 * n, vb / 4 * n, sizeof(Ctrl)};
+    void* arrays[kStateArrays] = {ctx->posA, ctx->vaA, ctx->adA, ctx->oidA, ctx->pres, ctx->ctrl};
     CopyPlan plan;
-    size_t off = 0;
-    for (int k = 0; k < 6; ++k) {
-        if (k == 5) off = state_ctrl_offset(ctx);
-        if (save) plan.add(arrays[k], d + off, bytes[k]);
-        else plan.add(d + off, arrays[k], bytes[k]);
-        off += bytes[k];
+    for (int k = 0; k < kStateArrays - (ctrl ? 0 : 1); ++k) {
+        if (save) plan.add(arrays[k], d + S.off[k], S.bytes[k]);
+        else plan.add(d + S.off[k], arrays[k], S.bytes[k]);
     }
     return plan;
 }
@@ -2157,9 +2182,9 @@ static rrsph_status save_state(rrsph_ctx* ctx, void* dst) { return enqueue_copie
 
 // The arrays of the state saved in blob, in place (layout of state_plan).
 static StateView state_view(const rrsph_ctx* ctx, void* blob) {
-    const size_t n = ctx->P.n, pb = pos_bytes(ctx), vb = real4_bytes(ctx);
+    const StateLayout S(ctx);
     char* d = (char*)blob;
-    return StateView{d, d + pb * n, d + (pb + vb) * n, (uint32_t*)(d + (pb + 2 * vb) * n)};
+    return StateView{d, d + S.off[1], d + S.off[2], (uint32_t*)(d + S.off[3])};
 }
 
 static rrsph_status restore_state(rrsph_ctx* ctx, const void* src, bool keys = true) {
@@ -2283,6 +2308,44 @@ static rrsph_status tape_build_lists(rrsph_ctx* ctx) {
     return RRSPH_OK;
 }
 
+// While a batched tape launches steps: a step reads the kept state before it
+// and leaves the kept state after it, the first from and the last to the
+// context's arrays (saving a copy after every step took 6.1 us and a launch
+// gap of the 100 of a step of 134,042 particles, 21 at 943,906 in 3D).
+struct TapeStates {
+    rrsph_ctx* c;
+    double2* pos;
+    void *va, *ad, *pres;
+    uint32_t* oid;
+    explicit TapeStates(rrsph_ctx* ctx)
+        : c(ctx), pos(ctx->posA), va(ctx->vaA), ad(ctx->adA), pres(ctx->pres), oid(ctx->oidA) {}
+    ~TapeStates() { context_arrays(); }
+    void context_arrays() {
+        c->posA = pos;
+        c->vaA = va;
+        c->adA = ad;
+        c->pres = pres;
+        c->oidA = oid;
+        c->out = rrsph_ctx::Out{};
+    }
+    // in, out: saved states, or null for the context's arrays
+    void step(char* in, char* out) {
+        const StateLayout S(c);
+        context_arrays();
+        if (out)
+            c->out = rrsph_ctx::Out{(double2*)out, out + S.off[1], out + S.off[2], out + S.off[4],
+                                    (uint32_t*)(out + S.off[3]), (Ctrl*)(out + S.off[5])};
+        else if (in)
+            c->out = rrsph_ctx::Out{pos, va, ad, pres, oid, nullptr};
+        if (!in) return;
+        c->posA = (double2*)in;
+        c->vaA = in + S.off[1];
+        c->adA = in + S.off[2];
+        c->oidA = (uint32_t*)(in + S.off[3]);
+        c->pres = in + S.off[4];
+    }
+};
+
 constexpr uint32_t kHaltCheck = 64;  // tape steps between two looks at the control block
 
 // Launch steps [k0, k1) of the tape, reading the control block back every
@@ -2295,6 +2358,7 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
     AdjTape& T = ctx->adj;
     const TapeSkin skin(ctx);
     const TapeBuildLists own(ctx);
+    TapeStates states(ctx);
     const size_t n = ctx->P.n;
     // the forward keeps the states of the last segment (of every step with
     // keep_all): the reverse pass starts there and needs no replay of it
@@ -2305,6 +2369,20 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
     // ranges fit one; the next step's sort overwrites them only after that
     if (forward && T.keep_all && T.lists)  // the builds before k0 (those launched after a halt left no lists)
         T.nseg_lists = k0 > 0 ? (uint32_t)(T.seg_build[k0 - 1] + 1) : 0u;
+    const bool chained = forward && T.batched();
+    // a halt leaves the state before the halted step in the context's arrays
+    auto finish = [&](rrsph_status st) -> rrsph_status {
+        states.context_arrays();
+        if (chained && ctx->host_ctrl->halted) {
+            const uint64_t at = committed_steps(*ctx->host_ctrl) - base;
+            if (at > k0 && at < k1) {
+                const rrsph_status s2 =
+                    enqueue_copies(ctx, state_plan(ctx, (char*)seg_base + (size_t)at * T.blob, false, false));
+                if (s2 != RRSPH_OK) return s2;
+            }
+        }
+        return st;
+    };
     CopyPlan pending;
     auto flush = [&]() -> rrsph_status {
         if (pending.n == 0) return RRSPH_OK;
@@ -2330,8 +2408,11 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
             if (st != RRSPH_OK) return st;
             HIP_TRY(hipMemcpyAsync(ctx->host_ctrl, ctx->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, ctx->stream));
             HIP_TRY(hipStreamSynchronize(ctx->stream));
-            if (ctx->host_ctrl->halted) return sync_status(ctx);
+            if (ctx->host_ctrl->halted) return finish(sync_status(ctx));
         }
+        if (chained)  // (a batched tape keeps state k in slot k)
+            states.step(k > k0 ? (char*)seg_base + (size_t)k * T.blob : nullptr,
+                        k + 1 < k1 ? (char*)seg_base + (size_t)(k + 1) * T.blob : nullptr);
         if (forward && k % T.every == 0) {
             if (T.lists && k > 0) {  // the build interval from the displacements so far
                 HIP_TRY(hipMemcpyAsync(ctx->host_ctrl, ctx->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, ctx->stream));
@@ -2343,12 +2424,11 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
         }
         const bool keep = forward ? k >= last0 : true;  // seg holds this step's state
         const size_t slot = forward ? k - last0 : k - kslot;
-        // a batched tape's records come from the kept control blocks, so a range
-        // that resumes at a halted step keeps the state saved before the halt
-        // (the halted step left the state as it was, but not the control block)
-        const bool kept = forward && T.batched() && k == k0 && k0 > 0;
+        // a batched tape's steps leave their states where they are kept, and a
+        // range that resumes at a halted step has the state before it there
         if (keep) {
-            if (!kept) st = save((char*)seg_base + slot * T.blob);
+            if (!chained || k == 0) st = save((char*)seg_base + slot * T.blob);
+            else st = flush();
             if (st != RRSPH_OK) return st;
             if (!forward && k + 1 == k1) {  // the state before the segment's last step is all the adjoint needs
                 // that step is not launched: a list step reads the lists of the segment's last build; a
@@ -2395,7 +2475,7 @@ static rrsph_status adjoint_run(rrsph_ctx* ctx, uint32_t k0, uint32_t k1, bool f
         }
     }
     if (const rrsph_status st = flush(); st != RRSPH_OK) return st;
-    return sync_status(ctx);
+    return finish(sync_status(ctx));
 }
 
 // adjoint_run with its halts handled: a step that changed more cells than
