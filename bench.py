@@ -525,12 +525,13 @@ def main():
 
     # dominant kernel of the FP32 step
     pk = r32["per_kernel_ms"]
-    # time per step of each kernel class: the prologue, the sort (three
-    # launches of each radix kernel), reorder and list build run on build
-    # steps only when the step uses neighbour lists
+    # time per step of each kernel class: the prologue, the sort (with lists
+    # the counting sort: one launch of each class; else three of each radix
+    # kernel), reorder and list build run on build steps only when the step
+    # uses neighbour lists
     ls = r32["list_stats"]
     build_frac = ls["builds"] / max(ls["builds"] + ls["list_steps"], 1) if ls["interval"] else 1.0
-    per_step = {k: pk[k] * (3 if "radix" in k else 1) * (build_frac if ("radix" in k or k in (
+    per_step = {k: pk[k] * (3 if "radix" in k and not ls["interval"] else 1) * (build_frac if ("radix" in k or k in (
         "step_prologue", "reorder_kernel", "list_build_kernel")) else 1.0) for k in pk if pk[k] > 0}
     dom = max(per_step, key=per_step.get)
     pair_ms = pk["pair_kernel"]

@@ -9,8 +9,9 @@ through the hand-written adjoint of the RRSPH_HIP step.
 of steps, the checkpoint interval and the gauge definition.  The forward
 re-uploads the initial state, sets the Fourier piston
 x(t) = sum_k a_k sin(k w t) + b_k cos(k w t) and runs the steps keeping a
-checkpoint every `every` steps; the backward replays each segment from its
-checkpoint and runs the step adjoints in reverse (rrsph_hip_adjoint_*).
+checkpoint every `every` steps, and every state where they fit the device;
+the backward runs the step adjoints in reverse (rrsph_hip_adjoint_*), and
+replays a segment from its checkpoint where its states were not kept.
 Tensors live on the host: the coefficients and gauge histories are small,
 the particle state never leaves the GPU.
 """

@@ -36,8 +36,8 @@
 // Step kernels: [density_sum_list] -> pair_list -> integrate_list (in place;
 // it also writes the next step's records, so no reorder runs between builds;
 // with a constant dt and no wave maker the pair pass integrates: fused_step_begin),
-// the first of them with the step's prologue (list_step_begin).  A build step runs list_prologue -> radix
-// sort -> reorder_list_kernel -> list_build_kernel -> the same step kernels
+// the first of them with the step's prologue (list_step_begin).  A build step runs list_prologue -> counting
+// sort (cell_sort.hpp) -> reorder_list_kernel -> list_build_kernel -> the same step kernels
 // on the reordered copy, integrating into A.
 #pragma once
 

@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -124,8 +125,8 @@ struct AdjTape {
     bool seg_last = false;               // seg holds the last segment's states (kept by the forward)
     // seg holds the state before every step of the run (and the sorts):
     // the forward keeps them all when they fit in half the free device
-    // memory (with list steps: together with the lists of a build in every
-    // step, so that the lists cannot run out), and the reverse pass replays
+    // memory (with list steps: together with their lists, see tape_fits), and
+    // the reverse pass replays
     // nothing (943,906-particle basin, 12 steps in two segments: 23.6 -> 20.2 ms)
     bool keep_all = false;
     // the cell sort each step of seg ran with (keys, permutation): the reverse
@@ -139,15 +140,17 @@ struct AdjTape {
     double *eta = nullptr, *zs = nullptr, *ws = nullptr;  // nsteps x kMaxGauges
     double *eta_bar = nullptr, *partials = nullptr, *piston_sum = nullptr;
     double *lam[2] = {nullptr, nullptr}, *direct = nullptr, *drho_adj = nullptr;
-    double4* out_adj = nullptr;          // 2D: out_a (n); 3D: the AdjRec3 records (n)
+    double4* out_adj = nullptr;          // 2D: out_a (n), or with lists the AdjRec2 records; 3D: the AdjRec3 records
     uint32_t* flag = nullptr;
-    // 3D with neighbour lists: the tape runs list steps.  The forward builds
+    // With neighbour lists the tape runs list steps.  The forward builds
     // at every checkpoint step and records which steps built; a replay
     // repeats that schedule, so it repeats its steps exactly.  The segment
-    // in hand keeps the lists (and sorted cell keys) of each of its builds;
-    // the reverse step of a list step reads its state in the slot order of
-    // its build (identity reorder) and that build's lists.
+    // in hand (with keep_all the run) keeps the lists (and sorted cell keys)
+    // of each of its builds; the reverse step of a list step reads its state
+    // in the slot order of its build and that build's lists.
     bool lists = false;
+    bool may_list = false;               // tape_lists when the buffers were allocated
+    bool no_room = false;                // a kept tape could not allocate a build's lists
     std::vector<uint8_t> builds;         // per step: the step built lists
     struct Lists {
         uint32_t *nbl = nullptr, *nbc = nullptr, *keys = nullptr;
@@ -251,7 +254,9 @@ struct rrsph_ctx {
     bool list_mode = false;
     bool all_terms = false;             // artificial viscosity, XSPH and the wall force are all on
     int lanes = 1;                      // lanes per particle of the 2D list passes
-    bool list_suspended = false;        // the adjoint's tapes and replays run without lists
+    bool list_suspended = false;        // 2D tapes without lists, and their replays
+    bool tape_keep = true;              // false: a kept tape ran out of room for its lists
+    size_t tape_lists_max = ~(size_t)0; // the most builds whose lists a kept tape allocates (RRSPH_HIP_TAPE_LISTS)
     uint32_t *nbl = nullptr, *nbc = nullptr;
     void* rec = nullptr;                // records of the list pass (ListRec per slot)
     void* dens = nullptr;               // 3D: records of the summation density pass (real4 per slot)
@@ -1370,6 +1375,7 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
         // the counting sort's scan passes over every cell of the grid: 12 bytes a
         // cell, so that 4 cells a particle take what one radix pass does (24 bytes
         // a particle read twice and written once); sparser grids keep the radix sort
+        if (const char* e2 = std::getenv("RRSPH_HIP_TAPE_LISTS")) ctx->tape_lists_max = std::strtoull(e2, nullptr, 10);
         const char* sort = std::getenv("RRSPH_HIP_BUILD_SORT");
         if ((uint64_t)ctx->P.ncells <= 4ull * n && !(sort && std::strcmp(sort, "radix") == 0)) {
             const size_t blocks = scan_blocks(ctx->P.ncells);
@@ -2289,7 +2295,7 @@ static rrsph_status tape_build_lists(rrsph_ctx* ctx) {
     const size_t n = ctx->P.n, rows = ctx->P.list_cap + kListPad;
     if (T.nseg_lists == T.seg_lists.size()) {
         AdjTape::Lists L;
-        hipError_t e = hipSuccess;
+        hipError_t e = T.keep_all && T.nseg_lists >= ctx->tape_lists_max ? hipErrorOutOfMemory : hipSuccess;
         L.nbl = dalloc<uint32_t>(rows * n, e);
         L.nbc = dalloc<uint32_t>(n, e);
         L.keys = dalloc<uint32_t>(n, e);
@@ -2298,6 +2304,8 @@ static rrsph_status tape_build_lists(rrsph_ctx* ctx) {
             void* got[] = {L.nbl, L.nbc, L.keys};
             for (void* p : got)
                 if (p) (void)hipFree(p);
+            (void)hipGetLastError();
+            T.no_room = T.keep_all;
             return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc (adjoint lists): ") + hipGetErrorString(e));
         }
         T.seg_lists.push_back(L);
@@ -2615,13 +2623,9 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
 rrsph_status rrsph_hip_adjoint_forward(rrsph_ctx* ctx, uint32_t nsteps, uint32_t checkpoint_every,
                                        const rrsph_gauge_spec* spec, double* eta) {
     if (!ctx) return RRSPH_ERR_INVALID_ARGUMENT;
-    if (ctx->P.dim == 3 || tape_lists(ctx)) {
-        rrsph_status st = adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
-        ctx->need_full = true;
-        return st;
-    }
-    ListSuspend guard(ctx);
-    return adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
+    const rrsph_status st = adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
+    if (ctx->P.dim == 3 || list_active(ctx)) ctx->need_full = true;  // the next step builds lists of its own
+    return st;
 }
 
 rrsph_status rrsph_hip_adjoint_backward(rrsph_ctx* ctx, const double* eta_bar, double* grad_a, double* grad_b,
@@ -2662,6 +2666,22 @@ static rrsph_status tape_records_and_gauges(rrsph_ctx* ctx) {
     return RRSPH_OK;
 }
 
+// Whether every state and sort of the tape, and with list steps the lists
+// of a build in every fourth step and every checkpoint, fit in half the free
+// memory.  (A kept tape that builds more often and finds no room for a
+// build's lists starts over: in 3D with one segment's states, in 2D on sorted
+// steps if all their states fit.)
+static bool tape_fits(const rrsph_ctx* ctx, bool lists) {
+    const AdjTape& T = ctx->adj;
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
+    const double n = ctx->P.n, steps = T.nsteps;
+    const double builds = lists ? steps / 4 + (double)((T.nsteps + T.every - 1) / T.every) + 1 : 0.0;
+    const double all_b = steps * ((double)state_bytes(ctx) + 256 + 8 * n) +
+                         builds * 4 * n * (double)(ctx->P.list_cap + kListPad + 2);
+    return all_b <= 0.5 * (double)free_b;
+}
+
 // The buffers of a tape of T.nsteps steps with a checkpoint every T.every.
 static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     AdjTape& T = ctx->adj;
@@ -2674,14 +2694,8 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     hipError_t e = hipSuccess;
     T.ck.assign(nck + 1, nullptr);
     for (auto& p : T.ck) p = dalloc<char>(T.blob, e);
-    {
-        // every step's state and sort when they fit in half the free memory
-        // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's, and replays)
-        size_t free_b = 0, total_b = 0;
-        const size_t lists_b = T.lists ? (size_t)(ctx->P.list_cap + kListPad + 2) * n * sizeof(uint32_t) : 0;
-        const double all_b = (double)nsteps * (double)(T.blob + 2 * n * sizeof(uint32_t) + lists_b);
-        T.keep_all = !T.segments && hipMemGetInfo(&free_b, &total_b) == hipSuccess && all_b <= 0.5 * (double)free_b;
-    }
+    // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's states, and replays)
+    T.keep_all = !T.segments && (ctx->tape_keep || !T.lists) && tape_fits(ctx, T.lists);
     uint32_t cap = T.keep_all ? nsteps : T.every;  // states seg holds
     const bool alloc_ok = e == hipSuccess;
     T.seg = dalloc<char>(T.blob * cap, e);
@@ -2751,21 +2765,26 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
     // loop allocates once (the 943,906-particle basin, 12 steps: 32.4 -> 24.3 ms; the tank, 60 steps: 13.0 -> 10.0); another shape frees them first
     const char* store = std::getenv("RRSPH_HIP_ADJ_STORE");
     const bool segments = store && std::strcmp(store, "segments") == 0;
-    const bool lists = tape_lists(ctx);
+    const bool may_list = tape_lists(ctx);
     AdjTape& T = ctx->adj;
     T.valid = false;
-    if (T.allocated && T.nsteps == nsteps && T.every == std::min(checkpoint_every, nsteps) && T.lists == lists &&
+    if (T.allocated && T.nsteps == nsteps && T.every == std::min(checkpoint_every, nsteps) && T.may_list == may_list &&
         T.segments == segments) {
         drop_tape_graph(T);  // captured with the last run's gauges and piston
     } else {
         free_tape(T);
         T.nsteps = nsteps;
         T.every = std::min(checkpoint_every, nsteps);
-        T.lists = lists;
         T.segments = segments;
+        T.may_list = may_list;
+        // in 2D sorted steps whose states can all be kept beat list steps that replay
+        T.lists = may_list && (ctx->P.dim == 3 || segments || (ctx->tape_keep && tape_fits(ctx, true)) ||
+                               !tape_fits(ctx, false));
         st = alloc_tape(ctx);
         if (st != RRSPH_OK) return st;
     }
+    std::optional<ListSuspend> guard;
+    if (ctx->P.dim == 2 && !T.lists) guard.emplace(ctx);
     const size_t n = ctx->P.n;
     const uint32_t nck = (uint32_t)T.ck.size() - 1;
     T.spec = G;
@@ -2775,14 +2794,20 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
     std::fill(T.seg_build.begin(), T.seg_build.end(), -1);
     T.nseg_lists = 0;
     T.force_build = ~0ull;
+    const uint64_t interval = ctx->list_interval;
     st = adjoint_run_checked(ctx, 0, nsteps, true, T.seg);
-    if (st != RRSPH_OK && T.lists && ctx->P.dim == 2 && ctx->host_ctrl->halted &&
-        ctx->host_ctrl->status == kStatusListOverflow) {
+    const bool overflowed = T.lists && ctx->P.dim == 2 && ctx->host_ctrl->halted &&
+                            ctx->host_ctrl->status == kStatusListOverflow;
+    if (st != RRSPH_OK && (overflowed || T.no_room)) {
         // a list ran out of room: the run starts over on sorted steps, which
-        // the context keeps to from here (as resume_halt has it)
+        // the context keeps to from here (as resume_halt has it); no memory for
+        // a build's lists: see tape_fits
         st = restore_state_sync(ctx, T.ck[0]);
         if (st != RRSPH_OK) return st;
-        ctx->list_mode = false;
+        if (overflowed) ctx->list_mode = false;
+        else ctx->tape_keep = false;
+        ctx->list_interval = interval;  // (the schedule of a run that had not been tried)
+        free_tape(T);
         ctx->err.clear();
         return adjoint_forward_impl(ctx, nsteps, checkpoint_every, spec, eta);
     }

@@ -68,6 +68,24 @@ def test_kept_list_tapes_equal_their_replays(monkeypatch, dim, precision, skin):
         assert np.max(np.abs(g1[f] - g0[f])) <= tol * np.max(np.abs(g0[f]))
 
 
+@pytest.mark.parametrize("dim", [2, 3])
+def test_a_kept_tape_without_memory_for_lists_starts_over(monkeypatch, dim):
+    """In 2D on sorted steps, whose states all fit, in 3D with one segment's states: the results of such runs."""
+    res = {}
+    other = ("RRSPH_HIP_LIST", "0") if dim == 2 else ("RRSPH_HIP_ADJ_STORE", "segments")
+    for name, var, value in (("short", "RRSPH_HIP_TAPE_LISTS", "2"), ("other", *other)):
+        with monkeypatch.context() as m:
+            m.setenv(var, value)
+            run, prm = _run(dim, H.FP64)
+            res[name] = _gradients(run, prm)
+            run.sim.close()
+    for k in (0, 1, 2):
+        a, b = res["short"][k], res["other"][k]
+        for f in ("r", "v", "rho") if k else (None,):
+            x, y = (a, b) if f is None else (a[f], b[f])
+            assert np.array_equal(x, y), (k, f)
+
+
 def _smooth_viscosity(lay):  # without the switch between approaching and parting pairs, as a kink
     lay.params.artificial_shear_visc, lay.params.artificial_bulk_visc = 0.0, 0.5
     lay.state["itype"][7:4000:531] = 0  # and a few particles that no longer exist
