@@ -109,19 +109,12 @@ __global__ void __launch_bounds__(kBlock) smooth_gauge_partials3(uint32_t n, con
     gauge_block_store(G.g, L, partials);
 }
 
-// lam[oid].r += sum_g eta_bar[g] d eta_g / d r (state in sorted order).
-__global__ void __launch_bounds__(kBlock) smooth_gauge_grad3(uint32_t n, const double4* __restrict__ pos,
-                                                             const uint32_t* __restrict__ oid, GaugeSpec3 G,
-                                                             const double* __restrict__ eta_bar,
-                                                             const double* __restrict__ zsum,
-                                                             const double* __restrict__ wsum,
-                                                             double* __restrict__ lam) {
-    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const double4 p = pos[s];
-    if ((int)p.w != G.g.ptype) return;
+// (gx, gy, gz) = sum_g eta_bar[g] d eta_g / d r at p; false outside every window.
+__device__ __forceinline__ bool gauge_gradient3(const GaugeSpec3& G, const double4& p,
+                                                const double* __restrict__ eta_bar, const double* __restrict__ zsum,
+                                                const double* __restrict__ wsum, double& gx, double& gy, double& gz) {
     const double inv_r2 = 1.0 / (G.g.radius * G.g.radius);
-    double gx = 0, gy = 0, gz = 0;
+    gx = gy = gz = 0;
     bool seen = false;  // inside a window: only those particles update lam
     for (uint32_t g = 0; g < G.g.n; ++g) {
         double dx, dz;
@@ -137,7 +130,22 @@ __global__ void __launch_bounds__(kBlock) smooth_gauge_grad3(uint32_t n, const d
         gx += c * dx;
         gz += c * dz;
     }
-    if (!seen) return;
+    return seen;
+}
+
+// lam[oid].r += sum_g eta_bar[g] d eta_g / d r (state in sorted order).
+__global__ void __launch_bounds__(kBlock) smooth_gauge_grad3(uint32_t n, const double4* __restrict__ pos,
+                                                             const uint32_t* __restrict__ oid, GaugeSpec3 G,
+                                                             const double* __restrict__ eta_bar,
+                                                             const double* __restrict__ zsum,
+                                                             const double* __restrict__ wsum,
+                                                             double* __restrict__ lam) {
+    const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
+    if (s >= n) return;
+    const double4 p = pos[s];
+    if ((int)p.w != G.g.ptype) return;
+    double gx, gy, gz;
+    if (!gauge_gradient3(G, p, eta_bar, zsum, wsum, gx, gy, gz)) return;
     double* l = lam + kLam3 * (size_t)oid[s];
     l[0] += gx;
     l[1] += gy;
@@ -157,8 +165,13 @@ __global__ void __launch_bounds__(kBlock) state_keys3_kernel(StepParams P, const
 // whole_step reverse (WholeStep.cpp:19-61 with the boundary motion of
 // cl/TimeIntegration.cl:190-245).  piston_sum[g] += adjoint of paddle g's
 // velocity (one entry per paddle of this step).
-template <class R>
+// PREDICT: B's positions, velocities and indices are a kept state in the
+// step's slot order and ad its last accelerations; the prediction, pressure
+// and p / rho^2 that reorder3_kernel gives are made here (943,906 particles
+// FP32: a reorder of 27 us and 64 before, 67 now).
+template <class R, bool PREDICT>
 __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, StateB3<R> B,
+                                                    const real4<R>* __restrict__ ad,
                                                     const double* __restrict__ lam_in, AdjRec3<R>* __restrict__ rec,
                                                     double* __restrict__ direct, double* __restrict__ piston_sum,
                                                     const uint32_t* __restrict__ home, float4* __restrict__ nearf) {
@@ -205,10 +218,21 @@ __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, Sta
         if (t == 0) oa.x = oa.y = oa.z = 0.0;  // no neighbours, no acceleration dependence
         oa.w = P.density_treatment != 0 ? rb * vdt + db : 0.0;
         AdjRec3<R> r;
+        const real4<R> va = B.va[s];
+        real4<R> pr;
+        R pw;
+        if constexpr (PREDICT) {
+            R p;
+            pr = predict3<R>(P, va, 1, ad[s], (R)T.dt_pred, pw, p);
+            B.pred[s] = pr;
+            B.pres[s] = p;
+        } else {
+            pr = B.pred[s];
+            pw = B.pw[s];
+        }
         if constexpr (sizeof(R) == 4) {
-            const real4<R> va = B.va[s];
-            r.vp = make_float4(va.x, va.y, va.z, B.pw[s]);
-            r.u = B.pred[s];
+            r.vp = make_float4(va.x, va.y, va.z, pw);
+            r.u = pr;
             r.oa = make_float4((float)oa.x, (float)oa.y, (float)oa.z, (float)oa.w);
             r.ox = make_float4((float)ox.x, (float)ox.y, (float)ox.z, 0.f);
         } else {
@@ -216,9 +240,9 @@ __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, Sta
             r.ox = ox.x;
             r.oy = ox.y;
             r.oz = ox.z;
-            r.pw = B.pw[s];
-            r.v = B.va[s];
-            r.u = B.pred[s];
+            r.pw = pw;
+            r.v = va;
+            r.u = pr;
         }
         rec[s] = r;
         if (nearf) nearf[s] = near3<float>(P, ps, (float)t, home[s]);  // type in w
@@ -250,7 +274,8 @@ __global__ void __launch_bounds__(kBlock) adj_prep3(StepParams P, AdjStep T, Sta
 // predict and EOS reverse; writes lam_out.  Every lane of a block runs the
 // wave-uniform walk (lanes past n walk empty ranges).  LISTS: the
 // neighbours come from the lists of the build the step read (nbl, nbc, in
-// B's slot order) instead of the cell walk.
+// B's slot order) instead of the cell walk, and the gradient of the gauges of
+// the state it reverses into is added (eta_bar null: none).
 template <class R, bool LISTS>
 __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, StateB3<R> B,
                                                     const uint32_t* __restrict__ skey,
@@ -260,7 +285,10 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
                                                     const AdjRec3<R>* __restrict__ rec,
                                                     const double* __restrict__ direct, double* __restrict__ lam_out,
                                                     uint32_t* __restrict__ overflow_flag,
-                                                    const float4* __restrict__ nearf) {
+                                                    const float4* __restrict__ nearf, GaugeSpec3 G,
+                                                    const double* __restrict__ eta_bar,
+                                                    const double* __restrict__ zsum,
+                                                    const double* __restrict__ wsum) {
     // FP32 step over lists: entries decided and hits' r_i - r_k taken from
     // the near records (16 bytes, as the list pass does) instead of the FP64
     // positions (32 bytes)
@@ -381,6 +409,14 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
     double l[kLam3];
     adj_predict<3>(P, T.dt_pred, S, prk.w, pres_k, vak.w, direct + kDirect3 * (size_t)s, l);
     l[kLam3 - 1] = 0.0;
+    if (LISTS && eta_bar && tk == G.g.ptype) {
+        double gx, gy, gz;
+        if (gauge_gradient3(G, pk, eta_bar, zsum, wsum, gx, gy, gz)) {
+            l[0] += gx;
+            l[1] += gy;
+            l[2] += gz;
+        }
+    }
     double2* out = (double2*)(lam_out + kLam3 * (size_t)B.oid[s]);
 #pragma unroll
     for (uint32_t c = 0; c < kLam3 / 2; ++c) out[c] = make_double2(l[2 * c], l[2 * c + 1]);

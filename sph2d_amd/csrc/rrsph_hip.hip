@@ -158,7 +158,6 @@ struct AdjTape {
     std::vector<Lists> seg_lists;        // lists of the segment's builds (allocated on demand, reused)
     uint32_t nseg_lists = 0;             // builds of the segment in hand
     std::vector<int32_t> seg_build;      // per seg slot: the build (index in seg_lists) its step read
-    uint32_t* iota = nullptr;            // identity permutation
     float4* nearf = nullptr;             // FP32 step: near records of the reverse step's state (n)
     uint64_t force_build = ~0ull;        // tape step that must build (after a stale-list halt)
     // the forward's sorted step with the incremental re-sort, its record and
@@ -1193,7 +1192,6 @@ void free_tape(AdjTape& T) {
             if (p) (void)hipFree(p);
     }
     T.seg_lists.clear();
-    if (T.iota) (void)hipFree(T.iota);
     if (T.nearf) (void)hipFree(T.nearf);
     void* ptrs[] = {T.seg, T.eta, T.zs, T.ws, T.eta_bar, T.partials, T.piston_sum, T.lam[0], T.lam[1], T.direct,
                     T.drho_adj, T.out_adj, T.flag, T.rec, T.uctrl, T.seg_keys, T.seg_perm};
@@ -1238,8 +1236,8 @@ void enqueue_state_keys(rrsph_ctx* ctx) {
 // The reverse of one step on its re-sorted state (state precision R, adjoint
 // arithmetic FP64): whole_step reverse, then the pair gather.  In 2D over
 // lists the step's saved state src is read in place, through perm if the step
-// was a build (else null), and the gradient of the gauges of that state comes
-// with the pair gather (eta_bar, zs, ws: their row, or null).  8 lanes a
+// was a build (else null; in 3D only then), and the gradient of the gauges of
+// that state comes with the pair gather (eta_bar, zs, ws: their row, or null).  8 lanes a
 // particle below 25,000, where the list passes take them (setup_params).
 constexpr uint32_t kAdjLanes8 = 25000;
 template <class R>
@@ -1264,29 +1262,39 @@ static void enqueue_reverse_step(rrsph_ctx* ctx, const AdjStep& S, Ctrl* uc, con
         else pair(adj_pair_list<2>, group_blocks_per_xcd<2>(P.n));
         return;
     }
-    if (keys) {  // the sort step k ran with, saved by the replay: reorder only
+    const bool in_order = lists && !perm;  // (3D) src is in the slot order of its build
+    if (!in_order && keys) {  // the sort step k ran with, saved by the replay: reorder only
         ctx->sorted_keys = keys;
         ctx->sorted_perm = perm;
         enqueue_util_reorder<R>(ctx, src, uc);
-    } else {
+    } else if (!in_order) {
         enqueue_util_sort<R>(ctx, uc);
     }
     if (P.dim == 3) {
         StateB3<R> B = stateB3<R>(ctx, ctx->pred_scratch, ctx->pw_scratch, ctx->pres_scratch);
+        if (in_order) {
+            B.pos = (double4*)src->pos;
+            B.va = (real4<R>*)src->va;
+            B.oid = src->oid;
+        }
         AdjRec3<R>* rec = (AdjRec3<R>*)T.out_adj;
         // FP32 step over lists: near records relative to the home cells of
         // the build (its sorted keys) for the pair adjoint's walk
         float4* nearf = lists && sizeof(R) == 4 ? T.nearf : nullptr;
-        adj_prep3<R><<<nb, kBlock, 0, ctx->stream>>>(P, S, B, lam_in, rec, T.direct, psum,
-                                                     nearf ? lists->keys : nullptr, nearf);
+        auto prep = [&](auto kernel) {
+            kernel<<<nb, kBlock, 0, ctx->stream>>>(P, S, B, in_order ? (const real4<R>*)src->ad : nullptr, lam_in, rec,
+                                                   T.direct, psum, nearf ? lists->keys : nullptr, nearf);
+        };
+        if (in_order) prep(adj_prep3<R, true>);
+        else prep(adj_prep3<R, false>);
         if (lists)
             adj_pair3<R, true><<<nb_xcd, kBlock, 0, ctx->stream>>>(P, S, B, ctx->sorted_keys, ctx->LB, lists->nbl,
                                                                    lists->nbc, rec, T.direct, lam_out, T.flag,
-                                                                   nearf);
+                                                                   nearf, T.spec, eta_bar, zs, ws);
         else
             adj_pair3<R, false><<<nb_xcd, kBlock, 0, ctx->stream>>>(P, S, B, ctx->sorted_keys, ctx->LB, nullptr,
                                                                     nullptr, rec, T.direct, lam_out, T.flag,
-                                                                    nullptr);
+                                                                    nullptr, GaugeSpec3{}, nullptr, nullptr, nullptr);
     } else {
         StateB<R> B = stateB<R>(ctx, ctx->pred_scratch, ctx->pres_scratch);
         adj_prep<R><<<nb, kBlock, 0, ctx->stream>>>(P, S, B, lam_in, T.out_adj, T.drho_adj, T.direct, psum);
@@ -2716,7 +2724,6 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     T.seg_sorted.assign(cap, 0);
     T.builds.assign(nsteps, 0);
     T.seg_build.assign(cap, -1);
-    if (T.lists && d3) T.iota = dalloc<uint32_t>(n, e);
     if (T.lists && d3 && ctx->fp32) T.nearf = dalloc<float4>(n, e);
     T.eta = dalloc<double>((size_t)nsteps * kMaxGauges, e);
     T.zs = dalloc<double>((size_t)nsteps * kMaxGauges, e);
@@ -2741,11 +2748,6 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     if (e != hipSuccess) {
         free_tape(ctx->adj);
         return fail(ctx, RRSPH_ERR_HIP, std::string("hipMalloc (adjoint tape): ") + hipGetErrorString(e));
-    }
-    if (T.iota) {
-        std::vector<uint32_t> id(n);
-        for (size_t i = 0; i < n; ++i) id[i] = (uint32_t)i;
-        HIP_TRY(hipMemcpy(T.iota, id.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice));
     }
     T.allocated = true;
     return RRSPH_OK;
@@ -2919,9 +2921,9 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
             }
             // sort and reorder state k exactly as its step did (predict with its dt)
             const uint32_t* sk = sorted ? T.seg_keys + slot * n : (lists ? lists->keys : nullptr);
-            const uint32_t* sp = sorted ? T.seg_perm + slot * n : (lists ? T.iota : nullptr);
-            // the loss term of state k: in 2D over lists with the pair gather
-            const bool with_gauges = !d3 && lists && k >= 1;
+            const uint32_t* sp = sorted ? T.seg_perm + slot * n : nullptr;
+            // the loss term of state k: over lists with the pair gather
+            const bool with_gauges = lists && k >= 1;
             const size_t row = k >= 1 ? (size_t)(k - 1) * kMaxGauges : 0;
             const double *eb = with_gauges ? T.eta_bar + row : nullptr, *zs = T.zs + row, *ws = T.ws + row;
             if (ctx->fp32)
