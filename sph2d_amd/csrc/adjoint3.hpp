@@ -322,7 +322,7 @@ __global__ void __launch_bounds__(kBlock) adj_pair3(StepParams P, AdjStep T, Sta
     bool overflow = false;
     uint32_t* my = hits + threadIdx.x;
     // Over lists in FP64 the wave fetches the records of its lanes' next hits
-    // together (WaveGather) while it works on this round's: lanes loading their
+    // together (WaveGather) while it works on their last ones: lanes loading their
     // own made 10 accesses of up to 64 lines a hit, which bound the loop
     // (509,126 particles 503 -> 427 us).  In FP32, 5 accesses a hit, it made no
     // difference (943,906 particles: 623 us, 638 and with two records in flight
