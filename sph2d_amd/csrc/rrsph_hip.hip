@@ -924,13 +924,18 @@ rrsph_status rollback_fused_step(rrsph_ctx* ctx) {
     return RRSPH_OK;
 }
 
+// A halt that the host answers by running the halted step again (resume_halt), none of rrsph_status.
+bool rerun_status(uint32_t status) {
+    return status == kStatusResort || status == kStatusRebuild || status == kStatusListOverflow ||
+           status == kStatusUnfused;
+}
+
 // Read the control block after the stream drained and turn it into a status.
 rrsph_status sync_status(rrsph_ctx* ctx) {
     HIP_TRY(hipMemcpyAsync(ctx->host_ctrl, ctx->ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     const Ctrl& c = *ctx->host_ctrl;
-    const bool rerun = c.status == kStatusResort || c.status == kStatusRebuild || c.status == kStatusListOverflow;
-    if (c.halted && c.status != 0 && !rerun) {
+    if (c.halted && c.status != 0 && !rerun_status(c.status)) {
         if (c.rollback) {
             if (const rrsph_status st = rollback_fused_step(ctx); st != RRSPH_OK) return st;
         }
@@ -1625,7 +1630,7 @@ static void adapt_list_interval(rrsph_ctx* ctx) {
 static rrsph_status resume_halt(rrsph_ctx* ctx, bool* resumed) {
     Ctrl& c = *ctx->host_ctrl;
     *resumed = false;
-    if (!c.halted) return RRSPH_OK;
+    if (!c.halted || !rerun_status(c.status)) return RRSPH_OK;
     const uint64_t at = committed_steps(c);  // the step that halted
     if (c.status == kStatusResort) {
         note_resort_overflow(ctx, at);
@@ -1635,11 +1640,9 @@ static rrsph_status resume_halt(rrsph_ctx* ctx, bool* resumed) {
         ctx->fuse = false;
         drop_list_graphs(ctx);  // (the stream is idle)
         ctx->need_full = true;
-    } else if (c.status == kStatusListOverflow) {
+    } else {                     // kStatusListOverflow
         ctx->list_mode = false;  // more candidates than a list holds: sort every step from here
         ctx->need_full = true;
-    } else {
-        return RRSPH_OK;
     }
     c.halted = 0;
     c.status = 0;
