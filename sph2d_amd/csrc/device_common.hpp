@@ -108,8 +108,8 @@ struct StepParams {
     // constants of the pair terms, so that no wave divides for them
     double inv_h;           // 1 / h
     double c_q1, c_q2, w_q2;  // cubic spline pieces: f / h^2, f / (2 h), f / 6
-    // list pair terms (list_step.hpp): a = c2 (b2 x - a2) x from x = vr /
-    // (d^2 + eta^2), and the factors of the summed terms
+    // list pair terms (list_step.hpp): a = (b2 x - a2) x from x = vr / (d^2 +
+    // eta^2), and the factors of the summed terms
     double lp_a2, lp_b2, lp_mF, lp_mW;
     int32_t skf_density, skf_intf, skf_av, skf_xsph, skf_ap;
     double eos_B;

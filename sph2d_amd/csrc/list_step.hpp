@@ -945,23 +945,29 @@ __device__ __forceinline__ void for_each_listed(const StepParams& P, const float
 // 2D and 3D, arranged for instruction count, which bounds the passes (a
 // wave of the 2D FP32 pass issued 1,797 VALU instructions, 47 of its 58 us
 // at 1M particles):
-//   * with t = max(1 - q/2, 0) and u = max(1 - q, 0), both free clamps of one
-//     multiply-add, the spline is W = 4f/3 (t^3 - u^3 / 2) and grad W = diff
-//     (-2f/h) (t^2 - u^2) / |r| on both pieces, without selects; constant
-//     factors are applied once per particle (lp_mF, lp_mW);
-//   * an entry that is no neighbour gets |r| = 4 h, where both vanish;
+//   * with t = h - |r| / 2 the outer piece is W = f / h^3 (4/3 t^3) and grad W
+//     = diff (-2f / h^3) t^2 / |r|, the inner one with the same scales 2/3 h^3 -
+//     |r|^2 t and t - |r| / 4; one comparison selects both, and the scales are
+//     applied once per particle (lp_mF, lp_mW).  At most one operand of each
+//     instruction is uniform: a second would take vector registers, which
+//     spills in FP64.  (With u = h - |r| above 0 the inner piece is the
+//     outer less multiples of u^2 and u^3, without the comparison; but the
+//     difference loses the bits of close pairs: FP32 gradients off by up to
+//     6.9e-6 of their value at q = 0.02 to 0.05 and 8.7e-7 at 0.2 to 0.4, 2e-7
+//     here);
+//   * an entry that is no neighbour gets |r| = 2 h, where both vanish;
 //   * artificial viscosity from x = min(vr, 0) / (d^2 + eta^2), mu = h x:
 //     the term is zero by itself where particles separate.
 // CONT: continuity density; ALL: artificial viscosity, XSPH and the wall
 // force are all on (else each by its switch).
 template <class R, bool CONT, bool ALL> struct ListPair {
     static constexpr bool cont = CONT;
-    R ht, hu, hfar, a2, b2, eta2, lj_r0, lj_D;
+    R h, h2, h23, a2, b2, eta2, lj_r0, lj_D;
     bool lj_on, av_on, xsph_on;
     __device__ explicit ListPair(const StepParams& P)
-        : ht((R)(-0.5 * P.inv_h)), hu((R)(-P.inv_h)), hfar((R)(4.0 * P.h)), a2((R)P.lp_a2), b2((R)P.lp_b2),
-          eta2((R)P.av_eta2), lj_r0((R)P.lj_r0), lj_D((R)P.lj_D), lj_on(ALL || P.lj_on), av_on(ALL || P.av_on),
-          xsph_on(ALL || P.xsph_on) {}
+        : h((R)P.h), h2((R)(2.0 * P.h)), h23((R)(2.0 / 3.0 * P.h * P.h * P.h)), a2((R)P.lp_a2),
+          b2((R)P.lp_b2), eta2((R)P.av_eta2), lj_r0((R)P.lj_r0), lj_D((R)P.lj_D), lj_on(ALL || P.lj_on),
+          av_on(ALL || P.av_on), xsph_on(ALL || P.xsph_on) {}
 };
 // What a pair gives, but for the direction: the gradient factor F (grad W =
 // diff F lp_mF / m), the XSPH weight w of fluid neighbours (W / (rho_i +
@@ -971,7 +977,6 @@ template <class R> struct ListTerm {
     R F, w, coef, rinv;
     bool wall;
 };
-template <class R> __device__ __forceinline__ R clamp01(R v) { return fmin(fmax(v, R(0)), R(1)); }
 // min(a, b) for b not NaN; the median takes no canonicalising instruction
 __device__ __forceinline__ float running_min(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, -INFINITY); }
 __device__ __forceinline__ double running_min(double a, double b) { return b < a ? b : a; }
@@ -980,12 +985,11 @@ __device__ __forceinline__ double running_min(double a, double b) { return b < a
 template <class R, class K_>
 __device__ __forceinline__ ListTerm<R> list_pair(const K_& K, bool take, R d2, R vr, R zi, R zj, R pw, R& xmin) {
     ListTerm<R> T;
-    // coincident particles: |r| = 0 and t = u, so F = 0
     T.rinv = fast_rsqrt<R>(d2 + (sizeof(R) == 4 ? R(1e-30f) : R(1e-200)));
-    const R dist = take ? d2 * T.rinv : K.hfar;
-    const R t = clamp01<R>(fma(dist, K.ht, R(1))), u = clamp01<R>(fma(dist, K.hu, R(1)));
-    const R t2 = t * t, u2 = u * u;
-    T.F = T.rinv * (t2 - u2);
+    const R dist = take ? d2 * T.rinv : K.h2;
+    const R t = fma(dist, R(-0.5), K.h), t2 = t * t;
+    const bool inner = dist <= K.h;  // (then taken, and d2 = |r|^2)
+    T.F = inner ? fma(dist, R(-0.25), t) : T.rinv * t2;
     const R inv_rs = fast_rcp<R>(fabs(zi) + fabs(zj));
     T.coef = pw;
     if (K.av_on) {
@@ -993,8 +997,9 @@ __device__ __forceinline__ ListTerm<R> list_pair(const K_& K, bool take, R d2, R
         xmin = running_min(xmin, x);
         T.coef += (K.b2 * x - K.a2) * x * inv_rs;
     }
-    T.w = K.xsph_on && zi > R(0) ? (t2 * t - R(0.5) * (u2 * u)) * inv_rs : R(0);
-    T.wall = K.lj_on && zj > R(0) && zi < R(0) && dist < K.lj_r0;
+    const R w = inner ? fma(-d2, t, K.h23) : t2 * t * R(4.0 / 3.0);
+    T.w = K.xsph_on && zi > R(0) ? w * inv_rs : R(0);
+    T.wall = K.lj_on && take && zj > R(0) && zi < R(0) && dist < K.lj_r0;
     return T;
 }
 // The wall force's factor on diff (0 for coincident particles).
@@ -1175,11 +1180,13 @@ __device__ __forceinline__ bool fused_pair_begin(const StepParams& P, Ctrl* next
 // pair_fast_kernel), the dt maxima, and the fields for the integrator.  With
 // continuity it also writes the pressure of the current density (the
 // reference's p array).
+// In FP64 with 8 lanes a bound of 3 waves per SIMD, about as many as 25,000
+// particles give: 4 spill (17.7 us a step of 11,842 particles, 16.5 with 3).
 // FUSED: see fused_step_begin.  200 steps of 6,923 particles (FP64) take 2.35 ms
 // so, 2.88 with an integrator of their own (4 us of a step's 14, and a launch
 // gap); 30 of 134,603 (summation, FP32) 1.50 against 1.58.
 template <class R, bool FIRST, int LPP, bool CONT, bool ALL, bool FUSED>
-__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? (FUSED ? 3 : 4) : LPP == 1 ? (FUSED ? 5 : 6) : 1)
+__global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? (FUSED || LPP == 8 ? 3 : 4) : LPP == 1 ? (FUSED ? 5 : 6) : 1)
     pair_list_kernel(StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec,
                      R* __restrict__ pres, const uint32_t* __restrict__ nbl, const uint32_t* __restrict__ nbc,
                      real4<R>* __restrict__ der, real2<R>* __restrict__ xs,

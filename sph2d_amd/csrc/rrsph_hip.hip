@@ -1008,8 +1008,8 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     P.w_q2 = P.f_cubic / 6.0;
     P.lp_a2 = 2.0 * h * (p.artificial_shear_visc * p.eos_sound_vel);
     P.lp_b2 = 2.0 * h * h * p.artificial_bulk_visc;
-    P.lp_mF = -2.0 * P.f_cubic / h * p.mass;
-    P.lp_mW = 2.0 * p.average_velocity_coef * p.mass * (4.0 / 3.0 * P.f_cubic);
+    P.lp_mF = -2.0 * P.f_cubic * p.mass / (h * h * h);
+    P.lp_mW = 2.0 * p.average_velocity_coef * p.mass * P.f_cubic / (h * h * h);
     P.skf_density = p.density_skf;
     P.skf_intf = p.intf_skf;
     P.skf_av = p.artificial_viscosity_skf;
