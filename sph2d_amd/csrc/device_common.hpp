@@ -108,6 +108,7 @@ struct StepParams {
     // constants of the pair terms, so that no wave divides for them
     double inv_h;           // 1 / h
     double c_q1, c_q2, w_q2;  // cubic spline pieces: f / h^2, f / (2 h), f / 6
+    double g_gauss, g_wend, g_desb;  // of the other kernels' gradients: -2 / h^2, -5 f / h^2, -3 f / h^2
     // list pair terms (list_step.hpp): a = (b2 x - a2) x from x = vr / (d^2 +
     // eta^2), and the factors of the summed terms
     double lp_a2, lp_b2, lp_mF, lp_mW;

@@ -1289,34 +1289,36 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? (FUSED || LPP == 8 ? 
 }
 
 // W and the gradient factor F (grad W = (r_i - r_j) F) of kernel type skf at
-// |r| = dist, with rinv = 1 / |r| (infinite for coincident particles) and
-// q = |r| / h: the pieces of kernel_w and kernel_gradf (physics.hpp) without
-// their divisions.
+// q = |r| / h, iq = h / |r| (infinite for coincident particles): the pieces
+// of kernel_w and kernel_gradf (physics.hpp) without their divisions, with
+// 1 / h^2 in the gradients' factors.  Wendland's s^4 - (2 q + 1) s^3 is
+// q times -5/2 s^3, without the difference (q iq is 1 but for q's rounding,
+// which offsets part of what that does to s^3).
 template <class R>
-__device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R dist, R rinv, R q, R& W, R& F) {
-    const R t = R(2) - q, ih = K.inv_h;
+__device__ __forceinline__ void kernel_wf(const StepParams& P, int skf, R q, R iq, R& W, R& F) {
+    const R t = R(2) - q;
     switch (skf) {
     case 2:
-        W = K.f_gauss * exp(-q * q);
-        F = R(-2) * ih * ih * W;
+        W = (R)P.f_gauss * exp(-q * q);
+        F = (R)P.g_gauss * W;
         break;
     case 3: {
-        const R s = R(0.5) * t, s3 = s * s * s, g = R(2) * q + R(1);
-        W = q > R(2) ? R(0) : K.f_wend * (s3 * s) * g;
-        F = q < R(1.e-6f) || q >= R(2) ? R(0) : R(2) * K.f_wend * ih * rinv * (s3 * s - g * s3);
+        const R s = R(0.5) * t, s3 = s * s * s;
+        W = q > R(2) ? R(0) : (R)P.f_wend * (s3 * s) * (R(2) * q + R(1));
+        F = q < R(1.e-6f) || q >= R(2) ? R(0) : (R)P.g_wend * (s3 * (q * iq));
         break;
     }
     case 4:
-        W = q <= R(2) ? K.f_desb * (t * t * t) : R(0);
-        F = q < R(2) ? K.f_desb * rinv * ih * (R(-3) * t * t) : R(0);
+        W = q <= R(2) ? (R)P.f_desb * (t * t * t) : R(0);
+        F = q < R(2) ? (R)P.g_desb * (t * t) * iq : R(0);
         break;
     default:
         if (q <= R(1)) {
-            W = K.f_cubic * (R(2) / R(3) - q * q + q * q * q * R(0.5));
-            F = K.f_cubic * (ih * ih) * (R(-2) + R(1.5) * q);
+            W = (R)P.f_cubic * (R(2) / R(3) - q * q + q * q * q * R(0.5));
+            F = (R)P.c_q1 * (R(-2) + R(1.5) * q);
         } else {
-            W = q <= R(2) ? K.f_cubic * (R(1) / R(6) * (t * t * t)) : R(0);
-            F = q <= R(2) ? -K.f_cubic * rinv * ih * (t * t * R(0.5)) : R(0);
+            W = q <= R(2) ? (R)P.f_cubic * (R(1) / R(6) * (t * t * t)) : R(0);
+            F = q <= R(2) ? (R)P.c_q1 * (t * t * R(-0.5)) * iq : R(0);
         }
         break;
     }
@@ -1328,9 +1330,11 @@ __device__ __forceinline__ void kernel_wf(const KernelConsts<R>& K, int skf, R d
 // pair_kernel on the same FP64 positions.  An entry gathers the neighbour's
 // position, state and pred record; entries in groups of G as in
 // for_each_listed.  Terms whose kernel type is the pressure's share one
-// evaluation, and no term divides: the cell walk over ~55 candidates with a
-// division or more per term took 167 us at 187,530 particles (FP64, Wendland
-// kernels, delta-SPH, artificial pressure), the ~20 entries of a list 42.
+// evaluation, and but for the wall force no term divides: the cell walk over
+// ~55 candidates with a division or more per term took 167 us at 187,530
+// particles (FP64, Wendland kernels, delta-SPH, artificial pressure), the ~20
+// entries of a list 45.  The reciprocal root and 1 / h alone would leave |r| / h
+// with half as much error again (43 us).
 template <class R, bool FIRST, int LPP>
 __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_general_kernel(
     StepParams P, Ctrl* next, Ctrl* cur, ListState<R> X, const ListRec<R>* __restrict__ rec, R* __restrict__ pres,
@@ -1400,14 +1404,17 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                 const R d2 = (R)(dxd * dxd + dyd * dyd);
                 const bool apart = d2 > R(0);
                 const R rinv = apart ? fast_rsqrt<R>(d2) : R(INFINITY);
-                const R dist = apart ? d2 * rinv : R(0);
-                const R q = dist * K.inv_h;
+                // |r| and |r| / h within half a unit of the last place, as sqrt and a
+                // division give them: near the cut-off the kernels amplify their errors
+                const R r1 = d2 * rinv;
+                const R dist = apart ? fma(fma(-r1, r1, d2), R(0.5) * rinv, r1) : R(0);
+                const R q1 = dist * K.inv_h, q = fma(fma(-q1, K.h, dist), K.inv_h, q1), iq = K.h * rinv;
                 R W, F;
-                kernel_wf<R>(K, P.skf_intf, dist, rinv, q, W, F);
+                kernel_wf<R>(P, P.skf_intf, q, iq, W, F);
                 // continuity density with v and rho of the current step
                 if (cont) {
                     R Wd = W, Fd = F;
-                    if (P.skf_density != P.skf_intf) kernel_wf<R>(K, P.skf_density, dist, rinv, q, Wd, Fd);
+                    if (P.skf_density != P.skf_intf) kernel_wf<R>(P, P.skf_density, q, iq, Wd, Fd);
                     const R gx = dx * Fd, gy = dy * Fd;
                     drho += m * ((va[u].x - vaj.x) * gx + (va[u].y - vaj.y) * gy);
                     if (delta) {
@@ -1417,9 +1424,9 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                 }
                 // Lennard-Jones wall force on fluid from boundary particles
                 if (P.lj_on && tj > 0 && ti < 0 && dist < lj_r0) {
-                    const R rn = lj_r0 * rinv;
+                    const R rn = lj_r0 / dist;  // (few pairs, and its 12th power)
                     const R rn2 = rn * rn, rn4 = rn2 * rn2;
-                    const R f = lj_D * (rn4 * rn4 * rn4 - rn4) * (rinv * rinv);
+                    const R f = lj_D * (rn4 * rn4 * rn4 - rn4) / d2;
                     ax -= dx * f;
                     ay -= dy * f;
                 }
@@ -1429,7 +1436,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                                           : pr[u].w + prj.w;
                 if (P.art_pressure && (pr[u].w < R(0) || prj.w < R(0))) {
                     R Wa = W, Fa = F;
-                    if (P.skf_ap != P.skf_intf) kernel_wf<R>(K, P.skf_ap, dist, rinv, q, Wa, Fa);
+                    if (P.skf_ap != P.skf_intf) kernel_wf<R>(P, P.skf_ap, q, iq, Wa, Fa);
                     const R api = pr[u].w < R(0) ? -(R)P.ap_coef * pr[u].w : R(0);
                     const R apj = prj.w < R(0) ? -(R)P.ap_coef * prj.w : R(0);
                     pf += (api + apj) * pow(Wa * ap_iw, (R)P.ap_index);
@@ -1444,7 +1451,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                         const R mu = K.h * vr * fast_rcp<R>(d2 + eta2);
                         amu = fmax(amu, fabs(mu));
                         R Wv = W, Fv = F;
-                        if (P.skf_av != P.skf_intf) kernel_wf<R>(K, P.skf_av, dist, rinv, q, Wv, Fv);
+                        if (P.skf_av != P.skf_intf) kernel_wf<R>(P, P.skf_av, q, iq, Wv, Fv);
                         cx += Fv * ((beta * mu - alpha_c) * mu * R(2) * inv_rs) * m;
                     }
                 }
@@ -1452,7 +1459,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                 ay += dy * cx;
                 if (P.xsph_on && ti > 0) {
                     R Wx = W, Fx = F;
-                    if (P.skf_xsph != P.skf_intf) kernel_wf<R>(K, P.skf_xsph, dist, rinv, q, Wx, Fx);
+                    if (P.skf_xsph != P.skf_intf) kernel_wf<R>(P, P.skf_xsph, q, iq, Wx, Fx);
                     const R c = two_eps_m * inv_rs * Wx;
                     avx += dvx * c;
                     avy += dvy * c;

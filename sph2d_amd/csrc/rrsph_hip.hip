@@ -1006,6 +1006,9 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     P.c_q1 = P.f_cubic / (h * h);
     P.c_q2 = 0.5 * P.f_cubic / h;
     P.w_q2 = P.f_cubic / 6.0;
+    P.g_gauss = -2.0 / (h * h);
+    P.g_wend = (double)(-5.0L * P.f_wend / ((long double)h * h));
+    P.g_desb = (double)(-3.0L * P.f_desb / ((long double)h * h));
     P.lp_a2 = 2.0 * h * (p.artificial_shear_visc * p.eos_sound_vel);
     P.lp_b2 = 2.0 * h * h * p.artificial_bulk_visc;
     P.lp_mF = -2.0 * P.f_cubic * p.mass / (h * h * h);
