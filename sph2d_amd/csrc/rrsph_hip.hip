@@ -151,6 +151,7 @@ struct AdjTape {
     bool lists = false;
     bool may_list = false;               // tape_lists when the buffers were allocated
     bool no_room = false;                // a kept tape could not allocate a build's lists
+    size_t max_lists = 0;                // ... or may not: the builds whose lists fit (tape_memory)
     std::vector<uint8_t> builds;         // per step: the step built lists
     struct Lists {
         uint32_t *nbl = nullptr, *nbc = nullptr, *keys = nullptr;
@@ -2309,7 +2310,8 @@ static rrsph_status tape_build_lists(rrsph_ctx* ctx) {
     const size_t n = ctx->P.n, rows = ctx->P.list_cap + kListPad;
     if (T.nseg_lists == T.seg_lists.size()) {
         AdjTape::Lists L;
-        hipError_t e = T.keep_all && T.nseg_lists >= ctx->tape_lists_max ? hipErrorOutOfMemory : hipSuccess;
+        hipError_t e = T.keep_all && T.nseg_lists >= std::min(T.max_lists, ctx->tape_lists_max) ? hipErrorOutOfMemory
+                                                                                                : hipSuccess;
         L.nbl = dalloc<uint32_t>(rows * n, e);
         L.nbc = dalloc<uint32_t>(n, e);
         L.keys = dalloc<uint32_t>(n, e);
@@ -2680,20 +2682,28 @@ static rrsph_status tape_records_and_gauges(rrsph_ctx* ctx) {
     return RRSPH_OK;
 }
 
+// What a tape that keeps every state may take: half the free memory, or what
+// RRSPH_HIP_TAPE_MEMORY says (bytes; a process that shares the device).
+static double tape_memory() {
+    if (const char* e = std::getenv("RRSPH_HIP_TAPE_MEMORY")) return std::strtod(e, nullptr);
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess ? 0.5 * (double)free_b : 0.0;
+}
+// Bytes of every state and sort of the tape, and of one build's lists.
+static double tape_state_bytes(const rrsph_ctx* ctx) {
+    return (double)ctx->adj.nsteps * ((double)state_bytes(ctx) + 256 + 8.0 * ctx->P.n);
+}
+static double tape_list_bytes(const rrsph_ctx* ctx) { return 4.0 * ctx->P.n * (double)(ctx->P.list_cap + kListPad + 2); }
+
 // Whether every state and sort of the tape, and with list steps the lists
-// of a build in every fourth step and every checkpoint, fit in half the free
-// memory.  (A kept tape that builds more often and finds no room for a
-// build's lists starts over: in 3D with one segment's states, in 2D on sorted
-// steps if all their states fit.)
+// of a build in every fourth step and every checkpoint, fit in tape_memory.
+// (A kept tape that builds more often than fits (max_lists), or finds no
+// memory for a build's lists, starts over: in 3D with one segment's states,
+// in 2D on sorted steps if all their states fit.)
 static bool tape_fits(const rrsph_ctx* ctx, bool lists) {
     const AdjTape& T = ctx->adj;
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
-    const double n = ctx->P.n, steps = T.nsteps;
-    const double builds = lists ? steps / 4 + (double)((T.nsteps + T.every - 1) / T.every) + 1 : 0.0;
-    const double all_b = steps * ((double)state_bytes(ctx) + 256 + 8 * n) +
-                         builds * 4 * n * (double)(ctx->P.list_cap + kListPad + 2);
-    return all_b <= 0.5 * (double)free_b;
+    const double builds = lists ? T.nsteps / 4.0 + (double)((T.nsteps + T.every - 1) / T.every) + 1 : 0.0;
+    return tape_state_bytes(ctx) + builds * tape_list_bytes(ctx) <= tape_memory();
 }
 
 // The buffers of a tape of T.nsteps steps with a checkpoint every T.every.
@@ -2710,6 +2720,7 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     for (auto& p : T.ck) p = dalloc<char>(T.blob, e);
     // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's states, and replays)
     T.keep_all = !T.segments && (ctx->tape_keep || !T.lists) && tape_fits(ctx, T.lists);
+    if (T.batched()) T.max_lists = (size_t)std::max(0.0, (tape_memory() - tape_state_bytes(ctx)) / tape_list_bytes(ctx));
     uint32_t cap = T.keep_all ? nsteps : T.every;  // states seg holds
     const bool alloc_ok = e == hipSuccess;
     T.seg = dalloc<char>(T.blob * cap, e);

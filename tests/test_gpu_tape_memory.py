@@ -1,0 +1,58 @@
+"""A tape that keeps every state admits its lists by a likely number of builds; where a run builds more often, the lists
+stay within the same bound (here set by RRSPH_HIP_TAPE_MEMORY, by default half the free memory), and the run starts over
+as one whose tape fits."""
+import numpy as np
+import pytest
+
+from sph2d_amd import generators as G
+from sph2d_amd import hip as H
+from sph2d_amd.adjoint import DifferentiableRun
+
+pytestmark = pytest.mark.gpu
+STEPS, MIB = 40, 1 << 20
+
+
+def _layout(dim):
+    if dim == 2:
+        return G.adjoint_tank(delta=0.0035, length=1.5), [0.03, 0.1], None
+    return G.piston_basin_3d(delta=0.03, length=1.0, width=0.8), [0.1, 0.2], [0.3, 0.5]
+
+
+def _gradients(dim):
+    import torch
+
+    lay, xs, zs = _layout(dim)
+    prm = lay.params
+    spec = H.gauge_spec(xs, radius=3 * prm.delta, tau=prm.delta / 4, y_ref=prm.depth, zs=zs)
+    run = DifferentiableRun(H.HipStep(prm, precision=H.FP64), dict(lay.state), STEPS, 8, spec, prm.piston_omega)
+    run.sim.upload(*(lay.state[f] for f in ("r", "v", "rho", "itype")))
+    a, b = np.array(prm.piston_a), np.array(prm.piston_b)
+    free = torch.cuda.mem_get_info()[0]
+    eta = run.forward(a, b)
+    used = free - torch.cuda.mem_get_info()[0]
+    g = run.backward(2 * (eta - prm.depth), len(a))
+    stats = run.sim.list_stats()
+    run.sim.close()
+    return eta, g, used, stats
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_lists_of_a_kept_tape_stay_within_its_bound(monkeypatch, dim):
+    n = _layout(dim)[0].params.ntotal
+    monkeypatch.setenv("RRSPH_HIP_LIST_SKIN", "0.0002")  # every step builds
+    # bytes of the kept states and sorts of FP64 steps, of a build's lists (their capacity: max_neighbours with the
+    # skin, 8 more and 8 rows of padding), and of the rest of the tape (checkpoints, adjoints, records)
+    states = STEPS * n * (124 if dim == 2 else 140)
+    lists = 4 * n * (_layout(dim)[0].params.max_neighbours + 19)
+    rest = 6 * n * 120 + n * 400 + 16 * MIB
+    bound = states + (STEPS // 4 + STEPS // 8 + 2) * lists  # builds in every fourth step and at the checkpoints, and one
+    monkeypatch.setenv("RRSPH_HIP_TAPE_MEMORY", str(bound))
+    eta, g, used, stats = _gradients(dim)
+    print("tape memory", dim, "n", n, "bound MiB", bound / MIB, "used", used / MIB, stats, flush=True)
+    assert stats["builds"] > STEPS // 4 + STEPS // 8 + 2  # it ran out
+    assert used <= bound + rest
+    monkeypatch.setenv(*(("RRSPH_HIP_LIST", "0") if dim == 2 else ("RRSPH_HIP_ADJ_STORE", "segments")))
+    eta0, g0, *_ = _gradients(dim)
+    assert np.array_equal(eta, eta0)
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(g[f], g0[f]), f
