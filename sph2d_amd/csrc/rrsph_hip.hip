@@ -255,7 +255,7 @@ struct rrsph_ctx {
     bool all_terms = false;             // artificial viscosity, XSPH and the wall force are all on
     int lanes = 1;                      // lanes per particle of the 2D list passes
     bool list_suspended = false;        // 2D tapes without lists, and their replays
-    bool tape_keep = true;              // false: a kept tape ran out of room for its lists
+    uint32_t no_keep_steps = 0, no_keep_every = 0;  // the shape of the last tape if its lists ran out of room when it kept them all
     size_t tape_lists_max = ~(size_t)0; // the most builds whose lists a kept tape allocates (RRSPH_HIP_TAPE_LISTS)
     uint32_t *nbl = nullptr, *nbc = nullptr;
     void* rec = nullptr;                // records of the list pass (ListRec per slot)
@@ -2706,6 +2706,11 @@ static bool tape_fits(const rrsph_ctx* ctx, bool lists) {
     return tape_state_bytes(ctx) + builds * tape_list_bytes(ctx) <= tape_memory();
 }
 
+// Whether a tape of this shape has not just run out of room for its lists.
+static bool tape_may_keep(const rrsph_ctx* ctx) {
+    return ctx->no_keep_steps != ctx->adj.nsteps || ctx->no_keep_every != ctx->adj.every;
+}
+
 // The buffers of a tape of T.nsteps steps with a checkpoint every T.every.
 static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     AdjTape& T = ctx->adj;
@@ -2719,7 +2724,7 @@ static rrsph_status alloc_tape(rrsph_ctx* ctx) {
     T.ck.assign(nck + 1, nullptr);
     for (auto& p : T.ck) p = dalloc<char>(T.blob, e);
     // (RRSPH_HIP_ADJ_STORE=segments keeps one segment's states, and replays)
-    T.keep_all = !T.segments && (ctx->tape_keep || !T.lists) && tape_fits(ctx, T.lists);
+    T.keep_all = !T.segments && (tape_may_keep(ctx) || !T.lists) && tape_fits(ctx, T.lists);
     if (T.batched()) T.max_lists = (size_t)std::max(0.0, (tape_memory() - tape_state_bytes(ctx)) / tape_list_bytes(ctx));
     uint32_t cap = T.keep_all ? nsteps : T.every;  // states seg holds
     const bool alloc_ok = e == hipSuccess;
@@ -2796,8 +2801,9 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
         T.every = std::min(checkpoint_every, nsteps);
         T.segments = segments;
         T.may_list = may_list;
+        if (tape_may_keep(ctx)) ctx->no_keep_steps = ctx->no_keep_every = 0;
         // in 2D sorted steps whose states can all be kept beat list steps that replay
-        T.lists = may_list && (ctx->P.dim == 3 || segments || (ctx->tape_keep && tape_fits(ctx, true)) ||
+        T.lists = may_list && (ctx->P.dim == 3 || segments || (tape_may_keep(ctx) && tape_fits(ctx, true)) ||
                                !tape_fits(ctx, false));
         st = alloc_tape(ctx);
         if (st != RRSPH_OK) return st;
@@ -2824,7 +2830,7 @@ static rrsph_status adjoint_forward_impl(rrsph_ctx* ctx, uint32_t nsteps, uint32
         st = restore_state_sync(ctx, T.ck[0]);
         if (st != RRSPH_OK) return st;
         if (overflowed) ctx->list_mode = false;
-        else ctx->tape_keep = false;
+        else ctx->no_keep_steps = T.nsteps, ctx->no_keep_every = T.every;
         ctx->list_interval = interval;  // (the schedule of a run that had not been tried)
         free_tape(T);
         ctx->err.clear();

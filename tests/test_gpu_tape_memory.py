@@ -56,3 +56,34 @@ def test_lists_of_a_kept_tape_stay_within_its_bound(monkeypatch, dim):
     assert np.array_equal(eta, eta0)
     for f in ("r", "v", "rho"):
         assert np.array_equal(g[f], g0[f]), f
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_a_run_that_fits_keeps_its_lists_after_one_that_did_not(monkeypatch, dim):
+    """What ran out of room is a run of one shape; a shorter one on the same context keeps its states and lists."""
+    monkeypatch.setenv("RRSPH_HIP_LIST_SKIN", "0.0002")  # every step builds
+    lay, xs, zs = _layout(dim)
+    prm = lay.params
+    spec = H.gauge_spec(xs, radius=3 * prm.delta, tau=prm.delta / 4, y_ref=prm.depth, zs=zs)
+    a, b = np.array(prm.piston_a), np.array(prm.piston_b)
+    c = np.random.default_rng(7).normal(0.0, 1.0, (16, 2))
+    out = []
+    for long_run_first in (True, False):
+        monkeypatch.setenv("RRSPH_HIP_TAPE_LISTS", "20")
+        run = DifferentiableRun(H.HipStep(prm, precision=H.FP64), dict(lay.state), STEPS, 8, spec, prm.piston_omega)
+        if long_run_first:
+            run.forward(a, b)
+            assert run.sim.list_stats()["builds"] > 20  # it ran out
+        run.nsteps = 16
+        for _ in range(2):  # by the second run the schedule is a build in every step
+            before = run.sim.list_stats()
+            eta = run.forward(a, b)
+            g = run.backward(c, len(a))
+            after = run.sim.list_stats()
+        # the forward's steps built their lists, and the reverse pass replayed none
+        assert after["builds"] - before["builds"] == 16 and after["list_steps"] == before["list_steps"]
+        out.append((eta, g))
+        run.sim.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    for f in ("r", "v", "rho"):
+        assert np.array_equal(out[0][1][f], out[1][1][f]), f
