@@ -1,6 +1,8 @@
 """A tape that keeps every state admits its lists by a likely number of builds; where a run builds more often, the lists
 stay within the same bound (here set by RRSPH_HIP_TAPE_MEMORY, by default half the free memory), and the run starts over
 as one whose tape fits."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -18,18 +20,22 @@ def _layout(dim):
     return G.piston_basin_3d(delta=0.03, length=1.0, width=0.8), [0.1, 0.2], [0.3, 0.5]
 
 
-def _gradients(dim):
-    import torch
+def _free_memory(sim):
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert sim.L.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0  # of the HIP runtime the library links
+    return free.value
 
+
+def _gradients(dim):
     lay, xs, zs = _layout(dim)
     prm = lay.params
     spec = H.gauge_spec(xs, radius=3 * prm.delta, tau=prm.delta / 4, y_ref=prm.depth, zs=zs)
     run = DifferentiableRun(H.HipStep(prm, precision=H.FP64), dict(lay.state), STEPS, 8, spec, prm.piston_omega)
     run.sim.upload(*(lay.state[f] for f in ("r", "v", "rho", "itype")))
     a, b = np.array(prm.piston_a), np.array(prm.piston_b)
-    free = torch.cuda.mem_get_info()[0]
+    free = _free_memory(run.sim)
     eta = run.forward(a, b)
-    used = free - torch.cuda.mem_get_info()[0]
+    used = free - _free_memory(run.sim)
     g = run.backward(2 * (eta - prm.depth), len(a))
     stats = run.sim.list_stats()
     run.sim.close()
