@@ -197,6 +197,7 @@ struct rrsph_ctx {
     bool stepped = false;
     bool fields_valid = false;  // der (list steps: adA) / xs hold the last step's fields in A's slot order
     bool list_fields = false;   // the last step was a list or build step
+    bool pres_in_order = true;  // false: pres is in the slot order of a step that failed
     uint32_t passes = 0;
     uint32_t ntiles = 0;
     // buffers
@@ -939,6 +940,13 @@ rrsph_status sync_status(rrsph_ctx* ctx) {
     if (c.halted && c.status != 0 && !rerun_status(c.status)) {
         if (c.rollback) {
             if (const rrsph_status st = rollback_fused_step(ctx); st != RRSPH_OK) return st;
+        } else if (c.status == RRSPH_ERR_TOO_MANY_NEIGHBOURS || c.status == RRSPH_ERR_NEVER_ENDING) {
+            // the step has left its fields (with lists A.ad, which the next step
+            // would have started from) and pressures in the slot order that it
+            // sorted into, and the state in the one before; a list step (some
+            // displacement counted since its build) sorted nothing
+            ctx->pres_in_order = ctx->list_fields && c.disp_acc > 0.0;
+            ctx->fields_valid = ctx->fields_valid && ctx->pres_in_order;
         }
         return fail(ctx, (rrsph_status)c.status, status_message(c.status));
     }
@@ -1482,6 +1490,7 @@ rrsph_status rrsph_hip_upload(rrsph_ctx* ctx, const double* r, const double* v, 
     ctx->uploaded = true;
     ctx->stepped = false;
     ctx->fields_valid = false;
+    ctx->pres_in_order = true;
     ctx->need_full = true;
     // step indices restart: forget the overflow history
     ctx->full_until = ctx->launched;
@@ -1733,22 +1742,23 @@ rrsph_status rrsph_hip_get_time(rrsph_ctx* ctx, double* time, double* dt, uint64
 static rrsph_status enqueue_unpack(rrsph_ctx* ctx) {
     const size_t dim = ctx->P.dim;
     const uint32_t nb = grid_blocks(ctx->P.n, kBlock);
+    const void* pres = ctx->stepped && ctx->pres_in_order ? ctx->pres : nullptr;  // null: the equation of state's of rho
     if (dim == 3) {
         if (ctx->fp32)
             download3_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(
-                ctx->P, stateA3<float>(ctx), ctx->stepped ? (const float*)ctx->pres : nullptr, ctx->st_r, ctx->st_v,
+                ctx->P, stateA3<float>(ctx), (const float*)pres, ctx->st_r, ctx->st_v,
                 ctx->st_rho, ctx->st_p, ctx->st_itype);
         else
             download3_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(
-                ctx->P, stateA3<double>(ctx), ctx->stepped ? (const double*)ctx->pres : nullptr, ctx->st_r,
+                ctx->P, stateA3<double>(ctx), (const double*)pres, ctx->st_r,
                 ctx->st_v, ctx->st_rho, ctx->st_p, ctx->st_itype);
     } else if (ctx->fp32) {
         download_kernel<float><<<nb, kBlock, 0, ctx->stream>>>(
-            ctx->P, stateA<float>(ctx), ctx->stepped ? (const float*)ctx->pres : nullptr, ctx->st_r, ctx->st_v,
+            ctx->P, stateA<float>(ctx), (const float*)pres, ctx->st_r, ctx->st_v,
             ctx->st_rho, ctx->st_p, ctx->st_itype);
     } else {
         download_kernel<double><<<nb, kBlock, 0, ctx->stream>>>(
-            ctx->P, stateA<double>(ctx), ctx->stepped ? (const double*)ctx->pres : nullptr, ctx->st_r, ctx->st_v,
+            ctx->P, stateA<double>(ctx), (const double*)pres, ctx->st_r, ctx->st_v,
             ctx->st_rho, ctx->st_p, ctx->st_itype);
     }
     HIP_TRY(hipGetLastError());
@@ -1786,7 +1796,7 @@ rrsph_status rrsph_hip_set_export_fields(rrsph_ctx* ctx, int32_t enable) {
 rrsph_status rrsph_hip_fields(rrsph_ctx* ctx, double* a, double* drho, double* av, double* arvmu) {
     if (!ctx || !ctx->stepped) return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: no step taken yet");
     if (!ctx->fields_valid)
-        return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: no step taken since the state was restored");
+        return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: no fields of the current state (it was restored, or the last step failed)");
     if (ctx->fused && !ctx->export_fields)
         return fail(ctx, RRSPH_ERR_INVALID_ARGUMENT, "RRSPH_HIP: enable rrsph_hip_set_export_fields before stepping");
     const size_t n = ctx->P.n, dim = ctx->P.dim;
@@ -2212,6 +2222,7 @@ static rrsph_status restore_state(rrsph_ctx* ctx, const void* src, bool keys = t
     if (const rrsph_status st = enqueue_copies(ctx, state_plan(ctx, const_cast<void*>(src), false)); st != RRSPH_OK)
         return st;
     ctx->fields_valid = false;  // der / xs belong to whatever step ran last
+    ctx->pres_in_order = true;
     // the next step's cell keys from the restored positions, and a full sort
     ctx->need_full = true;
     if (!keys) return RRSPH_OK;  // the caller reorders with a saved sort and launches no step
