@@ -2943,6 +2943,10 @@ static rrsph_status adjoint_backward_impl(rrsph_ctx* ctx, const double* eta_bar,
             // list steps: the build whose lists step k read, its state in that build's slot order
             const int32_t b = T.lists ? T.seg_build[slot] : -1;
             const AdjTape::Lists* lists = b >= 0 ? &T.seg_lists[(size_t)b] : nullptr;
+            // a replay does not launch a segment's last step: one that builds is
+            // reversed by the cell walk, in 3D FP32 with FP64 separations where
+            // lists have the near records' FP32, and so it is on kept tapes
+            if (T.batched() && d3 && ctx->fp32 && T.builds[k] && k + 1 == (int)n1 && n1 < N) lists = nullptr;
             // a step reordered with a saved sort reads its state where it was
             // saved; one that sorts again needs it in A (and its cell keys)
             char* blob = (char*)T.seg + slot * T.blob;
