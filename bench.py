@@ -310,7 +310,7 @@ def leg_3d(steps, delta, renorm_every=30):
         g.step(steps)
         torch.cuda.synchronize()
         wall = time.perf_counter() - t0
-        per_kernel, _ = g.profile_steps(2)
+        per_kernel, _ = g.profile_steps(8)  # (pair_ms: in pairs of fused steps with the integration)
         sort_stats = g.sort_stats()
         list_stats = g.list_stats()
         g.set_export_fields(True)

@@ -293,7 +293,9 @@ void* rrsph_hip_stream(rrsph_ctx* ctx);           /* hipStream_t the context lau
 rrsph_status rrsph_hip_set_graph(rrsph_ctx* ctx, int32_t enable);
 /* Runs nsteps steps with HIP events around every launch on the context's
  * stream; fills average milliseconds per launch for each kernel class
- * (names via rrsph_hip_kernel_class_name) and the total wall time. */
+ * (names via rrsph_hip_kernel_class_name; 0 for one that no step launched) and
+ * the total wall time.  The steps are those that rrsph_hip_step takes: where it
+ * fuses pairs of list steps, the pair pass's time holds the integration. */
 rrsph_status rrsph_hip_profile_steps(rrsph_ctx* ctx, uint32_t nsteps, double* avg_ms, uint32_t n_classes,
                                      double* total_ms);
 uint32_t rrsph_hip_kernel_class_count(void);

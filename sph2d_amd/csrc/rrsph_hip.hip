@@ -2023,10 +2023,15 @@ rrsph_status rrsph_hip_profile_steps(rrsph_ctx* ctx, uint32_t nsteps, double* av
     HIP_TRY(hipEventCreate(&t1));
     HIP_TRY(hipEventRecord(t0, ctx->stream));
     const uint64_t first = committed_steps(*ctx->host_ctrl);
+    bool second = false;  // the second of a fused pair
     for (uint32_t k = 0; k < nsteps; ++k) {
         if (list_active(ctx)) {
             const bool build = next_is_build(ctx, first + k);
-            enqueue_list_step(ctx, &prof, build ? kBuildStep : kPlainStep);
+            // as launch_steps: two list steps in a row are fused where the context fuses
+            const bool pair = !build && !second && ctx->fuse && k + 1 < nsteps &&
+                              !next_is_build(ctx, first + k + 1);
+            enqueue_list_step(ctx, &prof, build ? kBuildStep : second ? kFusedSecond : pair ? kFusedFirst : kPlainStep);
+            second = pair;
             if (build) {
                 ctx->build_at = first + k;
                 ++ctx->n_build;
