@@ -159,13 +159,14 @@ __global__ void __launch_bounds__(kBlock) reorder_list_kernel(StepParams P, cons
 // What several blocks of a step raise lies outside the published words: the
 // flags at the end of Ctrl, and maxima in slots, a set per parity of the step
 // index - displacement slots dslots (the integrator of step k fills set k,
-// the first kernel of step k + 1 reads it and clears the other) and dt
-// reduction slots maxslots (the pair pass of step k fills set k, its
-// integrator reads it and clears the other).  A set is few slots, each in a
-// 256-byte line of its own: every block of the next kernel reads them all, at
-// addresses known before any other load returns, without a reduction across
-// lanes or a barrier (256 adjacent slots, reduced by shuffles through LDS,
-// held every block up for about 1.5 us).
+// the first kernel of step k + 1 reads it and clears the other; where steps
+// fuse, four sets by the index modulo 4) and dt reduction slots, the kernels'
+// maxslots (the pair pass of step k fills set k, its integrator reads it and
+// clears the other).  A set is few slots, each in a 256-byte line of its own:
+// every block of the next kernel reads them all, at addresses known before any
+// other load returns, without a reduction across lanes or a barrier (256
+// adjacent slots, reduced by shuffles through LDS, held every block up for
+// about 1.5 us).
 constexpr uint32_t kSlots = 16, kSlotStride = 32;      // 64-bit words between slots
 constexpr uint32_t kSlotSet = kSlots * kSlotStride;    // words of a set
 constexpr uint32_t kDtSet = 2 * kSlotSet;              // a dt set: largest a^2, then largest mu
@@ -435,9 +436,10 @@ __device__ __forceinline__ int clamped_cell(double r, double rmin, double cell, 
 // the lane's column of an LDS buffer first; when a lane's column might
 // overflow, the wave writes the buffered rows out together, so that the
 // stores of a row are contiguous (written straight from the walk, they left
-// lines partly written in L2).  Bound by vector instructions now, about 7 per
-// candidate and 10 per entry: 3D 455 -> 339 us at 555,686 particles, 2020 ->
-// 1593 at 2,899,370; 2D 113 -> 90 at 1,020,263, 22 -> 17 at 22,662.
+// lines partly written in L2).  3D 455 -> 339 us at 555,686 particles, 2020 ->
+// 1593 at 2,899,370; 2D 113 -> 90 at 1,020,263, 22 -> 17 at 22,662.  Vector
+// instructions, about 7 per candidate and 10 per entry, take 43 of 93 us in 2D at
+// 1,020,263 particles and 1.86 of 3.15 ms in 3D at 6,595,366.
 //
 // The FP32 reach exceeds list_reach by build_margin (relative, of the square),
 // above the rounding of positions `cells` cells from the wave's reference (half
@@ -942,9 +944,9 @@ __device__ __forceinline__ void for_each_listed(const StepParams& P, const float
 }
 
 // The cubic configuration's pair terms (fast_pair_term) for list entries,
-// 2D and 3D, arranged for instruction count, which bounds the passes (a
-// wave of the 2D FP32 pass issued 1,797 VALU instructions, 47 of its 58 us
-// at 1M particles):
+// 2D and 3D, arranged for instruction count, the largest share of the FP32
+// passes' time (a wave of the 2D pass issues 1,557 VALU instructions, 40 of its
+// 59 us at 1M particles):
 //   * with t = h - |r| / 2 the outer piece is W = f / h^3 (4/3 t^3) and grad W
 //     = diff (-2f / h^3) t^2 / |r|, the inner one with the same scales 2/3 h^3 -
 //     |r|^2 t and t - |r| / 4; one comparison selects both, and the scales are

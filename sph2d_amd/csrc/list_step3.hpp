@@ -19,7 +19,7 @@
 //
 // Step kernels: [density_sum_list3] -> pair_list3_kernel ->
 // integrate_list3_kernel (in place), the first of them with the step's
-// prologue (list_step_begin).  A build step runs list_prologue -> radix sort
+// prologue (list_step_begin).  A build step runs list_prologue -> counting sort
 // -> reorder_list3_kernel -> list_build3_kernel -> the same step kernels on
 // the reordered copy, integrating into A.
 #pragma once
@@ -521,7 +521,8 @@ __device__ __forceinline__ double step_listed3(const StepParams& P, const Ctrl& 
 // the dt maxima and the fields for the integrator.  Entries in rounds of G,
 // the records gathered by each lane in FP32 (6 in flight: 706 us per pass at
 // 2,899,370 particles, summation; 724 at 8, 793 at 4; by the wave, two lanes a
-// record, 807: the pass is bound by instructions there) and by the wave in
+// record, 807: vector instructions take two thirds of the pass's time, 1.04 of
+// 1.53 ms at 6,595,366 particles) and by the wave in
 // FP64 (555,686 particles, summation: 224 us per pass with 4 in flight, 235
 // with 3, 253 with 2; 310 when each lane gathered its own; 943,906 particles,
 // continuity, which gathers the velocity too: 515 with 3, 576 with 2, 633 by

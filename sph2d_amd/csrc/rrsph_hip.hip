@@ -262,8 +262,8 @@ struct rrsph_ctx {
     void* rec = nullptr;                // records of the list pass (ListRec per slot)
     void* dens = nullptr;               // 3D: records of the summation density pass (real4 per slot)
     uint32_t* home = nullptr;           // each slot's cell at the last build
-    unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima, a set per step parity)
-    unsigned long long* dtslots = nullptr; // list steps: dt maxima (likewise)
+    unsigned long long* dslots = nullptr;  // list steps: largest displacement (block maxima; 2 sets by step index, 4 where steps fuse)
+    unsigned long long* dtslots = nullptr; // list steps: dt maxima (2 sets by step index)
     uint32_t* cell_count = nullptr;         // builds with the counting sort: cell counts (zero between builds), scan sums
     float4* cand = nullptr;                 // 3D builds: candidate records (FP32 home-relative position, z cell)
     ListGraphs list_graphs;             // of plain runs
@@ -798,8 +798,8 @@ rrsph_status launch_list_run(rrsph_ctx* ctx, bool build, uint32_t steps) {
             enqueue_list_step(ctx, nullptr, kind);
         }
     };
-    // a taped step is followed by a copy of its state to an address of its
-    // own, and every run sets new piston coefficients, which a graph would hold
+    // a taped step reads and leaves its state at addresses of its own, and every
+    // run sets new piston coefficients, which a graph would hold
     if (!ctx->use_graph || ctx->taping) {
         enqueue();
         return RRSPH_OK;
@@ -1144,8 +1144,11 @@ rrsph_status setup_params(rrsph_ctx* ctx, const rrsph_params_c& p) {
     // of the cut-off: a wider one makes builds rarer and lists longer, and in
     // 3D the lists grow faster.  Per 50 steps of 1,020,263 particles (FP32): 5250
     // us at 0.125, 5050 at 0.15, 5380 at 0.18; below 25,000 particles, where a
-    // pass is bound by latency, per 200 steps of 6,923: 3940 at 0.125, 3870 at
-    // 0.15, 3640 at 0.23, 3620 at 0.26; 3D, per 25 steps of 555,686 (FP64):
+    // pass is bound by latency, 0.23 (a step at 0.15, 0.23 and 0.27, FP64: dam
+    // breaks of 2,213 particles 9.0, 8.9 and 9.0 us, of 6,923 10.1, 9.5 and 9.6, of
+    // 14,813 12.3, 11.5 and 11.1; flumes of 11,842 18.5, 17.2 and 17.0, of 20,400
+    // 20.7, 19.0 and 18.4, of 27,229 20.7, 20.3 and 19.8, of 46,894 23.8, 24.1
+    // and 24.7); 3D, per 25 steps of 555,686 (FP64):
     // 11110 at 0.06, 11100 at 0.08, 11520 at 0.1, 11630 at 0.125
     double skin_frac = d3 ? 0.08 : P.n < 25000 ? 0.23 : 0.15;
     if (const char* e = std::getenv("RRSPH_HIP_LIST_SKIN")) skin_frac = std::strtod(e, nullptr);
@@ -1397,9 +1400,13 @@ rrsph_status rrsph_hip_create(const rrsph_params_c* params, rrsph_ctx** out) {
             ctx->ctrl_alt = dalloc<Ctrl>(1, e);
         }
         ctx->dtslots = dalloc<unsigned long long>(2 * kDtSet, e);
-        // the counting sort's scan passes over every cell of the grid: 12 bytes a
-        // cell, so that 4 cells a particle take what one radix pass does (24 bytes
-        // a particle read twice and written once); sparser grids keep the radix sort
+        // the counting sort's scan passes over every cell of the grid (16 bytes a
+        // cell: read twice, cleared, the start written), which the radix sort does
+        // not; sparser grids keep that one.  Steps that all build, counting and
+        // radix, us: 1,020,263 particles 222 and 250 with 2 cells a particle, 235
+        // and 256 with 4, 266 and 269 with 8, 326 and 306 with 16; 187,530
+        // particles 76 and 112 with 4, 148 and 153 with 64; the line is where
+        // the largest still gains
         if (const char* e2 = std::getenv("RRSPH_HIP_TAPE_LISTS")) ctx->tape_lists_max = std::strtoull(e2, nullptr, 10);
         const char* sort = std::getenv("RRSPH_HIP_BUILD_SORT");
         if ((uint64_t)ctx->P.ncells <= 4ull * n && !(sort && std::strcmp(sort, "radix") == 0)) {
@@ -2623,8 +2630,10 @@ rrsph_status rrsph_hip_set_piston(rrsph_ctx* ctx, double omega, uint32_t nharm, 
 // Whether a tape runs list steps (builds at its checkpoints and by the
 // displacements, the schedule recorded for the replays).
 // In 2D: 60 steps of 134,042 particles forward and back 10.2 -> 8.2 ms, 40 of
-// 18,544 4.1 -> 2.4 and of 5,040, the smallest measured, 4.0 -> 2.2.  Below
-// 4,096 tapes keep to sorted steps, as contexts without lists do.
+// 18,544 4.1 -> 2.4 and of 5,040 4.0 -> 2.2.  The line is not one of speed (40
+// steps of 474 particles would take 1.6 ms instead of 3.5, of 3,649 1.6 instead
+// of 3.7): list tapes are tested from 4,237 particles on, and smaller runs keep
+// the sorted steps that theirs are tested with.
 constexpr uint32_t kTapeListMin2 = 4096;
 static bool tape_lists(const rrsph_ctx* ctx) {
     if (!list_active(ctx)) return false;
