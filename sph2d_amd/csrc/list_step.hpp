@@ -1332,10 +1332,9 @@ __device__ __forceinline__ void kernel_wf(const StepParams& P, int skf, R q, R i
 // pair_kernel on the same FP64 positions.  An entry gathers the neighbour's
 // position, state and pred record; entries in groups of G as in
 // for_each_listed.  Terms whose kernel type is the pressure's share one
-// evaluation, and but for the wall force no term divides: the cell walk over
-// ~55 candidates with a division or more per term took 167 us at 187,530
-// particles (FP64, Wendland kernels, delta-SPH, artificial pressure), the ~20
-// entries of a list 45.  The reciprocal root and 1 / h alone would leave |r| / h
+// evaluation, and no term divides: the cell walk over ~55 candidates with a
+// division or more per term took 167 us at 187,530 particles (FP64, Wendland
+// kernels, delta-SPH, artificial pressure), the ~20 entries of a list 45.  The reciprocal root and 1 / h alone would leave |r| / h
 // with half as much error again (43 us).
 template <class R, bool FIRST, int LPP>
 __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_general_kernel(
@@ -1426,9 +1425,9 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                 }
                 // Lennard-Jones wall force on fluid from boundary particles
                 if (P.lj_on && tj > 0 && ti < 0 && dist < lj_r0) {
-                    const R rn = lj_r0 / dist;  // (few pairs, and its 12th power)
+                    const R r2 = lj_r0 * rinv, rn = fma(fma(-r2, dist, lj_r0), rinv, r2);  // (its 12th power)
                     const R rn2 = rn * rn, rn4 = rn2 * rn2;
-                    const R f = lj_D * (rn4 * rn4 * rn4 - rn4) / d2;
+                    const R f = lj_D * (rn4 * rn4 * rn4 - rn4) * (rinv * rinv);
                     ax -= dx * f;
                     ay -= dy * f;
                 }
