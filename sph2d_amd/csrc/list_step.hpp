@@ -1044,6 +1044,17 @@ __device__ __forceinline__ void list_dt_maxima(const StepParams& P, double a2, R
     if (P.dt_method == 2 && P.dt_dynamic_mode == 1) block_max_to_slots(a2, mu, slots, slots + kSlotSet, lb);
 }
 
+// The summed density of a particle that no longer exists, which has no
+// neighbours: its own term, renormalised by itself (w0 = W(0)).  Its record holds
+// 0 instead, the sign of its type, so that the integrator works it out again.
+template <class R> __device__ __forceinline__ R dead_density(const StepParams& P, R w0, R rho_old, bool renorm) {
+    const R m = (R)P.mass, rho = m * w0;
+    return renorm ? rho / (m / rho_old * w0) : rho;
+}
+template <class R> __device__ __forceinline__ R density_w0(const StepParams& P) {
+    return kernel_w<R>(kernel_consts<R>(P), P.skf_density, R(0));
+}
+
 // Summation density from the lists (Density.h:25-61): rho = m W(0) +
 // sum m W_ij, p = EOS(rho), into the pred records (the forces use this rho)
 // and the pressure array; renormalised on the steps that ask for it
@@ -1108,7 +1119,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list(StepParams P, Ctrl* n
                 if (capped) take = take_capped<LPP>(take, g.l, cap, hits, overflow);
                 const R w = take ? kernel_w<R>(K, P.skf_density, pair_dist<R>(dx, dy, 0.0)) : R(0);
                 rho += m * w;
-                if (renorm) wsum += m / va[u].z * w;
+                if (renorm && take) wsum += m / va[u].z * w;
             }
 #pragma unroll
             for (uint32_t u = 0; u < G; ++u) e[u] = en[u];
@@ -1283,8 +1294,10 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? (FUSED || LPP == 8 ? 
             const real4<R> d{ax, ay, drho, amu};
             const real2<R> x{xx, xy};
             real4<R> pr{};
-            if (!CONT) pr.z = fabs(prj.z);  // the summed density
-            moved2 = step_listed<R>(P, c, s, X.pos[s], X.va[s], pr, 0u, O.home[s], d, x, dt, O, outside, bad);
+            const real4<R> va = X.va[s];
+            if constexpr (!CONT)  // the summed density
+                pr.z = (int)va.w != 0 ? fabs(prj.z) : dead_density<R>(P, density_w0<R>(P), va.z, cur->cur_renorm != 0);
+            moved2 = step_listed<R>(P, c, s, X.pos[s], va, pr, 0u, O.home[s], d, x, dt, O, outside, bad);
         }
         finish_listed(P, O.flags, step, outside, bad, moved2, dslots, lb);
     }
@@ -1568,6 +1581,8 @@ __global__ void __launch_bounds__(kBlock) integrate_list_kernel(StepParams P, Ct
     if (live) {
         const bool reordered = A.oid != X.oid;
         const uint32_t oid = reordered || step_needs_oid(P, c, (int)va.w) ? X.oid[s] : 0u;
+        if (P.density_treatment == 0 && (int)va.w == 0)
+            pr.z = dead_density<R>(P, density_w0<R>(P), va.z, c.cur_renorm != 0);
         moved2 = step_listed<R>(P, c, s, p0, va, pr, oid, h, d, x, dt, ListOut<R>{A.pos, A.va, rec, home, key_next, next, false},
                                 outside, bad);
         if (reordered) A.oid[s] = oid;

@@ -364,6 +364,10 @@ struct ListRowsVector {
     }
 };
 
+template <class R> __device__ __forceinline__ R density_w0_3(const StepParams& P) {
+    return (R)P.f_cubic * (R(2) / R(3));
+}
+
 // Summation density from the lists (Density.h:25-61) with the
 // renormalisation of the steps that ask for it (ModelParams.tex:124-133):
 // rho into rec.pr.w (sign-typed), p / rho^2 into rec.nr.w, p into pres.
@@ -391,7 +395,7 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
     const uint32_t s = live ? s0 : P.n - 1;
     const R m = (R)P.mass, inv_h = (R)(1.0 / P.h), w_q1 = (R)P.f_cubic, w_q2 = (R)(P.f_cubic / 6.0);
     const real4<R> dj = dens[s];
-    const R w0 = w_q1 * (R(2) / R(3));
+    const R w0 = density_w0_3<R>(P);
     R rho = m * w0;
     const bool renorm = step_renorm(P, step);
     R wsum = renorm && dj.w != R(0) ? m / fabs(dj.w) * w0 : R(0);
@@ -442,12 +446,10 @@ __global__ void __launch_bounds__(kBlock) density_sum_list3(StepParams P, Ctrl* 
         });
     }
     if (!live) return;
-    // a particle that died since the build has no sums to renormalise (its
-    // record's density is 0): it keeps the plain sum, so that its records,
-    // which the lists of its former neighbours still name, stay finite
-    if (renorm && wsum > R(0)) rho = rho / wsum;
-    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const int itype = (int)X.pos[s].w;
+    if (itype == 0) rho = dead_density<R>(P, w0, X.va[s].w, renorm);  // (its record's density is 0)
+    else if (renorm) rho = rho / wsum;
+    if (overflow) atomicOr(&next->nbr_overflow, 1u);
     const R p = eos_p<R>(rho, (R)P.rho0, (R)P.eos_B);
     ListRec<R> r = rec[s];
     r.pr.w = typed_rho<R>(rho, itype);
@@ -662,8 +664,10 @@ __global__ void __launch_bounds__(kBlock, 3) pair_list3_kernel(
             c.cur_first = step == 0;
             const real4<R> d{ax, ay, az, drho}, x{mW * S.xx, mW * S.xy, mW * S.xz, amu};
             real4<R> pr{};
-            pr.w = fabs(rj.pr.w);  // the summed density
-            moved2 = step_listed3<R>(P, c, s, X.pos[s], vaj, pr, 0u, O.home[s], d, x, cur->cur_dt_const, O, outside,
+            const double4 p0 = X.pos[s];
+            pr.w = (int)p0.w != 0 ? fabs(rj.pr.w)  // the summed density
+                                  : dead_density<R>(P, density_w0_3<R>(P), vaj.w, cur->cur_renorm != 0);
+            moved2 = step_listed3<R>(P, c, s, p0, vaj, pr, 0u, O.home[s], d, x, cur->cur_dt_const, O, outside,
                                      bad);
         }
         finish_listed(P, O.flags, step, outside, bad, moved2, dslots, lb);
@@ -701,6 +705,8 @@ __global__ void __launch_bounds__(kBlock) integrate_list3_kernel(StepParams P, C
     if (live) {
         const bool reordered = A.oid != X.oid;
         const uint32_t oid = reordered || step_needs_oid(P, c, (int)p0.w) ? X.oid[s] : 0u;
+        if (P.density_treatment == 0 && (int)p0.w == 0)
+            pr.w = dead_density<R>(P, density_w0_3<R>(P), va.w, c.cur_renorm != 0);
         moved2 = step_listed3<R>(P, c, s, p0, va, pr, oid, h, d, x, dt,
                                  ListOut3<R>{A.pos, A.va, rec, dens, home, key_next, next, false}, outside, bad);
         if (reordered) A.oid[s] = oid;
