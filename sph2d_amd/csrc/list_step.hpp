@@ -72,6 +72,10 @@ template <class R> __device__ __forceinline__ R typed_rho(R rho, int itype) {
     return itype > 0 ? rho : (itype < 0 ? -rho : R(0));
 }
 
+// The density back from its record where the type is at hand: a flow that breaks
+// up may predict a negative one, whose sign a fabs would lose.
+template <class R> __device__ __forceinline__ R untyped_rho(R z, int itype) { return itype > 0 ? z : -z; }
+
 // The near record of a particle at pos with velocity (vx, vy) and home cell
 // `home` (a cell key cx ncy + cy).
 template <class R> __device__ __forceinline__ real4<R> near_record(const StepParams& P, double2 pos, R vx, R vy,
@@ -1385,7 +1389,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
     if (tj == 0) cnt = 0;
     if (cnt) {
         const bool cont = P.density_treatment != 0, delta = P.density_treatment == 2;
-        const R rhohj = fabs(prj.z), pjres = prj.w * (rhohj * rhohj);
+        const R rhohj = untyped_rho<R>(prj.z, tj), pjres = prj.w * (rhohj * rhohj);
         const R alpha_c = (R)P.av_alpha * (R)P.av_c, beta = (R)P.av_beta, eta2 = (R)P.av_eta2;
         const R two_eps_m = R(2) * (R)P.xsph_eps * m, lj_r0 = (R)P.lj_r0, lj_D = (R)P.lj_D;
         const R dhc2m = R(2) * (R)P.dhc * m, ap_iw = P.art_pressure ? (R)(1.0 / P.ap_wdelta) : R(0);
@@ -1445,7 +1449,7 @@ __global__ void __launch_bounds__(kBlock, sizeof(R) == 8 ? 3 : 1) pair_list_gene
                     ay -= dy * f;
                 }
                 // pressure: p / rho^2 of both from the pred records
-                const R rhohi = fabs(pr[u].z);
+                const R rhohi = untyped_rho<R>(pr[u].z, ti);
                 R pf = P.intf_approx == 1 ? (pjres + pr[u].w * (rhohi * rhohi)) * fast_rcp<R>(rhohj * rhohi)
                                           : pr[u].w + prj.w;
                 if (P.art_pressure && (pr[u].w < R(0) || prj.w < R(0))) {
